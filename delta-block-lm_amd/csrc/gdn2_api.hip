@@ -541,10 +541,15 @@ size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
         c = chunk_checkpoint_bytes(shape->batch, shape->time, shape->heads);
     else if (wide_eligible_shape(shape, chunk))
         c = wide_checkpoint_bytes(shape->batch, shape->time, shape->heads);
-    const size_t q = seq_checkpoint_bytes(shape);
-    return c > q ? c : q;
+    const size_t f = fc_checkpoint_bytes(shape->batch, shape->time, shape->heads, (int)shape->keys,
+                                         (int)shape->values, true);
+    return std::max(std::max(c, f), seq_checkpoint_bytes(shape));
 }
 
+// The f32 chunk kernels' backward walks windows of chunks that fit whatever
+// workspace it is given, so their share is capped: 64 MiB holds 2048 chunks of
+// 64 x 64, enough to fill the chip, and keeps every shape whose other needs fit
+// the library's fixed scratch within it (gdn_scalar_backward_noalloc).
 size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
     if (check_shape(shape) || check_chunk(chunk)) return 0;
     size_t c = 0;
@@ -552,15 +557,21 @@ size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
         c = chunk_workspace_bytes(shape->batch, shape->time, shape->heads);
     else if (wide_eligible_shape(shape, chunk))
         c = wide_workspace_bytes(shape->batch, shape->time, shape->heads);
-    const size_t q = seq_workspace_bytes(shape);
-    return c > q ? c : q;
+    const size_t f = fc_workspace_bytes(shape->batch, shape->time, shape->heads, (int)shape->keys,
+                                        (int)shape->values);
+    return std::max(std::max(c, std::min(f, (size_t)GDN2_NOALLOC_SCRATCH_BYTES)), seq_workspace_bytes(shape));
 }
 
 // The chunk-WY MFMA kernels take bf16 q/k/v with d_k = d_v = 64 (gdn2_chunk.hip)
 // or 128 (gdn2_chunk_wide.hip), chunk 64, unit channel stride and 16-byte
-// aligned token rows; everything else runs the token-sequential kernels.
-// Forward and backward apply the same rule, so the checkpoint format always
-// matches.
+// aligned token rows.  Everything else runs the f32 scalar-gate chunk kernels
+// (gdn2_chunk_fs.hip) from 17 tokens on, and the token-sequential kernels
+// (gdn2_seq.hip) up to 16: there one workgroup per head walks one chunk's tokens
+// in less time than three launches take (forward at 64 heads of 64 x 64 f32,
+// token-sequential against chunked: 11 and 17 us at T = 8, 13 and 17 at 16, 21
+// and 19 at 32, 62 and 30 at 128; backward 18 and 26, 29 and 25, 49 and 28, 172
+// and 42; at 2048 heads T = 16 takes 58 and 74 forward).  Forward and backward
+// apply the same rule, so the checkpoint format always matches.
 
 static bool use_chunk_path(const gdn2_shape *shape, int chunk, const gdn2_view *q,
                            const gdn2_view *k, const gdn2_view *v) {
@@ -589,6 +600,32 @@ static ChunkArgs chunk_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_
     a.valid = make_view(valid);
     a.reset = make_view(reset);
     return a;
+}
+
+static bool use_seq_path(const gdn2_shape *shape) { return shape->time <= FC_C; }
+
+// The f32 scalar-gate chunk path's argument block.  Its 4-channel reads need
+// unit channel stride, a width of whole fours and rows aligned to four elements.
+static FcArgs fs_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_view *k,
+                      const gdn2_view *v, const gdn2_view *beta, const gdn2_view *g,
+                      const gdn2_view *valid, const gdn2_view *reset, const gdn2_view *dout,
+                      void *checkpoint, void *workspace) {
+    FcArgs f{};
+    f.s = seq_args(s, q, k, v, beta, beta, beta, valid, reset);
+    f.s.beta = make_view(beta);
+    f.s.g = make_view(g);
+    f.s.dout = make_view(dout);
+    f.in_bf16 = q->dtype == GDN2_BF16;
+    f.nc = (f.s.T + FC_C - 1) / FC_C;
+    f.scalar = 1;
+    auto vec = [&](const gdn2_view *x, int64_t w) {
+        return x && x->stride[3] == 1 && w % 4 == 0 && ((uintptr_t)x->data & (f.in_bf16 ? 7 : 15)) == 0 &&
+               x->stride[0] % 4 == 0 && x->stride[1] % 4 == 0 && x->stride[2] % 4 == 0;
+    };
+    f.vec = (vec(q, s->keys) ? 1 : 0) | (vec(k, s->keys) ? 2 : 0) | (vec(v, s->values) ? 4 : 0) |
+            (vec(dout, s->values) ? 8 : 0);
+    fc_bind(f, checkpoint, workspace);
+    return f;
 }
 
 static int check_scalar_inputs(const gdn2_view *q, const gdn2_view *k, const gdn2_view *v,
@@ -635,18 +672,28 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
         chunk_bind_checkpoint(c, checkpoint);
         return launch_status(launch_chunk_fwd(c, (hipStream_t)stream, ev), "gdn_scalar_scan");
     }
-    SeqArgs a = seq_args(shape, q, k, v, beta, beta, beta, valid, reset);
-    a.scalar = 1;
-    a.beta = make_view(beta);
-    a.g = make_view(g);
-    a.initial = make_view(initial);
-    a.out = output;
-    a.out_bf16 = output_dtype == GDN2_BF16;
-    a.final_state = final_state;
-    a.scores = scores;
-    seq_bind_checkpoint(a, checkpoint);
-    return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
-                         "gdn_scalar_scan");
+    if (use_seq_path(shape)) {
+        SeqArgs a = seq_args(shape, q, k, v, beta, beta, beta, valid, reset);
+        a.scalar = 1;
+        a.beta = make_view(beta);
+        a.g = make_view(g);
+        a.initial = make_view(initial);
+        a.out = output;
+        a.out_bf16 = output_dtype == GDN2_BF16;
+        a.final_state = final_state;
+        a.scores = scores;
+        seq_bind_checkpoint(a, checkpoint);
+        return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
+                             "gdn_scalar_scan");
+    }
+    FcArgs f = fs_args(shape, q, k, v, beta, g, valid, reset, nullptr, checkpoint, nullptr);
+    f.s.initial = make_view(initial);
+    f.s.out = output;
+    f.s.out_bf16 = output_dtype == GDN2_BF16;
+    f.s.final_state = final_state;
+    f.s.scores = scores;
+    const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
+    return launch_status(launch_fs_fwd(f, (hipStream_t)stream, ev), "gdn_scalar_scan");
 }
 
 int gdn_scalar_backward(const gdn2_shape *shape, int chunk, const gdn2_view *q,
@@ -739,23 +786,36 @@ static int scalar_backward_impl(const gdn2_shape *shape, int chunk, const gdn2_v
                                   : launch_chunk_bwd(c, (hipStream_t)stream, ev),
                              "gdn_scalar_backward");
     }
-    SeqArgs a = seq_args(shape, q, k, v, beta, beta, beta, valid, reset);
-    a.scalar = 1;
-    a.beta = make_view(beta);
-    a.g = make_view(g);
-    seq_bind_checkpoint(a, checkpoint);
-    if (d_output) a.dout = make_view(d_output);
-    a.dfinal = d_final_state;
-    a.dscores = d_scores;
-    a.dq = dq;
-    a.dk = dk;
-    a.dv = dv;
-    a.dbeta = dbeta;
-    a.dg = dg;
-    a.dinitial = d_initial;
-    a.replay = (float *)workspace;
-    return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
-                         "gdn_scalar_backward");
+    if (use_seq_path(shape)) {
+        SeqArgs a = seq_args(shape, q, k, v, beta, beta, beta, valid, reset);
+        a.scalar = 1;
+        a.beta = make_view(beta);
+        a.g = make_view(g);
+        seq_bind_checkpoint(a, checkpoint);
+        if (d_output) a.dout = make_view(d_output);
+        a.dfinal = d_final_state;
+        a.dscores = d_scores;
+        a.dq = dq;
+        a.dk = dk;
+        a.dv = dv;
+        a.dbeta = dbeta;
+        a.dg = dg;
+        a.dinitial = d_initial;
+        a.replay = (float *)workspace;
+        return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
+                             "gdn_scalar_backward");
+    }
+    FcArgs f = fs_args(shape, q, k, v, beta, g, valid, reset, d_output, const_cast<void *>(checkpoint), workspace);
+    f.s.dfinal = d_final_state;
+    f.s.dscores = d_scores;
+    f.s.dq = dq;
+    f.s.dk = dk;
+    f.s.dv = dv;
+    f.s.dbeta = dbeta;
+    f.s.dg = dg;
+    f.s.dinitial = d_initial;
+    const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
+    return launch_status(launch_fs_bwd(f, workspace_bytes, (hipStream_t)stream, ev), "gdn_scalar_backward");
 }
 
 extern "C" {

@@ -5,6 +5,10 @@
 
 namespace gdn2 {
 
+// Four floats of a checkpoint or workspace array: the scalar-gate entry points
+// take buffers of any alignment (16-byte accesses to global memory need four).
+typedef float fc_u4 __attribute__((ext_vector_type(4), aligned(4)));
+
 constexpr int FC_C = 16;    // tokens per chunk
 constexpr int FC_MAX = 128;  // largest d_k and d_v
 
@@ -37,6 +41,10 @@ struct FcArgs {
     int in_bf16;  // q, k, v, dO and dq, dk, dv are bf16 (else f32)
     float *st, *tm, *dl, *fw, *fk, *fu, *gv;
     float *ds, *n;
+    int w0, wn;
+    float *carry;
+    int scalar;  // the scalar-gate path's layout
+    int vec;     // its 4-channel reads: bit 0 q, 1 k, 2 v, 3 dO
 };
 
 inline int64_t fc_chunks(int64_t B, int64_t T, int64_t H) { return B * H * ((T + FC_C - 1) / FC_C); }
@@ -44,20 +52,20 @@ __host__ __device__ inline int fc_kp(int K) { return (K + 15) & ~15; }
 inline size_t fc_pad4(size_t x) { return (x + 3) & ~(size_t)3; }
 
 // The checkpoint's arrays in order, in floats, for n chunks.
-inline void fc_checkpoint_parts(int64_t n, int K, int V, size_t part[7]) {
+inline void fc_checkpoint_parts(int64_t n, int K, int V, size_t part[7], bool scalar = false) {
     const size_t KP = fc_kp(K), VP = fc_kp(V);
     part[0] = n * KP * VP;              // st
     part[1] = fc_pad4(n * FC_C * FC_C); // tm
-    part[2] = fc_pad4(n * FC_C * V);    // dl
+    part[2] = scalar ? 0 : fc_pad4(n * FC_C * V);  // dl
     part[3] = n * FC_C * KP;            // fw
     part[4] = n * FC_C * KP;            // fk
     part[5] = n * FC_C * VP;            // fu
     part[6] = n * KP;                   // gv
 }
 
-inline size_t fc_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V) {
+inline size_t fc_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V, bool scalar = false) {
     size_t part[7], total = 0;
-    fc_checkpoint_parts(fc_chunks(B, T, H), K, V, part);
+    fc_checkpoint_parts(fc_chunks(B, T, H), K, V, part, scalar);
     for (size_t x : part) total += x;
     return total * sizeof(float);
 }
@@ -70,20 +78,30 @@ inline size_t fc_workspace_bytes(int64_t B, int64_t T, int64_t H, int K, int V) 
 inline void fc_bind(FcArgs &a, void *ck, void *ws) {
     const int64_t n = fc_chunks(a.s.B, a.s.T, a.s.H);
     size_t part[7];
-    fc_checkpoint_parts(n, a.s.K, a.s.V, part);
+    fc_checkpoint_parts(n, a.s.K, a.s.V, part, a.scalar != 0);
     float *p = static_cast<float *>(ck);
     float **dst[7] = {&a.st, &a.tm, &a.dl, &a.fw, &a.fk, &a.fu, &a.gv};
     for (int i = 0; i < 7; ++i) {
         *dst[i] = p;
         p += part[i];
     }
+    a.w0 = 0;
+    a.wn = a.nc;
     if (ws) {
         a.ds = static_cast<float *>(ws);
         a.n = a.ds + n * fc_kp(a.s.K) * fc_kp(a.s.V);
     }
 }
 
+// The state scan over the chunks (the adjoint scan over the window when rev).
+void launch_fc_scan(const FcArgs &a, bool rev, hipStream_t stream);
+
 hipError_t launch_fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
 hipError_t launch_fc_bwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
+// Scalar gates.  The backward takes any workspace of at least one chunk window
+// and the carry (fs_min_workspace_bytes); the whole of fc_workspace_bytes is one
+// window.
+hipError_t launch_fs_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
+hipError_t launch_fs_bwd(const FcArgs &a, size_t ws_bytes, hipStream_t stream, const hipEvent_t *ev);
 
 }  // namespace gdn2

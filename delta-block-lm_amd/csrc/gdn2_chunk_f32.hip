@@ -413,12 +413,12 @@ __global__ void __launch_bounds__(Fc<FK>::NT) fc_prep_kernel(FcArgs a) {
 // read from global memory into registers D chunks ahead.
 template <int KT>
 struct FcScanOps {
-    float4 w, g, a;  // A operands (token n, keys 16 tau + 4 g ..), gv rows, U or N rows
+    fc_u4 w, g, a;   // A operands (token n, keys 16 tau + 4 g ..), gv rows, U or N rows
     float k[4];      // A operands (tokens 4 g + s, key 16 tau + n)
 };
 
 template <int KT, bool REV>
-__device__ __forceinline__ void fc_scan_load(const FcArgs &a, int64_t ci, int cg, int VT, int tau,
+__device__ __forceinline__ void fc_scan_load(const FcArgs &a, int64_t ci, int64_t wi, int cg, int VT, int tau,
                                              FcScanOps<KT> &o) {
     // Every load is issued (past the value tiles the lanes read tile 0, their
     // values unused), so no load sits behind a branch and the compiler's
@@ -427,59 +427,75 @@ __device__ __forceinline__ void fc_scan_load(const FcArgs &a, int64_t ci, int cg
     const int l = lane_id(), g = l >> 4, n = l & 15, cc = cg < VT ? cg : 0;
     const float *fw = a.fw + ci * C * KP, *fk = a.fk + ci * C * KP;
     const float *rw = REV ? fk : fw, *ck = REV ? fw : fk;
-    o.w = *reinterpret_cast<const float4 *>(&rw[n * KP + 16 * tau + 4 * g]);
-    o.g = *reinterpret_cast<const float4 *>(&a.gv[ci * KP + 16 * tau + 4 * g]);
+    o.w = *reinterpret_cast<const fc_u4 *>(&rw[n * KP + 16 * tau + 4 * g]);
+    o.g = *reinterpret_cast<const fc_u4 *>(&a.gv[ci * KP + 16 * tau + 4 * g]);
 #pragma unroll
     for (int s = 0; s < 4; ++s) o.k[s] = ck[(4 * g + s) * KP + 16 * tau + n];
-    o.a = REV ? *reinterpret_cast<const float4 *>(&a.n[(((ci * VT + cc) * KT + tau) * 64 + l) * 4])
-              : *reinterpret_cast<const float4 *>(&a.fu[((ci * VT + cc) * 64 + l) * 4]);
+    o.a = REV ? *reinterpret_cast<const fc_u4 *>(&a.n[(((wi * VT + cc) * KT + tau) * 64 + l) * 4])
+              : *reinterpret_cast<const fc_u4 *>(&a.fu[((ci * VT + cc) * 64 + l) * 4]);
 }
 
-template <int KT, bool REV>
+// DELTA (scalar gates, forward): v is the chunk's edits delta; wave 0 leaves it
+// where U was, in U's layout.  The workgroups of one (batch, head) read the same
+// factors, so they take block indices of one residue mod 8 and share an XCD's L2.
+template <int KT, bool REV, bool DELTA>
 __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
     __shared__ float4 vpart[2][KT][64];  // each wave's part of v, by step parity
     const SeqArgs &s = a.s;
     const int K = s.K, V = s.V, VT = (V + 15) / 16;
     const int tau = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wg = blockIdx.x, bh = wg / VT, cg = wg % VT, b = bh / s.H, h = bh % s.H;
+    const int wg = blockIdx.x, cg = (wg >> 3) % VT, bh = (wg & 7) + 8 * (wg / (8 * VT));
+    if (bh >= s.B * s.H) return;
+    const int b = bh / s.H, h = bh % s.H;
     const int l = lane_id(), g = l >> 4, n = l & 15, j = 16 * cg + n;
     const bool jv = j < V;
+    const int steps = REV ? a.wn : a.nc;
+    const int64_t co = (((int64_t)bh * VT + cg) * KT + tau) * 64 + l;  // this lane's piece of the carry
     f32x4 X;
+    if (REV && a.w0 + a.wn < a.nc) {
+        const fc_u4 x = *reinterpret_cast<const fc_u4 *>(&a.carry[co * 4]);
+        X = f32x4{x.x, x.y, x.z, x.w};
+    } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int i = 16 * tau + 4 * g + r;
-        float x = 0.f;
-        if (i < K && jv) {
-            if (!REV) x = s.initial.data ? ld4<float>(s.initial, b, h, i, j) : 0.f;
-            else x = s.dfinal ? s.dfinal[((int64_t)bh * K + i) * V + j] : 0.f;
+        for (int r = 0; r < 4; ++r) {
+            const int i = 16 * tau + 4 * g + r;
+            float x = 0.f;
+            if (i < K && jv) {
+                if (!REV) x = s.initial.data ? ld4<float>(s.initial, b, h, i, j) : 0.f;
+                else x = s.dfinal ? s.dfinal[((int64_t)bh * K + i) * V + j] : 0.f;
+            }
+            X[r] = x;
         }
-        X[r] = x;
     }
     // A ring of D chunks' operands in registers: chunk step + D is loaded (the
     // last chunk again past the end) as soon as step's operands are used.
     constexpr int D = 4;
     FcScanOps<KT> ring[D];
-    auto chunk_at = [&](int step) {
-        const int sc = step < a.nc ? step : a.nc - 1;
-        return (int64_t)bh * a.nc + (REV ? a.nc - 1 - sc : sc);
+    auto chunk_at = [&](int step) {  // within the window (forward: all chunks)
+        const int sc = step < steps ? step : steps - 1;
+        return REV ? steps - 1 - sc : sc;
+    };
+    auto load = [&](int step, FcScanOps<KT> &o) {
+        const int cw = chunk_at(step);
+        fc_scan_load<KT, REV>(a, (int64_t)bh * a.nc + (REV ? a.w0 : 0) + cw, (int64_t)bh * a.wn + cw, cg, VT, tau, o);
     };
 #pragma unroll
-    for (int d = 0; d < D; ++d) fc_scan_load<KT, REV>(a, chunk_at(d), cg, VT, tau, ring[d]);
+    for (int d = 0; d < D; ++d) load(d, ring[d]);
     float *keep = REV ? a.ds : a.st;
-    for (int s0 = 0; s0 < a.nc; s0 += D) {
+    for (int s0 = 0; s0 < steps; s0 += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             const int step = s0 + d;
-            if (step >= a.nc) break;
-            const int64_t ci = chunk_at(step);
+            if (step >= steps) break;
+            const int64_t ci = (int64_t)bh * (REV ? a.wn : a.nc) + chunk_at(step);
             const FcScanOps<KT> &cur = ring[d];
             // the state before (forward) / the adjoint after (reverse) this chunk
             {
                 float kx[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) kx[r] = (16 * tau + 4 * g + r < K && jv) ? X[r] : 0.f;
-                *reinterpret_cast<float4 *>(&keep[(((ci * VT + cg) * KT + tau) * 64 + l) * 4]) =
-                    make_float4(kx[0], kx[1], kx[2], kx[3]);
+                *reinterpret_cast<fc_u4 *>(&keep[(((ci * VT + cg) * KT + tau) * 64 + l) * 4]) =
+                    fc_u4{kx[0], kx[1], kx[2], kx[3]};
             }
             // this tile's part of v[t][j], t = 4 g + r: -W' S (+ U in tile 0) or Ktil X
             f32x4 vp = (!REV && tau == 0) ? f32x4{cur.a.x, cur.a.y, cur.a.z, cur.a.w} : zero4();
@@ -500,6 +516,8 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
                     v += f32x4{t.x, t.y, t.z, t.w};
                 }
             }
+            if (DELTA && tau == 0)
+                *reinterpret_cast<fc_u4 *>(&a.fu[((ci * VT + cg) * 64 + l) * 4]) = fc_u4{v[0], v[1], v[2], v[3]};
             // S <- diag(gv) S + Ktil^T v, or X <- diag(gv) X + N - W'^T v
             const float gq[4] = {cur.g.x, cur.g.y, cur.g.z, cur.g.w};
             const float an[4] = {cur.a.x, cur.a.y, cur.a.z, cur.a.w};
@@ -510,8 +528,12 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
             for (int q = 0; q < 4; ++q)
                 x = __builtin_amdgcn_mfma_f32_16x16x4f32(REV ? -cur.k[q] : cur.k[q], v[q], x, 0, 0, 0);
             X = x;
-            fc_scan_load<KT, REV>(a, chunk_at(step + D), cg, VT, tau, ring[d]);
+            load(step + D, ring[d]);
         }
+    }
+    if (REV && a.w0 > 0) {
+        *reinterpret_cast<fc_u4 *>(&a.carry[co * 4]) = fc_u4{X[0], X[1], X[2], X[3]};
+        return;
     }
     float *fin = REV ? s.dinitial : s.final_state;
     if (fin)
@@ -522,19 +544,25 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
         }
 }
 
-template <bool REV>
-static void launch_fc_scan(const FcArgs &a, hipStream_t stream) {
-    const int KT = fc_kp(a.s.K) / 16;
-    const dim3 grid(a.s.B * a.s.H * ((a.s.V + 15) / 16)), block(64 * KT);
-    switch (KT) {
-        case 1: hipLaunchKernelGGL((fc_scan_kernel<1, REV>), grid, block, 0, stream, a); break;
-        case 2: hipLaunchKernelGGL((fc_scan_kernel<2, REV>), grid, block, 0, stream, a); break;
-        case 3: hipLaunchKernelGGL((fc_scan_kernel<3, REV>), grid, block, 0, stream, a); break;
-        case 4: hipLaunchKernelGGL((fc_scan_kernel<4, REV>), grid, block, 0, stream, a); break;
-        case 5: hipLaunchKernelGGL((fc_scan_kernel<5, REV>), grid, block, 0, stream, a); break;
-        case 6: hipLaunchKernelGGL((fc_scan_kernel<6, REV>), grid, block, 0, stream, a); break;
-        case 7: hipLaunchKernelGGL((fc_scan_kernel<7, REV>), grid, block, 0, stream, a); break;
-        default: hipLaunchKernelGGL((fc_scan_kernel<8, REV>), grid, block, 0, stream, a); break;
+template <int KT>
+static void launch_fc_scan_kt(const FcArgs &a, bool rev, hipStream_t stream) {
+    const int bh = a.s.B * a.s.H, VT = (a.s.V + 15) / 16;
+    const dim3 grid(8 * VT * ((bh + 7) / 8)), block(64 * KT);
+    if (rev) hipLaunchKernelGGL((fc_scan_kernel<KT, true, false>), grid, block, 0, stream, a);
+    else if (a.scalar) hipLaunchKernelGGL((fc_scan_kernel<KT, false, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((fc_scan_kernel<KT, false, false>), grid, block, 0, stream, a);
+}
+
+void launch_fc_scan(const FcArgs &a, bool rev, hipStream_t stream) {
+    switch (fc_kp(a.s.K) / 16) {
+        case 1: launch_fc_scan_kt<1>(a, rev, stream); break;
+        case 2: launch_fc_scan_kt<2>(a, rev, stream); break;
+        case 3: launch_fc_scan_kt<3>(a, rev, stream); break;
+        case 4: launch_fc_scan_kt<4>(a, rev, stream); break;
+        case 5: launch_fc_scan_kt<5>(a, rev, stream); break;
+        case 6: launch_fc_scan_kt<6>(a, rev, stream); break;
+        case 7: launch_fc_scan_kt<7>(a, rev, stream); break;
+        default: launch_fc_scan_kt<8>(a, rev, stream); break;
     }
 }
 
@@ -1009,7 +1037,7 @@ static void fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev) {
     hipLaunchKernelGGL(fc_prep_kernel<FK>, dim3(n), dim3(Fc<FK>::NT), 0, stream, a);
     fmark(ev, 1, stream);
     fmark(ev, 2, stream);
-    launch_fc_scan<false>(a, stream);
+    launch_fc_scan(a, false, stream);
     fmark(ev, 3, stream);
     fmark(ev, 4, stream);
     bool narrow = false;
@@ -1028,7 +1056,7 @@ static void fc_bwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev) {
     hipLaunchKernelGGL(fc_bprep_kernel<FK>, dim3(n), dim3(Fc<FK>::NT), 0, stream, a);
     fmark(ev, 1, stream);
     fmark(ev, 2, stream);
-    launch_fc_scan<true>(a, stream);
+    launch_fc_scan(a, true, stream);
     fmark(ev, 3, stream);
     fmark(ev, 4, stream);
     bool narrow = false;

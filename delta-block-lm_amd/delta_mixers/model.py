@@ -15,7 +15,7 @@ The convolution and every norm are the library's HIP operators (float32, as the
 reference's); projections and the MLP are GEMMs in `compute_dtype` (bfloat16 by
 default, float32 master weights).  In bfloat16, q/k/v enter the scan as bf16 and
 take the chunk-WY MFMA path (d_k = d_v = 64, chunk 64); in float32 the scan runs
-the token-sequential kernels.
+the f32 scalar-gate chunk kernels.
 
 With `fused` (the default for bfloat16) each block is one autograd node whose
 backward is written out: the GEMMs stay torch (hipBLASLt) calls and everything
