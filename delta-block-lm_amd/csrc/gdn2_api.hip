@@ -216,76 +216,47 @@ static bool rows_aligned(const gdn2_view *v) {
            v->stride[1] % 8 == 0 && v->stride[2] % 8 == 0;
 }
 
-// The channel-wise op runs the 16-token chunk-WY MFMA kernels
-// (gdn2_chunk_cw.hip) for bf16 q/k/v with d_k = d_v = 64 and aligned rows,
-// whatever the chunk argument (the chunking changes no result).  Forward and backward apply the
-// same rule, so the checkpoint format always matches.
-static bool use_cw_path(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *k,
+// The channel-wise ops run the f32 chunk kernels (gdn2_chunk_f32.hip) whatever
+// the dtype, the width (d_k, d_v <= 128), the strides and the chunk argument:
+// bf16 inputs are read as their exact f32 values and dq, dk, dv written as bf16.
+// Calls with bf16 q/k/v of d_k = d_v = 64 and aligned rows keep two terms of
+// their contract (include/gdn2.h): alpha >= 0, and aligned d_output rows.
+static bool bf16_rows64(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *k,
                         const gdn2_view *v) {
-    return cw_eligible_shape(shape) && q->dtype == GDN2_BF16 && rows_aligned(q) &&
+    return shape->keys == 64 && shape->values == 64 && q->dtype == GDN2_BF16 && rows_aligned(q) &&
            rows_aligned(k) && rows_aligned(v);
 }
 
-// Otherwise f32 or bf16 q/k/v of any width (d_k, d_v <= 128) run the f32 chunk
-// kernels (gdn2_chunk_f32.hip; any element strides; bf16 inputs are read as
-// their exact f32 values and the gradients written back as bf16), again
-// whatever the chunk argument.
-static bool use_fc_path(const gdn2_shape *shape, const gdn2_view *q) {
-    return fc_eligible_shape(shape) && (q->dtype == GDN2_F32 || q->dtype == GDN2_BF16);
+static int check_rows64_adjoint(bool rows64, const gdn2_view *d_output) {
+    if (rows64 && d_output && d_output->data && !rows_aligned(d_output))
+        return fail(GDN2_ERR_ARGUMENT,
+                    "d_output needs unit channel stride and 16-byte aligned rows on the "
+                    "chunked path (bf16, d_k = d_v = 64)");
+    return GDN2_OK;
 }
 
-// The checkpoint and workspace sizes do not depend on the dtype: each is the
-// largest that any kernel family eligible for the shape needs.
 static size_t training_checkpoint_bytes(const gdn2_shape *s) {
-    const size_t c = cw_eligible_shape(s) ? cw_checkpoint_bytes(s->batch, s->time, s->heads) : 0;
-    const size_t f = fc_eligible_shape(s) ? fc_checkpoint_bytes(s->batch, s->time, s->heads,
-                                                                (int)s->keys, (int)s->values)
-                                          : 0;
-    const size_t q = seq_checkpoint_bytes(s);
-    return std::max(c, std::max(f, q));
+    return fc_checkpoint_bytes(s->batch, s->time, s->heads, (int)s->keys, (int)s->values, false);
 }
 
 static size_t training_workspace_bytes(const gdn2_shape *s) {
-    const size_t c = cw_eligible_shape(s) ? cw_workspace_bytes(s->batch, s->time, s->heads) : 0;
-    const size_t f = fc_eligible_shape(s) ? fc_workspace_bytes(s->batch, s->time, s->heads,
-                                                               (int)s->keys, (int)s->values)
-                                          : 0;
-    const size_t q = seq_workspace_bytes(s);
-    return std::max(c, std::max(f, q));
+    return fc_workspace_bytes(s->batch, s->time, s->heads, (int)s->keys, (int)s->values);
 }
 
 // The f32 chunk path's argument block over the token-sequential one.
-static FcArgs fc_args(const SeqArgs &s, const gdn2_view *q, void *checkpoint, void *workspace) {
+static FcArgs fc_args(const SeqArgs &s, const gdn2_view *q, bool rows64, void *checkpoint, void *workspace) {
     FcArgs f{};
     f.s = s;
     f.in_bf16 = q->dtype == GDN2_BF16;
+    f.scalar = s.scalar;
+    f.nonneg = rows64;
     f.nc = (s.T + FC_C - 1) / FC_C;
+    const int es = f.in_bf16 ? 2 : 4;
+    f.vec = fc_vec_view(s.q, es, s.K) && fc_vec_view(s.k, es, s.K) && fc_vec_view(s.v, es, s.V) &&
+            (!s.dout.data || fc_vec_view(s.dout, es, s.V)) && (int64_t)s.H * std::max(s.K, s.V) < (1 << 24) &&
+            (s.scalar || (fc_vec_view(s.alpha, 4, s.K) && fc_vec_view(s.erase, 4, s.K) && fc_vec_view(s.write, 4, s.V)));
     fc_bind(f, checkpoint, workspace);
     return f;
-}
-
-static ChunkArgs cw_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_view *k,
-                         const gdn2_view *v, const gdn2_view *alpha, const gdn2_view *erase,
-                         const gdn2_view *write, const gdn2_view *valid, const gdn2_view *reset) {
-    ChunkArgs a{};
-    a.B = (int)s->batch;
-    a.T = (int)s->time;
-    a.H = (int)s->heads;
-    a.nc = (a.T + CW_C - 1) / CW_C;
-    a.q = (const uint16_t *)q->data;
-    a.k = (const uint16_t *)k->data;
-    a.v = (const uint16_t *)v->data;
-    for (int d = 0; d < 3; ++d) {
-        a.qs[d] = q->stride[d];
-        a.ks[d] = k->stride[d];
-        a.vs[d] = v->stride[d];
-    }
-    a.alpha = make_view(alpha);
-    a.erase = make_view(erase);
-    a.write = make_view(write);
-    a.valid = make_view(valid);
-    a.reset = make_view(reset);
-    return a;
 }
 
 extern "C" {
@@ -296,7 +267,7 @@ const char *gdn2_last_error(void) { return gdn2::last_error(); }
 
 size_t gdn2_training_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
     if (check_shape(shape) || check_chunk(chunk)) return 0;
-    return training_checkpoint_bytes(shape);  // large enough for either kernel family
+    return training_checkpoint_bytes(shape);
 }
 
 size_t gdn2_training_workspace_bytes(const gdn2_shape *shape, int chunk) {
@@ -322,31 +293,15 @@ int gdn2_training_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q,
     if (checkpoint_bytes < training_checkpoint_bytes(shape))
         return fail(GDN2_ERR_WORKSPACE, "checkpoint needs %zu bytes, got %zu",
                     training_checkpoint_bytes(shape), checkpoint_bytes);
-    if (use_cw_path(shape, q, k, v)) {
-        ChunkArgs c = cw_args(shape, q, k, v, alpha, erase, write, valid, reset);
-        c.initial = make_view(initial);
-        c.out = output;
-        c.out_bf16 = output_dtype == GDN2_BF16;
-        c.final_state = final_state;
-        c.scores = scores;
-        cw_bind_checkpoint(c, checkpoint);
-        const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
-        return launch_status(launch_cw_fwd(c, (hipStream_t)stream, ev), "gdn2_training_scan");
-    }
     SeqArgs a = seq_args(shape, q, k, v, alpha, erase, write, valid, reset);
     a.initial = make_view(initial);
     a.out = output;
     a.out_bf16 = output_dtype == GDN2_BF16;
     a.final_state = final_state;
     a.scores = scores;
-    if (use_fc_path(shape, q)) {
-        const FcArgs f = fc_args(a, q, checkpoint, nullptr);
-        const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
-        return launch_status(launch_fc_fwd(f, (hipStream_t)stream, ev), "gdn2_training_scan");
-    }
-    seq_bind_checkpoint(a, checkpoint);
-    return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
-                         "gdn2_training_scan");
+    const FcArgs f = fc_args(a, q, bf16_rows64(shape, q, k, v), checkpoint, nullptr);
+    const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
+    return launch_status(launch_fc_fwd(f, (hipStream_t)stream, ev), "gdn2_training_scan");
 }
 
 int gdn2_training_backward(const gdn2_shape *shape, int chunk, const gdn2_view *q,
@@ -372,30 +327,8 @@ int gdn2_training_backward(const gdn2_shape *shape, int chunk, const gdn2_view *
     if (workspace_bytes < training_workspace_bytes(shape))
         return fail(GDN2_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu",
                     training_workspace_bytes(shape), workspace_bytes);
-    if (use_cw_path(shape, q, k, v)) {
-        if (d_output && d_output->data && !rows_aligned(d_output))
-            return fail(GDN2_ERR_ARGUMENT,
-                        "d_output needs unit channel stride and 16-byte aligned rows on the "
-                        "chunked path (bf16, d_k = d_v = 64)");
-        ChunkArgs c = cw_args(shape, q, k, v, alpha, erase, write, valid, reset);
-        cw_bind_checkpoint(c, const_cast<void *>(checkpoint));
-        cw_bind_workspace(c, workspace);
-        if (d_output && d_output->data) {
-            c.dout = (const uint16_t *)d_output->data;
-            for (int d = 0; d < 3; ++d) c.ds[d] = d_output->stride[d];
-        }
-        c.dfinal = d_final_state;
-        c.dscores = d_scores;
-        c.dq = dq;
-        c.dk = dk;
-        c.dv = dv;
-        c.dalpha = dalpha;
-        c.derase = derase;
-        c.dwrite = dwrite;
-        c.dinitial = d_initial;
-        const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
-        return launch_status(launch_cw_bwd(c, (hipStream_t)stream, ev), "gdn2_training_backward");
-    }
+    const bool rows64 = bf16_rows64(shape, q, k, v);
+    GDN2_TRY(check_rows64_adjoint(rows64, d_output));
     SeqArgs a = seq_args(shape, q, k, v, alpha, erase, write, valid, reset);
     if (d_output) a.dout = make_view(d_output);
     a.dfinal = d_final_state;
@@ -407,15 +340,9 @@ int gdn2_training_backward(const gdn2_shape *shape, int chunk, const gdn2_view *
     a.derase = derase;
     a.dwrite = dwrite;
     a.dinitial = d_initial;
-    if (use_fc_path(shape, q)) {
-        const FcArgs f = fc_args(a, q, const_cast<void *>(checkpoint), workspace);
-        const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
-        return launch_status(launch_fc_bwd(f, (hipStream_t)stream, ev), "gdn2_training_backward");
-    }
-    seq_bind_checkpoint(a, checkpoint);
-    a.replay = (float *)workspace;
-    return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
-                         "gdn2_training_backward");
+    const FcArgs f = fc_args(a, q, rows64, const_cast<void *>(checkpoint), workspace);
+    const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
+    return launch_status(launch_fc_bwd(f, (hipStream_t)stream, ev), "gdn2_training_backward");
 }
 
 size_t gdn2_scan_checkpoint_bytes(const gdn2_shape *shape) {
@@ -441,31 +368,15 @@ int gdn2_scan(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *k, c
     if (checkpoint_bytes < training_checkpoint_bytes(shape))
         return fail(GDN2_ERR_WORKSPACE, "checkpoint needs %zu bytes, got %zu",
                     training_checkpoint_bytes(shape), checkpoint_bytes);
-    if (use_cw_path(shape, q, k, v)) {
-        ChunkArgs c = cw_args(shape, q, k, v, alpha, erase, write, nullptr, nullptr);
-        c.doc = 1;
-        c.doc_start = make_view(doc_start);
-        c.doc_end = make_view(doc_end);
-        c.out = output;
-        c.out_bf16 = output_dtype == GDN2_BF16;
-        cw_bind_checkpoint(c, checkpoint);
-        const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
-        return launch_status(launch_cw_fwd(c, (hipStream_t)stream, ev), "gdn2_scan");
-    }
     SeqArgs a = seq_args(shape, q, k, v, alpha, erase, write, nullptr, nullptr);
     a.doc = 1;
     a.doc_start = make_view(doc_start);
     a.doc_end = make_view(doc_end);
     a.out = output;
     a.out_bf16 = output_dtype == GDN2_BF16;
-    if (use_fc_path(shape, q)) {
-        const FcArgs f = fc_args(a, q, checkpoint, nullptr);
-        const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
-        return launch_status(launch_fc_fwd(f, (hipStream_t)stream, ev), "gdn2_scan");
-    }
-    seq_bind_checkpoint(a, checkpoint);
-    return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
-                         "gdn2_scan");
+    const FcArgs f = fc_args(a, q, bf16_rows64(shape, q, k, v), checkpoint, nullptr);
+    const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
+    return launch_status(launch_fc_fwd(f, (hipStream_t)stream, ev), "gdn2_scan");
 }
 
 int gdn2_backward(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *k,
@@ -487,30 +398,8 @@ int gdn2_backward(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *
     if (workspace_bytes < training_workspace_bytes(shape))
         return fail(GDN2_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu",
                     training_workspace_bytes(shape), workspace_bytes);
-    if (use_cw_path(shape, q, k, v)) {
-        if (d_output && d_output->data && !rows_aligned(d_output))
-            return fail(GDN2_ERR_ARGUMENT,
-                        "d_output needs unit channel stride and 16-byte aligned rows on the "
-                        "chunked path (bf16, d_k = d_v = 64)");
-        ChunkArgs c = cw_args(shape, q, k, v, alpha, erase, write, nullptr, nullptr);
-        c.doc = 1;
-        c.doc_start = make_view(doc_start);
-        c.doc_end = make_view(doc_end);
-        cw_bind_checkpoint(c, const_cast<void *>(checkpoint));
-        cw_bind_workspace(c, workspace);
-        if (d_output && d_output->data) {
-            c.dout = (const uint16_t *)d_output->data;
-            for (int d = 0; d < 3; ++d) c.ds[d] = d_output->stride[d];
-        }
-        c.dq = dq;
-        c.dk = dk;
-        c.dv = dv;
-        c.dalpha = dalpha;
-        c.derase = derase;
-        c.dwrite = dwrite;
-        const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
-        return launch_status(launch_cw_bwd(c, (hipStream_t)stream, ev), "gdn2_backward");
-    }
+    const bool rows64 = bf16_rows64(shape, q, k, v);
+    GDN2_TRY(check_rows64_adjoint(rows64, d_output));
     SeqArgs a = seq_args(shape, q, k, v, alpha, erase, write, nullptr, nullptr);
     a.doc = 1;
     a.doc_start = make_view(doc_start);
@@ -522,15 +411,9 @@ int gdn2_backward(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *
     a.dalpha = dalpha;
     a.derase = derase;
     a.dwrite = dwrite;
-    if (use_fc_path(shape, q)) {
-        const FcArgs f = fc_args(a, q, const_cast<void *>(checkpoint), workspace);
-        const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
-        return launch_status(launch_fc_bwd(f, (hipStream_t)stream, ev), "gdn2_backward");
-    }
-    seq_bind_checkpoint(a, checkpoint);
-    a.replay = (float *)workspace;
-    return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
-                         "gdn2_backward");
+    const FcArgs f = fc_args(a, q, rows64, const_cast<void *>(checkpoint), workspace);
+    const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
+    return launch_status(launch_fc_bwd(f, (hipStream_t)stream, ev), "gdn2_backward");
 }
 
 size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
@@ -604,28 +487,15 @@ static ChunkArgs chunk_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_
 
 static bool use_seq_path(const gdn2_shape *shape) { return shape->time <= FC_C; }
 
-// The f32 scalar-gate chunk path's argument block.  Its 4-channel reads need
-// unit channel stride, a width of whole fours and rows aligned to four elements.
-static FcArgs fs_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_view *k,
-                      const gdn2_view *v, const gdn2_view *beta, const gdn2_view *g,
-                      const gdn2_view *valid, const gdn2_view *reset, const gdn2_view *dout,
-                      void *checkpoint, void *workspace) {
-    FcArgs f{};
-    f.s = seq_args(s, q, k, v, beta, beta, beta, valid, reset);
-    f.s.beta = make_view(beta);
-    f.s.g = make_view(g);
-    f.s.dout = make_view(dout);
-    f.in_bf16 = q->dtype == GDN2_BF16;
-    f.nc = (f.s.T + FC_C - 1) / FC_C;
-    f.scalar = 1;
-    auto vec = [&](const gdn2_view *x, int64_t w) {
-        return x && x->stride[3] == 1 && w % 4 == 0 && ((uintptr_t)x->data & (f.in_bf16 ? 7 : 15)) == 0 &&
-               x->stride[0] % 4 == 0 && x->stride[1] % 4 == 0 && x->stride[2] % 4 == 0;
-    };
-    f.vec = (vec(q, s->keys) ? 1 : 0) | (vec(k, s->keys) ? 2 : 0) | (vec(v, s->values) ? 4 : 0) |
-            (vec(dout, s->values) ? 8 : 0);
-    fc_bind(f, checkpoint, workspace);
-    return f;
+// The token-sequential argument block of the scalar-gate op.
+static SeqArgs scalar_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_view *k,
+                           const gdn2_view *v, const gdn2_view *beta, const gdn2_view *g,
+                           const gdn2_view *valid, const gdn2_view *reset) {
+    SeqArgs a = seq_args(s, q, k, v, beta, beta, beta, valid, reset);
+    a.scalar = 1;
+    a.beta = make_view(beta);
+    a.g = make_view(g);
+    return a;
 }
 
 static int check_scalar_inputs(const gdn2_view *q, const gdn2_view *k, const gdn2_view *v,
@@ -672,28 +542,20 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
         chunk_bind_checkpoint(c, checkpoint);
         return launch_status(launch_chunk_fwd(c, (hipStream_t)stream, ev), "gdn_scalar_scan");
     }
+    SeqArgs a = scalar_args(shape, q, k, v, beta, g, valid, reset);
+    a.initial = make_view(initial);
+    a.out = output;
+    a.out_bf16 = output_dtype == GDN2_BF16;
+    a.final_state = final_state;
+    a.scores = scores;
     if (use_seq_path(shape)) {
-        SeqArgs a = seq_args(shape, q, k, v, beta, beta, beta, valid, reset);
-        a.scalar = 1;
-        a.beta = make_view(beta);
-        a.g = make_view(g);
-        a.initial = make_view(initial);
-        a.out = output;
-        a.out_bf16 = output_dtype == GDN2_BF16;
-        a.final_state = final_state;
-        a.scores = scores;
         seq_bind_checkpoint(a, checkpoint);
         return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_scan");
     }
-    FcArgs f = fs_args(shape, q, k, v, beta, g, valid, reset, nullptr, checkpoint, nullptr);
-    f.s.initial = make_view(initial);
-    f.s.out = output;
-    f.s.out_bf16 = output_dtype == GDN2_BF16;
-    f.s.final_state = final_state;
-    f.s.scores = scores;
     const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
-    return launch_status(launch_fs_fwd(f, (hipStream_t)stream, ev), "gdn_scalar_scan");
+    return launch_status(launch_fs_fwd(fc_args(a, q, false, checkpoint, nullptr), (hipStream_t)stream, ev),
+                         "gdn_scalar_scan");
 }
 
 int gdn_scalar_backward(const gdn2_shape *shape, int chunk, const gdn2_view *q,
@@ -786,36 +648,26 @@ static int scalar_backward_impl(const gdn2_shape *shape, int chunk, const gdn2_v
                                   : launch_chunk_bwd(c, (hipStream_t)stream, ev),
                              "gdn_scalar_backward");
     }
+    SeqArgs a = scalar_args(shape, q, k, v, beta, g, valid, reset);
+    if (d_output) a.dout = make_view(d_output);
+    a.dfinal = d_final_state;
+    a.dscores = d_scores;
+    a.dq = dq;
+    a.dk = dk;
+    a.dv = dv;
+    a.dbeta = dbeta;
+    a.dg = dg;
+    a.dinitial = d_initial;
     if (use_seq_path(shape)) {
-        SeqArgs a = seq_args(shape, q, k, v, beta, beta, beta, valid, reset);
-        a.scalar = 1;
-        a.beta = make_view(beta);
-        a.g = make_view(g);
         seq_bind_checkpoint(a, checkpoint);
-        if (d_output) a.dout = make_view(d_output);
-        a.dfinal = d_final_state;
-        a.dscores = d_scores;
-        a.dq = dq;
-        a.dk = dk;
-        a.dv = dv;
-        a.dbeta = dbeta;
-        a.dg = dg;
-        a.dinitial = d_initial;
         a.replay = (float *)workspace;
         return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_backward");
     }
-    FcArgs f = fs_args(shape, q, k, v, beta, g, valid, reset, d_output, const_cast<void *>(checkpoint), workspace);
-    f.s.dfinal = d_final_state;
-    f.s.dscores = d_scores;
-    f.s.dq = dq;
-    f.s.dk = dk;
-    f.s.dv = dv;
-    f.s.dbeta = dbeta;
-    f.s.dg = dg;
-    f.s.dinitial = d_initial;
     const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
-    return launch_status(launch_fs_bwd(f, workspace_bytes, (hipStream_t)stream, ev), "gdn_scalar_backward");
+    return launch_status(launch_fs_bwd(fc_args(a, q, false, const_cast<void *>(checkpoint), workspace), workspace_bytes,
+                                       (hipStream_t)stream, ev),
+                         "gdn_scalar_backward");
 }
 
 extern "C" {

@@ -63,22 +63,9 @@ struct ChunkArgs {
     // Wide path (d_k = d_v = 128, value blocks of 64): per-chunk |k_t|^2 and the
     // value blocks' partial |delta_t|^2 (forward checkpoint).
     float *ck_kk, *ck_ddp;
-    // Channel-wise path (16-token chunks): the gates alpha, erase [B,T,H,K] and
-    // write [B,T,H,V] (f32 views), the chunk-local cumulative log decay checkpoint,
-    // and the per-channel gate gradients.
-    View alpha, erase, write;
-    struct CwGate *ck_cwg;
-    float *ck_lam;
-    float *ck_tf;  // T = (I + A)^-1 per 16-token chunk, f32
-    float *ck_p;   // P (decay-weighted q.k overlaps, lower, same segment) per chunk, f32
     // Lo parts (x - bf16(x)) of the chunk-start states and the chunk-end state
     // adjoints, kept by the scan when non-null.
     uint16_t *ck_state_lo, *ws_dstate_lo;
-    // Document limits (int32 [B,T] views, inclusive) in place of valid/reset:
-    // a token is live when end >= start and resets the state when start == t.
-    int doc;
-    View doc_start, doc_end;
-    float *dalpha, *derase, *dwrite;
     // Factored chunk map (the scan of gdn2_chunk_lr.hip): -W'^T [D][C] and
     // Ktil = lam K [C][D] (bf16), U^T [D][C] and the map's diagonal [D] (f32).
     uint16_t *lr_wt, *lr_kt;
@@ -94,7 +81,7 @@ struct ChunkArgs {
 // A kernel that walks many chunks calls this at the top of each chunk: behind
 // the opaque move the compiler reloads the fields a chunk uses with scalar
 // loads, instead of holding every field in SGPRs across the loop, where they
-// spill into VGPR lanes.  (In the one-chunk cw_bgrad it measured 3% slower.)
+// spill into VGPR lanes.
 __device__ inline const ChunkArgs &chunk_args_reloaded() {
     typedef const __attribute__((address_space(4))) ChunkArgs KernArgs;
     KernArgs *p = (KernArgs *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -150,85 +137,9 @@ inline void chunk_bind_workspace(ChunkArgs &a, void *ws) {
     a.ws_n = reinterpret_cast<float *>(p);
 }
 
-// ---- channel-wise path: per-channel gates, 16-token chunks, d_k = d_v = 64 ------
-constexpr int CW_C = 16;  // tokens per chunk
-struct CwGate {
-    float val[CW_C];
-    int seg[CW_C];  // resets at or before the token within the chunk
-};
-
-inline bool cw_eligible_shape(const gdn2_shape *s) {
-    return s->keys == CHUNK_D && s->values == CHUNK_D;
-}
-
-inline int64_t cw_chunk_count(int64_t B, int64_t T, int64_t H) {
-    return B * H * ((T + CW_C - 1) / CW_C);
-}
-
-// Checkpoint per chunk: S0^T (bf16 hi/lo, 64x64), T and P (f32 16x16), CwGate,
-// the cumulative log decay Lambda (f32 16x64), delta (f32 16x64), and the
-// factored chunk map: -W'^T and Ktil (bf16 hi and lo, 16x64 each), U^T (f32
-// 16x64), b_15 (f32 64).
-constexpr size_t CWK_STATE = (size_t)CHUNK_D * CHUNK_D * 2;
-constexpr size_t CWK_T = (size_t)CW_C * CW_C * 4;
-constexpr size_t CWK_GATE = sizeof(CwGate);
-constexpr size_t CWK_LAM = (size_t)CW_C * CHUNK_D * 4;
-constexpr size_t CWK_DELTA = (size_t)CW_C * CHUNK_D * 4;
-constexpr size_t CWK_LRW = (size_t)CW_C * CHUNK_D * 2 * 2;  // hi and lo
-constexpr size_t CWK_LRU = (size_t)CW_C * CHUNK_D * 4;
-constexpr size_t CWK_LRG = (size_t)CHUNK_D * 4;
-constexpr size_t CWK_MAPN = (size_t)CHUNK_D * CHUNK_D * 4;
-constexpr size_t CWK_CHUNK = 2 * CWK_STATE + 2 * CWK_T + CWK_GATE + CWK_LAM + CWK_DELTA + 2 * CWK_LRW +
-                             CWK_LRU + CWK_LRG;
-constexpr size_t CWW_CHUNK = 2 * CWK_STATE + CWK_MAPN;  // backward: dS^T (bf16 hi/lo), N^T (f32)
-
-inline size_t cw_checkpoint_bytes(int64_t B, int64_t T, int64_t H) {
-    return (size_t)cw_chunk_count(B, T, H) * CWK_CHUNK;
-}
-inline size_t cw_workspace_bytes(int64_t B, int64_t T, int64_t H) {
-    return (size_t)cw_chunk_count(B, T, H) * CWW_CHUNK;
-}
-
-inline void cw_bind_checkpoint(ChunkArgs &a, void *ck) {
-    const int64_t n = (int64_t)a.B * a.H * a.nc;
-    char *p = static_cast<char *>(ck);
-    a.ck_state = reinterpret_cast<uint16_t *>(p);
-    p += n * CWK_STATE;
-    a.ck_state_lo = reinterpret_cast<uint16_t *>(p);
-    p += n * CWK_STATE;
-    a.ck_tf = reinterpret_cast<float *>(p);
-    p += n * CWK_T;
-    a.ck_p = reinterpret_cast<float *>(p);
-    p += n * CWK_T;
-    a.ck_cwg = reinterpret_cast<CwGate *>(p);
-    p += n * CWK_GATE;
-    a.ck_lam = reinterpret_cast<float *>(p);
-    p += n * CWK_LAM;
-    a.ck_delta = reinterpret_cast<float *>(p);
-    p += n * CWK_DELTA;
-    a.lr_wt = reinterpret_cast<uint16_t *>(p);
-    p += n * CWK_LRW;
-    a.lr_kt = reinterpret_cast<uint16_t *>(p);
-    p += n * CWK_LRW;
-    a.lr_u = reinterpret_cast<float *>(p);
-    p += n * CWK_LRU;
-    a.lr_gv = reinterpret_cast<float *>(p);
-}
-
-inline void cw_bind_workspace(ChunkArgs &a, void *ws) {
-    const int64_t n = (int64_t)a.B * a.H * a.nc;
-    char *p = static_cast<char *>(ws);
-    a.ws_dstate = reinterpret_cast<uint16_t *>(p);
-    a.ws_dstate_lo = reinterpret_cast<uint16_t *>(p + n * CWK_STATE);
-    a.ws_n = reinterpret_cast<float *>(p + 2 * n * CWK_STATE);
-}
-
 // The affine scan over a.nc chunks of per-chunk 64 x 64 maps (gdn2_chunk.hip),
 // forward (state) or reverse (adjoint).
 hipError_t launch_chunk_scan(const ChunkArgs &a, bool reverse, hipStream_t stream);
-
-hipError_t launch_cw_fwd(const ChunkArgs &a, hipStream_t stream, const hipEvent_t *ev);
-hipError_t launch_cw_bwd(const ChunkArgs &a, hipStream_t stream, const hipEvent_t *ev);
 
 // ---- wide path: d_k = d_v = WIDE_D, value blocks of 64 -------------------------
 constexpr int WIDE_D = 128;
@@ -306,21 +217,20 @@ hipError_t launch_wide_bwd(const ChunkArgs &a, hipStream_t stream, const hipEven
 // Factored affine scan (gdn2_chunk_lr.hip) over chunks of one (batch, head):
 //   forward  X_next = diag(gv) X + Ktil^T (U - W' X),   X0 = initial state
 //   reverse  X_prev = diag(gv) X + N - W'^T (Ktil X),   X0 = final-state adjoint
-// with X before each step to ckpt[c] (X^T, bf16 hi and, when ckpt_lo is set, lo).
+// with X before each step to ckpt[c] and ckpt_lo[c] (X^T, bf16 hi and lo).
 struct LrScanArgs {
     int nc, B, H, vd;      // chunks per head, batch, heads, state columns
-    const uint16_t *wt;    // -W'^T per chunk [kd][ct] bf16 (kd x ct = 64 x 16: hi, then lo)
-    const uint16_t *kt;    // per chunk: kd = 128, K [ct][kd] bf16 (Ktil = lam K);
-                           // kd = 64, Ktil [ct][kd] bf16 hi, then lo
+    const uint16_t *wt;    // -W'^T per chunk [kd][ct] bf16
+    const uint16_t *kt;    // per chunk K [ct][kd] bf16 (Ktil = lam K)
     const float *u;        // U^T per chunk [vd][ct] f32 (forward)
     const float *n;        // N^T per chunk [vd][kd] f32 (reverse)
-    const float *gv;       // per chunk: the map's diagonal [kd] f32; kd = 128: then lam [ct]
+    const float *gv;       // per chunk: the map's diagonal [kd], then lam [ct], f32
     uint16_t *ckpt, *ckpt_lo;  // X^T per chunk [vd][kd] bf16
     View x0;               // [B,H,kd,vd] strided (data may be null: zero)
     float *xout;           // [B,H,kd,vd] dense (may be null)
     int reverse;
 };
-// kd x ct in {128 x 64, 64 x 16}; hipErrorInvalidValue for other shapes.
+// kd x ct = 128 x 64; hipErrorInvalidValue for other shapes.
 hipError_t launch_lr_scan(const LrScanArgs &p, int kd, int ct, hipStream_t stream);
 
 // Compute units of the current device (queried once per device); sizes the

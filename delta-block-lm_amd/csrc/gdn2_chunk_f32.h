@@ -1,4 +1,5 @@
-// Chunked channel-wise GDN-2 in f32 (d_k, d_v <= 128, 16-token chunks).
+// Chunked GDN-2 in f32 (d_k, d_v <= 128, 16-token chunks): channel-wise gates
+// (gdn2_chunk_f32.hip) and scalar gates (gdn2_chunk_fs.hip).
 #pragma once
 
 #include "gdn2_seq.h"
@@ -9,12 +10,7 @@ namespace gdn2 {
 // take buffers of any alignment (16-byte accesses to global memory need four).
 typedef float fc_u4 __attribute__((ext_vector_type(4), aligned(4)));
 
-constexpr int FC_C = 16;    // tokens per chunk
-constexpr int FC_MAX = 128;  // largest d_k and d_v
-
-inline bool fc_eligible_shape(const gdn2_shape *s) {
-    return s->keys <= FC_MAX && s->values <= FC_MAX;
-}
+constexpr int FC_C = 16;  // tokens per chunk
 
 // The token-sequential argument block (shapes, views, outputs, gradients)
 // plus the chunk path's checkpoint and workspace arrays, each indexed by
@@ -22,50 +18,67 @@ inline bool fc_eligible_shape(const gdn2_shape *s) {
 //   st     S at the chunk start, tile-packed: [VT][KT][4][16][4], element
 //          (((vt * KT + tau) * 4 + g) * 16 + n) * 4 + r = S[16 tau + 4 g + r][16 vt + n]
 //          (forward scan -> out, bgrad)
-//   tm     T = (I + A)^-1, [16][16]                       (prep -> out, bgrad)
-//   dl     the edits delta, [16][V]                       (out -> bprep, bgrad)
+//   tm     T = (I + A)^-1, [16][16]                          (prep -> bgrad)
+//   pm     P, [16][16]                          (prep -> out, bprep, bgrad)
+//   dm     the pair decays D, [16][16], scalar gates only    (prep -> bgrad)
 //   fw, fk the factored map: W' = T (b . e . k) and Ktil = lam . k, [16][KP] each
-//   fu     U = T (w . v), lane-packed for the scan: [VT][4][16][4], element
-//          ((vt * 4 + g) * 16 + n) * 4 + r = U[4 g + r][16 vt + n]
+//   fq     Qhat = b . q, [16][KP]                      (prep -> out, bprep)
+//   fu     U = T (w . v), lane-packed: [VT][4][16][4], element
+//          ((vt * 4 + g) * 16 + n) * 4 + r = U[4 g + r][16 vt + n]; the forward
+//          scan overwrites it with the edits delta (-> out, bprep, bgrad)
 //   gv     b_15 (the map's diagonal), [KP]
+//   gb     per token: valid, reset, |k|^2, and with scalar gates beta, b, lam; [16][8]
 // KP = d_k and VP = d_v rounded up to 16 (VT = VP / 16): the key axis of the
 // map's factors is padded with zeros to whole 16-row MFMA tiles for the scans.
 // KT = KP / 16.  A scan wave stores its 16 x 16 tile of S as one 16-byte piece
 // per lane, its accumulator registers as they are.  Backward workspace: ds, the
-// state adjoint at each chunk end, and n, the adjoint map's additive term, both
-// tile-packed like st.  st, ds and n are zero outside K x V.  Every array starts
-// on a 16-byte boundary.
+// state adjoint at each chunk end, and n, the adjoint map's additive term,
+// both tile-packed like st, for the window of chunks w0 .. w0 + wn - 1 of each
+// (batch, head) (index bh * wn + c - w0; all nc chunks unless the scalar-gate
+// path walks windows); carry is the adjoint before the window, tile-packed, one
+// state per (batch, head).  st, ds and n are zero outside K x V.  Every array
+// starts on a 16-byte boundary when the caller's buffer does.
 struct FcArgs {
     SeqArgs s;
     int nc;
     int in_bf16;  // q, k, v, dO and dq, dk, dv are bf16 (else f32)
-    float *st, *tm, *dl, *fw, *fk, *fu, *gv;
+    int vec;      // every input of the call passes fc_vec_view
+    int scalar;   // scalar gates
+    int nonneg;   // a negative alpha poisons its sequence with NaN
+    float *st, *tm, *pm, *dm, *fw, *fk, *fq, *fu, *gv, *gb;
     float *ds, *n;
     int w0, wn;
     float *carry;
-    int scalar;  // the scalar-gate path's layout
-    int vec;     // its 4-channel reads: bit 0 q, 1 k, 2 v, 3 dO
 };
 
 inline int64_t fc_chunks(int64_t B, int64_t T, int64_t H) { return B * H * ((T + FC_C - 1) / FC_C); }
 __host__ __device__ inline int fc_kp(int K) { return (K + 15) & ~15; }
-inline size_t fc_pad4(size_t x) { return (x + 3) & ~(size_t)3; }
 
-// The checkpoint's arrays in order, in floats, for n chunks.
-inline void fc_checkpoint_parts(int64_t n, int K, int V, size_t part[7], bool scalar = false) {
-    const size_t KP = fc_kp(K), VP = fc_kp(V);
-    part[0] = n * KP * VP;              // st
-    part[1] = fc_pad4(n * FC_C * FC_C); // tm
-    part[2] = scalar ? 0 : fc_pad4(n * FC_C * V);  // dl
-    part[3] = n * FC_C * KP;            // fw
-    part[4] = n * FC_C * KP;            // fk
-    part[5] = n * FC_C * VP;            // fu
-    part[6] = n * KP;                   // gv
+// The inputs that the kernels read by whole 16-channel tiles from a uniform base
+// with 32-bit offsets: unit channel stride, 4-channel pieces aligned to their
+// size, and rows less than 2^24 elements apart.
+inline bool fc_vec_view(const View &v, int bytes, int64_t W) {
+    return v.s3 == 1 && W % 16 == 0 && ((uintptr_t)v.data & (4 * bytes - 1)) == 0 && v.s0 % 4 == 0 &&
+           v.s1 % 4 == 0 && v.s2 % 4 == 0 && v.s1 < (1 << 24);
 }
 
-inline size_t fc_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V, bool scalar = false) {
-    size_t part[7], total = 0;
-    fc_checkpoint_parts(fc_chunks(B, T, H), K, V, part, scalar);
+constexpr int FC_PARTS = 10;
+// The checkpoint's arrays in order, in floats, for n chunks (each a multiple of
+// four).
+inline void fc_checkpoint_parts(int64_t n, int K, int V, bool scalar, size_t part[FC_PARTS]) {
+    const size_t KP = fc_kp(K), VP = fc_kp(V);
+    part[0] = n * KP * VP;                      // st
+    part[1] = part[2] = n * FC_C * FC_C;        // tm, pm
+    part[3] = scalar ? n * FC_C * FC_C : 0;     // dm
+    part[4] = part[5] = part[6] = n * FC_C * KP;  // fw, fk, fq
+    part[7] = n * FC_C * VP;                    // fu
+    part[8] = n * KP;                           // gv
+    part[9] = n * FC_C * 8;                     // gb
+}
+
+inline size_t fc_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V, bool scalar) {
+    size_t part[FC_PARTS], total = 0;
+    fc_checkpoint_parts(fc_chunks(B, T, H), K, V, scalar, part);
     for (size_t x : part) total += x;
     return total * sizeof(float);
 }
@@ -77,11 +90,11 @@ inline size_t fc_workspace_bytes(int64_t B, int64_t T, int64_t H, int K, int V) 
 
 inline void fc_bind(FcArgs &a, void *ck, void *ws) {
     const int64_t n = fc_chunks(a.s.B, a.s.T, a.s.H);
-    size_t part[7];
-    fc_checkpoint_parts(n, a.s.K, a.s.V, part, a.scalar != 0);
+    size_t part[FC_PARTS];
+    fc_checkpoint_parts(n, a.s.K, a.s.V, a.scalar != 0, part);
     float *p = static_cast<float *>(ck);
-    float **dst[7] = {&a.st, &a.tm, &a.dl, &a.fw, &a.fk, &a.fu, &a.gv};
-    for (int i = 0; i < 7; ++i) {
+    float **dst[FC_PARTS] = {&a.st, &a.tm, &a.pm, &a.dm, &a.fw, &a.fk, &a.fq, &a.fu, &a.gv, &a.gb};
+    for (int i = 0; i < FC_PARTS; ++i) {
         *dst[i] = p;
         p += part[i];
     }
@@ -93,14 +106,16 @@ inline void fc_bind(FcArgs &a, void *ck, void *ws) {
     }
 }
 
-// The state scan over the chunks (the adjoint scan over the window when rev).
+// The stages that both gate forms share: the state scan over the chunks (the
+// adjoint scan over the window when rev), out, and bprep over the window.
 void launch_fc_scan(const FcArgs &a, bool rev, hipStream_t stream);
+void launch_fc_out(const FcArgs &a, hipStream_t stream);
+void launch_fc_bprep(const FcArgs &a, hipStream_t stream);
 
 hipError_t launch_fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
 hipError_t launch_fc_bwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
-// Scalar gates.  The backward takes any workspace of at least one chunk window
-// and the carry (fs_min_workspace_bytes); the whole of fc_workspace_bytes is one
-// window.
+// Scalar gates.  The backward takes any workspace that holds one chunk window
+// and the carry; the whole of fc_workspace_bytes is one window.
 hipError_t launch_fs_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
 hipError_t launch_fs_bwd(const FcArgs &a, size_t ws_bytes, hipStream_t stream, const hipEvent_t *ev);
 

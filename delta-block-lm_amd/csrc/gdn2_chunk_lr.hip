@@ -8,8 +8,7 @@
 // CT x VD update and N the adjoint's additive term.  Streaming the factors
 // instead of the dense KD x KD map moves (2 KD CT + 4 VD CT) bytes per chunk
 // and head in place of (2 KD KD + 4 KD VD): for d = 128, C = 64 that is 64 KiB
-// instead of 96 KiB, and for the channel-wise 16-token chunks 8 KiB instead of
-// 24 KiB.  Both directions run two products per step,
+// instead of 96 KiB.  Both directions run two products per step,
 //   phase 1  V = Ad - Qm X        (CT x 16 per wave, reduction over KD)
 //   phase 2  X = gv X + Pm^T V + N (KD x 16 per wave, reduction over CT)
 // forward: Qm = -W', Pm = Ktil, Ad = U, N = 0; reverse: Qm = Ktil, Pm = -W',
@@ -98,47 +97,35 @@ __device__ __forceinline__ void lr_split(const f32x4 &x, lr_v4s &hi, lr_v4s &lo)
     }
 }
 
-template <int KD_, int CT_, int NCW_, int NPROD_, int R_, bool BWD_, bool LO_, bool WHL_, bool KLAM_>
+template <int KD_, int CT_, int NCW_, int R_, bool BWD_>
 struct LrCfg {
-    static constexpr int KD = KD_, CT = CT_, NCW = NCW_, NPROD = NPROD_, R = R_;
-    static constexpr bool BWD = BWD_, LO = LO_;  // LO: the checkpoint keeps lo parts
-    static constexpr bool WHL = WHL_;            // -W'^T comes as hi and lo
-    // KLAM: Ktil = diag(lam) K with one lam per token (scalar gates) comes as the
-    // bf16 rows of K (exact) and lam (f32, after gv); lam scales the f32 tile V
-    // instead (Ktil^T V = K^T (lam V), Ktil X = lam (K X)).  Otherwise Ktil comes
-    // as bf16 hi and lo.
-    static constexpr bool KLAM = KLAM_;
+    static constexpr int KD = KD_, CT = CT_, NCW = NCW_, R = R_;
+    static constexpr int NPROD = 3;  // producer waves: one per stream
+    static constexpr bool BWD = BWD_;
+    // Ktil = diag(lam) K with one lam per token comes as the bf16 rows of K (exact)
+    // and lam (f32, after gv); lam scales the f32 tile V instead (Ktil^T V = K^T
+    // (lam V), Ktil X = lam (K X)).
     static constexpr int WT_NCH = CT * 2 / 16;              // -W'^T [KD][CT] bf16
     static constexpr int KT_NCH = KD * 2 / 16;              // Ktil [CT][KD] bf16
     static constexpr int AUX_NCH = (BWD ? KD : CT) * 4 / 16;  // N^T [cols][KD] or U^T [cols][CT] f32
-    // The factors arrive as bf16 hi and lo tiles, the lo tile right after the hi
-    // tile in memory and in the LDS slot (rows KD.. of -W'^T, CT.. of Ktil).
-    static constexpr int WT_BYTES = KD * CT * 2;            // one term
+    static constexpr int WT_BYTES = KD * CT * 2;
     static constexpr int KT_BYTES = CT * KD * 2;
-    static constexpr int WT_TERMS = WHL ? 2 : 1;
     static constexpr int AUX_BYTES = NCW * 16 * AUX_NCH * 16;
     static constexpr int GV_BYTES = 1024;                   // KD f32 (KD <= 256)
-    static constexpr int KT_TERMS = KLAM ? 1 : 2;
-    static constexpr int GV_FLOATS = KD + (KLAM ? CT : 0);  // gv, then lam
-    static constexpr int WT_OPS = WT_TERMS * WT_BYTES / 1024, KT_OPS = KT_TERMS * KT_BYTES / 1024,
-                         AUX_OPS = AUX_BYTES / 1024;
-    static constexpr int SLOT = WT_TERMS * WT_BYTES + KT_TERMS * KT_BYTES + AUX_BYTES + GV_BYTES;
+    static constexpr int GV_FLOATS = KD + CT;  // gv, then lam
+    static constexpr int WT_OPS = WT_BYTES / 1024, KT_OPS = KT_BYTES / 1024, AUX_OPS = AUX_BYTES / 1024;
+    static constexpr int SLOT = WT_BYTES + KT_BYTES + AUX_BYTES + GV_BYTES;
     static constexpr int XS_NCH = KD * 2 / 16;                  // X^T staging rows [16 cols][KD] bf16
     static constexpr int XS_BYTES = 16 * KD * 2;                // one term (hi or lo)
-    static constexpr int LDS_BYTES = R * SLOT + NCW * (LO ? 2 : 1) * XS_BYTES;
+    static constexpr int LDS_BYTES = R * SLOT + NCW * 2 * XS_BYTES;
     // LDS-DMA operations each producer issues per chunk
-    static constexpr int OPS0 = NPROD == 1 ? WT_OPS + KT_OPS + AUX_OPS + 1 : WT_OPS;
-    static constexpr int OPS1 = NPROD == 1 ? 0 : KT_OPS;
-    static constexpr int OPS2 = NPROD == 1 ? 0 : AUX_OPS + 1;
+    static constexpr int OPS0 = WT_OPS, OPS1 = KT_OPS, OPS2 = AUX_OPS + 1;
     static_assert(WT_BYTES % 1024 == 0 && KT_BYTES % 1024 == 0 && AUX_BYTES % 1024 == 0, "1 KiB DMA units");
     static_assert(GV_FLOATS * 4 <= GV_BYTES && GV_FLOATS % 4 == 0, "gv and lam fit one DMA unit");
-    static_assert(NPROD == 1 || NPROD == 3, "one producer, or one per stream");
     static_assert((R - 1) * OPS0 <= 63 && (R - 1) * OPS1 <= 63 && (R - 1) * OPS2 <= 63,
                   "prefetched chunks fit the memory counter");
     static_assert(LDS_BYTES <= 160 * 1024, "ring and staging fit LDS");
-    static_assert(KD % 32 == 0 && (CT == 16 || CT % 32 == 0), "tile shapes");
-    // The lo tile reuses the hi tile's swizzle: lr_swz repeats every 16 rows.
-    static_assert(KD % 16 == 0 && CT % 16 == 0, "lo tiles start on a swizzle period");
+    static_assert(KD % 32 == 0 && CT % 32 == 0, "tile shapes");
 };
 
 }  // namespace
@@ -170,15 +157,15 @@ __global__ void __launch_bounds__(64 * (Cfg::NCW + Cfg::NPROD)) lr_scan_kernel(L
             const int sc = min(s, p.nc - 1);
             const int64_t cix = (int64_t)bh * p.nc + chunk_of(sc);
             char *slot = lr_ring + (s % R) * Cfg::SLOT;
-            if (Cfg::NPROD == 1 || pw == 0)
-                dma_tile(reinterpret_cast<const char *>(p.wt + cix * Cfg::WT_TERMS * KD * CT), Cfg::WT_OPS,
+            if (pw == 0)
+                dma_tile(reinterpret_cast<const char *>(p.wt + cix * KD * CT), Cfg::WT_OPS,
                          Cfg::WT_NCH, slot);
-            if (Cfg::NPROD == 1 || pw == 1)
-                dma_tile(reinterpret_cast<const char *>(p.kt + cix * Cfg::KT_TERMS * CT * KD), Cfg::KT_OPS,
-                         Cfg::KT_NCH, slot + Cfg::WT_TERMS * Cfg::WT_BYTES);
-            if (Cfg::NPROD == 1 || pw == 2) {
+            if (pw == 1)
+                dma_tile(reinterpret_cast<const char *>(p.kt + cix * CT * KD), Cfg::KT_OPS,
+                         Cfg::KT_NCH, slot + Cfg::WT_BYTES);
+            if (pw == 2) {
                 const float *aux = BWD ? p.n + (cix * p.vd + colbase) * KD : p.u + (cix * p.vd + colbase) * CT;
-                char *ax = slot + Cfg::WT_TERMS * Cfg::WT_BYTES + Cfg::KT_TERMS * Cfg::KT_BYTES;
+                char *ax = slot + Cfg::WT_BYTES + Cfg::KT_BYTES;
                 dma_tile(reinterpret_cast<const char *>(aux), Cfg::AUX_OPS, Cfg::AUX_NCH, ax);
                 if (l < Cfg::GV_FLOATS / 4)
                     __builtin_amdgcn_global_load_lds((lr_gptr)(p.gv + cix * Cfg::GV_FLOATS + 4 * l),
@@ -211,8 +198,7 @@ __global__ void __launch_bounds__(64 * (Cfg::NCW + Cfg::NPROD)) lr_scan_kernel(L
         // wave's LDS rows [16 columns][KD] to the checkpoint in whole 16-byte pieces
         // (eight lanes per column row), so each store instruction writes full lines.
         bf16x8_t xh[KD / 32], xl[KD / 32];
-        char *xsw = lr_ring + R * Cfg::SLOT + w * (Cfg::LO ? 2 : 1) * Cfg::XS_BYTES;
-        constexpr bool lo_out = Cfg::LO;
+        char *xsw = lr_ring + R * Cfg::SLOT + w * 2 * Cfg::XS_BYTES;
 #pragma unroll
         for (int kk = 0; kk < KD / 32; ++kk) {
             lr_v4s h0, l0, h1, l1;
@@ -222,49 +208,42 @@ __global__ void __launch_bounds__(64 * (Cfg::NCW + Cfg::NPROD)) lr_scan_kernel(L
             xl[kk] = lr_cat(l0, l1);
             *reinterpret_cast<lr_v4s *>(xsw + lr_off(n, 32 * kk + 4 * g, 2, Cfg::XS_NCH)) = h0;
             *reinterpret_cast<lr_v4s *>(xsw + lr_off(n, 32 * kk + 16 + 4 * g, 2, Cfg::XS_NCH)) = h1;
-            if (lo_out) {
-                *reinterpret_cast<lr_v4s *>(xsw + Cfg::XS_BYTES + lr_off(n, 32 * kk + 4 * g, 2, Cfg::XS_NCH)) = l0;
-                *reinterpret_cast<lr_v4s *>(xsw + Cfg::XS_BYTES + lr_off(n, 32 * kk + 16 + 4 * g, 2, Cfg::XS_NCH)) = l1;
-            }
+            *reinterpret_cast<lr_v4s *>(xsw + Cfg::XS_BYTES + lr_off(n, 32 * kk + 4 * g, 2, Cfg::XS_NCH)) = l0;
+            *reinterpret_cast<lr_v4s *>(xsw + Cfg::XS_BYTES + lr_off(n, 32 * kk + 16 + 4 * g, 2, Cfg::XS_NCH)) = l1;
         }
         {
             uint16_t *ck = p.ckpt + (cix * p.vd + colbase + 16 * w) * KD;
-            uint16_t *cl = lo_out ? p.ckpt_lo + (cix * p.vd + colbase + 16 * w) * KD : nullptr;
+            uint16_t *cl = p.ckpt_lo + (cix * p.vd + colbase + 16 * w) * KD;
 #pragma unroll
             for (int i = 0; i < Cfg::XS_BYTES / 1024; ++i) {
                 const int q = 64 * i + l, r = q / Cfg::XS_NCH, y = q % Cfg::XS_NCH;
                 const int off = r * Cfg::XS_NCH * 16 + ((y ^ lr_swz(r, Cfg::XS_NCH)) << 4);
                 *reinterpret_cast<uint4 *>(ck + 8 * q) = *reinterpret_cast<const uint4 *>(xsw + off);
-                if (lo_out)
-                    *reinterpret_cast<uint4 *>(cl + 8 * q) = *reinterpret_cast<const uint4 *>(xsw + Cfg::XS_BYTES + off);
+                *reinterpret_cast<uint4 *>(cl + 8 * q) = *reinterpret_cast<const uint4 *>(xsw + Cfg::XS_BYTES + off);
             }
         }
         lr_barrier();  // slot s has landed
         const char *slot = lr_ring + (s % R) * Cfg::SLOT;
-        const char *wt = slot, *kt = slot + Cfg::WT_TERMS * Cfg::WT_BYTES, *ax = kt + Cfg::KT_TERMS * Cfg::KT_BYTES;
-        constexpr bool WHL = Cfg::WHL, KLAM = Cfg::KLAM;
+        const char *wt = slot, *kt = slot + Cfg::WT_BYTES, *ax = kt + Cfg::KT_BYTES;
         const float *gv = reinterpret_cast<const float *>(ax + Cfg::AUX_BYTES);
-        const float *lam = gv + KD;  // KLAM: lam of the chunk's tokens
-        constexpr int WL = Cfg::WT_BYTES, KL = Cfg::KT_BYTES;  // offsets of the lo tiles
+        const float *lam = gv + KD;  // of the chunk's tokens
         // Phase 1's LDS reads first (none depends on X), then phase 2's, so their
         // latencies overlap each other and the products.
-        constexpr int NP = CT >= 32 ? CT / 32 : 1;
-        bf16x8_t qa[CT / 16][KD / 32], qal[CT / 16][KD / 32] = {};  // phase 1 A operands (Qm hi, lo)
+        constexpr int NP = CT / 32;
+        bf16x8_t qa[CT / 16][KD / 32];  // phase 1 A operands (Qm)
         f32x4 ad[CT / 16], nb[KD / 16], gq[KD / 16];
 #pragma unroll
         for (int tt = 0; tt < CT / 16; ++tt)
 #pragma unroll
             for (int kk = 0; kk < KD / 32; ++kk) {
-                if (BWD) {  // Qm = Ktil (KLAM: K) rows: token 16 tt + n, keys 32 kk + 4 g (+ 16)
+                if (BWD) {  // Qm = K rows: token 16 tt + n, keys 32 kk + 4 g (+ 16)
                     const int o0 = lr_off(16 * tt + n, 32 * kk + 4 * g, 2, Cfg::KT_NCH);
                     const int o1 = lr_off(16 * tt + n, 32 * kk + 16 + 4 * g, 2, Cfg::KT_NCH);
                     qa[tt][kk] = lr_cat(lr_ld8(kt + o0), lr_ld8(kt + o1));
-                    if (!KLAM) qal[tt][kk] = lr_cat(lr_ld8(kt + KL + o0), lr_ld8(kt + KL + o1));
                 } else {  // Qm = -W' read across -W'^T rows (keys 32 kk + 4 g + e (+ 16), token 16 tt + n)
                     const int r = 32 * kk + 4 * g + (n >> 2), e = 16 * tt + 4 * (n & 3);
                     const int o0 = lr_off(r, e, 2, Cfg::WT_NCH), o1 = lr_off(r + 16, e, 2, Cfg::WT_NCH);
                     qa[tt][kk] = lr_cat(lr_tr16(wt + o0), lr_tr16(wt + o1));
-                    if (WHL) qal[tt][kk] = lr_cat(lr_tr16(wt + WL + o0), lr_tr16(wt + WL + o1));
                 }
             }
         if (!BWD)
@@ -284,7 +263,7 @@ __global__ void __launch_bounds__(64 * (Cfg::NCW + Cfg::NPROD)) lr_scan_kernel(L
                 nb[rt] = f32x4{nv.x, nv.y, nv.z, nv.w};
             }
         }
-        // phase 1: V = Ad - Qm X (token tiles tt), three terms of the hi/lo pairs
+        // phase 1: V = Ad - Qm X (token tiles tt), both terms of X
         f32x4 V[CT / 16];
 #pragma unroll
         for (int tt = 0; tt < CT / 16; ++tt) V[tt] = BWD ? zero4() : ad[tt];
@@ -293,13 +272,10 @@ __global__ void __launch_bounds__(64 * (Cfg::NCW + Cfg::NPROD)) lr_scan_kernel(L
 #pragma unroll
             for (int tt = 0; tt < CT / 16; ++tt) {
                 V[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[tt][kk], xh[kk], V[tt], 0, 0, 0);
-                if ((BWD && !KLAM) || (!BWD && WHL))
-                    V[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qal[tt][kk], xh[kk], V[tt], 0, 0, 0);
                 V[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[tt][kk], xl[kk], V[tt], 0, 0, 0);
             }
-        // KLAM: V (token rows 16 tt + 4 g + i) times lam, before its split -- the
-        // reverse's K X becomes Ktil X, the forward's V enters Ktil^T V as lam V.
-        if constexpr (KLAM)
+        // V (token rows 16 tt + 4 g + i) times lam, before its split -- the reverse's
+        // K X becomes Ktil X, the forward's V enters Ktil^T V as lam V.
 #pragma unroll
             for (int tt = 0; tt < CT / 16; ++tt) {
                 const float4 lm = *reinterpret_cast<const float4 *>(lam + 16 * tt + 4 * g);
@@ -307,58 +283,33 @@ __global__ void __launch_bounds__(64 * (Cfg::NCW + Cfg::NPROD)) lr_scan_kernel(L
             }
         // phase 2: X = gv X + Pm^T V + N (row tiles rt)
         bf16x8_t vh[NP], vl[NP];
-        lr_v4s vh4 = {0, 0, 0, 0}, vl4 = {0, 0, 0, 0};
-        if constexpr (CT >= 32) {
 #pragma unroll
-            for (int q = 0; q < NP; ++q) {
-                lr_v4s h0, l0, h1, l1;
-                lr_split(V[2 * q], h0, l0);
-                lr_split(V[2 * q + 1], h1, l1);
-                vh[q] = lr_cat(h0, h1);
-                vl[q] = lr_cat(l0, l1);
-            }
-        } else {
-            lr_split(V[0], vh4, vl4);
+        for (int q = 0; q < NP; ++q) {
+            lr_v4s h0, l0, h1, l1;
+            lr_split(V[2 * q], h0, l0);
+            lr_split(V[2 * q + 1], h1, l1);
+            vh[q] = lr_cat(h0, h1);
+            vl[q] = lr_cat(l0, l1);
         }
 #pragma unroll
         for (int rt = 0; rt < KD / 16; ++rt) {
             f32x4 acc;
 #pragma unroll
             for (int i = 0; i < 4; ++i) acc[i] = gq[rt][i] * X[rt][i] + (BWD ? nb[rt][i] : 0.f);
-            if constexpr (CT >= 32) {
 #pragma unroll
-                for (int q = 0; q < NP; ++q) {
-                    bf16x8_t pa, pal = {};
-                    if (BWD) {  // Pm = -W': -W'^T rows 16 rt + n, tokens 32 q + 4 g (+ 16)
-                        const int o0 = lr_off(16 * rt + n, 32 * q + 4 * g, 2, Cfg::WT_NCH);
-                        const int o1 = lr_off(16 * rt + n, 32 * q + 16 + 4 * g, 2, Cfg::WT_NCH);
-                        pa = lr_cat(lr_ld8(wt + o0), lr_ld8(wt + o1));
-                        if (WHL) pal = lr_cat(lr_ld8(wt + WL + o0), lr_ld8(wt + WL + o1));
-                    } else {  // Pm = Ktil (KLAM: K) read across its rows (tokens 32 q + 4 g + e (+ 16), key 16 rt + n)
-                        const int r = 32 * q + 4 * g + (n >> 2), e = 16 * rt + 4 * (n & 3);
-                        const int o0 = lr_off(r, e, 2, Cfg::KT_NCH), o1 = lr_off(r + 16, e, 2, Cfg::KT_NCH);
-                        pa = lr_cat(lr_tr16(kt + o0), lr_tr16(kt + o1));
-                        if (!KLAM) pal = lr_cat(lr_tr16(kt + KL + o0), lr_tr16(kt + KL + o1));
-                    }
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vh[q], acc, 0, 0, 0);
-                    if ((!BWD && !KLAM) || (BWD && WHL))
-                        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pal, vh[q], acc, 0, 0, 0);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vl[q], acc, 0, 0, 0);
+            for (int q = 0; q < NP; ++q) {
+                bf16x8_t pa;
+                if (BWD) {  // Pm = -W': -W'^T rows 16 rt + n, tokens 32 q + 4 g (+ 16)
+                    const int o0 = lr_off(16 * rt + n, 32 * q + 4 * g, 2, Cfg::WT_NCH);
+                    const int o1 = lr_off(16 * rt + n, 32 * q + 16 + 4 * g, 2, Cfg::WT_NCH);
+                    pa = lr_cat(lr_ld8(wt + o0), lr_ld8(wt + o1));
+                } else {  // Pm = K read across its rows (tokens 32 q + 4 g + e (+ 16), key 16 rt + n)
+                    const int r = 32 * q + 4 * g + (n >> 2), e = 16 * rt + 4 * (n & 3);
+                    const int o0 = lr_off(r, e, 2, Cfg::KT_NCH), o1 = lr_off(r + 16, e, 2, Cfg::KT_NCH);
+                    pa = lr_cat(lr_tr16(kt + o0), lr_tr16(kt + o1));
                 }
-            } else {  // 16 tokens: one 16x16x16 product per term
-                lr_v4s pa4, pal4 = {0, 0, 0, 0};
-                if (BWD) {
-                    const int o = lr_off(16 * rt + n, 4 * g, 2, Cfg::WT_NCH);
-                    pa4 = lr_ld8(wt + o);
-                    if (WHL) pal4 = lr_ld8(wt + WL + o);
-                } else {
-                    const int o = lr_off(4 * g + (n >> 2), 16 * rt + 4 * (n & 3), 2, Cfg::KT_NCH);
-                    pa4 = lr_tr16(kt + o);
-                    pal4 = lr_tr16(kt + KL + o);
-                }
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa4, vh4, acc, 0, 0, 0);
-                if (!BWD || WHL) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pal4, vh4, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(pa4, vl4, acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vh[q], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, vl[q], acc, 0, 0, 0);
             }
             X[rt] = acc;
         }
@@ -386,16 +337,8 @@ static hipError_t launch_lr(const LrScanArgs &p, hipStream_t stream) {
 }
 
 hipError_t launch_lr_scan(const LrScanArgs &p, int kd, int ct, hipStream_t stream) {
-    if (p.vd % 16 != 0) return hipErrorInvalidValue;
-    // every configuration keeps the checkpoint's lo part; d = 128 streams -W'^T as hi only
-    if (p.ckpt_lo == nullptr) return hipErrorInvalidValue;
-    if (kd == 128 && ct == 64 && p.vd % 32 == 0)
-        return p.reverse ? launch_lr<LrCfg<128, 64, 2, 3, 2, true, true, false, true>>(p, stream)
-                         : launch_lr<LrCfg<128, 64, 2, 3, 3, false, true, false, true>>(p, stream);
-    if (kd == 64 && ct == 16 && p.vd % 16 == 0)
-        return p.reverse ? launch_lr<LrCfg<64, 16, 1, 1, 5, true, true, true, false>>(p, stream)
-                         : launch_lr<LrCfg<64, 16, 1, 1, 7, false, true, true, false>>(p, stream);
-    return hipErrorInvalidValue;
+    if (p.ckpt_lo == nullptr || kd != 128 || ct != 64 || p.vd % 32 != 0) return hipErrorInvalidValue;
+    return p.reverse ? launch_lr<LrCfg<128, 64, 2, 2, true>>(p, stream) : launch_lr<LrCfg<128, 64, 2, 3, false>>(p, stream);
 }
 
 }  // namespace gdn2
