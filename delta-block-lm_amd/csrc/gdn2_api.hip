@@ -430,7 +430,7 @@ size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
 }
 
 // The f32 chunk kernels' backward walks windows of chunks that fit whatever
-// workspace it is given, so their share is capped: 64 MiB holds 2048 chunks of
+// workspace it is given, so their share is capped: 64 MiB holds 4064 chunks of
 // 64 x 64, enough to fill the chip, and keeps every shape whose other needs fit
 // the library's fixed scratch within it (gdn_scalar_backward_noalloc).
 size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {

@@ -15,28 +15,27 @@ constexpr int FC_C = 16;  // tokens per chunk
 // The token-sequential argument block (shapes, views, outputs, gradients)
 // plus the chunk path's checkpoint and workspace arrays, each indexed by
 // chunk ci = (b * H + h) * nc + c:
-//   st     S at the chunk start, tile-packed: [VT][KT][4][16][4], element
+//   st     S at the chunk start, packed tiles: [VT][KT][4][16][4], element
 //          (((vt * KT + tau) * 4 + g) * 16 + n) * 4 + r = S[16 tau + 4 g + r][16 vt + n]
 //          (forward scan -> out, bgrad)
 //   tm     T = (I + A)^-1, [16][16]                          (prep -> bgrad)
-//   pm     P, [16][16]                          (prep -> out, bprep, bgrad)
+//   pm     P, [16][16]                  (prep -> out, adjoint scan, bgrad)
 //   dm     the pair decays D, [16][16], scalar gates only    (prep -> bgrad)
-//   fw, fk the factored map: W' = T (b . e . k) and Ktil = lam . k, [16][KP] each
-//   fq     Qhat = b . q, [16][KP]                      (prep -> out, bprep)
-//   fu     U = T (w . v), lane-packed: [VT][4][16][4], element
-//          ((vt * 4 + g) * 16 + n) * 4 + r = U[4 g + r][16 vt + n]; the forward
-//          scan overwrites it with the edits delta (-> out, bprep, bgrad)
+//   fw, fk, fq  the factored map W' = T (b . e . k) and Ktil = lam . k, and Qhat =
+//          b . q, packed tiles: [KT][4][16][4], element
+//          ((tau * 4 + g) * 16 + n) * 4 + r = W'[4 g + r][16 tau + n]
+//   fu     U = T (w . v), packed tiles [VT][4][16][4]; the forward scan overwrites
+//          it with the edits delta (-> out, bgrad)
 //   gv     b_15 (the map's diagonal), [KP]
-//   gb     per token: valid, reset, |k|^2, and with scalar gates beta, b, lam; [16][8]
-// KP = d_k and VP = d_v rounded up to 16 (VT = VP / 16): the key axis of the
-// map's factors is padded with zeros to whole 16-row MFMA tiles for the scans.
-// KT = KP / 16.  A scan wave stores its 16 x 16 tile of S as one 16-byte piece
-// per lane, its accumulator registers as they are.  Backward workspace: ds, the
-// state adjoint at each chunk end, and n, the adjoint map's additive term,
-// both tile-packed like st, for the window of chunks w0 .. w0 + wn - 1 of each
-// (batch, head) (index bh * wn + c - w0; all nc chunks unless the scalar-gate
-// path walks windows); carry is the adjoint before the window, tile-packed, one
-// state per (batch, head).  st, ds and n are zero outside K x V.  Every array
+//   gb     rows of one value per token: valid, reset, |k|^2, and with scalar gates
+//          beta, b, lam; [8][16]
+// KP = d_k and VP = d_v rounded up to 16 (KT = KP / 16, VT = VP / 16): the tiles
+// are padded with zeros to whole 16 x 16 MFMA tiles.  Backward workspace: ds, the
+// state adjoint at each chunk end, packed like st, and, with a score adjoint, sc,
+// the coefficients c and c' per token [2][16], for the window of chunks w0 .. w0 +
+// wn - 1 of each (batch, head) (index bh * wn + c - w0; all nc chunks unless the
+// scalar-gate path walks windows); carry is the adjoint before the window, packed,
+// one state per (batch, head).  st and ds are zero outside K x V.  Every array
 // starts on a 16-byte boundary when the caller's buffer does.
 struct FcArgs {
     SeqArgs s;
@@ -46,7 +45,7 @@ struct FcArgs {
     int scalar;   // scalar gates
     int nonneg;   // a negative alpha poisons its sequence with NaN
     float *st, *tm, *pm, *dm, *fw, *fk, *fq, *fu, *gv, *gb;
-    float *ds, *n;
+    float *ds, *sc;
     int w0, wn;
     float *carry;
 };
@@ -83,9 +82,11 @@ inline size_t fc_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V,
     return total * sizeof(float);
 }
 
+// Floats of the workspace per chunk.
+inline int64_t fc_ws_chunk(int K, int V) { return (int64_t)fc_kp(K) * fc_kp(V) + 2 * FC_C; }
+
 inline size_t fc_workspace_bytes(int64_t B, int64_t T, int64_t H, int K, int V) {
-    const int64_t n = fc_chunks(B, T, H);
-    return 2 * (size_t)n * fc_kp(K) * fc_kp(V) * sizeof(float);
+    return (size_t)(fc_chunks(B, T, H) * fc_ws_chunk(K, V)) * sizeof(float);
 }
 
 inline void fc_bind(FcArgs &a, void *ck, void *ws) {
@@ -102,15 +103,15 @@ inline void fc_bind(FcArgs &a, void *ck, void *ws) {
     a.wn = a.nc;
     if (ws) {
         a.ds = static_cast<float *>(ws);
-        a.n = a.ds + n * fc_kp(a.s.K) * fc_kp(a.s.V);
+        a.sc = a.ds + n * fc_kp(a.s.K) * fc_kp(a.s.V);
     }
 }
 
-// The stages that both gate forms share: the state scan over the chunks (the
-// adjoint scan over the window when rev), out, and bprep over the window.
-void launch_fc_scan(const FcArgs &a, bool rev, hipStream_t stream);
+// The stages that both gate forms share: the state scan over the chunks, out, and
+// the adjoint scan over the window (with the score adjoint's coefficients).
+void launch_fc_scan(const FcArgs &a, hipStream_t stream);
 void launch_fc_out(const FcArgs &a, hipStream_t stream);
-void launch_fc_bprep(const FcArgs &a, hipStream_t stream);
+void launch_fc_adjoint(const FcArgs &a, hipStream_t stream);
 
 hipError_t launch_fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
 hipError_t launch_fc_bwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);

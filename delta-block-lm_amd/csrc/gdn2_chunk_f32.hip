@@ -27,19 +27,19 @@
 // score adjoints and carries the adjoints of F and G back through the products
 // that formed them, which is exact for zero gates too.
 //
-// Five kernels: prep (A, T, P, the map's factors; one wave per chunk), the scan
-// over the chunks of each (batch, head) (states and edits forward, state adjoints
-// in reverse), out, bprep (the adjoint map's additive term N) and bgrad (every
-// gradient; one wave per 16-channel tile).  All products are
-// v_mfma_f32_16x16x4f32 (exact f32 products) on operands read in their layout
-// (gdn2_chunk_f32_dev.h).
+// Five kernels: prep (A, T, P, the map's factors), the state scan over the chunks
+// of each (batch, head), out, the adjoint scan
+//   X <- diag(b_15) X + Qhat^T dO - W'^T (P^T dO + c delta + Ktil X)
+// and bgrad (every gradient); a wave takes one 16-channel tile of a chunk, or of a
+// head in the scans.  All products are v_mfma_f32_16x16x4f32 (exact f32 products)
+// on operands read in their layout (gdn2_chunk_f32_dev.h).
 //
 // Kernels of a forward + backward, against the LDS-tiled kernels before them
 // (f32 pair sums on the VALU; bf16 64 x 64 calls on bf16 hi/lo MFMA):
-//   f32 B8 T512 H4 K32 V64    82 us, was 141 (floor of its 43 MB 9 us)
-//   bf16 B16 T509 H8 64 x 64  275 us, was 366 (173 MB, 35 us)
-// A lone chunk per head (B1 T128 H4 K32 V64) takes 41 us, was 65: six launches
-// of 4 to 10 us.
+//   f32 B8 T512 H4 K32 V64    75 us, was 141 (floor of its 43 MB 9 us)
+//   bf16 B16 T509 H8 64 x 64  221 us, was 366 (173 MB, 35 us)
+// A lone sequence per head (B1 T128 H4 K32 V64) takes 34 us, was 65: five launches
+// of 4 to 9 us.  bgrad (92 us of the 221) moves 255 MB, 52 us of a copy's rate.
 #include "gdn2_chunk_f32_dev.h"
 
 #include <algorithm>
@@ -93,13 +93,13 @@ struct FcCol {
     __device__ __forceinline__ float ug8() const { return g >= 2 ? 1.f : x8; }   // lam = G8 ug8
 };
 
-// Gates of masked tokens: 1 on padding, 0 on a reset; NaN for a negative gate
-// where the call's contract asks for alpha >= 0.  code: 0 padding, 1 valid, 2 a
-// valid reset.
-__device__ __forceinline__ float fc_gate(float a, float code, int nonneg) {
-    a = (nonneg && a < 0.f) ? __builtin_nanf("") : a;
-    return code == 1.f ? a : (code == 0.f ? 1.f : 0.f);
+// The decay of a token from its gate: 1 on padding, 0 on a reset; NaN for a gate
+// below `least` (0 where the call's contract asks for alpha >= 0, else -inf).
+__device__ __forceinline__ float fc_gate(float a, bool live, float masked, float least) {
+    a = a < least ? __builtin_nanf("") : a;
+    return live ? a : masked;
 }
+__device__ __forceinline__ float fc_least(const FcArgs &a) { return a.nonneg ? 0.f : -__builtin_inff(); }
 
 template <int KM>
 struct FcGradSmem {
@@ -112,140 +112,142 @@ struct FcGradSmem {
 
 }  // namespace
 
-// ---- prep: gates, A, T, P and the factored map, one wave per chunk ----------------
-template <int KM, bool BF, bool VEC>
-__global__ void __launch_bounds__(64) fc_prep_kernel(FcArgs a) {
+// ---- prep: gates, A, T, P and the factored map ------------------------------------
+// Wave w takes key tile w (its terms of A and P, Ktil, Qhat and W') and value
+// tile w (U); blockDim is 64 max(KT, VT).  The terms of A meet in wave 0, which
+// inverts, and those of P in the last wave.  (One wave per chunk measured 50 us
+// where this takes 37 at 4096 chunks of 64 x 64: it holds 192 registers and waits
+// for one tile's reads after another.)
+struct FcPrepSmem {
+    f32x4 A[8][64], P[8][64];  // each key tile's terms, in acc layout
+    float la[C * FC_LA];
+    f32x4 t[64];
+    float ksq[8][C];
+};
+
+template <bool BF, bool VEC>
+__global__ void __launch_bounds__(512) fc_prep_kernel(FcArgs a) {
+    __shared__ FcPrepSmem sm;
     const SeqArgs &s = a.s;
     const int64_t ci = blockIdx.x;
     const int bh = blockIdx.x / a.nc, c = blockIdx.x % a.nc, b = bh / s.H, h = bh % s.H;
-    const int K = s.K, V = s.V, KP = fc_kp(K), KT = KP >> 4, VT = (V + 15) >> 4;
-    const int l = lane_id(), g = l >> 4, n = l & 15;
-    const bool o1 = n & 1, o2 = n & 2, o4 = n & 4;
-    const FcSrc<BF, VEC> sk(s.k, b, h, c, s.T, K), sq(s.q, b, h, c, s.T, K), sv(s.v, b, h, c, s.T, V);
-    const FcSrc<false, VEC> sa(s.alpha, b, h, c, s.T, K), se(s.erase, b, h, c, s.T, K), sw(s.write, b, h, c, s.T, V);
+    const int K = s.K, V = s.V, KT = fc_kp(K) >> 4, VT = (V + 15) >> 4, NW = blockDim.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id(), g = l >> 4, n = l & 15;
     bool on, rst;
     fc_flags(s, b, c, on, rst);
-    const float code = on ? (rst ? 2.f : 1.f) : 0.f;
-    const f32x4 code4 = fc_rows(code, g);
-    f32x4 A4 = zero4(), A8 = zero4(), P4 = zero4(), P8 = zero4(), be[KM];
-    float qa[6] = {}, qp[10] = {}, ksq = 0.f;  // pairs inside four tokens: (1,0) (2,0) (2,1) (3,0) (3,1) (3,2), then (a,a)
-    float *fk = a.fk + ci * C * KP, *fq = a.fq + ci * C * KP;
-#pragma unroll
-    for (int tau = 0; tau < KM; ++tau) {
-        be[tau] = zero4();
-        if (tau >= KT) continue;
-        const f32x4 kf = fc_keep(sk.frag(tau), on), qf = fc_keep(sq.frag(tau), on), ef = fc_keep(se.frag(tau), on);
-        const f32x4 af = sa.frag(tau);
-        f32x4 k = fc_keep4(sk.col(tau), code4), q = fc_keep4(sq.col(tau), code4), e = fc_keep4(se.col(tau), code4);
-        f32x4 al = sa.col(tau);
+    const bool live = on && !rst;
+    const float masked = on ? 0.f : 1.f, least = fc_least(a);
+    f32x4 u = zero4(), be = zero4();
+    if (w < VT)
+        u = FcSrc<BF, VEC>(s.v, b, h, c, s.T, V).col(w) * FcSrc<false, VEC>(s.write, b, h, c, s.T, V).col(w);
+    if (w < KT) {
+        const FcSrc<BF, VEC> sk(s.k, b, h, c, s.T, K), sq(s.q, b, h, c, s.T, K);
+        const FcSrc<false, VEC> sa(s.alpha, b, h, c, s.T, K), se(s.erase, b, h, c, s.T, K);
+        f32x4 kf = sk.frag(w), qf = sq.frag(w), ef = se.frag(w), af = sa.frag(w);
+        f32x4 k = sk.col(w), q = sq.col(w), e = se.col(w), al = sa.col(w);
+        const bool o1 = n & 1, o2 = n & 2, o4 = n & 4;
+        const f32x4 on4 = fc_rows(on ? 1.f : 0.f, g), live4 = fc_rows(live ? 1.f : 0.f, g);
+        kf = fc_keep(kf, on), qf = fc_keep(qf, on), ef = fc_keep(ef, on);
+        k = fc_keep4(k, on4), q = fc_keep4(q, on4), e = fc_keep4(e, on4);
         f32x4 e4, e8, q4, q8, k4, k8;
+        float ksq = 0.f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             ksq += kf[r] * kf[r];
-            const FcLevels x = fc_levels(fc_gate(af[r], code, a.nonneg), o1, o2, o4);
+            const FcLevels x = fc_levels(fc_gate(af[r], live, masked, least), o1, o2, o4);
             const float eh = ef[r] * kf[r];
             e4[r] = eh * x.f4, e8[r] = eh * x.f8;
             q4[r] = qf[r] * x.f4, q8[r] = qf[r] * x.f8;
             k4[r] = kf[r] * x.g4, k8[r] = kf[r] * x.g8;
-            al[r] = fc_gate(al[r], code4[r], a.nonneg);
+            al[r] = fc_gate(al[r], live4[r] != 0.f, 1.f - on4[r], least);
         }
-        A4 = fc_mma4(e4, k4, A4);
-        A8 = fc_mma4(e8, k8, A8);
-        P4 = fc_mma4(q4, k4, P4);
-        P8 = fc_mma4(q8, k8, P8);
-        const FcCol x(al, g);
+        const f32x4 A4 = fc_mma4(e4, k4, zero4()), A8 = fc_mma4(e8, k8, zero4());
+        const f32x4 P4 = fc_mma4(q4, k4, zero4()), P8 = fc_mma4(q8, k8, zero4());
+        ksq = fc_group_sum(ksq);
+        if (g == 0) sm.ksq[w][n] = ksq;
+        // the pairs inside the lane's four tokens, summed over the channels
+        const f32x4 eh = e * k;
         const float y10 = k[0] * al[1], y20 = y10 * al[2], y30 = y20 * al[3], y21 = k[1] * al[2], y31 = y21 * al[3],
                     y32 = k[2] * al[3];
-        const f32x4 eh = e * k;
-        qa[0] += eh[1] * y10, qa[1] += eh[2] * y20, qa[2] += eh[2] * y21;
-        qa[3] += eh[3] * y30, qa[4] += eh[3] * y31, qa[5] += eh[3] * y32;
-        qp[0] += q[1] * y10, qp[1] += q[2] * y20, qp[2] += q[2] * y21;
-        qp[3] += q[3] * y30, qp[4] += q[3] * y31, qp[5] += q[3] * y32;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) qp[6 + i] += q[i] * k[i];
-        const float bo = x.uf4() * x.uf8(), lo = x.ug4() * x.ug8();
-        const f32x4 bt = x.f4 * bo;
-        be[tau] = bt * eh;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            fk[(4 * g + i) * KP + 16 * tau + n] = x.g4[i] * lo * k[i];
-            fq[(4 * g + i) * KP + 16 * tau + n] = bt[i] * q[i];
-        }
-        if (g == 3) a.gv[ci * KP + 16 * tau + n] = 16 * tau + n < K ? bt[3] : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < 6; ++i) qa[i] = fc_row_sum(qa[i]);
-#pragma unroll
-    for (int i = 0; i < 10; ++i) qp[i] = fc_row_sum(qp[i]);
-    // rows t = 4 g + i, column s = n: the level by the quads of t and s
-    const int sq4 = n >> 2, sc = n & 3;
-    const bool diag = sq4 == g, near = sq4 < g && (sq4 >> 1) == (g >> 1), far = sq4 < g && !near;
-    f32x4 A, P;
-    {
-        const float a1[4] = {0.f, sc == 0 ? qa[0] : 0.f, sc == 0 ? qa[1] : (sc == 1 ? qa[2] : 0.f),
-                             sc == 0 ? qa[3] : (sc == 1 ? qa[4] : (sc == 2 ? qa[5] : 0.f))};
-        const float p1[4] = {sc == 0 ? qp[6] : 0.f, sc == 0 ? qp[0] : (sc == 1 ? qp[7] : 0.f),
-                             sc == 0 ? qp[1] : (sc == 1 ? qp[2] : (sc == 2 ? qp[8] : 0.f)),
-                             sc == 0 ? qp[3] : (sc == 1 ? qp[4] : (sc == 2 ? qp[5] : qp[9]))};
+        const float a10 = fc_row_sum(eh[1] * y10), a20 = fc_row_sum(eh[2] * y20), a21 = fc_row_sum(eh[2] * y21);
+        const float a30 = fc_row_sum(eh[3] * y30), a31 = fc_row_sum(eh[3] * y31), a32 = fc_row_sum(eh[3] * y32);
+        const float p10 = fc_row_sum(q[1] * y10), p20 = fc_row_sum(q[2] * y20), p21 = fc_row_sum(q[2] * y21);
+        const float p30 = fc_row_sum(q[3] * y30), p31 = fc_row_sum(q[3] * y31), p32 = fc_row_sum(q[3] * y32);
+        const float p00 = fc_row_sum(q[0] * k[0]), p11 = fc_row_sum(q[1] * k[1]), p22 = fc_row_sum(q[2] * k[2]),
+                    p33 = fc_row_sum(q[3] * k[3]);
+        // rows t = 4 g + i, column s = n: the level by the quads of t and s
+        const int sq4 = n >> 2, sc = n & 3;
+        const bool diag = sq4 == g, near = (sq4 < g) & ((sq4 >> 1) == (g >> 1)), far = (sq4 < g) & !near;
+        const bool c0 = sc == 0, c1 = sc == 1, c2 = sc == 2;
+        const f32x4 ad = {0.f, c0 ? a10 : 0.f, c0 ? a20 : (c1 ? a21 : 0.f), c0 ? a30 : (c1 ? a31 : (c2 ? a32 : 0.f))};
+        const f32x4 pd = {c0 ? p00 : 0.f, c0 ? p10 : (c1 ? p11 : 0.f), c0 ? p20 : (c1 ? p21 : (c2 ? p22 : 0.f)),
+                          c0 ? p30 : (c1 ? p31 : (c2 ? p32 : p33))};
+        f32x4 A, P;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            A[i] = diag ? a1[i] : (near ? A4[i] : (far ? A8[i] : 0.f));
-            P[i] = diag ? p1[i] : (near ? P4[i] : (far ? P8[i] : 0.f));
+            const float ax = far ? A8[i] : 0.f, px = far ? P8[i] : 0.f, ay = near ? A4[i] : ax, py = near ? P4[i] : px;
+            A[i] = diag ? ad[i] : ay;
+            P[i] = diag ? pd[i] : py;
         }
+        sm.A[w][l] = A;
+        sm.P[w][l] = P;
+        const FcCol x(al, g);
+        const f32x4 bt = x.f4 * (x.uf4() * x.uf8());
+        be = bt * eh;
+        fc_p4(a.fk + (ci * KT + w) * 256, 16 * l, x.g4 * (x.ug4() * x.ug8()) * k);
+        fc_p4(a.fq + (ci * KT + w) * 256, 16 * l, bt * q);
+        if (g == 3) *fc_at(a.gv + (ci * KT + w) * 16, 4 * n) = 16 * w + n < K ? bt[3] : 0.f;
     }
-    const f32x4 t = fc_inverse(A, g, n);
-    *reinterpret_cast<fc_u4 *>(a.tm + ci * C * C + n * C + 4 * g) = t;
-    fc_put_rows(a.pm + ci * C * C, P, g, n);
-    ksq = fc_group_sum(ksq);
-    if (g == 0)
-        *reinterpret_cast<fc_u4 *>(a.gb + (ci * C + n) * 8) = f32x4{on ? 1.f : 0.f, rst ? 1.f : 0.f, ksq, 0.f};
-#pragma unroll
-    for (int tau = 0; tau < KM; ++tau)
-        if (tau < KT) fc_put_w(a, ci, KP, tau, t, be[tau], g, n);
-    for (int vt = 0; vt < VT; ++vt) fc_put_u(a, ci, VT, vt, t, fc_keep4(sv.col(vt) * sw.col(vt), code4));
+    __syncthreads();
+    if (w == 0) {
+        f32x4 A = sm.A[0][l];
+        for (int x = 1; x < KT; ++x) A += sm.A[x][l];
+        const f32x4 t = fc_inverse(A, sm.la, g, n);
+        sm.t[l] = t;
+        fc_p4(a.tm + ci * C * C, (n * C + 4 * g) * 4, t);
+    }
+    if (w == NW - 1) {
+        f32x4 P = sm.P[0][l];
+        float ksq = sm.ksq[0][n];
+        for (int x = 1; x < KT; ++x) P += sm.P[x][l], ksq += sm.ksq[x][n];
+        FcOff(C).put(a.pm + ci * C * C, P);
+        if (g < 3) *fc_at(a.gb + ci * C * 8 + C * g, 4 * n) = g == 0 ? (on ? 1.f : 0.f) : (g == 1 ? (rst ? 1.f : 0.f) : ksq);
+    }
+    __syncthreads();
+    const f32x4 t = sm.t[l];
+    if (w < KT) fc_p4(a.fw + (ci * KT + w) * 256, 16 * l, fc_mma4(t, be, zero4()));
+    if (w < VT)
+        fc_p4(a.fu + (ci * VT + w) * 256, 16 * l, fc_mma4(t, fc_keep4(u, fc_rows(on ? 1.f : 0.f, g)), zero4()));
 }
 
-// ---- the scan over the chunks of one (batch, head) -----------------------------
+// ---- the scans over the chunks of one (batch, head) -----------------------------
 // One workgroup per (batch, head, 16 value columns j = 16 cg + l % 16), one wave
-// per 16-row key tile tau = w, on v_mfma_f32_16x16x4f32 (exact f32 products).
-// Wave tau holds its tile of the state in the accumulator layout: lane l
-// (g = l / 16, n = l % 16) holds S[16 tau + 4 g + r][j] in register r.
-// Per chunk, forward:  v = U - W' S,          S <- diag(gv) S + Ktil^T v
-//            reverse:  v = Ktil X,            X <- diag(gv) X + N - W'^T v
-// v sums over the key axis: each wave forms its tile's part (four k = 4 MFMA
-// steps whose k-slice {4 g + s} makes register s of the lane's own accumulator
+// per 16-row key tile tau = w.  Wave tau holds its tile of the state in the
+// accumulator layout: lane l (g = l / 16, n = l % 16) holds S[16 tau + 4 g + r][j]
+// in register r.  Per chunk,
+//   forward:  v = U - W' S,                  S <- diag(gv) S + Ktil^T v
+//   reverse:  v = P^T dO + c delta + Ktil X,  X <- diag(gv) X + Qhat^T dO - W'^T v
+// v sums over the key axis: each wave forms its tile's part (the accumulator is
 // the B operand), the parts meet in LDS (double-buffered by step parity, one
-// barrier per step) and every wave adds them in tile order, so all waves hold
-// the same v; each then updates its own tile, v's accumulator rows as the B
-// operand.  The A operands (W' or Ktil rows, gv, the lane-packed U or N) are
-// read from global memory into registers D chunks ahead.
-template <int KT>
+// barrier per step) and every wave adds them in tile order, so all waves hold the
+// same v; each then updates its own tile, v's accumulator rows as the B operand.
+// The other operands are read from global memory into registers D chunks ahead.
+// The scans are bound by the bytes they stream (at 128 heads of 64 x 64, 28 KiB
+// per chunk forward, 4.1 TB/s).  An additive term N of the adjoint map, formed by
+// a kernel of its own, cost 16 KiB written and read per chunk: that kernel and the
+// scan took 27 and 42 us where the scan with the products inside takes 46.
+template <bool REV>
 struct FcScanOps {
-    fc_u4 w, g, a;   // A operands (token n, keys 16 tau + 4 g ..), gv rows, U or N rows
-    float k[4];      // A operands (tokens 4 g + s, key 16 tau + n)
+    f32x4 w;           // A operand, tokens n, keys 16 tau + 4 g ..: W' or Ktil across
+    f32x4 g, k, a;     // gv rows; Ktil or W', A operand over the tokens; U or Qhat
+    f32x4 d, p;        // reverse: dO columns j, P rows
+    f32x4 on;
 };
-
-template <int KT, bool REV>
-__device__ __forceinline__ void fc_scan_load(const FcArgs &a, int64_t ci, int64_t wi, int cg, int VT, int tau,
-                                             FcScanOps<KT> &o) {
-    // Every load is issued (past the value tiles the lanes read tile 0, their
-    // values unused), so no load sits behind a branch and the compiler's
-    // memory-counter waits stay exact across the prefetch ring.
-    constexpr int KP = 16 * KT;
-    const int l = lane_id(), g = l >> 4, n = l & 15, cc = cg < VT ? cg : 0;
-    const float *fw = a.fw + ci * C * KP, *fk = a.fk + ci * C * KP;
-    const float *rw = REV ? fk : fw, *ck = REV ? fw : fk;
-    o.w = *reinterpret_cast<const fc_u4 *>(&rw[n * KP + 16 * tau + 4 * g]);
-    o.g = *reinterpret_cast<const fc_u4 *>(&a.gv[ci * KP + 16 * tau + 4 * g]);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) o.k[s] = ck[(4 * g + s) * KP + 16 * tau + n];
-    o.a = REV ? *reinterpret_cast<const fc_u4 *>(&a.n[(((wi * VT + cc) * KT + tau) * 64 + l) * 4])
-              : *reinterpret_cast<const fc_u4 *>(&a.fu[((ci * VT + cc) * 64 + l) * 4]);
-}
 
 // The workgroups of one (batch, head) read the same factors, so they take block
 // indices of one residue mod 8 and share an XCD's L2.
-template <int KT, bool REV>
+// SC: with a score adjoint.
+template <int KT, bool REV, bool BF, bool VEC, bool SC>
 __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
     __shared__ float4 vpart[2][KT][64];  // each wave's part of v, by step parity
     const SeqArgs &s = a.s;
@@ -255,13 +257,13 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
     if (bh >= s.B * s.H) return;
     const int b = bh / s.H, h = bh % s.H;
     const int l = lane_id(), g = l >> 4, n = l & 15, j = 16 * cg + n;
-    const bool jv = j < V;
+    const bool jv = j < V, has_do = REV && s.dout.data != nullptr;
+    const View dov = has_do ? s.dout : s.v;  // a missing dO reads v, zeroed where it is used
     const int steps = REV ? a.wn : a.nc;
-    const int64_t co = (((int64_t)bh * VT + cg) * KT + tau) * 64 + l;  // this lane's piece of the carry
+    float *carry = a.carry + (((int64_t)bh * VT + cg) * KT + tau) * 256;
     f32x4 X;
     if (REV && a.w0 + a.wn < a.nc) {
-        const fc_u4 x = *reinterpret_cast<const fc_u4 *>(&a.carry[co * 4]);
-        X = f32x4{x.x, x.y, x.z, x.w};
+        X = fc_g4(carry, 16 * l);
     } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -275,71 +277,107 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
         }
     }
     // A ring of D chunks' operands in registers: chunk step + D is loaded (the
-    // last chunk again past the end) as soon as step's operands are used.
+    // last chunk again past the end) as soon as step's operands are used.  No load
+    // sits behind a branch that lanes or steps take differently.
     constexpr int D = 4;
-    FcScanOps<KT> ring[D];
+    FcScanOps<REV> ring[D];
     auto chunk_at = [&](int step) {  // within the window (forward: all chunks)
         const int sc = step < steps ? step : steps - 1;
         return REV ? steps - 1 - sc : sc;
     };
-    auto load = [&](int step, FcScanOps<KT> &o) {
-        const int cw = chunk_at(step);
-        fc_scan_load<KT, REV>(a, (int64_t)bh * a.nc + (REV ? a.w0 : 0) + cw, (int64_t)bh * a.wn + cw, cg, VT, tau, o);
-    };
-#pragma unroll
-    for (int d = 0; d < D; ++d) load(d, ring[d]);
-    float *keep = REV ? a.ds : a.st;
-    for (int s0 = 0; s0 < steps; s0 += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const int step = s0 + d;
-            if (step >= steps) break;
-            const int64_t ci = (int64_t)bh * (REV ? a.wn : a.nc) + chunk_at(step);
-            const FcScanOps<KT> &cur = ring[d];
-            // the state before (forward) / the adjoint after (reverse) this chunk
-            {
-                float kx[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) kx[r] = (16 * tau + 4 * g + r < K && jv) ? X[r] : 0.f;
-                *reinterpret_cast<fc_u4 *>(&keep[(((ci * VT + cg) * KT + tau) * 64 + l) * 4]) =
-                    fc_u4{kx[0], kx[1], kx[2], kx[3]};
-            }
-            // this tile's part of v[t][j], t = 4 g + r: -W' S (+ U in tile 0) or Ktil X
-            f32x4 vp = (!REV && tau == 0) ? f32x4{cur.a.x, cur.a.y, cur.a.z, cur.a.w} : zero4();
-            const float wq[4] = {cur.w.x, cur.w.y, cur.w.z, cur.w.w};
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                vp = __builtin_amdgcn_mfma_f32_16x16x4f32(REV ? wq[q] : -wq[q], X[q], vp, 0, 0, 0);
-            f32x4 v = vp;
-            if (KT > 1) {
-                const int par = step & 1;
-                vpart[par][tau][l] = make_float4(vp[0], vp[1], vp[2], vp[3]);
-                __syncthreads();
-                float4 t0 = vpart[par][0][l];
-                v = f32x4{t0.x, t0.y, t0.z, t0.w};
-#pragma unroll
-                for (int u = 1; u < KT; ++u) {
-                    const float4 t = vpart[par][u][l];
-                    v += f32x4{t.x, t.y, t.z, t.w};
-                }
-            }
-            if (!REV && tau == 0)  // v is the chunk's edits delta: where U was, in U's layout
-                *reinterpret_cast<fc_u4 *>(&a.fu[((ci * VT + cg) * 64 + l) * 4]) = fc_u4{v[0], v[1], v[2], v[3]};
-            // S <- diag(gv) S + Ktil^T v, or X <- diag(gv) X + N - W'^T v
-            const float gq[4] = {cur.g.x, cur.g.y, cur.g.z, cur.g.w};
-            const float an[4] = {cur.a.x, cur.a.y, cur.a.z, cur.a.w};
-            f32x4 x;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) x[r] = gq[r] * X[r] + (REV ? an[r] : 0.f);
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                x = __builtin_amdgcn_mfma_f32_16x16x4f32(REV ? -cur.k[q] : cur.k[q], v[q], x, 0, 0, 0);
-            X = x;
-            load(step + D, ring[d]);
+    const FcOff oc(C);
+    auto load = [&](int step, FcScanOps<REV> &o) {
+        const int c = (REV ? a.w0 : 0) + chunk_at(step);
+        const int64_t ci = (int64_t)bh * a.nc + c;
+        const float *fw = a.fw + (ci * KT + tau) * 256, *fk = a.fk + (ci * KT + tau) * 256;
+        o.w = fc_across(REV ? fk : fw);
+        o.g = fc_g4(a.gv + (ci * KT + tau) * 16, 16 * g);
+        o.k = fc_g4(REV ? fw : fk, 16 * l);
+        o.a = fc_g4(REV ? a.fq + (ci * KT + tau) * 256 : a.fu + (ci * VT + cg) * 256, 16 * l);
+        if (REV) {
+            o.d = FcSrc<BF, VEC>(dov, b, h, c, s.T, V).col(cg);
+            o.p = oc.get(a.pm + ci * C * C);
+            o.on = fc_gb4(a, ci, 0);
         }
+    };
+    // The loads are issued in ring order, the order in which the steps wait for
+    // them: a wait at the loop's head must not cover the whole ring because the
+    // scheduler put the first chunk's loads last.
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        load(d, ring[d]);
+        __builtin_amdgcn_sched_barrier(0);
     }
+    // A step's masked dO and, in tile 0, the terms of v known before X: U, or P^T dO
+    // + c delta.
+    f32x4 dnext = zero4(), base = zero4();
+    auto prepare = [&](int step, const FcScanOps<REV> &o) {
+        if (!REV) {
+            base = o.a;
+            return;
+        }
+        dnext = fc_keep(fc_keep4(o.d, o.on), has_do);
+        if (tau != 0) return;
+        base = zero4();
+        if (SC) {
+            const int cw = chunk_at(step);
+            base = fc_g4(a.sc + ((int64_t)bh * a.wn + cw) * 2 * C, 16 * g) *
+                   fc_g4(a.fu + (((int64_t)bh * a.nc + a.w0 + cw) * VT + cg) * 256, 16 * l);
+        }
+        base = fc_mma4(o.p, dnext, base);
+    };
+    prepare(0, ring[0]);
+    float *keep = REV ? a.ds : a.st;
+    auto advance = [&](int step, int d) __attribute__((always_inline)) {
+        const int cw = chunk_at(step);
+        const int64_t ci = (int64_t)bh * a.nc + (REV ? a.w0 : 0) + cw, wi = (int64_t)bh * (REV ? a.wn : a.nc) + cw;
+        const FcScanOps<REV> &cur = ring[d];
+        const f32x4 dnow = dnext;
+        // The state before (forward) / the adjoint after (reverse) this chunk; zero
+        // outside K x V, as X0 and every term of the map are.
+        fc_p4(keep + ((wi * VT + cg) * KT + tau) * 256, 16 * l, X);
+        // this tile's part of v[t][j], t = 4 g + r: -W' S (+ U in tile 0), or
+        // Ktil X (+ the step's base in tile 0).  The four-step products that
+        // wait for X or v run as two chains of two.
+        const f32x4 wm = REV ? cur.w : -cur.w;
+        f32x4 vp = fc_mma(wm[1], X[1], fc_mma(wm[0], X[0], tau == 0 ? base : zero4()));
+        vp += fc_mma(wm[3], X[3], fc_mma(wm[2], X[2], zero4()));
+        const int par = step & 1;
+        if (KT > 1) vpart[par][tau][l] = make_float4(vp[0], vp[1], vp[2], vp[3]);
+        // in the shadow of the exchange: what depends on neither X nor v
+        f32x4 x = cur.g * X, v = vp;
+        if (REV) x = fc_mma4(cur.a, dnow, x);
+        prepare(step + 1, ring[(d + 1) % D]);
+        if (KT > 1) {
+            __syncthreads();
+            float4 t0 = vpart[par][0][l];
+            v = f32x4{t0.x, t0.y, t0.z, t0.w};
+#pragma unroll
+            for (int u = 1; u < KT; ++u) {
+                const float4 t = vpart[par][u][l];
+                v += f32x4{t.x, t.y, t.z, t.w};
+            }
+        }
+        // forward: v is the chunk's edits delta, kept where U was
+        if (!REV && tau == 0) fc_p4(a.fu + (ci * VT + cg) * 256, 16 * l, v);
+        const f32x4 km = REV ? -cur.k : cur.k;
+        x = fc_mma(km[1], v[1], fc_mma(km[0], v[0], x));
+        X = x + fc_mma(km[3], v[3], fc_mma(km[2], v[2], zero4()));
+        __builtin_amdgcn_sched_barrier(0);
+        load(step + D, ring[d]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Whole rounds of the ring, then what is left: a round with exits between its
+    // steps would make every wait at its head cover the whole ring.
+    int s0 = 0;
+    for (; s0 + D <= steps; s0 += D)
+#pragma unroll
+        for (int d = 0; d < D; ++d) advance(s0 + d, d);
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+        if (s0 + d < steps) advance(s0 + d, d);
     if (REV && a.w0 > 0) {
-        *reinterpret_cast<fc_u4 *>(&a.carry[co * 4]) = fc_u4{X[0], X[1], X[2], X[3]};
+        fc_p4(carry, 16 * l, X);
         return;
     }
     float *fin = REV ? s.dinitial : s.final_state;
@@ -351,25 +389,28 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
         }
 }
 
-template <int KT>
-static void launch_fc_scan_kt(const FcArgs &a, bool rev, hipStream_t stream) {
-    const int bh = a.s.B * a.s.H, VT = (a.s.V + 15) / 16;
-    const dim3 grid(8 * VT * ((bh + 7) / 8)), block(64 * KT);
-    if (rev) hipLaunchKernelGGL((fc_scan_kernel<KT, true>), grid, block, 0, stream, a);
-    else hipLaunchKernelGGL((fc_scan_kernel<KT, false>), grid, block, 0, stream, a);
-}
-
-void launch_fc_scan(const FcArgs &a, bool rev, hipStream_t stream) {
-    switch (fc_kp(a.s.K) / 16) {
-        case 1: launch_fc_scan_kt<1>(a, rev, stream); break;
-        case 2: launch_fc_scan_kt<2>(a, rev, stream); break;
-        case 3: launch_fc_scan_kt<3>(a, rev, stream); break;
-        case 4: launch_fc_scan_kt<4>(a, rev, stream); break;
-        case 5: launch_fc_scan_kt<5>(a, rev, stream); break;
-        case 6: launch_fc_scan_kt<6>(a, rev, stream); break;
-        case 7: launch_fc_scan_kt<7>(a, rev, stream); break;
-        default: launch_fc_scan_kt<8>(a, rev, stream); break;
+// The score adjoint's coefficients per token, one wave per chunk: c = dscore |k| /
+// |delta| and c' = dscore |delta| / |k| (zero at a zero edit or key).
+__global__ void __launch_bounds__(64) fc_score_kernel(FcArgs a) {
+    const SeqArgs &s = a.s;
+    const int bh = blockIdx.x / a.wn, c = a.w0 + blockIdx.x % a.wn, VT = (s.V + 15) >> 4;
+    const int64_t ci = (int64_t)bh * a.nc + c, wi = blockIdx.x;
+    const int l = lane_id(), n = l & 15, tg = c * C + n;
+    f32x4 d2 = zero4();
+    for (int vt = 0; vt < VT; ++vt) {
+        const f32x4 d = fc_g4(a.fu + (ci * VT + vt) * 256, 16 * l);
+        d2 += d * d;
     }
+    float dsq = 0.f;  // token n's sum sits in group n / 4, register n % 4
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float x = __shfl(fc_row_sum(d2[i]), 16 * (n >> 2));
+        if ((n & 3) == i) dsq = x;
+    }
+    const float nk = sqrtf(fc_gb(a, ci, 2)), nd = sqrtf(dsq);
+    const float dsc = tg < s.T ? s.dscores[((int64_t)(bh / s.H) * s.T + tg) * s.H + bh % s.H] : 0.f;
+    const bool ok = fc_gb(a, ci, 0) != 0.f && nk > 0.f && nd > 0.f;
+    if (l < 2 * C) *fc_at(a.sc + wi * 2 * C, 4 * l) = !ok ? 0.f : (l < C ? dsc * nk / nd : dsc * nd / nk);
 }
 
 // ---- out: O = Qhat S0 + P delta and the scores, one wave per value tile -----------
@@ -379,22 +420,22 @@ __global__ void __launch_bounds__(512) fc_out_kernel(FcArgs a) {
     const SeqArgs &s = a.s;
     const int64_t ci = blockIdx.x;
     const int bh = blockIdx.x / a.nc, c = blockIdx.x % a.nc, b = bh / s.H, h = bh % s.H;
-    const int K = s.K, V = s.V, KP = fc_kp(K), KT = KP >> 4, VT = (V + 15) >> 4;
-    const int vt = threadIdx.x >> 6, l = lane_id(), g = l >> 4, n = l & 15;
-    const float *fq = a.fq + ci * C * KP + n * KP + 4 * g, *st = a.st + (ci * VT + vt) * KT * 256 + 4 * l;
+    const int K = s.K, V = s.V, KT = fc_kp(K) >> 4, VT = (V + 15) >> 4;
+    const int vt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id(), g = l >> 4, n = l & 15;
+    const float *fq = a.fq + ci * KT * 256, *st = a.st + (ci * VT + vt) * KT * 256;
     f32x4 q[KM], s0[KM];
 #pragma unroll
     for (int tau = 0; tau < KM; ++tau) {
         q[tau] = s0[tau] = zero4();
-        if (tau < KT) q[tau] = fc_g4(fq + 16 * tau), s0[tau] = fc_g4(st + 256 * tau);
+        if (tau < KT) q[tau] = fc_across(fq + 256 * tau), s0[tau] = fc_g4(st + 256 * tau, 16 * l);
     }
-    const f32x4 p = fc_g4(a.pm + ci * C * C + n * C + 4 * g), dl = fc_g4(a.fu + (ci * VT + vt) * 256 + 4 * l);
-    const f32x4 gb = fc_g4(a.gb + (ci * C + n) * 8);
+    const f32x4 p = fc_g4(a.pm + ci * C * C, (n * C + 4 * g) * 4), dl = fc_g4(a.fu + (ci * VT + vt) * 256, 16 * l);
+    const f32x4 on4 = fc_gb4(a, ci, 0);
     f32x4 o = zero4();
 #pragma unroll
     for (int tau = 0; tau < KM; ++tau) o = fc_mma4(q[tau], s0[tau], o);
     o = fc_mma4(p, dl, o);
-    fc_put<false, VEC>(s.out, s.out_bf16, s, b, h, c, V, vt, fc_keep4(o, fc_rows(gb[0], g)));
+    fc_put<false, VEC>(s.out, s.out_bf16, s, b, h, c, V, vt, fc_keep4(o, on4));
     if (!s.scores) return;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -405,40 +446,8 @@ __global__ void __launch_bounds__(512) fc_out_kernel(FcArgs a) {
     if (threadIdx.x < C && c * C + n < s.T) {
         float x = 0.f;
         for (int v = 0; v < VT; ++v) x += dd[v][n];
-        s.scores[((int64_t)b * s.T + c * C + n) * s.H + h] = gb[0] != 0.f ? sqrtf(gb[2] * x) : 0.f;
+        s.scores[((int64_t)b * s.T + c * C + n) * s.H + h] = fc_gb(a, ci, 0) != 0.f ? sqrtf(fc_gb(a, ci, 2) * x) : 0.f;
     }
-}
-
-// ---- bprep: N = Qhat^T dO - W'^T X, X = P^T dO + c delta, one wave per value tile
-template <int KM, bool BF, bool VEC>
-__global__ void __launch_bounds__(512) fc_bprep_kernel(FcArgs a) {
-    const SeqArgs &s = a.s;
-    const int bh = blockIdx.x / a.wn, cw = blockIdx.x % a.wn, c = a.w0 + cw, b = bh / s.H, h = bh % s.H;
-    const int64_t ci = (int64_t)bh * a.nc + c, wi = blockIdx.x;
-    const int K = s.K, V = s.V, KP = fc_kp(K), KT = KP >> 4, VT = (V + 15) >> 4;
-    const int vt = threadIdx.x >> 6, l = lane_id(), g = l >> 4, n = l & 15;
-    const float *fq = a.fq + ci * C * KP, *fw = a.fw + ci * C * KP;
-    const f32x4 gb = fc_g4(a.gb + (ci * C + n) * 8), p = fc_get_rows(a.pm + ci * C * C, g, n);
-    f32x4 q[KM], w[KM], dO = zero4();
-    if (s.dout.data) dO = FcSrc<BF, VEC>(s.dout, b, h, c, s.T, V).col(vt);
-#pragma unroll
-    for (int tau = 0; tau < KM; ++tau) {
-        q[tau] = w[tau] = zero4();
-        if (tau < KT) q[tau] = fc_get_col(fq, KP, tau, g, n), w[tau] = fc_get_col(fw, KP, tau, g, n);
-    }
-    dO = fc_keep4(dO, fc_rows(gb[0], g));
-    f32x4 x = zero4();
-    if (s.dscores) {
-        float cs, ck;
-        fc_score_adj(a, ci, b, h, c, VT, gb[0] != 0.f, gb[2], cs, ck);
-        x = fc_rows(cs, g) * fc_g4(a.fu + (ci * VT + vt) * 256 + 4 * l);
-    }
-    x = -fc_mma4(p, dO, x);
-#pragma unroll
-    for (int tau = 0; tau < KM; ++tau)
-        if (tau < KT)
-            *reinterpret_cast<fc_u4 *>(a.n + ((wi * VT + vt) * KT + tau) * 256 + 4 * l) =
-                fc_mma4(w[tau], x, fc_mma4(q[tau], dO, zero4()));
 }
 
 // ---- bgrad: every gradient of one chunk -----------------------------------------
@@ -461,29 +470,29 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fc_bgrad_kernel(FcAr
     const SeqArgs &s = a.s;
     const int64_t ci = blockIdx.x;
     const int bh = blockIdx.x / a.nc, c = blockIdx.x % a.nc, b = bh / s.H, h = bh % s.H;
-    const int K = s.K, V = s.V, KP = fc_kp(K), KT = KP >> 4, VT = (V + 15) >> 4, NW = blockDim.x >> 6;
-    const int w = threadIdx.x >> 6, l = lane_id(), g = l >> 4, n = l & 15;
+    const int K = s.K, V = s.V, KT = fc_kp(K) >> 4, VT = (V + 15) >> 4, NW = blockDim.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id(), g = l >> 4, n = l & 15;
     const FcSrc<BF, VEC> sdo(s.dout, b, h, c, s.T, V);
     const bool has_do = s.dout.data != nullptr;
-    const f32x4 gb = fc_g4(a.gb + (ci * C + n) * 8);
-    const bool on = gb[0] != 0.f;
-    const f32x4 on4 = fc_rows(gb[0], g);
-    float cs = 0.f, ck = 0.f;
-    if (s.dscores) fc_score_adj(a, ci, b, h, c, VT, on, gb[2], cs, ck);
+    const bool on = fc_gb(a, ci, 0) != 0.f;
+    const f32x4 on4 = fc_gb4(a, ci, 0), rst4 = fc_gb4(a, ci, 1);
+    f32x4 cs4 = zero4(), ck4 = zero4();
+    if (s.dscores) cs4 = fc_g4(a.sc + ci * 2 * C, 16 * g), ck4 = fc_g4(a.sc + ci * 2 * C + C, 16 * g);
     const float *st = a.st + ci * KT * VT * 256, *ds = a.ds + ci * KT * VT * 256;
     if (w < VT) {  // ddelta and dR of value tile w
-        const f32x4 p = fc_get_rows(a.pm + ci * C * C, g, n), tb = fc_get_rows(a.tm + ci * C * C, g, n);
-        const f32x4 dl = fc_g4(a.fu + (ci * VT + w) * 256 + 4 * l);
+        const FcOff oc(C);
+        const f32x4 p = oc.get(a.pm + ci * C * C), tb = oc.get(a.tm + ci * C * C);
+        const f32x4 dl = fc_g4(a.fu + (ci * VT + w) * 256, 16 * l);
         const f32x4 v = FcSrc<BF, VEC>(s.v, b, h, c, s.T, V).col(w), wr = FcSrc<false, VEC>(s.write, b, h, c, s.T, V).col(w);
         f32x4 dO = has_do ? sdo.col(w) : zero4(), kf[KM], dsn[KM];
-        const float *fk = a.fk + ci * C * KP + n * KP + 4 * g;
+        const float *fk = a.fk + ci * KT * 256;
 #pragma unroll
         for (int tau = 0; tau < KM; ++tau) {
             kf[tau] = dsn[tau] = zero4();
-            if (tau < KT) kf[tau] = fc_g4(fk + 16 * tau), dsn[tau] = fc_g4(ds + (w * KT + tau) * 256 + 4 * l);
+            if (tau < KT) kf[tau] = fc_across(fk + 256 * tau), dsn[tau] = fc_g4(ds + (w * KT + tau) * 256, 16 * l);
         }
         dO = fc_keep4(dO, on4);
-        f32x4 dd = fc_mma4(p, dO, fc_rows(cs, g) * dl);
+        f32x4 dd = fc_mma4(p, dO, cs4 * dl);
 #pragma unroll
         for (int tau = 0; tau < KM; ++tau) dd = fc_mma4(kf[tau], dsn[tau], dd);
         const f32x4 dr = fc_mma4(tb, dd, zero4());                                           // rows t, column j
@@ -528,7 +537,7 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fc_bgrad_kernel(FcAr
 #pragma unroll
         for (int vt = 0; vt < KM; ++vt)
             if (vt < VT) {
-                const f32x4 s0 = fc_get_across(st, KT, w, vt, g, n), d1 = fc_get_across(ds, KT, w, vt, g, n);
+                const f32x4 s0 = fc_across(st + (vt * KT + w) * 256), d1 = fc_across(ds + (vt * KT + w) * 256);
                 const f32x4 d = *reinterpret_cast<const f32x4 *>(&sm.dl[n * LD + 16 * vt + 4 * g]);
                 const f32x4 r = *reinterpret_cast<const f32x4 *>(&sm.dr[n * LD + 16 * vt + 4 * g]);
                 Qg = fc_mma4(yf[vt], s0, Qg);
@@ -541,12 +550,11 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fc_bgrad_kernel(FcAr
     }
     __syncthreads();
     if (w >= KT) return;
-    const f32x4 rst4 = fc_rows(gb[1], g), ck4 = fc_rows(ck, g);
     k = fc_keep4(k, on4);
     q = fc_keep4(q, on4);
     e = fc_keep4(e, on4);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) al[i] = fc_gate(al[i], on4[i] + rst4[i], a.nonneg);
+    for (int i = 0; i < 4; ++i) al[i] = fc_gate(al[i], on4[i] > rst4[i], 1.f - on4[i], fc_least(a));
     const f32x4 eh = e * k;
     const FcCol x(al, g);
     const f32x4 f8 = x.f4 * x.uf4(), g8 = x.g4 * x.ug4();
@@ -633,14 +641,10 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fc_bgrad_kernel(FcAr
 }
 
 // ---- launches -------------------------------------------------------------------
-template <int KM, bool BF, bool VEC>
+template <bool BF, bool VEC>
 static void fc_prep(const FcArgs &a, hipStream_t stream) {
-    hipLaunchKernelGGL((fc_prep_kernel<KM, BF, VEC>), dim3(a.s.B * a.s.H * a.nc), dim3(64), 0, stream, a);
-}
-template <int KM, bool BF, bool VEC>
-static void fc_bprep(const FcArgs &a, hipStream_t stream) {
-    hipLaunchKernelGGL((fc_bprep_kernel<KM, BF, VEC>), dim3(a.s.B * a.s.H * a.wn), dim3(64 * ((a.s.V + 15) / 16)), 0,
-                       stream, a);
+    const int KT = fc_kp(a.s.K) / 16, VT = (a.s.V + 15) / 16;
+    hipLaunchKernelGGL((fc_prep_kernel<BF, VEC>), dim3(a.s.B * a.s.H * a.nc), dim3(64 * std::max(KT, VT)), 0, stream, a);
 }
 template <int KM, bool BF, bool VEC>
 static void fc_bgrad(const FcArgs &a, hipStream_t stream) {
@@ -662,14 +666,52 @@ void launch_fc_out(const FcArgs &a, hipStream_t stream) {
     else fc_out<8>(a, stream);
 }
 
-void launch_fc_bprep(const FcArgs &a, hipStream_t stream) { FC_DISPATCH(fc_kp(a.s.K) / 16, fc_bprep, a, stream); }
+template <bool REV, bool BF, bool VEC, bool SC>
+static void fc_scan(const FcArgs &a, hipStream_t stream) {
+    const int bh = a.s.B * a.s.H, VT = (a.s.V + 15) / 16, KT = fc_kp(a.s.K) / 16;
+    const dim3 grid(8 * VT * ((bh + 7) / 8)), block(64 * KT);
+#define FC_SCAN(N)                                                                                        \
+    case N: hipLaunchKernelGGL((fc_scan_kernel<N, REV, BF, VEC, SC>), grid, block, 0, stream, a); break
+    switch (KT) {
+        FC_SCAN(1);
+        FC_SCAN(2);
+        FC_SCAN(3);
+        FC_SCAN(4);
+        FC_SCAN(5);
+        FC_SCAN(6);
+        FC_SCAN(7);
+        FC_SCAN(8);
+    }
+#undef FC_SCAN
+}
+
+void launch_fc_scan(const FcArgs &a, hipStream_t stream) { fc_scan<false, false, false, false>(a, stream); }
+
+void launch_fc_adjoint(const FcArgs &a, hipStream_t stream) {
+    if (a.s.dscores) {  // the reads of any layout only
+        hipLaunchKernelGGL(fc_score_kernel, dim3(a.s.B * a.s.H * a.wn), dim3(64), 0, stream, a);
+        if (a.in_bf16) fc_scan<true, true, false, true>(a, stream);
+        else fc_scan<true, false, false, true>(a, stream);
+    } else if (a.in_bf16 && a.vec) {
+        fc_scan<true, true, true, false>(a, stream);
+    } else if (a.in_bf16) {
+        fc_scan<true, true, false, false>(a, stream);
+    } else if (a.vec) {
+        fc_scan<true, false, true, false>(a, stream);
+    } else {
+        fc_scan<true, false, false, false>(a, stream);
+    }
+}
 
 hipError_t launch_fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev) {
     fc_mark(ev, 0, stream);
-    FC_DISPATCH(fc_kp(a.s.K) / 16, fc_prep, a, stream);
+    if (a.in_bf16 && a.vec) fc_prep<true, true>(a, stream);
+    else if (a.in_bf16) fc_prep<true, false>(a, stream);
+    else if (a.vec) fc_prep<false, true>(a, stream);
+    else fc_prep<false, false>(a, stream);
     fc_mark(ev, 1, stream);
     fc_mark(ev, 2, stream);
-    launch_fc_scan(a, false, stream);
+    launch_fc_scan(a, stream);
     fc_mark(ev, 3, stream);
     fc_mark(ev, 4, stream);
     launch_fc_out(a, stream);
@@ -678,11 +720,10 @@ hipError_t launch_fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *
 }
 
 hipError_t launch_fc_bwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev) {
-    fc_mark(ev, 0, stream);
-    launch_fc_bprep(a, stream);
+    fc_mark(ev, 0, stream);  // no prep stage: the adjoint scan forms its map's terms
     fc_mark(ev, 1, stream);
     fc_mark(ev, 2, stream);
-    launch_fc_scan(a, true, stream);
+    launch_fc_adjoint(a, stream);
     fc_mark(ev, 3, stream);
     fc_mark(ev, 4, stream);
     FC_DISPATCH(std::max(fc_kp(a.s.K), (a.s.V + 15) & ~15) / 16, fc_bgrad, a, stream);

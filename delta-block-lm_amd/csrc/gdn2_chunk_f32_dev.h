@@ -11,7 +11,8 @@
 //   acc   rows 4 g + i, column n (the accumulator); register i is also an A or B
 //         operand whose reduction slice is {4 g + i}, so products chain in
 //         registers, and a [token][channel] accumulator has the layout of a col
-// A tile-packed state (a 16-byte piece per lane) is a B operand as it is loaded.
+// A packed tile (the col or acc registers as one 16-byte piece per lane, 1 KiB) is
+// read back the same way in one load, or across (fc_across) as a frag in four.
 #pragma once
 
 #include "gdn2_chunk_f32.h"
@@ -26,7 +27,7 @@ constexpr int C = FC_C;
 template <int CTRL>
 __device__ __forceinline__ float fc_dpp(float x) {
     return __builtin_bit_cast(
-        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, true));
 }
 // Sum over the 16 lanes n of a lane group, in all of them.
 __device__ __forceinline__ float fc_row_sum(float x) {
@@ -61,7 +62,39 @@ __device__ __forceinline__ f32x4 fc_keep4(f32x4 x, const f32x4 &on) {
     for (int i = 0; i < 4; ++i) x[i] = on[i] != 0.f ? x[i] : 0.f;
     return x;
 }
-__device__ __forceinline__ f32x4 fc_g4(const float *p) { return *reinterpret_cast<const fc_u4 *>(p); }
+// Accesses at a 32-bit byte offset from a uniform base: one instruction, with the
+// base in scalar registers.
+__device__ __forceinline__ const float *fc_at(const float *p, uint32_t bytes) {
+    return reinterpret_cast<const float *>(reinterpret_cast<const char *>(p) + bytes);
+}
+__device__ __forceinline__ float *fc_at(float *p, uint32_t bytes) {
+    return reinterpret_cast<float *>(reinterpret_cast<char *>(p) + bytes);
+}
+__device__ __forceinline__ f32x4 fc_g4(const float *p, uint32_t bytes) {
+    return *reinterpret_cast<const fc_u4 *>(fc_at(p, bytes));
+}
+__device__ __forceinline__ void fc_p4(float *p, uint32_t bytes, const f32x4 &x) {
+    *reinterpret_cast<fc_u4 *>(fc_at(p, bytes)) = x;
+}
+// Byte offsets of this lane's col elements (rows 4 g + i, column n) in rows of ld
+// floats.
+struct FcOff {
+    uint32_t o[4];
+    __device__ __forceinline__ explicit FcOff(uint32_t ld) {
+        const uint32_t l = lane_id(), g = l >> 4, n = l & 15;
+        o[0] = (4 * g * ld + n) * 4;
+#pragma unroll
+        for (int i = 1; i < 4; ++i) o[i] = o[i - 1] + 4 * ld;
+    }
+    __device__ __forceinline__ f32x4 get(const float *p, int tile = 0) const {
+        p += 16 * tile;
+        return f32x4{*fc_at(p, o[0]), *fc_at(p, o[1]), *fc_at(p, o[2]), *fc_at(p, o[3])};
+    }
+    __device__ __forceinline__ void put(float *p, const f32x4 &x, int tile = 0) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *fc_at(p + 16 * tile, o[i]) = x[i];
+    }
+};
 
 // Reads of one chunk of a [token][channel] input, unmasked.  VEC (fc_vec_view on
 // every input of the call): unit channel stride, a width of whole 16-channel
@@ -91,13 +124,13 @@ struct FcSrc {
     }
     __device__ __forceinline__ f32x4 frag(int tau) const {
         if (VEC) {
-            const char *p = base + fo + 16 * ES * tau;
+            const char *p = base + 16 * ES * tau;  // uniform
             if (BF) {
-                const uint2 x = *reinterpret_cast<const uint2 *>(p);
+                const uint2 x = *reinterpret_cast<const uint2 *>(p + fo);
                 return f32x4{__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u),
                              __uint_as_float(x.y << 16), __uint_as_float(x.y & 0xffff0000u)};
             }
-            return *reinterpret_cast<const f32x4 *>(p);
+            return *reinterpret_cast<const f32x4 *>(p + fo);
         }
         const int l = lane_id();
         f32x4 x;
@@ -111,8 +144,10 @@ struct FcSrc {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             if (VEC) {
-                const char *p = base + ((uint32_t)min(4 * g + q, last) * s1 + n * ES) + 16 * ES * tau;
-                x[q] = BF ? bf16_to_f32(*reinterpret_cast<const bf16_t *>(p)) : *reinterpret_cast<const float *>(p);
+                const char *p = base + 16 * ES * tau;  // uniform
+                const uint32_t o = (uint32_t)min(4 * g + q, last) * s1 + n * ES;
+                x[q] = BF ? bf16_to_f32(*reinterpret_cast<const bf16_t *>(p + o))
+                          : *reinterpret_cast<const float *>(p + o);
             } else {
                 x[q] = at(4 * g + q, 16 * tau + n);
             }
@@ -128,108 +163,80 @@ __device__ __forceinline__ void fc_put(void *dst, int bf16, const SeqArgs &s, in
     const int l = lane_id(), g = l >> 4, ch = 16 * tile + (l & 15);
     const int64_t o0 = (((int64_t)b * s.T + c * C) * s.H + h) * W;
     const int left = s.T - c * C;
+    if (VEC) {
+        const int es = bf16 ? 2 : 4;
+        char *p = static_cast<char *>(dst) + o0 * es;
+        const uint32_t row = (uint32_t)(s.H * W) * es, o = 4 * g * row + ch * es;
+        if (left >= C) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (bf16) *reinterpret_cast<bf16_t *>(p + (o + i * row)) = f32_to_bf16(x[i]);
+                else *reinterpret_cast<float *>(p + (o + i * row)) = x[i];
+            }
+            return;
+        }
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        if (4 * g + i < left && (VEC || ch < W)) {
-            if (VEC) {
-                const uint32_t o = (uint32_t)(4 * g + i) * (uint32_t)(s.H * W) + ch;
-                if (bf16) *reinterpret_cast<bf16_t *>(static_cast<char *>(dst) + o0 * 2 + o * 2u) = f32_to_bf16(x[i]);
-                else *reinterpret_cast<float *>(static_cast<char *>(dst) + o0 * 4 + o * 4u) = x[i];
-            } else {
-                store_out(dst, bf16, o0 + (int64_t)(4 * g + i) * s.H * W + ch, x[i]);
-            }
-        }
+        if (4 * g + i < left && ch < W) store_out(dst, bf16, o0 + (int64_t)(4 * g + i) * s.H * W + ch, x[i]);
 }
 
 // Token n's valid and reset flags (lane (g, n); the document limits in place of
 // the masks when given).
 __device__ __forceinline__ void fc_flags(const SeqArgs &s, int b, int c, bool &on, bool &rst) {
-    const int tg = c * C + (lane_id() & 15);
-    on = rst = false;
-    if (tg < s.T) {
-        if (s.doc) {
-            const int st = static_cast<const int *>(s.doc_start.data)[b * s.doc_start.s0 + tg * s.doc_start.s1];
-            const int en = static_cast<const int *>(s.doc_end.data)[b * s.doc_end.s0 + tg * s.doc_end.s1];
-            on = en >= st;
-            rst = on && st == tg;
-        } else {
-            on = ld4<float>(s.valid, b, tg, 0, 0) != 0.f;
-            rst = on && ld4<float>(s.reset, b, tg, 0, 0) != 0.f;
-        }
-    }
+    // Both words are loaded without a branch (past the sequence, the last token's).
+    const int tg = c * C + (lane_id() & 15), t = min(tg, s.T - 1);
+    const View &v0 = s.doc ? s.doc_start : s.valid, &v1 = s.doc ? s.doc_end : s.reset;
+    const int x0 = static_cast<const int *>(v0.data)[b * v0.s0 + t * v0.s1];
+    const int x1 = static_cast<const int *>(v1.data)[b * v1.s0 + t * v1.s1];
+    const bool live = s.doc ? x1 >= x0 : (x0 << 1) != 0;  // x1 >= x0; a nonzero float
+    const bool cut = s.doc ? x0 == tg : (x1 << 1) != 0;
+    on = (tg < s.T) & live;
+    rst = on & cut;
 }
 
 // T = (I + A)^-1 for A strictly lower in acc layout; returns row n of T, columns
 // 4 g + r (the A operand of T x, and one 16-byte piece of the row-major T).
 // T (I + A) = I by rows: from the last column on, T_nq is final and leaves T_nj
-// -= T_nq A_qj for j < q (entries above the diagonal stay zero).
-__device__ __forceinline__ f32x4 fc_inverse(const f32x4 &A, int g, int n) {
+// -= T_nq A_qj for j < q (entries above the diagonal stay zero).  A's rows come
+// back from LDS (the wave's own 320 floats) as broadcast 16-byte reads.
+constexpr int FC_LA = 20;  // row stride
+__device__ __forceinline__ f32x4 fc_inverse(const f32x4 &A, float *la, int g, int n) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) la[(4 * g + i) * FC_LA + n] = A[i];
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own rows have landed
+    __builtin_amdgcn_wave_barrier();
     float x[C];
 #pragma unroll
     for (int j = 0; j < C; ++j) x[j] = j == n ? 1.f : 0.f;
 #pragma unroll
     for (int q = C - 1; q > 0; --q)
 #pragma unroll
-        for (int j = 0; j < q; ++j) x[j] -= x[q] * fc_lane(A[q & 3], 16 * (q >> 2) + j);
+        for (int j4 = 0; j4 < q; j4 += 4) {
+            const f32x4 r = *reinterpret_cast<const f32x4 *>(&la[q * FC_LA + j4]);
+#pragma unroll
+            for (int j = j4; j < j4 + 4 && j < q; ++j) x[j] -= x[q] * r[j - j4];
+        }
     f32x4 t;
 #pragma unroll
     for (int r = 0; r < 4; ++r) t[r] = g == 0 ? x[r] : (g == 1 ? x[4 + r] : (g == 2 ? x[8 + r] : x[12 + r]));
     return t;
 }
 
-// The map's factors from T (fc_inverse): W' tile tau from the col tile b . e . k,
-// U tile vt from the col tile w . v, and the 16 x 16 array tm.
-__device__ __forceinline__ void fc_put_w(const FcArgs &a, int64_t ci, int KP, int tau, const f32x4 &t, const f32x4 &x,
-                                         int g, int n) {
-    const f32x4 w = fc_mma4(t, x, zero4());
-    float *p = a.fw + ci * C * KP;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[(4 * g + i) * KP + 16 * tau + n] = w[i];
+// A packed tile read across: register i holds row n, column 4 g + i of a
+// [token][channel] tile (a frag), or row n, column 4 g + i of a state tile (four
+// one-word loads that together read the tile's 1 KiB once).
+__device__ __forceinline__ f32x4 fc_across(const float *tile) {
+    const uint32_t l = lane_id(), n = l & 15, o = ((n >> 2) * 64 + 16 * (l >> 4) + (n & 3)) * 4;
+    return f32x4{*fc_at(tile, o), *fc_at(tile, o + 16), *fc_at(tile, o + 32), *fc_at(tile, o + 48)};
 }
-__device__ __forceinline__ void fc_put_u(const FcArgs &a, int64_t ci, int VT, int vt, const f32x4 &t, const f32x4 &x) {
-    *reinterpret_cast<fc_u4 *>(a.fu + (ci * VT + vt) * 256 + 4 * lane_id()) = fc_mma4(t, x, zero4());
+// Row r of a chunk's gb block (16 tokens): lane (g, n)'s token n, or its rows 4 g + i.
+__device__ __forceinline__ float fc_gb(const FcArgs &a, int64_t ci, int r) {
+    return *fc_at(a.gb + ci * C * 8 + C * r, 4 * (lane_id() & 15));
 }
-__device__ __forceinline__ void fc_put_rows(float *p, const f32x4 &x, int g, int n) {  // acc -> [16][16]
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[(4 * g + i) * C + n] = x[i];
-}
-__device__ __forceinline__ f32x4 fc_get_rows(const float *p, int g, int n) {  // [16][16] -> acc
-    return f32x4{p[(4 * g) * C + n], p[(4 * g + 1) * C + n], p[(4 * g + 2) * C + n], p[(4 * g + 3) * C + n]};
-}
-__device__ __forceinline__ f32x4 fc_get_col(const float *p, int KP, int tau, int g, int n) {  // [16][KP] -> col
-    const float *x = p + 16 * tau + n;
-    return f32x4{x[(4 * g) * KP], x[(4 * g + 1) * KP], x[(4 * g + 2) * KP], x[(4 * g + 3) * KP]};
-}
-// Key tile tau of a tile-packed state across the stored tiles of value tile vt:
-// register i holds row 16 tau + n, column 16 vt + 4 g + i (four one-word loads
-// that together read the tile's 1 KiB once).
-__device__ __forceinline__ f32x4 fc_get_across(const float *st, int KT, int tau, int vt, int g, int n) {
-    const float *p = st + (vt * KT + tau) * 256 + (n >> 2) * 64 + 16 * g + (n & 3);
-    return f32x4{p[0], p[4], p[8], p[12]};
-}
-
-// Score adjoint coefficients of token n: cs = dscore |k| / |delta|, ck = dscore
-// |delta| / |k| (zero at a zero edit or key).
-__device__ void fc_score_adj(const FcArgs &a, int64_t ci, int b, int h, int c, int VT, bool on, float ksq, float &cs,
-                             float &ck) {
-    const SeqArgs &s = a.s;
-    const int l = lane_id(), n = l & 15, tg = c * C + n;
-    f32x4 d2 = zero4();
-    for (int vt = 0; vt < VT; ++vt) {
-        const f32x4 d = fc_g4(a.fu + (ci * VT + vt) * 256 + 4 * l);
-        d2 += d * d;
-    }
-    float dsq = 0.f;  // token n's sum sits in group n / 4, register n % 4
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float x = __shfl(fc_row_sum(d2[i]), 16 * (n >> 2));
-        if ((n & 3) == i) dsq = x;
-    }
-    const float nk = sqrtf(ksq), nd = sqrtf(dsq);
-    const float dsc = tg < s.T ? s.dscores[((int64_t)b * s.T + tg) * s.H + h] : 0.f;
-    const bool ok = on && nk > 0.f && nd > 0.f;
-    cs = ok ? dsc * nk / nd : 0.f;
-    ck = ok ? dsc * nd / nk : 0.f;
+__device__ __forceinline__ f32x4 fc_gb4(const FcArgs &a, int64_t ci, int r) {
+    return fc_g4(a.gb + ci * C * 8 + C * r, 16 * (lane_id() >> 4));
 }
 
 inline void fc_mark(const hipEvent_t *ev, int i, hipStream_t stream) {

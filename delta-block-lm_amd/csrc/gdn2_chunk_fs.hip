@@ -8,11 +8,11 @@
 // product of the forward and the backward is a 16 x 16 matrix product.  a_u is
 // exp(g_u), 1 on padding and 0 on a reset, and D, b_t = D from the chunk start
 // and lam_s = D to the chunk end are direct products, so an underflowed decay
-// needs no special case.  The map's factors, the states, the scans, out and
-// bprep are gdn2_chunk_f32.hip's; prep and bgrad are here.
+// needs no special case.  The map's factors, the states, the scans and out are
+// gdn2_chunk_f32.hip's; prep and bgrad are here.
 //
-// At B8 T512 H8 K = V = 64 in f32, forward + backward takes 139 us of kernels
-// (prep 22, scans 24 and 22, out 11, bprep 15, bgrad 44) against 885 us of the
+// At B8 T512 H8 K = V = 64 in f32, forward + backward takes 121 us of kernels
+// (prep 17, scans 20 and 29, out 11, bgrad 43) against 885 us of the
 // token-sequential kernels, which walk a head's tokens in one workgroup
 // (forward 226, backward 658); the floor of its 69 MB is 14 us.
 #include "gdn2_chunk_f32_dev.h"
@@ -59,6 +59,7 @@ struct FsGradSmem {
 // ---- prep: T, P, D and the factored map, one wave per chunk ---------------------
 template <int KM, bool BF, bool VEC>
 __global__ void __launch_bounds__(64) fs_prep_kernel(FcArgs a) {
+    __shared__ __align__(16) float la[C * FC_LA];
     const SeqArgs &s = a.s;
     const int64_t ci = blockIdx.x;
     const int bh = blockIdx.x / a.nc, c = blockIdx.x % a.nc, b = bh / s.H, h = bh % s.H;
@@ -67,28 +68,30 @@ __global__ void __launch_bounds__(64) fs_prep_kernel(FcArgs a) {
     const FcSrc<BF, VEC> sk(s.k, b, h, c, s.T, K), sq(s.q, b, h, c, s.T, K), sv(s.v, b, h, c, s.T, V);
     bool on, rst;
     fc_flags(s, b, c, on, rst);
-    const float beta = on ? ld4<float>(s.beta, b, tg, h, 0) : 0.f;
-    const float av = on ? (rst ? 0.f : expf(ld4<float>(s.g, b, tg, h, 0))) : 1.f;
+    const int tc = min(tg, s.T - 1);
+    const float bv = ld4<float>(s.beta, b, tc, h, 0), gl = ld4<float>(s.g, b, tc, h, 0);
+    const float beta = on ? bv : 0.f, av = on ? (rst ? 0.f : expf(gl)) : 1.f;
     const f32x4 on4 = fc_rows(on ? 1.f : 0.f, g);
     f32x4 kb[KM], qb[KM], kk = zero4(), qk = zero4();
     float ksq = 0.f, lam;
     const f32x4 d = fs_decay_rows(av, g, n, lam);
-    float *fk = a.fk + ci * C * KP + n * KP + 4 * g;
+    const FcOff oc(C);
 #pragma unroll
     for (int tau = 0; tau < KM; ++tau) {
-        kb[tau] = qb[tau] = zero4();
-        if (tau >= KT) continue;
-        const f32x4 kf = fc_keep(sk.frag(tau), on), qf = fc_keep(sq.frag(tau), on);
-        kb[tau] = fc_keep4(sk.col(tau), on4);
-        qb[tau] = fc_keep4(sq.col(tau), on4);
+        // Past the last key tile (vector reads) the last tile is read again and
+        // zeroed, so that no load of the chunk waits behind a branch.
+        const int tt = VEC ? min(tau, KT - 1) : tau;
+        const bool in = tau < KT;
+        const f32x4 kf = fc_keep(sk.frag(tt), on && in), qf = fc_keep(sq.frag(tt), on && in);
+        kb[tau] = fc_keep4(sk.col(tt), on4);
+        qb[tau] = fc_keep4(sq.col(tt), on4);
         kk = fc_mma4(kf, kf, kk);
         qk = fc_mma4(qf, kf, qk);  // row t = 4 g + i, column s = n
 #pragma unroll
         for (int r = 0; r < 4; ++r) ksq += kf[r] * kf[r];
-        *reinterpret_cast<fc_u4 *>(fk + 16 * tau) = lam * kf;
     }
     const float bn = fs_scan_mul(av);
-    const f32x4 be4 = fc_rows(beta, g), b4 = fc_rows(bn, g);
+    const f32x4 be4 = fc_rows(beta, g), b4 = fc_rows(bn, g), lam4 = fc_rows(lam, g);
     f32x4 A, P, D;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -96,25 +99,26 @@ __global__ void __launch_bounds__(64) fs_prep_kernel(FcArgs a) {
         P[i] = n <= 4 * g + i ? d[i] * qk[i] : 0.f;
         D[i] = n <= 4 * g + i ? d[i] : 0.f;
     }
-    const f32x4 t = fc_inverse(A, g, n);
-    *reinterpret_cast<fc_u4 *>(a.tm + ci * C * C + n * C + 4 * g) = t;
-    fc_put_rows(a.pm + ci * C * C, P, g, n);
-    fc_put_rows(a.dm + ci * C * C, D, g, n);
+    const f32x4 t = fc_inverse(A, la, g, n);
+    fc_p4(a.tm + ci * C * C, (n * C + 4 * g) * 4, t);
+    oc.put(a.pm + ci * C * C, P);
+    oc.put(a.dm + ci * C * C, D);
     ksq = fc_group_sum(ksq);
-    if (g < 2)
-        *reinterpret_cast<fc_u4 *>(a.gb + (ci * C + n) * 8 + 4 * g) =
-            g == 0 ? f32x4{on ? 1.f : 0.f, rst ? 1.f : 0.f, ksq, beta} : f32x4{bn, lam, 0.f, 0.f};
+    float *gb = a.gb + ci * C * 8;
+    *fc_at(gb + C * g, 4 * n) = g == 0 ? (on ? 1.f : 0.f) : (g == 1 ? (rst ? 1.f : 0.f) : (g == 2 ? ksq : beta));
+    if (g < 2) *fc_at(gb + C * (4 + g), 4 * n) = g == 0 ? bn : lam;
     const float b15 = fc_lane(bn, C - 1);
     for (int i = l; i < KP; i += 64) a.gv[ci * KP + i] = b15;
-    float *fq = a.fq + ci * C * KP;
 #pragma unroll
     for (int tau = 0; tau < KM; ++tau)
         if (tau < KT) {
-            fc_put_w(a, ci, KP, tau, t, b4 * be4 * kb[tau], g, n);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) fq[(4 * g + i) * KP + 16 * tau + n] = b4[i] * qb[tau][i];
+            const int64_t o = (ci * KT + tau) * 256;
+            fc_p4(a.fw + o, 16 * l, fc_mma4(t, b4 * be4 * kb[tau], zero4()));
+            fc_p4(a.fk + o, 16 * l, lam4 * kb[tau]);
+            fc_p4(a.fq + o, 16 * l, b4 * qb[tau]);
         }
-    for (int vt = 0; vt < VT; ++vt) fc_put_u(a, ci, VT, vt, t, be4 * fc_keep4(sv.col(vt), on4));
+    for (int vt = 0; vt < VT; ++vt)
+        fc_p4(a.fu + (ci * VT + vt) * 256, 16 * l, fc_mma4(t, be4 * fc_keep4(sv.col(vt), on4), zero4()));
 }
 
 // ---- bgrad: every gradient of one chunk -------------------------------------------
@@ -138,31 +142,31 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
     const SeqArgs &s = a.s;
     const int bh = blockIdx.x / a.wn, cw = blockIdx.x % a.wn, c = a.w0 + cw, b = bh / s.H, h = bh % s.H;
     const int64_t ci = (int64_t)bh * a.nc + c, wi = blockIdx.x;
-    const int K = s.K, V = s.V, KP = fc_kp(K), KT = KP >> 4, VT = (V + 15) >> 4, NW = blockDim.x >> 6;
-    const int w = threadIdx.x >> 6, l = lane_id(), g = l >> 4, n = l & 15, tg = c * C + n;
+    const int K = s.K, V = s.V, KT = fc_kp(K) >> 4, VT = (V + 15) >> 4, NW = blockDim.x >> 6;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = lane_id(), g = l >> 4, n = l & 15, tg = c * C + n;
     const FcSrc<BF, VEC> sdo(s.dout, b, h, c, s.T, V);
     const bool has_do = s.dout.data != nullptr;
-    const f32x4 gb = fc_g4(a.gb + (ci * C + n) * 8), gc = fc_g4(a.gb + (ci * C + n) * 8 + 4);
-    const float bn = gc[0], lam = gc[1];
-    const bool on = gb[0] != 0.f;
-    const f32x4 on4 = fc_rows(gb[0], g), be4 = fc_rows(gb[3], g);
-    float cs = 0.f, ck = 0.f;
-    if (s.dscores) fc_score_adj(a, ci, b, h, c, VT, on, gb[2], cs, ck);
+    const float bn = fc_gb(a, ci, 4), lam = fc_gb(a, ci, 5);
+    const bool on = fc_gb(a, ci, 0) != 0.f;
+    const f32x4 on4 = fc_gb4(a, ci, 0), be4 = fc_gb4(a, ci, 3);
+    f32x4 cs4 = zero4(), ck4 = zero4();
+    if (s.dscores) cs4 = fc_g4(a.sc + wi * 2 * C, 16 * g), ck4 = fc_g4(a.sc + wi * 2 * C + C, 16 * g);
     const float *st = a.st + ci * KT * VT * 256, *ds = a.ds + wi * KT * VT * 256;
-    const f32x4 p = fc_get_rows(a.pm + ci * C * C, g, n);
+    const FcOff oc(C);
+    const f32x4 p = oc.get(a.pm + ci * C * C);
     if (w < VT) {  // ddelta and dR of value tile w
-        const f32x4 tb = fc_get_rows(a.tm + ci * C * C, g, n);
-        const f32x4 dl = fc_g4(a.fu + (ci * VT + w) * 256 + 4 * l);
+        const f32x4 tb = oc.get(a.tm + ci * C * C);
+        const f32x4 dl = fc_g4(a.fu + (ci * VT + w) * 256, 16 * l);
         const f32x4 v = fc_keep4(FcSrc<BF, VEC>(s.v, b, h, c, s.T, V).col(w), on4);
         f32x4 dO = has_do ? sdo.col(w) : zero4(), kf[KM], dsn[KM];
-        const float *fk = a.fk + ci * C * KP + n * KP + 4 * g;
+        const float *fk = a.fk + ci * KT * 256;
 #pragma unroll
         for (int tau = 0; tau < KM; ++tau) {
             kf[tau] = dsn[tau] = zero4();
-            if (tau < KT) kf[tau] = fc_g4(fk + 16 * tau), dsn[tau] = fc_g4(ds + (w * KT + tau) * 256 + 4 * l);
+            if (tau < KT) kf[tau] = fc_across(fk + 256 * tau), dsn[tau] = fc_g4(ds + (w * KT + tau) * 256, 16 * l);
         }
         dO = fc_keep4(dO, on4);
-        f32x4 dd = fc_mma4(p, dO, fc_rows(cs, g) * dl);
+        f32x4 dd = fc_mma4(p, dO, cs4 * dl);
 #pragma unroll
         for (int tau = 0; tau < KM; ++tau) dd = fc_mma4(kf[tau], dsn[tau], dd);
         const f32x4 dr = fc_mma4(tb, dd, zero4());                                               // rows t, column j
@@ -196,7 +200,7 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
                 m = x < 2 ? fc_mma4(d, y, m) : fc_mma4(y, d, m);
             }
         const float *dm = a.dm + ci * C * C;
-        const f32x4 d = x < 2 ? fc_g4(dm + n * C + 4 * g) : fc_get_rows(dm, g, n);  // zero above the diagonal
+        const f32x4 d = x < 2 ? fc_g4(dm, (n * C + 4 * g) * 4) : oc.get(dm);  // zero above the diagonal
         f32x4 md = m * d;
         if (x & 1)
 #pragma unroll
@@ -227,7 +231,7 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
 #pragma unroll
         for (int vt = 0; vt < KM; ++vt)
             if (vt < VT) {
-                const f32x4 s0 = fc_get_across(st, KT, w, vt, g, n), d1 = fc_get_across(ds, KT, w, vt, g, n);
+                const f32x4 s0 = fc_across(st + (vt * KT + w) * 256), d1 = fc_across(ds + (vt * KT + w) * 256);
                 const f32x4 d = *reinterpret_cast<const f32x4 *>(&sm.dl[n * LD + 16 * vt + 4 * g]);
                 const f32x4 r = *reinterpret_cast<const f32x4 *>(&sm.dr[n * LD + 16 * vt + 4 * g]);
                 Qb = fc_mma4(bn * yf[vt], s0, Qb);
@@ -240,7 +244,6 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
     if (l == 0) sm.fr[w] = fr;
     __syncthreads();
     if (w < KT) {
-        const f32x4 ck4 = fc_rows(ck, g);
         const f32x4 dq = fc_mma4(sm.m[0][l], kb, Qb), de = fc_mma4(sm.m[1][l], kb, Ab);
         const f32x4 dk = fc_mma4(sm.m[2][l], qb, fc_mma4(sm.m[3][l], kb, Kl));
         if (s.dq) fc_put<BF, VEC>(s.dq, BF, s, b, h, c, K, w, fc_keep4(dq, on4));
@@ -278,7 +281,7 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
         dg += fc_lane(bn, C - 1) * f;
         const int64_t o = ((int64_t)b * s.T + tg) * s.H + h;
         if (s.dbeta) s.dbeta[o] = on ? db : 0.f;
-        if (s.dg) s.dg[o] = (on && gb[1] == 0.f) ? dg : 0.f;
+        if (s.dg) s.dg[o] = (on && fc_gb(a, ci, 1) == 0.f) ? dg : 0.f;
     }
 }
 
@@ -298,7 +301,7 @@ hipError_t launch_fs_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *
     FC_DISPATCH(fc_kp(a.s.K) / 16, fs_prep, a, stream);
     fc_mark(ev, 1, stream);
     fc_mark(ev, 2, stream);
-    launch_fc_scan(a, false, stream);
+    launch_fc_scan(a, stream);
     fc_mark(ev, 3, stream);
     fc_mark(ev, 4, stream);
     launch_fc_out(a, stream);
@@ -311,22 +314,21 @@ hipError_t launch_fs_bwd(const FcArgs &whole, size_t ws_bytes, hipStream_t strea
     const int bh = a.s.B * a.s.H, VT = (a.s.V + 15) / 16, KT = fc_kp(a.s.K) / 16;
     // Chunk windows, last first: as many chunks as the workspace holds, the
     // adjoint between two windows in the carry.
-    const int64_t state = (int64_t)KT * VT * 256, carry = bh * state * 4, per = 2 * bh * state * 4;
+    const int64_t state = (int64_t)KT * VT * 256, carry = bh * state * 4, per = bh * fc_ws_chunk(a.s.K, a.s.V) * 4;
     int64_t wn = (int64_t)ws_bytes / per;
     if (wn < a.nc) wn = ((int64_t)ws_bytes - carry) / per;
     if (wn < 1) return hipErrorInvalidValue;
     wn = std::min<int64_t>(wn, a.nc);
-    a.n = a.ds + wn * bh * state;
-    a.carry = a.n + wn * bh * state;
+    a.sc = a.ds + wn * bh * state;
+    a.carry = a.sc + wn * bh * 2 * C;
     for (int end = a.nc; end > 0; end = a.w0) {
         a.wn = (int)std::min<int64_t>(end, wn);
         a.w0 = end - a.wn;
         const hipEvent_t *e = end == a.nc ? ev : nullptr;
         fc_mark(e, 0, stream);
-        launch_fc_bprep(a, stream);
         fc_mark(e, 1, stream);
         fc_mark(e, 2, stream);
-        launch_fc_scan(a, true, stream);
+        launch_fc_adjoint(a, stream);
         fc_mark(e, 3, stream);
         fc_mark(e, 4, stream);
         FC_DISPATCH(std::max(KT, VT), fs_bgrad, a, stream);
