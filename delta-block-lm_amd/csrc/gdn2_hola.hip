@@ -13,13 +13,14 @@
 //     rank is the number of eligible candidates that beat it (exact top-k with
 //     no sort); it writes the cache positions before/after every chunk and the
 //     end of each key's visibility ("expiry");
-//   * read, query VJP: one wave per (batch, head, chunk); the chunk's slots
-//     (cache positions from the schedule + the chunk's own tokens) are gathered
-//     once into LDS, then each query is a wave-wide softmax over <= 80 slots;
-//   * key VJP: one wave per (batch, head, chunk) of keys.  A selected key stays
+//   * read, query VJP: one wave per (batch, head, chunk); the rows of the chunk's
+//     slots (cache positions from the schedule + the chunk's own tokens) go from
+//     memory into MFMA operands, and each query's softmax over <= 80 slots stays
+//     in the registers of four lanes;
+//   * key VJP: four waves per (batch, head, chunk) of keys.  A selected key stays
 //     in the cache without interruption until it is evicted, so its visible
-//     queries are the chunks from its own up to its expiry; the wave walks them
-//     with a slot map per chunk and accumulates dk, dv in registers from the
+//     queries are the chunks from its own up to its expiry; the waves walk them
+//     with a slot map per chunk and accumulate dk, dv in registers from the
 //     (probability, logit gradient) pairs the query VJP saved.  No atomics.
 //   * sink gradient: a fixed-order sum over tokens per head.
 #include <float.h>
@@ -92,565 +93,622 @@ __device__ __forceinline__ int64_t token(const HolaArgs &a, int b, int t, int h)
     return ((int64_t)b * a.T + t) * a.H + h;
 }
 
+// Orders a wave's own LDS traffic: what any lane wrote before is read after.
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // ---- schedule ---------------------------------------------------------------------
 
-// One wave per (batch, head), chunks in order.  The cache entries carry their
-// ranking key and document in LDS, and the next chunk's token words (valid,
-// document, score) are loaded while the current chunk is ranked, so a chunk
-// costs LDS work only.
-__global__ void __launch_bounds__(64) hola_schedule_kernel(HolaArgs a) {
-    __shared__ float cpos[kMaxCapacity], cpri[kMaxCapacity], cdoc[kMaxCapacity];
-    __shared__ float pos[kMaxSlots], pri[kMaxSlots], sdoc[kMaxSlots];
-    __shared__ __align__(16) uint64_t key[kMaxSlots];
-    __shared__ float npos[kMaxCapacity], npri[kMaxCapacity], ndoc[kMaxCapacity];
-    const int lane = threadIdx.x, bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
+__device__ __forceinline__ uint64_t lane_u64(uint64_t x, int lane) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, lane);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), lane);
+    return ((uint64_t)hi << 32) | lo;
+}
+
+// One workgroup per (batch, head), chunks in order: a serial chain, bound by the
+// instructions and LDS round trips of one chunk.  Wave 1 prepares chunks one ahead of
+// the chain: it loads their token words (valid, document, score; kAhead chunks
+// early) and leaves the eligible tokens in rank order.  Wave 0 holds the cache in
+// registers, lane r the entry of rank r, so the cache is sorted at all times: an
+// entry's new rank is the eligible entries before it plus the tokens that beat it,
+// and the tokens fill the free ranks in their order.  128 (batch, head) pairs, 32
+// chunks of 16, 64 entries: 23 us, against 62 where one wave compared every pair
+// of the 80 candidates through LDS.
+__global__ void __launch_bounds__(128) hola_schedule_kernel(HolaArgs a) {
+    constexpr int kAhead = 4;
+    // A chunk's tokens in rank order: ranking word (0 past them); position, word, document.
+    __shared__ __align__(16) uint32_t word[2][kMaxChunk];
+    __shared__ __align__(16) float4 tok[2][kMaxChunk];
+    __shared__ float2 about[2];  // tokens, eligible document
+    __shared__ __align__(16) float4 place[kMaxCapacity];  // position, ranking word, document
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
     float *sched = a.schedule + (int64_t)bh * (a.nc + 1) * a.cap;
-    if (lane < a.cap) {
-        cpos[lane] = -1.f;
-        cpri[lane] = cdoc[lane] = 0.f;
-        sched[lane] = -1.f;
-    }
-    // Candidate slots past capacity + chunk stay empty for good.
-    for (int sl = lane; sl < kMaxSlots; sl += 64) {
-        pos[sl] = -1.f;
-        pri[sl] = 0.f;
-        key[sl] = 0;
-    }
+    float *expiry = a.expiry ? a.expiry + (int64_t)b * a.T * a.H + h : nullptr;
+    float cpos = -1.f, cdoc = 0.f;
+    uint32_t cord = 0;
+    if (wave == 0 && lane < a.cap) sched[lane] = -1.f;
     // Token words of a chunk: lane j < chunk holds token first + j.
-    float tv = 0.f, td = 0.f, ts = 0.f;
+    struct Words {
+        float valid, doc, score;
+    };
     auto fetch = [&](int c) {
+        Words w{0.f, 0.f, 0.f};
         const int t = c * a.chunk + lane;
-        tv = td = ts = 0.f;
         if (lane < a.chunk && t < a.T) {
-            tv = ldf(a.valid, b, t);
-            td = ldf(a.docs, b, t);
-            if (!a.recency) ts = ldf(a.scores, b, t, h);
+            w.valid = ldf(a.valid, b, t);
+            w.doc = ldf(a.docs, b, t);
+            if (!a.recency) w.score = ldf(a.scores, b, t, h);
+        }
+        return w;
+    };
+    auto prepare = [&](int c, const Words &w) {
+        const int first = c * a.chunk, n = min(a.chunk, a.T - first), buf = c & 1;
+        // Only the document of the chunk's last PHYSICAL slot, padding included,
+        // is eligible.
+        const float last_doc = readlane_f(w.doc, n - 1);
+        // Ranking keys: the order-preserving bits of the score (or position)
+        // above the complemented position, so "beats" (higher key, ties to the
+        // earlier position) is one unsigned compare; ineligible tokens get key 0
+        // and never beat.
+        const float pos = (float)(first + lane);
+        const bool on = lane < n && w.valid >= 0.5f && w.doc == last_doc;
+        const uint32_t u = __float_as_uint(a.recency ? pos : w.score);
+        const uint32_t ord = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+        const uint64_t key =
+            on ? ((uint64_t)ord << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)(first + lane)) : 0;
+        int rank = 0;
+#pragma unroll
+        for (int j = 0; j < kMaxChunk; ++j) rank += lane_u64(key, j) > key;
+        const int count = __popcll(__ballot(on));
+        if (lane < kMaxChunk) word[buf][lane] = 0;
+        wave_fence();
+        if (on) {
+            word[buf][rank] = ord;
+            tok[buf][rank] = make_float4(pos, __uint_as_float(ord), w.doc, 0.f);
+        }
+        if (lane == 0) about[buf] = make_float2((float)count, last_doc);
+    };
+    auto merge = [&](int c) {
+        const int first = c * a.chunk, n = min(a.chunk, a.T - first), end = first + n, buf = c & 1;
+        const float2 ab = about[buf];
+        const int count = (int)ab.x;
+        if (lane < n && expiry) expiry[(int64_t)(first + lane) * a.H] = (float)end;
+        const bool on = cpos >= 0.f && cdoc == ab.y;
+        const uint64_t below = (1ull << lane) - 1;
+        int rank = __popcll(__ballot(on) & below);
+#pragma unroll
+        for (int j = 0; j < kMaxChunk; j += 4) {
+            const uint4 o = *reinterpret_cast<const uint4 *>(&word[buf][j]);
+            // Ties go to the earlier position, the cache's.
+            rank += (int)(o.x > cord) + (int)(o.y > cord) + (int)(o.z > cord) + (int)(o.w > cord);
+        }
+        place[lane] = make_float4(-1.f, 0.f, 0.f, 0.f);
+        wave_fence();
+        if (on && rank < a.cap) place[rank] = make_float4(cpos, __uint_as_float(cord), cdoc, 0.f);
+        wave_fence();
+        float4 e = place[lane];
+        const uint64_t used = __ballot(e.x >= 0.f);
+        const int next = __popcll(~used & below);
+        const float4 t = tok[buf][min(next, kMaxChunk - 1)];
+        const bool take = e.x < 0.f && next < count && lane < a.cap;
+        cpos = take ? t.x : e.x;
+        cord = __float_as_uint(take ? t.y : e.y);
+        cdoc = take ? t.z : e.z;
+        wave_fence();
+        if (lane < a.cap) {
+            sched += a.cap;
+            sched[lane] = cpos;
+            if (cpos >= 0.f && expiry)
+                expiry[(int64_t)(int)cpos * a.H] = (float)min(end + a.chunk, a.T);
         }
     };
-    fetch(0);
-    __syncthreads();
-    for (int c = 0; c < a.nc; ++c) {
-        const int first = c * a.chunk, end = min(first + a.chunk, a.T), n = end - first;
-        const float mv = tv, md = td, ms = ts;
-        if (c + 1 < a.nc) fetch(c + 1);
-        // The document of the chunk's last PHYSICAL slot, padding included.
-        const float last_doc = readlane_f(md, n - 1);
-        if (lane < n && a.expiry) a.expiry[token(a, b, first + lane, h)] = (float)end;
-        // Candidates: the cache, then the chunk's valid tokens; only the last
-        // slot's document is eligible.
-        if (lane < a.cap) {
-            const float p = cpos[lane];
-            const bool ok = p >= 0.f && cdoc[lane] == last_doc;
-            pos[lane] = ok ? p : -1.f;
-            pri[lane] = cpri[lane];
-            sdoc[lane] = cdoc[lane];
-        }
-        if (lane < a.chunk) {
-            const int t = first + lane;
-            const bool ok = lane < n && mv >= 0.5f && md == last_doc;
-            pos[a.cap + lane] = ok ? (float)t : -1.f;
-            pri[a.cap + lane] = a.recency ? (float)t : ms;
-            sdoc[a.cap + lane] = md;
-        }
-        if (lane < a.cap) npos[lane] = -1.f;
-        __syncthreads();
-        // Ranking keys: the order-preserving bits of the score (or position)
-        // above the complemented position, so "beats" (higher key, ties to
-        // the earlier position) is one unsigned compare; empty and ineligible
-        // slots get key 0 and never beat.
-        for (int sl = lane; sl < a.cap + a.chunk; sl += 64) {
-            const float p = pos[sl];
-            const uint32_t u = __float_as_uint(pri[sl]);
-            const uint32_t ord = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-            key[sl] = p >= 0.f ? ((uint64_t)ord << 32) | (uint64_t)(0xFFFFFFFFu - (uint32_t)p) : 0;
-        }
-        __syncthreads();
-        // Rank = number of eligible candidates that beat this one (higher key,
-        // then earlier position): an exact top-capacity with no sort.  Each
-        // lane ranks candidates lane and lane + 64 in one pass over the
-        // candidate list, read four at a time (empty slots never beat).
-        {
-            const int s1 = lane + 64;
-            const float p0 = pos[lane], c0 = pri[lane];
-            const float p1 = s1 < kMaxSlots ? pos[s1] : -1.f, c1 = s1 < kMaxSlots ? pri[s1] : 0.f;
-            const uint64_t k0 = key[lane], k1 = s1 < kMaxSlots ? key[s1] : 0;
-            int r0 = 0, r1 = 0;
-#pragma unroll 10
-            for (int o = 0; o < kMaxSlots; o += 2) {
-                const ulonglong2 ko = *reinterpret_cast<const ulonglong2 *>(&key[o]);
-                r0 += (ko.x > k0) + (ko.y > k0);
-                r1 += (ko.x > k1) + (ko.y > k1);
-            }
-            if (p0 >= 0.f && r0 < a.cap) {
-                npos[r0] = p0;
-                npri[r0] = c0;
-                ndoc[r0] = sdoc[lane];
-            }
-            if (p1 >= 0.f && r1 < a.cap) {
-                npos[r1] = p1;
-                npri[r1] = c1;
-                ndoc[r1] = sdoc[s1];
-            }
-        }
-        __syncthreads();
-        if (lane < a.cap) {
-            const float p = npos[lane];
-            cpos[lane] = p;
-            cpri[lane] = npri[lane];
-            cdoc[lane] = ndoc[lane];
-            sched[(int64_t)(c + 1) * a.cap + lane] = p;
-            if (p >= 0.f && a.expiry)
-                a.expiry[token(a, b, (int)p, h)] = (float)min(end + a.chunk, a.T);
-        }
-        __syncthreads();
+    Words ring[kAhead];
+    if (wave == 1) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) ring[u] = fetch(u);
     }
-    if (a.final_positions && lane < a.cap) a.final_positions[(int64_t)bh * a.cap + lane] = cpos[lane];
+    for (int c0 = 0; c0 <= a.nc; c0 += kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int c = c0 + u;
+            if (c > a.nc) continue;
+            if (wave == 1) {
+                if (c < a.nc) prepare(c, ring[u]);
+                ring[u] = fetch(c + kAhead);
+            } else if (c > 0) {
+                merge(c - 1);
+            }
+            __syncthreads();
+        }
+    }
+    if (wave == 0 && a.final_positions && lane < a.cap)
+        a.final_positions[(int64_t)bh * a.cap + lane] = cpos;
+}
+
+// ---- rows and products ------------------------------------------------------------
+//
+// Every product of the read and its VJP runs on v_mfma_f32_16x16x4f32 with both
+// operands in registers: lane 16 g + n gives row (column) n at the reduction
+// index of group g, and holds rows 4 g + i of column n of the result.  Slots (or
+// keys) and queries are the rows and columns, so a result's registers are at
+// once the operand of the next product over the slots (its reduction index
+// 4 g + i), and no tile goes through LDS.  Rows come straight from memory: they
+// are gathered in 64- to 256-byte pieces, and each is used by one wave only.
+
+constexpr int kSlotTiles = kMaxSlots / 16;
+typedef float hola_f4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef float hola_f2 __attribute__((ext_vector_type(2), aligned(4)));
+
+__device__ __forceinline__ f32x4 mma(float x, float y, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(x, y, c, 0, 0, 0);
+}
+
+__device__ __forceinline__ float group_sum(float x) {  // over the four lane groups
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+}
+
+// Row t (its first row where t < 0: the caller drops it) of a view.
+__device__ __forceinline__ const float *row_of(const View &x, int b, int t, int h) {
+    return reinterpret_cast<const float *>(x.data) + b * x.s0 + max(t, 0) * x.s1 + h * x.s2;
+}
+
+// Channels i .. i + E - 1 of a row of width w, and the same with the channels past the
+// width (and rows that are off) cleared; two steps, so that the loads of a whole
+// set of rows are in flight before any is looked at.  VEC: unit channel stride and
+// widths in whole float4, whatever the alignment.
+template <int E, bool VEC>
+__device__ __forceinline__ void load_row(const float *row, int64_t s3, int i, int w, float (&x)[E]) {
+    if (VEC) {
+        const float *p = row + (i < w ? i : 0);
+        if (E == 4) {
+            const hola_f4 v = *reinterpret_cast<const hola_f4 *>(p);
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[e] = v[e];
+        } else {
+            const hola_f2 v = *reinterpret_cast<const hola_f2 *>(p);
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[e] = v[e & 1];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) x[e] = row[(i + e < w ? i + e : 0) * s3];
+    }
+}
+template <int E, bool VEC>
+__device__ __forceinline__ void keep_row(int i, int w, bool on, float (&x)[E]) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) x[e] = on && (VEC ? i : i + e) < w ? x[e] : 0.f;
+}
+template <int E, bool VEC>
+__device__ __forceinline__ void store_row(float *row, int i, int w, const float (&x)[E]) {
+    if (VEC) {
+        if (i >= w) return;
+        if (E == 4) *reinterpret_cast<hola_f4 *>(row + i) = hola_f4{x[0], x[1], x[E - 2], x[E - 1]};
+        else *reinterpret_cast<hola_f2 *>(row + i) = hola_f2{x[0], x[1]};
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (i + e < w) row[i + e] = x[e];
+    }
+}
+
+// A row as the operand of a product over its channels: lane group g holds
+// channels 16 t + 4 g + q.
+template <int D, bool VEC>
+struct Frag {
+    float x[D / 16][4];
+    __device__ __forceinline__ void load(const View &v, int b, int t, int h, int w) {
+        const float *row = row_of(v, b, t, h);
+        const int g = lane_id() >> 4;
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i) load_row<4, VEC>(row, v.s3, 16 * i + 4 * g, w, x[i]);
+    }
+    __device__ __forceinline__ void keep(bool on, int w) {
+        const int g = lane_id() >> 4;
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i) keep_row<4, VEC>(16 * i + 4 * g, w, on, x[i]);
+    }
+    __device__ __forceinline__ float dot(const Frag &y) const {
+        float s = 0.f;
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) s += x[i][q] * y.x[i][q];
+        return group_sum(s);
+    }
+};
+
+// Channels of a product over rows: tile (blk, e) has channels 16 E blk + E m + e as its
+// rows m, so that a lane reads and writes E channels in one piece.
+template <int D>
+struct Chans {
+    static constexpr int E = D >= 64 ? 4 : 2, NB = D / (16 * E);
+    f32x4 x[NB][E];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+            for (int e = 0; e < E; ++e) x[k][e] = zero4();
+    }
+    // Column n (lane n's row of the result) to dst.
+    template <bool VEC>
+    __device__ __forceinline__ void store(float *row, int w, bool on) const {
+        const int g = lane_id() >> 4;
+#pragma unroll
+        for (int k = 0; k < NB; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float y[E];
+#pragma unroll
+                for (int e = 0; e < E; ++e) y[e] = on ? x[k][e][i] : 0.f;
+                store_row<E, VEC>(row, 16 * E * k + E * (4 * g + i), w, y);
+            }
+    }
+};
+// Four rows (reduction indices 4 g + q) as the operand of a product over rows.
+template <int D, bool VEC>
+struct Rows {
+    static constexpr int E = Chans<D>::E, NB = Chans<D>::NB;
+    float x[4][NB][E];
+    __device__ __forceinline__ void load(const View &v, int b, const int (&t)[4], int h, int w) {
+        const int n = lane_id() & 15;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float *row = row_of(v, b, t[q], h);
+#pragma unroll
+            for (int k = 0; k < NB; ++k) load_row<E, VEC>(row, v.s3, 16 * E * k + E * n, w, x[q][k]);
+        }
+    }
+    // out += these rows, row 4 g + q weighted by y[q] (column n); off rows (t < 0) are zero.
+    __device__ __forceinline__ void mix(const f32x4 &y, const int (&t)[4], int w, Chans<D> &out) {
+        const int n = lane_id() & 15;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int k = 0; k < NB; ++k) {
+                keep_row<E, VEC>(16 * E * k + E * n, w, t[q] >= 0, x[q][k]);
+#pragma unroll
+                for (int e = 0; e < E; ++e) out.x[k][e] = mma(x[q][k][e], y[q], out.x[k][e]);
+            }
+    }
+};
+
+// (batch, head, chunk) of a workgroup: neighbouring workgroups go to the 8 XCDs in
+// turn, so each XCD is given a contiguous range of the list, and a head's rows, which
+// all its chunks gather from, are read into one L2 instead of into all eight.
+__device__ __forceinline__ int chunk_of_block(int id, int blocks) {
+    const int x = id & 7, q = blocks >> 3, r = blocks & 7;
+    return x * q + min(x, r) + (id >> 3);
 }
 
 // ---- chunk slots ------------------------------------------------------------------
 
-constexpr int kReadWaves = 4;  // waves per chunk in the read and the query VJP
-constexpr int kReadThreads = 64 * kReadWaves;
-constexpr int kWaveQueries = kMaxChunk / kReadWaves;
-
-// Query tt of a chunk is handled by wave tt % 4 as its (tt / 4)-th query;
-// transposed query tiles keep each wave's four queries of one channel in one
-// 16-byte group.
-__device__ __forceinline__ int query_slot(int tt) { return ((tt & 3) << 2) | (tt >> 2); }
-
-// dst[j * LD + i] = x(b, pos_j, h, i) for rows j < MAXS (zero where j >= S,
-// pos_j < 0 or i >= w), by NT threads.  Loads go out 16 per thread at a time
-// before any is used, so a gather costs a few memory latencies rather than
-// one per row.
-template <int D, int LD, int MAXS, int NT = 64, bool TQ = false>
-__device__ __forceinline__ void gather_rows(const View &x, int b, int h, int w, const float *pos,
-                                            int S, float *dst) {
-    constexpr int PER = MAXS * D / NT, BATCH = 16;
-    static_assert(PER * NT == MAXS * D, "whole workgroups");
-    const int lane = threadIdx.x;
-    for (int n0 = 0; n0 < PER; n0 += BATCH) {
-        float r[BATCH];
+// Slots of a chunk (the cache before the chunk, then the chunk's tokens; empty or
+// invalid slots have position -1), one wave.
+struct SlotInfo {
+    float pos[kMaxSlots] __attribute__((aligned(16)));
+    float doc[kMaxSlots] __attribute__((aligned(16)));
+    __device__ __forceinline__ void stage(const HolaArgs &a, int b, int h, int c) {
+        const int lane = lane_id(), first = c * a.chunk, end = min(first + a.chunk, a.T);
+        const float *sched = a.schedule + ((int64_t)(b * a.H + h) * (a.nc + 1) + c) * a.cap;
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const int idx = lane + NT * (n0 + u), j = idx / D, i = idx % D;
-            r[u] = 0.f;
-            if (n0 + u < PER && j < S && i < w) {
-                const float p = pos[j];
-                if (p >= 0.f) r[u] = ldf(x, b, (int)p, h, i);
+        for (int r = 0; r < 2; ++r) {
+            const int j = lane + 64 * r;
+            if (j >= kMaxSlots) continue;
+            float p = -1.f;
+            if (j < a.cap) {
+                p = sched[j];
+            } else {
+                const int t = first + j - a.cap;
+                if (t < end && ldf(a.valid, b, t) >= 0.5f) p = (float)t;
             }
+            pos[j] = p;
+            doc[j] = p >= 0.f ? ldf(a.docs, b, (int)p) : 0.f;
         }
+        wave_fence();
+    }
+    __device__ __forceinline__ int at(int j) const { return (int)pos[j]; }
+    __device__ __forceinline__ void rows(int s, int (&t)[4]) const {
+        const f32x4 p = *reinterpret_cast<const f32x4 *>(&pos[16 * s + 4 * (lane_id() >> 4)]);
 #pragma unroll
-        for (int u = 0; u < BATCH; ++u) {
-            const int idx = lane + NT * (n0 + u), j = idx / D, i = idx % D;
-            if (n0 + u < PER) {
-                if (TQ) dst[i * MAXS + query_slot(j)] = r[u];
-                else dst[j * LD + i] = r[u];
-            }
+        for (int q = 0; q < 4; ++q) t[q] = (int)p[q];
+    }
+};
+
+// The chunk's query of a lane (query n of lane 16 g + n).
+struct Query {
+    int t;
+    bool in, act;  // inside the sequence; and valid
+    float doc;
+    __device__ __forceinline__ Query(const HolaArgs &a, int b, int c) {
+        const int first = c * a.chunk, end = min(first + a.chunk, a.T);
+        t = first + (lane_id() & 15);
+        in = t < end;
+        t = in ? t : first;
+        act = in && ldf(a.valid, b, t) >= 0.5f;
+        doc = ldf(a.docs, b, t);
+    }
+};
+
+// Products of the slots' rows with the chunk's queries' x: slot 16 s + 4 g + i, query n.
+template <int D, bool VEC>
+__device__ __forceinline__ void slot_dots(const View &y, int b, int h, int w, const SlotInfo &s, int slots,
+                                          const Frag<D, VEC> &x, f32x4 (&out)[kSlotTiles]) {
+    const int n = lane_id() & 15;
+    Frag<D, VEC> f[kSlotTiles];
+#pragma unroll
+    for (int k = 0; k < kSlotTiles; ++k)
+        if (16 * k < slots) f[k].load(y, b, s.at(16 * k + n), h, w);
+#pragma unroll
+    for (int k = 0; k < kSlotTiles; ++k) {
+        out[k] = zero4();
+        if (16 * k >= slots) continue;
+        f[k].keep(s.at(16 * k + n) >= 0, w);
+#pragma unroll
+        for (int i = 0; i < D / 16; ++i)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) out[k] = mma(f[k].x[i][q], x.x[i][q], out[k]);
+    }
+}
+
+// The slots' rows, for their weighted sums.
+template <int D, bool VEC>
+struct SlotRows {
+    Rows<D, VEC> r[kSlotTiles];
+    __device__ __forceinline__ void load(const View &y, int b, int h, int w, const SlotInfo &s, int slots) {
+#pragma unroll
+        for (int k = 0; k < kSlotTiles; ++k) {
+            int t[4];
+            s.rows(k, t);
+            if (16 * k < slots) r[k].load(y, b, t, h, w);
+        }
+    }
+    __device__ __forceinline__ void mix(const f32x4 (&p)[kSlotTiles], int w, const SlotInfo &s, int slots,
+                                        Chans<D> &out) {
+        out.clear();
+#pragma unroll
+        for (int k = 0; k < kSlotTiles; ++k) {
+            int t[4];
+            s.rows(k, t);
+            if (16 * k < slots) r[k].mix(p[k], t, w, out);
+        }
+    }
+};
+
+// Raw logits -> scaled, -FLT_MAX where the slot is not visible: empty, later than the
+// query, another document, or an inactive query.
+__device__ __forceinline__ void visible_logits(const HolaArgs &a, const SlotInfo &s, const Query &q,
+                                               f32x4 (&lg)[kSlotTiles]) {
+    const int g = lane_id() >> 4;
+#pragma unroll
+    for (int k = 0; k < kSlotTiles; ++k) {
+        const f32x4 p = *reinterpret_cast<const f32x4 *>(&s.pos[16 * k + 4 * g]);
+        const f32x4 d = *reinterpret_cast<const f32x4 *>(&s.doc[16 * k + 4 * g]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const bool vis = q.act && p[i] >= 0.f && p[i] <= (float)q.t && d[i] == q.doc;
+            lg[k][i] = vis ? lg[k][i] * a.scale : -FLT_MAX;
         }
     }
 }
 
-// PAD = 1 (the read): lanes reading different rows of one column hit
-// different banks.  PAD = 4 (the query VJP's MFMA products): an operand read
-// of 16 rows x 4 columns hits 64 distinct banks, one of 4 rows x 16 columns
-// (its dq product) each bank at most four times.
-template <int DK, int DV, int PAD = 1>
-struct SlotTiles {
-    static constexpr int LK = DK + PAD, LV = DV + PAD;
-    float K[kMaxSlots][LK];
-    float V[kMaxSlots][LV];
-    float QT[DK][kMaxChunk] __attribute__((aligned(16)));  // [channel][query_slot(tt)]
-    float pos[kMaxSlots], doc[kMaxSlots];
-    float tpos[kMaxChunk], tval[kMaxChunk], tdoc[kMaxChunk];
-};
-
-// Slots of chunk c (the cache before the chunk, then the chunk's tokens; empty
-// or invalid slots get position -1 and zero rows), and the chunk's queries.
-template <int DK, int DV, int PAD>
-__device__ void stage_slots(const HolaArgs &a, int b, int h, int c, SlotTiles<DK, DV, PAD> &s) {
-    const int lane = threadIdx.x, first = c * a.chunk, end = min(first + a.chunk, a.T);
+// One wave per (batch, head, chunk).  Bound by the gather of the slots' rows (40 KB
+// a chunk at 64 slots + 16 and widths of 64, out of the caches) and its latency.
+// B16 T512 H8, widths of 64: 31 us, against 86 with the tiles in LDS (four waves a
+// chunk) and VALU products; the rows and results alone are 14 us at copy rate.  Four
+// waves a SIMD hold all 4096 chunks at once (three: 33 us).
+template <int DK, int DV, bool VEC>
+__global__ void __launch_bounds__(64, DK + DV > 128 ? 2 : 4) hola_forward_kernel(HolaArgs a) {
+    __shared__ SlotInfo s;
+    const int g = lane_id() >> 4;
+    const int item = chunk_of_block(blockIdx.x, gridDim.x), c = item % a.nc, bh = item / a.nc;
+    const int b = bh / a.H, h = bh % a.H;
     const int slots = a.cap + a.chunk;
-    const float *sched = a.schedule + ((int64_t)(b * a.H + h) * (a.nc + 1) + c) * a.cap;
-    for (int j = lane; j < slots; j += kReadThreads) {
-        float p = -1.f;
-        if (j < a.cap) {
-            p = sched[j];
-        } else {
-            const int t = first + j - a.cap;
-            if (t < end && ldf(a.valid, b, t) >= 0.5f) p = (float)t;
-        }
-        s.pos[j] = p;
-        s.doc[j] = p >= 0.f ? ldf(a.docs, b, (int)p) : 0.f;
-    }
-    if (lane < kMaxChunk) {
-        const int t = first + lane;
-        const bool in = lane < a.chunk && t < end;
-        s.tpos[lane] = in ? (float)t : -1.f;
-        s.tval[lane] = in ? ldf(a.valid, b, t) : 0.f;
-        s.tdoc[lane] = in ? ldf(a.docs, b, t) : 0.f;
-    }
-    __syncthreads();
-    gather_rows<DK, DK + PAD, kMaxSlots, kReadThreads>(a.k, b, h, a.dk, s.pos, slots, &s.K[0][0]);
-    gather_rows<DV, DV + PAD, kMaxSlots, kReadThreads>(a.v, b, h, a.dv, s.pos, slots, &s.V[0][0]);
-    gather_rows<DK, DK, kMaxChunk, kReadThreads, true>(a.q, b, h, a.dk, s.tpos, kMaxChunk,
-                                                      &s.QT[0][0]);
-    __syncthreads();
-}
-
-// The four queries of a wave (tt = wave + 4u): token, activity, document.
-struct WaveQueries {
-    int t[kWaveQueries];
-    bool on[kWaveQueries], act[kWaveQueries];
-    float doc[kWaveQueries];
-};
-
-template <int DK, int DV, int PAD>
-__device__ __forceinline__ WaveQueries wave_queries(const SlotTiles<DK, DV, PAD> &s, int wave, int first,
-                                                    int n) {
-    WaveQueries w;
-#pragma unroll
-    for (int u = 0; u < kWaveQueries; ++u) {
-        const int tt = wave + kReadWaves * u;
-        w.t[u] = first + tt;
-        w.on[u] = tt < n;
-        w.act[u] = tt < n && s.tval[tt] >= 0.5f;
-        w.doc[u] = tt < n ? s.tdoc[tt] : 0.f;
-    }
-    return w;
-}
-
-// Scaled logits of the wave's queries against slot j (-FLT_MAX where the slot
-// is not visible: empty, later than the query, another document, or an
-// inactive query).  One K read and one 16-byte query read per channel.
-template <int DK, int DV>
-__device__ __forceinline__ void wave_logits(const HolaArgs &a, const SlotTiles<DK, DV> &s,
-                                            const WaveQueries &w, int wave, int j,
-                                            float (&lg)[kWaveQueries]) {
-    float acc[kWaveQueries] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int i = 0; i < DK; ++i) {
-        const float kv = s.K[j][i];
-        const float4 q4 = *reinterpret_cast<const float4 *>(&s.QT[i][4 * wave]);
-        acc[0] += q4.x * kv;
-        acc[1] += q4.y * kv;
-        acc[2] += q4.z * kv;
-        acc[3] += q4.w * kv;
-    }
-    const float p = s.pos[j], d = s.doc[j];
-#pragma unroll
-    for (int u = 0; u < kWaveQueries; ++u) {
-        const bool vis = w.act[u] && p >= 0.f && p <= (float)w.t[u] && d == w.doc[u];
-        lg[u] = vis ? acc[u] * a.scale : -FLT_MAX;
-    }
-}
-
-// [query slot][slot] tiles of a chunk (logits, probabilities, their adjoints):
-// row stride 84 floats (20 mod 64), so an MFMA A-operand read (16 rows x 4
-// columns) and an accumulator store hit 64 distinct banks.
-constexpr int kLP = kMaxSlots + 4;
-
-// Query tt of the chunk behind query slot qs (the inverse of query_slot).
-__device__ __forceinline__ int slot_query(int qs) { return (qs >> 2) + 4 * (qs & 3); }
-
-// X Y^T over the reduction width D on v_mfma_f32_16x16x4f32: X^T [D][16] in
-// query-slot columns (the chunk's queries or their output adjoints), Y [slot]
-// rows of stride LY (K or V); out[qs][slot] for the 16-slot tiles that cover
-// the slots, wave w taking tiles w, w + 4, ...  Lane (lg, ln) reduces over
-// k = 4 ks + lg and holds rows 4 lg + r of column 16 n + ln.
-template <int D, int LY>
-__device__ __forceinline__ void chunk_xyt(const float (*XT)[kMaxChunk], const float *Y, int slots, int wave,
-                                          float (*out)[kLP]) {
-    const int l = lane_id(), lg = l >> 4, ln = l & 15;
-    for (int n = wave; 16 * n < slots; n += kReadWaves) {
-        f32x4 acc = zero4();
-#pragma unroll 4
-        for (int ks = 0; ks < D / 4; ++ks)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(XT[4 * ks + lg][ln], Y[(16 * n + ln) * LY + 4 * ks + lg],
-                                                       acc, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) out[4 * lg + r][16 * n + ln] = acc[r];
-    }
-}
-
-// P Y over the slots on v_mfma_f32_16x16x4f32: P [qs][slot] (zero past the
-// slots), Y [slot][channel] rows of stride LY (zero past the slots); wave w
-// takes the 16-channel tiles w, w + 4, .. of the W used channels and stores row
-// qs (query slot_query(qs) of the chunk) of each to dst[token][channel] when the
-// query is inside the sequence, zero when it is inactive.
-template <int D, int LY>
-__device__ __forceinline__ void chunk_py(const HolaArgs &a, const float (*P)[kLP], const float *Y, int slots,
-                                         int wave, int b, int h, int first, int n, const float *tval, int W,
-                                         float *dst) {
-    const int l = lane_id(), lg = l >> 4, ln = l & 15, nks = (slots + 3) >> 2;
-    for (int ct = wave; ct < D / 16; ct += kReadWaves) {
-        f32x4 acc = zero4();
-        for (int ks = 0; ks < nks; ++ks)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(P[ln][4 * ks + lg], Y[(4 * ks + lg) * LY + 16 * ct + ln],
-                                                       acc, 0, 0, 0);
-        const int ch = 16 * ct + ln;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int tt = slot_query(4 * lg + r);
-            if (tt < n && ch < W)
-                dst[token(a, b, first + tt, h) * W + ch] = tval[tt] >= 0.5f ? acc[r] : 0.f;
-        }
-    }
-}
-
-// Scaled logit of the wave's query u against slot j from the chunk's raw
-// logits (-FLT_MAX where the slot is not visible: past the slots, empty, later
-// than the query, another document, or an inactive query).
-template <int DK, int DV, int PAD>
-__device__ __forceinline__ float visible_logit(const HolaArgs &a, const SlotTiles<DK, DV, PAD> &s,
-                                               const WaveQueries &w, const float (*L)[kLP], int wave, int u,
-                                               int j, int slots) {
-    if (j >= slots || !w.act[u]) return -FLT_MAX;
-    const float p = s.pos[j];
-    const bool vis = p >= 0.f && p <= (float)w.t[u] && s.doc[j] == w.doc[u];
-    return vis ? L[4 * wave + u][j] * a.scale : -FLT_MAX;
-}
-
-template <int DK, int DV>
-__global__ void __launch_bounds__(kReadThreads) hola_forward_kernel(HolaArgs a) {
-    __shared__ SlotTiles<DK, DV> s;
-    __shared__ float4 PT[kReadWaves][kMaxSlots];  // normalised probabilities, [slot][query]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = blockIdx.x % a.nc, bh = blockIdx.x / a.nc, b = bh / a.H, h = bh % a.H;
-    const int first = c * a.chunk, end = min(first + a.chunk, a.T), slots = a.cap + a.chunk;
-    stage_slots<DK, DV>(a, b, h, c, s);
+    const Query q(a, b, c);
+    Frag<DK, VEC> qf;
+    qf.load(a.q, b, q.t, h, a.dk);
+    s.stage(a, b, h, c);
+    qf.keep(q.in, a.dk);
+    f32x4 p[kSlotTiles];
+    slot_dots<DK, VEC>(a.k, b, h, a.dk, s, slots, qf, p);
+    SlotRows<DV, VEC> v;
+    v.load(a.v, b, h, a.dv, s, slots);
+    visible_logits(a, s, q, p);
     const float sink = ldf(a.sink, h);
-    const WaveQueries w = wave_queries(s, wave, first, end - first);
-    float lg[2][kWaveQueries];
+    float m = sink, sum = 0.f;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int j = lane + 64 * r;
-        if (j < slots) wave_logits(a, s, w, wave, j, lg[r]);
-        else
-            for (int u = 0; u < kWaveQueries; ++u) lg[r][u] = -FLT_MAX;
-    }
-    float m[kWaveQueries], inv[kWaveQueries], p0[kWaveQueries], p1[kWaveQueries];
+    for (int k = 0; k < kSlotTiles; ++k)
 #pragma unroll
-    for (int u = 0; u < kWaveQueries; ++u) m[u] = wave_max(fmaxf(sink, fmaxf(lg[0][u], lg[1][u])));
+        for (int i = 0; i < 4; ++i) m = fmaxf(m, p[k][i]);
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
 #pragma unroll
-    for (int u = 0; u < kWaveQueries; ++u) {
-        p0[u] = lg[0][u] > -FLT_MAX ? expf(lg[0][u] - m[u]) : 0.f;
-        p1[u] = lg[1][u] > -FLT_MAX ? expf(lg[1][u] - m[u]) : 0.f;
-    }
+    for (int k = 0; k < kSlotTiles; ++k)
 #pragma unroll
-    for (int u = 0; u < kWaveQueries; ++u) {
-        inv[u] = 1.f / (wave_sum(p0[u] + p1[u]) + expf(sink - m[u]));
-        // Normalised before the value product: finite values cannot overflow.
-        p0[u] *= inv[u];
-        p1[u] *= inv[u];
-    }
-    if (lane < slots) PT[wave][lane] = make_float4(p0[0], p0[1], p0[2], p0[3]);
-    if (lane + 64 < slots) PT[wave][lane + 64] = make_float4(p1[0], p1[1], p1[2], p1[3]);
-    __builtin_amdgcn_wave_barrier();
-    for (int j = lane; j < a.dv; j += 64) {
-        float o[kWaveQueries] = {0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < slots; ++k) {
-            const float vv = s.V[k][j];
-            const float4 p4 = PT[wave][k];
-            o[0] += p4.x * vv;
-            o[1] += p4.y * vv;
-            o[2] += p4.z * vv;
-            o[3] += p4.w * vv;
+        for (int i = 0; i < 4; ++i) {
+            p[k][i] = p[k][i] > -FLT_MAX ? expf(p[k][i] - m) : 0.f;
+            sum += p[k][i];
         }
+    const float inv = 1.f / (group_sum(sum) + expf(sink - m));
+    // Normalised before the value product: finite values cannot overflow.
 #pragma unroll
-        for (int u = 0; u < kWaveQueries; ++u)
-            if (w.on[u]) a.out[token(a, b, w.t[u], h) * a.dv + j] = w.act[u] ? o[u] : 0.f;
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int u = 0; u < kWaveQueries; ++u) {
-            if (!w.on[u]) continue;
-            const int64_t tok = token(a, b, w.t[u], h);
-            a.stats[2 * tok] = m[u];
-            a.stats[2 * tok + 1] = inv[u];
-        }
+    for (int k = 0; k < kSlotTiles; ++k) p[k] *= inv;
+    Chans<DV> o;
+    v.mix(p, a.dv, s, slots, o);
+    if (!q.in) return;
+    const int64_t tok = token(a, b, q.t, h);
+    o.template store<VEC>(a.out + tok * a.dv, a.dv, q.act);
+    if (g == 0) {
+        a.stats[2 * tok] = m;
+        a.stats[2 * tok + 1] = inv;
     }
 }
 
 // ---- backward ---------------------------------------------------------------------
 
-template <int DK, int DV>
-__global__ void __launch_bounds__(kReadThreads) hola_query_backward_kernel(HolaArgs a) {
-    __shared__ SlotTiles<DK, DV, 4> s;
-    __shared__ float L[kMaxChunk][kLP];   // logits, then logit gradients: [query slot][slot]
-    __shared__ float Dt[kMaxChunk][kLP];  // dO . v_slot: [query slot][slot]
-    __shared__ float GT[DV][kMaxChunk] __attribute__((aligned(16)));  // dO, [channel][query_slot]
-    __shared__ float O[kMaxChunk][DV + 1];
-    __shared__ float stat[kMaxChunk][2];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int c = blockIdx.x % a.nc, bh = blockIdx.x / a.nc, b = bh / a.H, h = bh % a.H;
-    const int first = c * a.chunk, end = min(first + a.chunk, a.T), slots = a.cap + a.chunk;
-    stage_slots<DK, DV>(a, b, h, c, s);
-    // The chunk's output adjoints (transposed), forward outputs and softmax
-    // statistics.
-    {
-        constexpr int PER = kMaxChunk * DV / kReadThreads;
-        float g[PER], o[PER];
+// One wave per (batch, head, chunk); bound as the read, plus the pairs that it
+// leaves for the key VJP (8 bytes a query and slot).
+// B16 T512 H8, widths of 64: 53 us, against 127 with the tiles in LDS; rows, pairs and
+// results are 29 us at copy rate.  Three waves a SIMD: four would spill.
+template <int DK, int DV, bool VEC>
+__global__ void __launch_bounds__(64, DK + DV > 128 ? 2 : 3) hola_query_backward_kernel(HolaArgs a) {
+    __shared__ SlotInfo s;
+    const int g = lane_id() >> 4;
+    const int item = chunk_of_block(blockIdx.x, gridDim.x), c = item % a.nc, bh = item / a.nc;
+    const int b = bh / a.H, h = bh % a.H;
+    const int slots = a.cap + a.chunk;
+    const Query q(a, b, c);
+    const int64_t tok = token(a, b, q.t, h);
+    const float m = a.stats[2 * tok], inv = a.stats[2 * tok + 1], sink = ldf(a.sink, h);
+    Frag<DK, VEC> qf;
+    Frag<DV, VEC> gf, of;
+    const View ov{a.fwd_out, (int64_t)a.T * a.H * a.dv, (int64_t)a.H * a.dv, a.dv, 1};
+    qf.load(a.q, b, q.t, h, a.dk);
+    of.load(ov, b, q.t, h, a.dv);
+    gf.load(a.dout.data ? a.dout : ov, b, q.t, h, a.dv);  // a null adjoint is zero
+    s.stage(a, b, h, c);
+    qf.keep(q.in, a.dk);
+    gf.keep(q.in && a.dout.data, a.dv);
+    of.keep(q.in, a.dv);
+    float delta = gf.dot(of);
+    delta = q.act ? delta : 0.f;
+    f32x4 lg[kSlotTiles], dp[kSlotTiles];
+    slot_dots<DK, VEC>(a.k, b, h, a.dk, s, slots, qf, lg);
+    slot_dots<DV, VEC>(a.v, b, h, a.dv, s, slots, gf, dp);
+    SlotRows<DK, VEC> kr;
+    kr.load(a.k, b, h, a.dk, s, slots);
+    visible_logits(a, s, q, lg);
+    if (g == 0 && q.in) {
+        a.aux[2 * tok] = delta;
+        a.aux[2 * tok + 1] = q.act ? -delta * expf(sink - m) * inv : 0.f;
+    }
+    // p and the logit gradient d = p (dO . v - delta) / sqrt(d_k), saved as pairs.
+    float *pairs = a.pairs + tok * slots * 2;
 #pragma unroll
-        for (int n = 0; n < PER; ++n) {
-            const int idx = tid + kReadThreads * n, tt = idx / DV, j = idx % DV, t = first + tt;
-            g[n] = o[n] = 0.f;
-            if (tt < end - first && j < a.dv) {
-                if (a.dout.data) g[n] = ldf(a.dout, b, t, h, j);
-                o[n] = a.fwd_out[token(a, b, t, h) * a.dv + j];
-            }
-        }
+    for (int k = 0; k < kSlotTiles; ++k) {
+        float pd[8];
 #pragma unroll
-        for (int n = 0; n < PER; ++n) {
-            const int idx = tid + kReadThreads * n, tt = idx / DV, j = idx % DV;
-            GT[j][query_slot(tt)] = g[n];
-            O[tt][j] = o[n];
+        for (int i = 0; i < 4; ++i) {
+            const bool on = lg[k][i] > -FLT_MAX;
+            const float p = on ? expf(lg[k][i] - m) * inv : 0.f;
+            const float d = on ? p * (dp[k][i] - delta) * a.scale : 0.f;
+            pd[2 * i] = p;
+            pd[2 * i + 1] = d;
+            dp[k][i] = d;
         }
-        if (tid < 2 * kMaxChunk) {
-            const int tt = tid >> 1, t = first + tt;
-            stat[tt][tid & 1] = tt < end - first ? a.stats[2 * token(a, b, t, h) + (tid & 1)] : 0.f;
+        const int j = 16 * k + 4 * g;
+        if (q.in && j + 3 < slots) {
+            *reinterpret_cast<hola_f4 *>(pairs + 2 * j) = hola_f4{pd[0], pd[1], pd[2], pd[3]};
+            *reinterpret_cast<hola_f4 *>(pairs + 2 * j + 4) = hola_f4{pd[4], pd[5], pd[6], pd[7]};
+        } else if (q.in) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (j + i < slots) {
+                    pairs[2 * (j + i)] = pd[2 * i];
+                    pairs[2 * (j + i) + 1] = pd[2 * i + 1];
+                }
         }
     }
-    __syncthreads();
-    // Raw logits and dO . v for every (query, slot) on MFMA.
-    chunk_xyt<DK, DK + 4>(s.QT, &s.K[0][0], slots, wave, L);
-    chunk_xyt<DV, DV + 4>(GT, &s.V[0][0], slots, wave, Dt);
-    const float sink = ldf(a.sink, h);
-    const WaveQueries w = wave_queries(s, wave, first, end - first);
-    float delta[kWaveQueries], m[kWaveQueries], inv[kWaveQueries];
-#pragma unroll
-    for (int u = 0; u < kWaveQueries; ++u) {
-        const int tt = wave + kReadWaves * u;
-        float dl = 0.f;
-        if (w.act[u])
-            for (int j = lane; j < DV; j += 64) dl += GT[j][query_slot(tt)] * O[tt][j];
-        delta[u] = wave_sum(dl);
-        m[u] = w.on[u] ? stat[tt][0] : 0.f;
-        inv[u] = w.on[u] ? stat[tt][1] : 0.f;
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int u = 0; u < kWaveQueries; ++u) {
-            if (!w.on[u]) continue;
-            const int64_t tok = token(a, b, w.t[u], h);
-            a.aux[2 * tok] = delta[u];
-            a.aux[2 * tok + 1] = w.act[u] ? -delta[u] * expf(sink - m[u]) * inv[u] : 0.f;
-        }
-    }
-    __syncthreads();
-    // Per slot (lanes): p and the logit gradient d = p (dO . v - delta) / sqrt(d_k),
-    // saved as pairs; the wave's rows of L take d (zero past the slots).
-#pragma unroll
-    for (int r = 0; r < 2; ++r) {
-        const int j = lane + 64 * r;
-        if (j >= kMaxSlots) continue;
-#pragma unroll
-        for (int u = 0; u < kWaveQueries; ++u) {
-            const float lgv = visible_logit(a, s, w, L, wave, u, j, slots);
-            const float p = lgv > -FLT_MAX ? expf(lgv - m[u]) * inv[u] : 0.f;
-            const float d = lgv > -FLT_MAX ? p * (Dt[4 * wave + u][j] - delta[u]) * a.scale : 0.f;
-            if (w.on[u] && j < slots)
-                reinterpret_cast<float2 *>(a.pairs)[token(a, b, w.t[u], h) * slots + j] = make_float2(p, d);
-            L[4 * wave + u][j] = d;
-        }
-    }
-    __syncthreads();
-    chunk_py<DK, DK + 4>(a, L, &s.K[0][0], slots, wave, b, h, first, end - first, s.tval, a.dk, a.gq);
+    Chans<DK> o;
+    kr.mix(dp, a.dk, s, slots, o);
+    if (q.in) o.template store<VEC>(a.gq + tok * a.dk, a.dk, q.act);
 }
 
-template <int DK, int DV>
-__global__ void __launch_bounds__(64) hola_key_backward_kernel(HolaArgs a) {
-    constexpr int RK = (DK + 63) / 64, RV = (DV + 63) / 64;
-    __shared__ int map[kMaxChunk];
-    __shared__ float Q[kMaxChunk][DK], G[kMaxChunk][DV];
-    __shared__ float2 PD[kMaxChunk][kMaxChunk];  // (probability, logit gradient) [query][key]
-    __shared__ float qpos[kMaxChunk];
-    const int lane = threadIdx.x;
-    const int c = blockIdx.x % a.nc, bh = blockIdx.x / a.nc, b = bh / a.H, h = bh % a.H;
-    const int first = c * a.chunk, end = min(first + a.chunk, a.T), n = end - first;
+// kKeyWaves waves per (batch, head, chunk) of keys: the query chunks that see the keys
+// run from the keys' own to the last expiry, up to the whole sequence, so wave w
+// takes every kKeyWaves-th of them (one wave would leave the early chunks' walks as
+// the kernel's tail) and the partial gradients are added pairwise through LDS.
+// B16 T512 H8, widths of 64: 38 us, against 99 with one wave on VALU products; 50 with
+// the workgroups in grid order (see chunk_of_block).
+constexpr int kKeyWaves = 4;
+
+template <int DK, int DV, bool VEC>
+__global__ void __launch_bounds__(64 * kKeyWaves) hola_key_backward_kernel(HolaArgs a) {
+    constexpr int NK = DK / 16, NV = DV / 16;
+    __shared__ float map[kKeyWaves][kMaxChunk];
+    __shared__ f32x4 part[kKeyWaves / 2][NK + NV][64];
+    const int l = lane_id(), wave = threadIdx.x >> 6, n = l & 15, g = l >> 4;
+    const int item = chunk_of_block(blockIdx.x, gridDim.x), c = item % a.nc, bh = item / a.nc;
+    const int b = bh / a.H, h = bh % a.H;
+    const int first = c * a.chunk, end = min(first + a.chunk, a.T), keys = end - first;
     const int slots = a.cap + a.chunk;
     const float *sched = a.schedule + (int64_t)bh * (a.nc + 1) * a.cap;
-    float dka[kMaxChunk][RK], dva[kMaxChunk][RV];
-#pragma unroll
-    for (int j = 0; j < kMaxChunk; ++j) {
-#pragma unroll
-        for (int r = 0; r < RK; ++r) dka[j][r] = 0.f;
-#pragma unroll
-        for (int r = 0; r < RV; ++r) dva[j][r] = 0.f;
-    }
+    Chans<DK> dka;
+    Chans<DV> dva;
+    dka.clear();
+    dva.clear();
     // Queries that can see a key of this chunk end at its expiry.
     float lastf = (float)end;
-    if (lane < n) lastf = fmaxf(lastf, a.expiry[token(a, b, first + lane, h)]);
+    if (l < keys) lastf = fmaxf(lastf, a.expiry[token(a, b, first + l, h)]);
     const int last = (int)wave_max(lastf);
-    for (int cq = c; cq * a.chunk < last; ++cq) {
-        const int q0 = cq * a.chunk, q1 = min(q0 + a.chunk, a.T), nq = q1 - q0;
-        // Where this chunk's keys sit among the slots of query chunk cq.
-        if (lane < kMaxChunk) {
-            map[lane] = -1;
-            qpos[lane] = lane < nq ? (float)(q0 + lane) : -1.f;
+    auto entry = [&](int cq) {
+        return l < a.cap && cq < a.nc ? sched[(int64_t)cq * a.cap + l] : -1.f;
+    };
+    float cached = entry(c + wave);
+    for (int cq = c + wave; cq * a.chunk < last; cq += kKeyWaves) {
+        const int q0 = cq * a.chunk, nq = min(q0 + a.chunk, a.T) - q0;
+        // Where key n sits among the slots of query chunk cq.
+        if (l < kMaxChunk) map[wave][l] = cq == c && l < keys ? (float)(a.cap + l) : -1.f;
+        wave_fence();
+        if (cq != c && cached >= (float)first && cached < (float)end)
+            map[wave][(int)cached - first] = (float)l;
+        wave_fence();
+        const int sl = (int)map[wave][n];
+        wave_fence();
+        cached = entry(cq + kKeyWaves);
+        // The chunk's queries and output adjoints, and the pairs of the mapped slots.
+        int t[4];
+        float p[4][2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            t[q] = 4 * g + q < nq ? q0 + 4 * g + q : -1;
+            const float *src = a.pairs + (token(a, b, max(t[q], q0), h) * slots + max(sl, 0)) * 2;
+            const hola_f2 v = *reinterpret_cast<const hola_f2 *>(src);
+            p[q][0] = v[0];
+            p[q][1] = v[1];
+        }
+        Rows<DK, VEC> qr;
+        Rows<DV, VEC> gr;
+        qr.load(a.q, b, t, h, a.dk);
+        if (a.dout.data) gr.load(a.dout, b, t, h, a.dv);
+        f32x4 pr, dl;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool on = sl >= 0 && t[q] >= 0;
+            pr[q] = on ? p[q][0] : 0.f;
+            dl[q] = on ? p[q][1] : 0.f;
+        }
+        qr.mix(dl, t, a.dk, dka);
+        if (a.dout.data) gr.mix(pr, t, a.dv, dva);
+    }
+    // Partial gradients of waves 2, 3 to 0, 1, then of 1 to 0.
+#pragma unroll
+    for (int half = kKeyWaves / 2; half > 0; half /= 2) {
+        if (wave >= half && wave < 2 * half) {
+#pragma unroll
+            for (int i = 0; i < NK; ++i) part[wave - half][i][l] = dka.x[i / Chans<DK>::E][i % Chans<DK>::E];
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                part[wave - half][NK + i][l] = dva.x[i / Chans<DV>::E][i % Chans<DV>::E];
         }
         __syncthreads();
-        if (cq == c) {
-            if (lane < n) map[lane] = a.cap + lane;
-        } else if (lane < a.cap) {
-            const float p = sched[(int64_t)cq * a.cap + lane];
-            if (p >= (float)first && p < (float)end) map[(int)p - first] = lane;
-        }
-        __syncthreads();
-        // The chunk's queries, output adjoints and the pairs of the mapped slots.
-        gather_rows<DK, DK, kMaxChunk>(a.q, b, h, a.dk, qpos, kMaxChunk, &Q[0][0]);
-        if (a.dout.data) gather_rows<DV, DV, kMaxChunk>(a.dout, b, h, a.dv, qpos, kMaxChunk, &G[0][0]);
-        else
-            for (int idx = lane; idx < kMaxChunk * DV; idx += 64) G[idx / DV][idx % DV] = 0.f;
-        {
-            constexpr int PER = kMaxChunk * kMaxChunk / 64;
-            float2 r[PER];
+        if (wave < half) {
 #pragma unroll
-            for (int u = 0; u < PER; ++u) {
-                const int idx = lane + 64 * u, tq = idx / kMaxChunk, j = idx % kMaxChunk;
-                const int sl = map[j];
-                r[u] = make_float2(0.f, 0.f);
-                if (tq < nq && sl >= 0)
-                    r[u] = reinterpret_cast<const float2 *>(a.pairs)[token(a, b, q0 + tq, h) * slots + sl];
-            }
+            for (int i = 0; i < NK; ++i) dka.x[i / Chans<DK>::E][i % Chans<DK>::E] += part[wave][i][l];
 #pragma unroll
-            for (int u = 0; u < PER; ++u) {
-                const int idx = lane + 64 * u;
-                PD[idx / kMaxChunk][idx % kMaxChunk] = r[u];
-            }
-        }
-        __syncthreads();
-        for (int tq = 0; tq < nq; ++tq) {
-            float qv[RK], gv[RV];
-#pragma unroll
-            for (int r = 0; r < RK; ++r) qv[r] = lane + 64 * r < DK ? Q[tq][lane + 64 * r] : 0.f;
-#pragma unroll
-            for (int r = 0; r < RV; ++r) gv[r] = lane + 64 * r < DV ? G[tq][lane + 64 * r] : 0.f;
-#pragma unroll
-            for (int j = 0; j < kMaxChunk; ++j) {
-                const float2 pd = PD[tq][j];
-#pragma unroll
-                for (int r = 0; r < RK; ++r) dka[j][r] += pd.y * qv[r];
-#pragma unroll
-                for (int r = 0; r < RV; ++r) dva[j][r] += pd.x * gv[r];
-            }
+            for (int i = 0; i < NV; ++i)
+                dva.x[i / Chans<DV>::E][i % Chans<DV>::E] += part[wave][NK + i][l];
         }
         __syncthreads();
     }
-#pragma unroll
-    for (int j = 0; j < kMaxChunk; ++j) {
-        if (j >= n) continue;
-        const int64_t tok = token(a, b, first + j, h);
-#pragma unroll
-        for (int r = 0; r < RK; ++r) {
-            const int i = lane + 64 * r;
-            if (i < a.dk) a.gk[tok * a.dk + i] = dka[j][r];
-        }
-#pragma unroll
-        for (int r = 0; r < RV; ++r) {
-            const int i = lane + 64 * r;
-            if (i < a.dv) a.gv[tok * a.dv + i] = dva[j][r];
-        }
-    }
+    if (wave != 0 || n >= keys) return;
+    const int64_t tok = token(a, b, first + n, h);
+    dka.template store<VEC>(a.gk + tok * a.dk, a.dk, true);
+    dva.template store<VEC>(a.gv + tok * a.dv, a.dv, true);
 }
 
 // dsink[h] = sum over (b, t) of aux[.][1], in a fixed order.
@@ -674,30 +732,38 @@ __global__ void __launch_bounds__(1024) hola_sink_kernel(HolaArgs a) {
 
 int pad_width(int64_t w) { return w <= 32 ? 32 : (w <= 64 ? 64 : 128); }
 
-template <template <int, int> class K>
+// Rows in whole float4 pieces: unit channel strides and widths of whole pieces.
+bool vec_rows(const HolaArgs &a) {
+    return a.q.s3 == 1 && a.k.s3 == 1 && a.v.s3 == 1 && (!a.dout.data || a.dout.s3 == 1) &&
+           a.dk % 4 == 0 && a.dv % 4 == 0;
+}
+
+template <template <int, int, bool> class K>
 void launch_widths(const HolaArgs &a, dim3 grid, hipStream_t st) {
     const int kp = pad_width(a.dk), vp = pad_width(a.dv);
-#define GDN2_HOLA_CASE(P, Q)                                                    \
-    if (kp == P && vp == Q) {                                                   \
-        hipLaunchKernelGGL((K<P, Q>::fn), grid, dim3(K<P, Q>::threads), 0, st, a); \
-        return;                                                                 \
+    const bool vec = vec_rows(a);
+#define GDN2_HOLA_CASE(P, Q)                                                                    \
+    if (kp == P && vp == Q) {                                                                   \
+        if (vec) hipLaunchKernelGGL((K<P, Q, true>::fn), grid, dim3(K<P, Q, true>::threads), 0, st, a); \
+        else hipLaunchKernelGGL((K<P, Q, false>::fn), grid, dim3(K<P, Q, false>::threads), 0, st, a);   \
+        return;                                                                                 \
     }
     GDN2_HOLA_CASE(32, 32) GDN2_HOLA_CASE(32, 64) GDN2_HOLA_CASE(32, 128)
     GDN2_HOLA_CASE(64, 32) GDN2_HOLA_CASE(64, 64) GDN2_HOLA_CASE(64, 128)
     GDN2_HOLA_CASE(128, 32) GDN2_HOLA_CASE(128, 64) GDN2_HOLA_CASE(128, 128)
 #undef GDN2_HOLA_CASE
 }
-template <int P, int Q> struct Fwd {
-    static constexpr auto fn = hola_forward_kernel<P, Q>;
-    static constexpr int threads = kReadThreads;
-};
-template <int P, int Q> struct QBwd {
-    static constexpr auto fn = hola_query_backward_kernel<P, Q>;
-    static constexpr int threads = kReadThreads;
-};
-template <int P, int Q> struct KBwd {
-    static constexpr auto fn = hola_key_backward_kernel<P, Q>;
+template <int P, int Q, bool VEC> struct Fwd {
+    static constexpr auto fn = hola_forward_kernel<P, Q, VEC>;
     static constexpr int threads = 64;
+};
+template <int P, int Q, bool VEC> struct QBwd {
+    static constexpr auto fn = hola_query_backward_kernel<P, Q, VEC>;
+    static constexpr int threads = 64;
+};
+template <int P, int Q, bool VEC> struct KBwd {
+    static constexpr auto fn = hola_key_backward_kernel<P, Q, VEC>;
+    static constexpr int threads = 64 * kKeyWaves;
 };
 
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
@@ -782,7 +848,7 @@ int gdn2_hola_schedule(const gdn2_hola_shape *shape, int recency, const gdn2_vie
     a.scores = make_view(scores);
     a.recency = recency != 0;
     a.schedule = schedule;
-    hipLaunchKernelGGL(hola_schedule_kernel, dim3(a.B * a.H), dim3(64), 0, (hipStream_t)stream, a);
+    hipLaunchKernelGGL(hola_schedule_kernel, dim3(a.B * a.H), dim3(128), 0, (hipStream_t)stream, a);
     return launch_status(hipGetLastError(), "gdn2_hola_schedule");
 }
 
@@ -814,7 +880,7 @@ int gdn2_hola_read(const gdn2_hola_shape *shape, int recency, const gdn2_view *q
     a.out = output;
     a.final_positions = final_positions;
     hipStream_t st = (hipStream_t)stream;
-    hipLaunchKernelGGL(hola_schedule_kernel, dim3(a.B * a.H), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(hola_schedule_kernel, dim3(a.B * a.H), dim3(128), 0, st, a);
     GDN2_TRY(launch_status(hipGetLastError(), "gdn2_hola_read (schedule)"));
     launch_widths<Fwd>(a, dim3(a.B * a.H * a.nc), st);
     return launch_status(hipGetLastError(), "gdn2_hola_read");
