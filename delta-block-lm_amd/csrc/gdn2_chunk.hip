@@ -214,17 +214,23 @@ __global__ void __launch_bounds__(NT) chunk_prep_kernel(ChunkArgs a) {
     __syncthreads();
     // Rows out, hi then lo: M = A_c^T row by row (the adjoint scan's map), and A_c
     // (the state scan's) read across it: lane (row 16 (w%4) + l%16, columns
-    // 32 (w/4) + 8 (l/16) ..) stores one 16-byte row piece.
+    // 32 (w/4) + ..) stores one 16-byte row piece.  The scans' column order: piece
+    // 4 kk + g of a row holds columns 32 kk + 4 g .. + 3, then 32 kk + 16 + 4 g .. + 3.
     {
-        const int r = tid >> 3, c0 = 8 * (tid & 7), l = lane_id();
+        const int r = tid >> 3, l = lane_id(), i = l & 15;
+        const int c0 = 32 * ((tid >> 2) & 1) + 4 * (tid & 3);
         uint16_t *mt = a.map_mt + (int64_t)ci * 2 * D * D, *mm = a.map_m + (int64_t)ci * 2 * D * D;
-        const int64_t fo = (int64_t)(16 * (w & 3) + (l & 15)) * D + 32 * (w >> 2) + 8 * (l >> 4);
+        const int64_t fo = (int64_t)(16 * (w & 3) + i) * D + 32 * (w >> 2) + 8 * (l >> 4);
 #pragma unroll
         for (int part = 0; part < 2; ++part) {
             const uint16_t *src = part == 0 ? Mt : Mtl;
-            *reinterpret_cast<uint4 *>(mt + part * D * D + r * D + c0) =
-                *reinterpret_cast<const uint4 *>(&src[r * LDB + c0]);
-            *reinterpret_cast<bf16x8_t *>(mm + part * D * D + fo) = frag_tr(src, 32 * (w >> 2), 16 * (w & 3));
+            const uint2 x = *reinterpret_cast<const uint2 *>(&src[r * LDB + c0]);
+            const uint2 y = *reinterpret_cast<const uint2 *>(&src[r * LDB + c0 + 16]);
+            *reinterpret_cast<uint4 *>(mt + part * D * D + r * D + 8 * (tid & 7)) = make_uint4(x.x, x.y, y.x, y.y);
+            const uint16_t *z = src + (32 * (w >> 2) + 4 * (l >> 4) + (i >> 2)) * LDB + 16 * (w & 3) + 4 * (i & 3);
+            const v4s a0 = lds_tr16(z), a1 = lds_tr16(z + 16 * LDB);
+            *reinterpret_cast<uint4 *>(mm + part * D * D + fo) =
+                __builtin_bit_cast(uint4, __builtin_shufflevector(a0, a1, 0, 1, 2, 3, 4, 5, 6, 7));
         }
     }
 }
@@ -397,30 +403,37 @@ __global__ void __launch_bounds__(NT) chunk_out_kernel(ChunkArgs a) {
 // evolve independently, so each head's scan is split over AS_SPLIT workgroups
 // of 16 AS_CW columns each (the workgroups of one head read the same maps; their
 // block indices differ by a multiple of B*H, so with B*H a multiple of the XCD
-// count they share an L2).  AS_CW + 3 waves per workgroup:
+// count, they share an L2).  AS_CW + 3 waves per workgroup:
 //   waves 0 .. AS_CW-1  compute: wave w owns state columns j0 + 16 w .. + 15 in
-//              MFMA accumulators; per step it writes X^T hi/lo into its LDS
-//              tiles (the B operand of the product and the writer's source),
-//              passes the step's barrier and forms N + M_hi X_hi + M_hi X_lo +
-//              M_lo X_hi (24 MFMAs, four independent accumulator tiles);
+//              MFMA accumulators and forms N + M_hi X_hi + M_hi X_lo + M_lo X_hi
+//              (24 MFMAs, four independent accumulator tiles);
 //   wave AS_CW      streams M (hi, then lo) into an LDS ring with LDS-DMA loads,
-//              AS_MRING - 1 chunks ahead;
+//              AS_MRING chunks ahead;
 //   wave AS_CW + 1  streams the workgroup's rows of N^T (f32) the same way;
 //   wave AS_CW + 2  copies each step's X^T tiles to the checkpoint.
-// The compute waves issue no global memory operations inside the loop.  LDS
-// rows are swizzled by 16-byte chunk against bank conflicts.
+// A step is a serial chain, so nothing but the product is left on it: the
+// accumulators of row tiles 2 kk and 2 kk + 1, converted to bf16, are the B operand of
+// the next product (a reduction index may be permuted: the maps' columns are stored
+// in that order), the step's M and N are in registers when it begins
+// (read from LDS during the step before), and the X^T tiles for the writer go to LDS
+// behind the first products.  One barrier a step: behind it the next chunk's M
+// and N are in their slots, this chunk's slots are free and the writer may read
+// this step's X^T.  Eight heads, 47 chunks of 64: 25.7 us, against 33 with X
+// taken through LDS and M read after the barrier (0.46 us a step, from 0.7); 128
+// heads, 8 chunks: 9.1 against 9.5.  A ring of five is slower (27.3 and 9.8).  The compute waves issue no global memory operations
+// inside the loop.  LDS rows are swizzled by 16-byte chunk against bank conflicts.
 namespace {
 constexpr int AS_CW = 2;               // compute waves per workgroup
 constexpr int AS_SPLIT = 4 / AS_CW;    // workgroups per head
-constexpr int AS_MRING = 3;
-constexpr int AS_NRING = 3;
+constexpr int AS_MRING = 4;
+constexpr int AS_NRING = 4;
 constexpr int AS_MOPS = 2 * D * D * 2 / 1024;       // LDS-DMA instructions per map (hi + lo, 1 KiB each)
 constexpr int AS_NOPS = 16 * AS_CW * D * 4 / 1024;  // per workgroup's rows of N^T (f32)
 constexpr int AS_THREADS = (AS_CW + 3) * 64;
 
 struct AsArgs {
     int nc, B, H;
-    const uint16_t *m;  // per chunk: M rows, bf16 hi [64][64] then lo [64][64]
+    const uint16_t *m;  // per chunk: M rows, bf16 hi [64][64] then lo [64][64], in the scans' column order
     const float *n;     // per chunk: N^T rows, f32 [64][64]
     uint16_t *ckpt, *ckpt_lo;  // X^T per chunk, bf16 hi and lo
     View x0;            // [B,H,64,64] strided (data may be null: zero)
@@ -428,13 +441,15 @@ struct AsArgs {
 };
 
 struct AsSmem {
-    uint4 m[AS_MRING][2 * D * D / 8];       // row r (hi rows 0..63, lo rows 64..127): chunk x at x ^ (r & 7)
+    uint4 m[AS_MRING][2 * D * D / 8];       // row r (hi rows 0..63, lo rows 64..127): chunk x at x ^ (r / 2 & 7)
     uint4 n[AS_NRING][16 * AS_CW * D / 4];  // N^T row j0 + j: chunk x (four f32) at x ^ (j & 15)
     uint16_t xs[2][AS_CW][2][16 * LDB];     // [step parity][compute wave][hi, lo]: X^T [col][row]
 };
 
 // s_waitcnt immediates (gfx9 encoding): vmcnt <= n only; lgkmcnt == 0 only.
-constexpr int as_vmcnt(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+constexpr int as_vmcnt(int n) {
+    return n > 63 ? as_vmcnt(63) : (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8);
+}
 constexpr int AS_LGKMCNT_ZERO = 15 | (3 << 14) | (7 << 4);
 
 __device__ __forceinline__ void as_barrier() {
@@ -457,28 +472,30 @@ __global__ void __launch_bounds__(AS_THREADS) affine_scan_kernel(AsArgs p) {
         const int sc = min(s, p.nc - 1);
         return (int64_t)bh * p.nc + (REV ? p.nc - 1 - sc : sc);
     };
-    if (w == AS_CW) {  // producer: M (hi and lo), AS_MRING - 1 chunks ahead
+    if (w == AS_CW) {  // producer: M (hi and lo), AS_MRING chunks ahead
         auto issue = [&](int s) {
             const uint16_t *M = p.m + chunk_of(s) * 2 * D * D;
             uint4 *slot = sm.m[s % AS_MRING];
 #pragma unroll
             for (int i = 0; i < AS_MOPS; ++i) {
                 const int q = 64 * i + l, r = q >> 3, x = q & 7;
-                __builtin_amdgcn_global_load_lds((gptr)(M + r * D + 8 * (x ^ (r & 7))), (lptr)(slot + 64 * i), 16,
-                                                 0, 0);
+                __builtin_amdgcn_global_load_lds((gptr)(M + r * D + 8 * (x ^ (r >> 1 & 7))), (lptr)(slot + 64 * i),
+                                                 16, 0, 0);
             }
         };
-        for (int s = 0; s < AS_MRING - 1; ++s) issue(s);
+        for (int s = 0; s < AS_MRING; ++s) issue(s);
+        __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_MRING - 1) * AS_MOPS));
+        as_barrier();  // chunk 0 has landed
         for (int s = 0; s < p.nc; ++s) {
-            // chunk s has landed once no more than the AS_MRING - 2 later maps are in flight
+            // chunk s + 1 has landed once no more than the AS_MRING - 2 later maps are in flight
             __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_MRING - 2) * AS_MOPS));
             as_barrier();
-            issue(s + AS_MRING - 1);  // into the slot that step s - 1 read
+            issue(s + AS_MRING);  // into the slot that held chunk s
         }
         __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
         return;
     }
-    if (w == AS_CW + 1) {  // producer: this workgroup's rows of N^T, AS_NRING - 1 chunks ahead
+    if (w == AS_CW + 1) {  // producer: this workgroup's rows of N^T, AS_NRING chunks ahead
         auto issue = [&](int s) {
             const float *N = p.n + chunk_of(s) * D * D + j0 * D;
             uint4 *slot = sm.n[s % AS_NRING];
@@ -489,16 +506,19 @@ __global__ void __launch_bounds__(AS_THREADS) affine_scan_kernel(AsArgs p) {
                                                  0, 0);
             }
         };
-        for (int s = 0; s < AS_NRING - 1; ++s) issue(s);
+        for (int s = 0; s < AS_NRING; ++s) issue(s);
+        __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_NRING - 1) * AS_NOPS));
+        as_barrier();
         for (int s = 0; s < p.nc; ++s) {
             __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_NRING - 2) * AS_NOPS));
             as_barrier();
-            issue(s + AS_NRING - 1);
+            issue(s + AS_NRING);
         }
         __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
         return;
     }
     if (w == AS_CW + 2) {  // writer: X^T before step s -> the checkpoint of chunk c(s)
+        as_barrier();
         for (int s = 0; s < p.nc; ++s) {
             as_barrier();
             const int64_t co = chunk_of(s) * D * D;
@@ -522,41 +542,88 @@ __global__ void __launch_bounds__(AS_THREADS) affine_scan_kernel(AsArgs p) {
     for (int tm = 0; tm < 4; ++tm)
 #pragma unroll
         for (int i = 0; i < 4; ++i) X[tm][i] = p.x0.data ? ld4<float>(p.x0, b, h, 16 * tm + 4 * g + i, j) : 0.f;
-    for (int s = 0; s < p.nc; ++s) {
-        uint16_t *xh = sm.xs[s & 1][w][0], *xl = sm.xs[s & 1][w][1];
-#pragma unroll
-        for (int tm = 0; tm < 4; ++tm) store_tile_t_split(xh + 16 * tm, xl + 16 * tm, LDB, X[tm]);
-        // The writer wave reads these tiles after the barrier, and the LDS writes of
-        // different waves may complete out of issue order: wait until they landed.
-        __builtin_amdgcn_s_waitcnt(AS_LGKMCNT_ZERO);
-        as_barrier();  // this step's M and N are in their slots; the writer may read X^T
+    // A step's M (A operands: columns 32 kk + 4 g + i, then 32 kk + 16 + 4 g + i) and N.
+    struct Step {
+        bf16x8_t mh[2][4], ml[2][4];
+        f32x4 n[4];
+    };
+    auto read = [&](int s, Step &m) {
         const uint4 *slot = sm.m[s % AS_MRING];
         const float4 *nslot = reinterpret_cast<const float4 *>(sm.n[s % AS_NRING]);
-        f32x4 Y[4], Z[4];
 #pragma unroll
         for (int tm = 0; tm < 4; ++tm) {  // N[16 tm + 4 g + i][j]: chunk 4 tm + g of N^T row j
             const float4 nv = nslot[jl * 16 + ((4 * tm + g) ^ (jl & 15))];
-            Y[tm] = f32x4{nv.x, nv.y, nv.z, nv.w};
-            Z[tm] = zero4();
+            m.n[tm] = f32x4{nv.x, nv.y, nv.z, nv.w};
         }
 #pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-            const bf16x8_t bh_ = frag(xh, LDB, 32 * kk), bl_ = frag(xl, LDB, 32 * kk);
+        for (int kk = 0; kk < 2; ++kk)
 #pragma unroll
             for (int tm = 0; tm < 4; ++tm) {
-                const int r = 16 * tm + n, q = 4 * kk + g;
-                const bf16x8_t mh = __builtin_bit_cast(bf16x8_t, slot[r * 8 + (q ^ (r & 7))]);
-                const bf16x8_t ml = __builtin_bit_cast(bf16x8_t, slot[512 + r * 8 + (q ^ (r & 7))]);
-                Y[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh, bh_, Y[tm], 0, 0, 0);
-                Z[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mh, bl_, Z[tm], 0, 0, 0);
-                Z[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ml, bh_, Z[tm], 0, 0, 0);
+                const int r = 16 * tm + n, o = 8 * r + ((4 * kk + g) ^ (r >> 1 & 7));
+                m.mh[kk][tm] = __builtin_bit_cast(bf16x8_t, slot[o]);
+                m.ml[kk][tm] = __builtin_bit_cast(bf16x8_t, slot[512 + o]);
             }
+    };
+    auto step = [&](int s, Step &m, Step &next) {
+        uint16_t *xh = sm.xs[s & 1][w][0], *xl = sm.xs[s & 1][w][1];
+        bf16x8_t bh_[2], bl_[2];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            uint32_t hi[4], lo[4];  // pairs of rows
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float x0 = X[2 * kk + e / 2][2 * (e & 1)], x1 = X[2 * kk + e / 2][2 * (e & 1) + 1];
+                hi[e] = bf16_pack2(x0, x1);
+                lo[e] = bf16_pack2(x0 - __uint_as_float(hi[e] << 16), x1 - __uint_as_float(hi[e] & 0xFFFF0000u));
+            }
+            const int o = n * LDB + 32 * kk + 4 * g;
+            *reinterpret_cast<uint2 *>(xh + o) = make_uint2(hi[0], hi[1]);
+            *reinterpret_cast<uint2 *>(xh + o + 16) = make_uint2(hi[2], hi[3]);
+            *reinterpret_cast<uint2 *>(xl + o) = make_uint2(lo[0], lo[1]);
+            *reinterpret_cast<uint2 *>(xl + o + 16) = make_uint2(lo[2], lo[3]);
+            bh_[kk] = __builtin_bit_cast(bf16x8_t, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+            bl_[kk] = __builtin_bit_cast(bf16x8_t, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        }
+        f32x4 Z[4];
+#pragma unroll
+        for (int tm = 0; tm < 4; ++tm) Z[tm] = zero4();
+        auto product = [&](int kk) {  // a tile's three products apart, none waits for the last
+#pragma unroll
+            for (int tm = 0; tm < 4; ++tm)
+                m.n[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m.mh[kk][tm], bh_[kk], m.n[tm], 0, 0, 0);
+#pragma unroll
+            for (int tm = 0; tm < 4; ++tm)
+                Z[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m.ml[kk][tm], bh_[kk], Z[tm], 0, 0, 0);
+#pragma unroll
+            for (int tm = 0; tm < 4; ++tm)
+                Z[tm] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(m.mh[kk][tm], bl_[kk], Z[tm], 0, 0, 0);
+        };
+        product(0);
+        __builtin_amdgcn_sched_barrier(0);
+        // The X^T tiles are in LDS, and this step's M and N are out of their slots.
+        __builtin_amdgcn_s_waitcnt(AS_LGKMCNT_ZERO);
+        as_barrier();
+        read(s + 1, next);
+        product(1);
+#pragma unroll
+        for (int i = 0; i < 12; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);  // LDS reads
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
         }
 #pragma unroll
         for (int tm = 0; tm < 4; ++tm)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) X[tm][i] = Y[tm][i] + Z[tm][i];
+            for (int i = 0; i < 4; ++i) X[tm][i] = m.n[tm][i] + Z[tm][i];
+    };
+    as_barrier();  // chunk 0's M and N are in their slots
+    Step even, odd;
+    read(0, even);
+    int s = 0;
+    for (; s + 1 < p.nc; s += 2) {
+        step(s, even, odd);
+        step(s + 1, odd, even);
     }
+    if (s < p.nc) step(s, even, odd);
     if (p.xout)
 #pragma unroll
         for (int tm = 0; tm < 4; ++tm)
