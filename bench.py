@@ -102,7 +102,7 @@ def traffic_from_counters(fetch_dir, write_dir, out_path, probe_bytes):
     import re
 
     def stage_of(name):
-        """The stage of a chunk-family kernel (chunk_, cw_, wide_, fc_ prefixes
+        """The stage of a chunk-family kernel (chunk_, wide_, fc_, fs_ prefixes
         share the stage names); the factored scans split into state_scan and
         adjoint_scan by their direction template argument; "neg" is the probe."""
         if "neg_kernel" in name:
@@ -115,11 +115,11 @@ def traffic_from_counters(fetch_dir, write_dir, out_path, probe_bytes):
             cfg = re.search(r"LrCfg<([^>]*)>", name)
             bwd = cfg is not None and cfg.group(1).split(",")[5].strip() == "true"
             return "adjoint_scan" if bwd else "state_scan"
-        if base == "fc_scan":  # fc_scan_kernel<KT, reverse>
-            return "adjoint_scan" if "true>" in name else "state_scan"
+        if base == "fc_scan":  # fc_scan_kernel<KT, reverse, ...>
+            return "adjoint_scan" if re.search(r"fc_scan_kernel<\d+, true", name) else "state_scan"
         if base == "affine_scan":  # affine_scan_kernel<reverse> (d = 64 dense maps)
             return "adjoint_scan" if "<true>" in name else "state_scan"
-        for pre in ("chunk_", "cw_", "wide_", "fc_"):
+        for pre in ("chunk_", "wide_", "fc_", "fs_"):
             if base.startswith(pre) and base[len(pre):] in ("prep", "out", "bprep", "bgrad"):
                 return "chunk_" + base[len(pre):]
         return None
