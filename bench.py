@@ -91,6 +91,31 @@ def load_profile(name):
     return data, "current"
 
 
+STAGES = ("chunk_prep", "state_scan", "chunk_out", "chunk_bprep", "adjoint_scan", "chunk_bgrad")
+
+
+def kernel_stage(name):
+    """(kernel, stage) of a profiler's kernel name: the library's own name of the
+    kernel without its suffix, and the stage that it is (the chunk_, wide_, fc_ and
+    fs_ families share the stage names; a scan is state_scan or adjoint_scan by its
+    direction argument).  (None, None) for a kernel of another library."""
+    import re
+
+    m = re.search(r"gdn2::(?:\(anonymous namespace\)::)?(\w+?)_kernel", name)
+    if not m:
+        return None, None
+    base = m.group(1)
+    reverse = {"lr_scan": r"LrCfg<[^<>]*\btrue *>",        # its last argument
+               "fc_scan": r"fc_scan_kernel<\d+, true\b",  # its second
+               "affine_scan": r"affine_scan_kernel<true>"}.get(base)
+    if reverse:
+        return base, "adjoint_scan" if re.search(reverse, name) else "state_scan"
+    for pre in ("chunk_", "wide_", "fc_", "fs_"):
+        if base.startswith(pre) and base[len(pre):] in ("prep", "out", "bprep", "bgrad"):
+            return base, "chunk_" + base[len(pre):]
+    return base, None
+
+
 def traffic_from_counters(fetch_dir, write_dir, out_path, probe_bytes):
     """Per-launch HBM bytes of each kernel from two rocprofv3 --pmc runs.
     FETCH_SIZE and WRITE_SIZE are in KiB per dispatch; each is scaled by the
@@ -99,30 +124,9 @@ def traffic_from_counters(fetch_dir, write_dir, out_path, probe_bytes):
     written = its size)."""
     import csv
     import glob
-    import re
 
     def stage_of(name):
-        """The stage of a chunk-family kernel (chunk_, wide_, fc_, fs_ prefixes
-        share the stage names); the factored scans split into state_scan and
-        adjoint_scan by their direction template argument; "neg" is the probe."""
-        if "neg_kernel" in name:
-            return "neg"
-        m = re.search(r"gdn2::(\w+?)_kernel", name)
-        if not m:
-            return None
-        base = m.group(1)
-        if base == "lr_scan":
-            cfg = re.search(r"LrCfg<([^>]*)>", name)
-            bwd = cfg is not None and cfg.group(1).split(",")[5].strip() == "true"
-            return "adjoint_scan" if bwd else "state_scan"
-        if base == "fc_scan":  # fc_scan_kernel<KT, reverse, ...>
-            return "adjoint_scan" if re.search(r"fc_scan_kernel<\d+, true", name) else "state_scan"
-        if base == "affine_scan":  # affine_scan_kernel<reverse> (d = 64 dense maps)
-            return "adjoint_scan" if "<true>" in name else "state_scan"
-        for pre in ("chunk_", "wide_", "fc_", "fs_"):
-            if base.startswith(pre) and base[len(pre):] in ("prep", "out", "bprep", "bgrad"):
-                return "chunk_" + base[len(pre):]
-        return None
+        return "neg" if "neg_kernel" in name else kernel_stage(name)[1]  # the probe
 
     def read(folder, counter):
         rows = {}
@@ -154,8 +158,7 @@ def traffic_from_counters(fetch_dir, write_dir, out_path, probe_bytes):
     out = {"sources": sources_digest(), "fetch_scale": f_scale, "write_scale": w_scale,
            "probe_bytes": probe_bytes, "bytes_per_launch": {}, "fetch_bytes": {},
            "write_bytes": {}}
-    for stage in ("chunk_prep", "state_scan", "chunk_out", "chunk_bprep", "adjoint_scan",
-                  "chunk_bgrad"):
+    for stage in STAGES:
         if stage in fetch and stage in write:
             fb = sum(v for v, _ in fetch[stage]) / len(fetch[stage]) * 1024.0 * f_scale
             wb = sum(v for v, _ in write[stage]) / len(write[stage]) * 1024.0 * w_scale
@@ -904,7 +907,6 @@ def mfma_from_counters(pmc_dir, out_path):
     reported beside its achieved fraction of the bf16 peak as the check."""
     import csv
     import glob
-    import re
 
     files = glob.glob(os.path.join(pmc_dir, "**", "*counter_collection.csv"), recursive=True)
     if not files:
@@ -914,16 +916,11 @@ def mfma_from_counters(pmc_dir, out_path):
         with open(path) as f:
             for r in csv.DictReader(f):
                 name = r["Kernel_Name"]
-                m = re.search(r"gdn2::(\w+?)_kernel", name)
-                key = m.group(1) if m else ("gemm" if ("Cijk" in name or "gemm" in name.lower())
-                                            else None)
+                base, stage = kernel_stage(name)
+                key = stage or base or ("gemm" if "Cijk" in name or "gemm" in name.lower()
+                                        else None)
                 if key is None:
                     continue
-                if key == "affine_scan":  # affine_scan_kernel<reverse>
-                    key = "affine_scan_rev" if "<true>" in name else "affine_scan_fwd"
-                elif key == "lr_scan":  # the factored scan: LrCfg<..., reverse, lo>
-                    args = name[name.find("LrCfg<") + 6:].split(",")
-                    key = "lr_scan_rev" if len(args) > 5 and args[5].strip() == "true" else "lr_scan_fwd"
                 d = per.setdefault(key, {}).setdefault(r.get("Dispatch_Id", r.get("Correlation_Id")),
                                                        {})
                 d[r["Counter_Name"]] = d.get(r["Counter_Name"], 0.0) + float(r["Counter_Value"])
@@ -935,14 +932,9 @@ def mfma_from_counters(pmc_dir, out_path):
                 if v.get("GRBM_GUI_ACTIVE") and "SQ_VALU_MFMA_BUSY_CYCLES" in v]
         if vals:
             busy[key] = sorted(vals)[len(vals) // 2]
-    names = {"chunk_prep": "chunk_prep", "chunk_out": "chunk_out", "chunk_bprep": "chunk_bprep",
-             "chunk_bgrad": "chunk_bgrad",
-             "wide_prep": "chunk_prep", "wide_out": "chunk_out", "wide_bprep": "chunk_bprep",
-             "wide_bgrad": "chunk_bgrad", "lr_scan_fwd": "state_scan", "lr_scan_rev": "adjoint_scan",
-             "affine_scan_fwd": "state_scan", "affine_scan_rev": "adjoint_scan"}
     out = {"sources": sources_digest(),
            "formula": "SQ_VALU_MFMA_BUSY_CYCLES / (GRBM_GUI_ACTIVE / 8 x 256 CUs x 4 SIMDs)",
-           "mfma_busy": {names[k]: v for k, v in busy.items() if k in names},
+           "mfma_busy": {k: busy[k] for k in STAGES if k in busy},
            "calibration_gemm_busy": busy.get("gemm")}
     text = json.dumps(out, indent=1)
     print(text)
