@@ -53,6 +53,24 @@ __device__ __forceinline__ f32x4 fc_mma4(const f32x4 &a, const f32x4 &b, f32x4 c
     for (int r = 0; r < 4; ++r) c = fc_mma(a[r], b[r], c);
     return c;
 }
+// x[0] = the sum of x[0] .. x[N - 1] (N a power of two), pairwise: each 16-channel
+// tile's product first and the tiles in a tree, as a chain of 64 or 128 f32 additions
+// has twice the error.
+template <int N>
+__device__ __forceinline__ void fc_tree(f32x4 (&x)[N]) {
+#pragma unroll
+    for (int w = 1; w < N; w *= 2)
+#pragma unroll
+        for (int i = 0; i < N; i += 2 * w) x[i] += x[i + w];
+}
+template <int N>
+__device__ __forceinline__ f32x4 fc_mma_tree(const f32x4 (&a)[N], const f32x4 (&b)[N]) {
+    f32x4 x[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = fc_mma4(a[i], b[i], zero4());
+    fc_tree(x);
+    return x[0];
+}
 __device__ __forceinline__ f32x4 fc_rows(float x, int g) {  // rows 4 g + i of a per-token value (lane n: token n)
     return f32x4{__shfl(x, 4 * g), __shfl(x, 4 * g + 1), __shfl(x, 4 * g + 2), __shfl(x, 4 * g + 3)};
 }

@@ -23,25 +23,39 @@ namespace gdn2 {
 
 namespace {
 
+// The decays are formed in f64 and rounded once.  One decay serves every channel
+// of a head, so its rounding does not average out over the channel sums, as the
+// token walk's does: f32 products were the largest term of the outputs' error
+// (1.6e-7 of 2.5e-7 at 64 x 64, in an emulation of the sums).
+__device__ __forceinline__ double fs_join(int hi, int lo) {
+    return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+__device__ __forceinline__ int fs_hi(double x) { return (int)(__builtin_bit_cast(uint64_t, x) >> 32); }
+__device__ __forceinline__ int fs_lo(double x) { return (int)__builtin_bit_cast(uint64_t, x); }
+template <int CTRL>  // x of the lane that CTRL names within the 16-lane row, 1 past its start
+__device__ __forceinline__ double fs_shifted(double x) {
+    return fs_join(__builtin_amdgcn_update_dpp(fs_hi(1.), fs_hi(x), CTRL, 0xF, 0xF, false),
+                   __builtin_amdgcn_update_dpp(0, fs_lo(x), CTRL, 0xF, 0xF, false));
+}
 // Inclusive product over the tokens of lanes 0 .. n of a 16-lane row.
-__device__ __forceinline__ float fs_scan_mul(float x) {
-    const int one = __builtin_bit_cast(int, 1.f);
-    x *= __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(one, __builtin_bit_cast(int, x), 0x111, 0xF, 0xF, false));
-    x *= __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(one, __builtin_bit_cast(int, x), 0x112, 0xF, 0xF, false));
-    x *= __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(one, __builtin_bit_cast(int, x), 0x114, 0xF, 0xF, false));
-    return x * __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(one, __builtin_bit_cast(int, x), 0x118, 0xF, 0xF, false));
+__device__ __forceinline__ double fs_scan_mul(double x) {
+    x *= fs_shifted<0x111>(x);
+    x *= fs_shifted<0x112>(x);
+    x *= fs_shifted<0x114>(x);
+    return x * fs_shifted<0x118>(x);
 }
 
 // D_ts at t = 4 g + i, s = n (t >= s, else unspecified), and lam_n = D_15,n.
-__device__ __forceinline__ f32x4 fs_decay_rows(float a, int g, int n, float &lam) {
+__device__ __forceinline__ f32x4 fs_decay_rows(double a, int g, int n, float &lam) {
     f32x4 d = zero4();
-    float p = 0.f;
+    double p = 0.;
 #pragma unroll
     for (int t = 0; t < C; ++t) {
-        p = t == n ? 1.f : p * fc_lane(a, t);
-        if ((t >> 2) == g) d[t & 3] = p;
+        const double at = fs_join(__builtin_amdgcn_readlane(fs_hi(a), t), __builtin_amdgcn_readlane(fs_lo(a), t));
+        p = t == n ? 1. : p * at;
+        if ((t >> 2) == g) d[t & 3] = (float)p;
     }
-    lam = p;
+    lam = (float)p;
     return d;
 }
 
@@ -70,10 +84,11 @@ __global__ void __launch_bounds__(64) fs_prep_kernel(FcArgs a) {
     fc_flags(s, b, c, on, rst);
     const int tc = min(tg, s.T - 1);
     const float bv = ld4<float>(s.beta, b, tc, h, 0), gl = ld4<float>(s.g, b, tc, h, 0);
-    const float beta = on ? bv : 0.f, av = on ? (rst ? 0.f : expf(gl)) : 1.f;
+    const float beta = on ? bv : 0.f;
+    const double av = on ? (rst ? 0. : exp((double)gl)) : 1.;
     const f32x4 on4 = fc_rows(on ? 1.f : 0.f, g);
-    f32x4 kb[KM], qb[KM], kk = zero4(), qk = zero4();
-    float ksq = 0.f, lam;
+    f32x4 kb[KM], qb[KM], kk[KM], qk[KM], ksq4 = zero4();
+    float lam;
     const f32x4 d = fs_decay_rows(av, g, n, lam);
     const FcOff oc(C);
 #pragma unroll
@@ -85,40 +100,49 @@ __global__ void __launch_bounds__(64) fs_prep_kernel(FcArgs a) {
         const f32x4 kf = fc_keep(sk.frag(tt), on && in), qf = fc_keep(sq.frag(tt), on && in);
         kb[tau] = fc_keep4(sk.col(tt), on4);
         qb[tau] = fc_keep4(sq.col(tt), on4);
-        kk = fc_mma4(kf, kf, kk);
-        qk = fc_mma4(qf, kf, qk);  // row t = 4 g + i, column s = n
-#pragma unroll
-        for (int r = 0; r < 4; ++r) ksq += kf[r] * kf[r];
+        kk[tau] = fc_mma4(kf, kf, zero4());
+        qk[tau] = fc_mma4(qf, kf, zero4());  // row t = 4 g + i, column s = n
+        ksq4 += kf * kf;
     }
-    const float bn = fs_scan_mul(av);
+    fc_tree(kk);
+    fc_tree(qk);
+    const float bn = (float)fs_scan_mul(av);
     const f32x4 be4 = fc_rows(beta, g), b4 = fc_rows(bn, g), lam4 = fc_rows(lam, g);
     f32x4 A, P, D;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        A[i] = n < 4 * g + i ? be4[i] * d[i] * kk[i] : 0.f;
-        P[i] = n <= 4 * g + i ? d[i] * qk[i] : 0.f;
+        A[i] = n < 4 * g + i ? be4[i] * d[i] * kk[0][i] : 0.f;
+        P[i] = n <= 4 * g + i ? d[i] * qk[0][i] : 0.f;
         D[i] = n <= 4 * g + i ? d[i] : 0.f;
     }
     const f32x4 t = fc_inverse(A, la, g, n);
     fc_p4(a.tm + ci * C * C, (n * C + 4 * g) * 4, t);
     oc.put(a.pm + ci * C * C, P);
     oc.put(a.dm + ci * C * C, D);
-    ksq = fc_group_sum(ksq);
+    const float ksq = fc_group_sum((ksq4[0] + ksq4[1]) + (ksq4[2] + ksq4[3]));
     float *gb = a.gb + ci * C * 8;
     *fc_at(gb + C * g, 4 * n) = g == 0 ? (on ? 1.f : 0.f) : (g == 1 ? (rst ? 1.f : 0.f) : (g == 2 ? ksq : beta));
     if (g < 2) *fc_at(gb + C * (4 + g), 4 * n) = g == 0 ? bn : lam;
     const float b15 = fc_lane(bn, C - 1);
     for (int i = l; i < KP; i += 64) a.gv[ci * KP + i] = b15;
+    // T - I: the products with T add the rest to the operand itself, which is the
+    // larger term.
+    f32x4 t1 = t;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) t1[r] = 4 * g + r == n ? 0.f : t[r];
 #pragma unroll
     for (int tau = 0; tau < KM; ++tau)
         if (tau < KT) {
             const int64_t o = (ci * KT + tau) * 256;
-            fc_p4(a.fw + o, 16 * l, fc_mma4(t, b4 * be4 * kb[tau], zero4()));
+            const f32x4 bk = b4 * be4 * kb[tau];
+            fc_p4(a.fw + o, 16 * l, bk + fc_mma4(t1, bk, zero4()));
             fc_p4(a.fk + o, 16 * l, lam4 * kb[tau]);
             fc_p4(a.fq + o, 16 * l, b4 * qb[tau]);
         }
-    for (int vt = 0; vt < VT; ++vt)
-        fc_p4(a.fu + (ci * VT + vt) * 256, 16 * l, fc_mma4(t, be4 * fc_keep4(sv.col(vt), on4), zero4()));
+    for (int vt = 0; vt < VT; ++vt) {
+        const f32x4 bv = be4 * fc_keep4(sv.col(vt), on4);
+        fc_p4(a.fu + (ci * VT + vt) * 256, 16 * l, bv + fc_mma4(t1, bv, zero4()));
+    }
 }
 
 // ---- bgrad: every gradient of one chunk -------------------------------------------
@@ -166,10 +190,11 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
             if (tau < KT) kf[tau] = fc_across(fk + 256 * tau), dsn[tau] = fc_g4(ds + (w * KT + tau) * 256, 16 * l);
         }
         dO = fc_keep4(dO, on4);
-        f32x4 dd = fc_mma4(p, dO, cs4 * dl);
+        const f32x4 dd = fc_mma4(p, dO, cs4 * dl) + fc_mma_tree<KM>(kf, dsn);
+        f32x4 t1 = tb;  // T - I, as in prep
 #pragma unroll
-        for (int tau = 0; tau < KM; ++tau) dd = fc_mma4(kf[tau], dsn[tau], dd);
-        const f32x4 dr = fc_mma4(tb, dd, zero4());                                               // rows t, column j
+        for (int i = 0; i < 4; ++i) t1[i] = 4 * g + i == n ? 0.f : tb[i];
+        const f32x4 dr = dd + fc_mma4(t1, dd, zero4());                                          // rows t, column j
         *reinterpret_cast<f32x4 *>(&sm.dr[n * LD + 16 * w + 4 * g]) = fc_mma4(dd, tb, zero4());  // rows j, column t
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -191,14 +216,18 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
     // The decayed adjoint tiles: 0 dP D and 1 dA D with column t (row s), 2 dP D
     // and 3 beta dA D with column s (row t); with the last two, E's terms.
     for (int x = w; x < 4; x += NW) {
-        f32x4 m = zero4();
+        f32x4 mv[KM];
 #pragma unroll
-        for (int vt = 0; vt < KM; ++vt)
+        for (int vt = 0; vt < KM; ++vt) {
+            mv[vt] = zero4();
             if (vt < VT) {
                 const f32x4 d = *reinterpret_cast<const f32x4 *>(&sm.dl[n * LD + 16 * vt + 4 * g]);
                 const f32x4 y = (x & 1) ? -*reinterpret_cast<const f32x4 *>(&sm.dr[n * LD + 16 * vt + 4 * g]) : yf[vt];
-                m = x < 2 ? fc_mma4(d, y, m) : fc_mma4(y, d, m);
+                mv[vt] = x < 2 ? fc_mma4(d, y, zero4()) : fc_mma4(y, d, zero4());
             }
+        }
+        fc_tree(mv);
+        const f32x4 m = mv[0];
         const float *dm = a.dm + ci * C * C;
         const f32x4 d = x < 2 ? fc_g4(dm, (n * C + 4 * g) * 4) : oc.get(dm);  // zero above the diagonal
         f32x4 md = m * d;
@@ -214,18 +243,23 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
         if (x == 3) {
             md = md * be4;
             const FcSrc<BF, VEC> sk(s.k, b, h, c, s.T, K);
-            f32x4 kk = zero4();
+            f32x4 kk[KM];
 #pragma unroll
-            for (int tau = 0; tau < KM; ++tau)
+            for (int tau = 0; tau < KM; ++tau) {
+                kk[tau] = zero4();
                 if (tau < KT) {
                     const f32x4 kf = fc_keep(sk.frag(tau), on);
-                    kk = fc_mma4(kf, kf, kk);
+                    kk[tau] = fc_mma4(kf, kf, kk[tau]);
                 }
-            sm.e[1][l] = md * kk;
+            }
+            fc_tree(kk);
+            sm.e[1][l] = md * kk[0];
         }
         sm.m[x][l] = md;
     }
-    f32x4 Qb = zero4(), Ab = zero4(), Kl = zero4();  // rows t, column key 16 w + n
+    f32x4 Qb[4], Ab[4], Kl[4];  // rows t, column key 16 w + n: four partial sums
+#pragma unroll
+    for (int i = 0; i < 4; ++i) Qb[i] = Ab[i] = Kl[i] = zero4();
     float fr = 0.f;
     if (w < KT)
 #pragma unroll
@@ -234,24 +268,27 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
                 const f32x4 s0 = fc_across(st + (vt * KT + w) * 256), d1 = fc_across(ds + (vt * KT + w) * 256);
                 const f32x4 d = *reinterpret_cast<const f32x4 *>(&sm.dl[n * LD + 16 * vt + 4 * g]);
                 const f32x4 r = *reinterpret_cast<const f32x4 *>(&sm.dr[n * LD + 16 * vt + 4 * g]);
-                Qb = fc_mma4(bn * yf[vt], s0, Qb);
-                Ab = fc_mma4(-bn * r, s0, Ab);
-                Kl = fc_mma4(lam * d, d1, Kl);
+                Qb[vt & 3] = fc_mma4(bn * yf[vt], s0, Qb[vt & 3]);
+                Ab[vt & 3] = fc_mma4(-bn * r, s0, Ab[vt & 3]);
+                Kl[vt & 3] = fc_mma4(lam * d, d1, Kl[vt & 3]);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) fr += s0[i] * d1[i];
             }
+    fc_tree(Qb);
+    fc_tree(Ab);
+    fc_tree(Kl);
     fr = fc_group_sum(fc_row_sum(fr));
     if (l == 0) sm.fr[w] = fr;
     __syncthreads();
     if (w < KT) {
-        const f32x4 dq = fc_mma4(sm.m[0][l], kb, Qb), de = fc_mma4(sm.m[1][l], kb, Ab);
-        const f32x4 dk = fc_mma4(sm.m[2][l], qb, fc_mma4(sm.m[3][l], kb, Kl));
+        const f32x4 dq = Qb[0] + fc_mma4(sm.m[0][l], kb, zero4()), de = Ab[0] + fc_mma4(sm.m[1][l], kb, zero4());
+        const f32x4 dk = Kl[0] + (fc_mma4(sm.m[2][l], qb, zero4()) + fc_mma4(sm.m[3][l], kb, zero4()));
         if (s.dq) fc_put<BF, VEC>(s.dq, BF, s, b, h, c, K, w, fc_keep4(dq, on4));
         if (s.dk) fc_put<BF, VEC>(s.dk, BF, s, b, h, c, K, w, fc_keep4(dk + be4 * de + ck4 * kb, on4));
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float ys = fc_row_sum(be4[i] * kb[i] * Ab[i] + qb[i] * Qb[i]);
-            const float zs = fc_row_sum(kb[i] * Kl[i]), kd = fc_row_sum(kb[i] * de[i]);
+            const float ys = fc_row_sum(be4[i] * kb[i] * Ab[0][i] + qb[i] * Qb[0][i]);
+            const float zs = fc_row_sum(kb[i] * Kl[0][i]), kd = fc_row_sum(kb[i] * de[i]);
             if (n == 0) sm.ys[w][4 * g + i] = ys, sm.zs[w][4 * g + i] = zs, sm.kd[w][4 * g + i] = kd;
         }
     }
@@ -270,7 +307,7 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
     }
     __syncthreads();
     if (threadIdx.x < C && tg < s.T) {
-        float db = 0.f, dg = wu, f = 0.f;
+        double db = 0., dg = wu, f = 0.;  // one thread a token, a term for every tile
         for (int x = 0; x < VT; ++x) db += sm.vd[x][n];
         for (int x = 0; x < KT; ++x) {
             db += sm.kd[x][n];
@@ -280,8 +317,8 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
         for (int x = 0; x < NW; ++x) f += sm.fr[x];
         dg += fc_lane(bn, C - 1) * f;
         const int64_t o = ((int64_t)b * s.T + tg) * s.H + h;
-        if (s.dbeta) s.dbeta[o] = on ? db : 0.f;
-        if (s.dg) s.dg[o] = (on && fc_gb(a, ci, 1) == 0.f) ? dg : 0.f;
+        if (s.dbeta) s.dbeta[o] = on ? (float)db : 0.f;
+        if (s.dg) s.dg[o] = (on && fc_gb(a, ci, 1) == 0.f) ? (float)dg : 0.f;
     }
 }
 
