@@ -110,11 +110,6 @@ int check_out_dtype(int32_t dt) {
     return GDN2_OK;
 }
 
-size_t seq_checkpoint_bytes(const gdn2_shape *s) {
-    return (size_t)seq_checkpoint_floats(s->batch, s->time, s->heads, (int)s->keys,
-                                         (int)s->values) * 4;
-}
-
 size_t seq_workspace_bytes(const gdn2_shape *s) {
     return (size_t)seq_workspace_floats(s->batch, s->heads, (int)s->keys, (int)s->values) * 4;
 }
@@ -174,7 +169,11 @@ SeqArgs seq_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_view *k, co
 // device's copy of the code object, held until the process ends.  Host code
 // never uses the array's name as an address: each device's address comes from
 // hipGetSymbolAddress, taken once per device with that device current.
-static __device__ __align__(256) unsigned char scratch[GDN2_NOALLOC_SCRATCH_BYTES];
+// The bytes past the public size take the f32 chunk kernels' words of a shape whose
+// other needs fill it: at most 1024, as the token walk needs 64 KiB or more for
+// each batch and head.
+constexpr size_t kScratchBytes = GDN2_NOALLOC_SCRATCH_BYTES + 4096;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
 constexpr int kMaxDevices = 64;
@@ -416,25 +415,16 @@ int gdn2_backward(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *
     return launch_status(launch_fc_bwd(f, (hipStream_t)stream, ev), "gdn2_backward");
 }
 
-size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
-    if (check_shape(shape) || check_chunk(chunk)) return 0;
-    // Large enough for whichever kernel family the call will select.
-    size_t c = 0;
-    if (chunk_eligible_shape(shape, chunk))
-        c = chunk_checkpoint_bytes(shape->batch, shape->time, shape->heads);
-    else if (wide_eligible_shape(shape, chunk))
-        c = wide_checkpoint_bytes(shape->batch, shape->time, shape->heads);
-    const size_t f = fc_checkpoint_bytes(shape->batch, shape->time, shape->heads, (int)shape->keys,
-                                         (int)shape->values, true);
-    return std::max(std::max(c, f), seq_checkpoint_bytes(shape));
-}
+}  // extern "C"
 
-// The f32 chunk kernels' backward walks windows of chunks that fit whatever
-// workspace it is given, so their share is capped: 64 MiB holds 4064 chunks of
+static bool use_seq_path(const gdn2_shape *shape) { return shape->time <= FC_C; }
+
+// The scalar-gate backward's workspace without the f32 chunk kernels' words (one per
+// batch and head).  Their backward walks windows of chunks that fit whatever
+// workspace it is given, so its share is capped: 64 MiB holds 4064 chunks of
 // 64 x 64, enough to fill the chip, and keeps every shape whose other needs fit
 // the library's fixed scratch within it (gdn_scalar_backward_noalloc).
-size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
-    if (check_shape(shape) || check_chunk(chunk)) return 0;
+static size_t scalar_workspace_base(const gdn2_shape *shape, int chunk) {
     size_t c = 0;
     if (chunk_eligible_shape(shape, chunk))
         c = chunk_workspace_bytes(shape->batch, shape->time, shape->heads);
@@ -443,6 +433,32 @@ size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
     const size_t f = fc_workspace_bytes(shape->batch, shape->time, shape->heads, (int)shape->keys,
                                         (int)shape->values);
     return std::max(std::max(c, std::min(f, (size_t)GDN2_NOALLOC_SCRATCH_BYTES)), seq_workspace_bytes(shape));
+}
+
+extern "C" {
+
+size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
+    if (check_shape(shape) || check_chunk(chunk)) return 0;
+    size_t c = 0;
+    if (chunk_eligible_shape(shape, chunk))
+        c = chunk_checkpoint_bytes(shape->batch, shape->time, shape->heads);
+    else if (wide_eligible_shape(shape, chunk))
+        c = wide_checkpoint_bytes(shape->batch, shape->time, shape->heads);
+    const int K = (int)shape->keys, V = (int)shape->values;
+    return std::max(c, use_seq_path(shape)
+                           ? fc_walk_checkpoint_bytes(shape->batch, shape->time, shape->heads, K, V)
+                           : fc_checkpoint_bytes(shape->batch, shape->time, shape->heads, K, V, true));
+}
+
+size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
+    if (check_shape(shape) || check_chunk(chunk)) return 0;
+    const size_t base = scalar_workspace_base(shape, chunk);
+    if (use_seq_path(shape)) return base;
+    const size_t words = fc_word_bytes(shape->batch, shape->heads);
+    const size_t f = fc_workspace_bytes(shape->batch, shape->time, shape->heads, (int)shape->keys,
+                                        (int)shape->values) + words;
+    return std::max(base, std::max(std::min(f, (size_t)GDN2_NOALLOC_SCRATCH_BYTES),
+                                   seq_workspace_bytes(shape) + words));
 }
 
 // The chunk-WY MFMA kernels take bf16 q/k/v with d_k = d_v = 64 (gdn2_chunk.hip)
@@ -485,8 +501,6 @@ static ChunkArgs chunk_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_
     return a;
 }
 
-static bool use_seq_path(const gdn2_shape *shape) { return shape->time <= FC_C; }
-
 // The token-sequential argument block of the scalar-gate op.
 static SeqArgs scalar_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_view *k,
                            const gdn2_view *v, const gdn2_view *beta, const gdn2_view *g,
@@ -496,6 +510,12 @@ static SeqArgs scalar_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_v
     a.beta = make_view(beta);
     a.g = make_view(g);
     return a;
+}
+
+// The token walk's arrays of a checkpoint.
+static void bind_walk(SeqArgs &a, const void *checkpoint) {
+    a.st = (float *)const_cast<void *>(checkpoint);
+    a.fu = a.st + (int64_t)a.B * a.H * a.nck * fc_kp(a.K) * fc_kp(a.V);
 }
 
 static int check_scalar_inputs(const gdn2_view *q, const gdn2_view *k, const gdn2_view *v,
@@ -549,7 +569,7 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
     a.final_state = final_state;
     a.scores = scores;
     if (use_seq_path(shape)) {
-        seq_bind_checkpoint(a, checkpoint);
+        bind_walk(a, checkpoint);
         return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_scan");
     }
@@ -581,7 +601,7 @@ int gdn_scalar_backward_noalloc(const gdn2_shape *shape, int chunk, const gdn2_v
                                 void *stream) {
     GDN2_TRY(check_shape(shape));
     GDN2_TRY(check_chunk(chunk));
-    const size_t need = gdn_scalar_workspace_bytes(shape, chunk);
+    const size_t need = scalar_workspace_base(shape, chunk);
     if (need > GDN2_NOALLOC_SCRATCH_BYTES)
         return fail(GDN2_ERR_WORKSPACE,
                     "gdn_scalar_backward_noalloc: this shape needs %zu bytes of scratch, above "
@@ -592,7 +612,7 @@ int gdn_scalar_backward_noalloc(const gdn2_shape *shape, int chunk, const gdn2_v
     GDN2_TRY(noalloc_scratch(&ws));
     return scalar_backward_impl(shape, chunk, q, k, v, beta, g, valid, reset, checkpoint,
                                 checkpoint_bytes, d_output, d_final_state, d_scores, dq, dk, dv,
-                                dbeta, dg, d_initial, ws, GDN2_NOALLOC_SCRATCH_BYTES, stream);
+                                dbeta, dg, d_initial, ws, kScratchBytes, stream);
 }
 
 }  // extern "C"
@@ -659,7 +679,7 @@ static int scalar_backward_impl(const gdn2_shape *shape, int chunk, const gdn2_v
     a.dg = dg;
     a.dinitial = d_initial;
     if (use_seq_path(shape)) {
-        seq_bind_checkpoint(a, checkpoint);
+        bind_walk(a, checkpoint);
         a.replay = (float *)workspace;
         return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_backward");
@@ -731,7 +751,6 @@ int gdn2_decode_step(const gdn2_shape *shape, const gdn2_view *q, const gdn2_vie
     a.out = output;
     a.out_bf16 = output_dtype == GDN2_BF16;
     a.scores = scores;
-    seq_bind_checkpoint(a, nullptr);
     return launch_status(launch_seq_decode(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                          "gdn2_decode_step");
 }

@@ -29,13 +29,18 @@ constexpr int FC_C = 16;  // tokens per chunk
 //   gv     b_15 (the map's diagonal), [KP]
 //   gb     rows of one value per token: valid, reset, |k|^2, and with scalar gates
 //          beta, b, lam; [8][16]
+// and, with scalar gates, one word per (batch, head):
+//   bad    the forward gave a value that is not finite (out); such a (batch, head)
+//          is walked by token afterwards (gdn2_chunk_fs.hip)
+// st and fu come first: they are all that the token walk keeps.
 // KP = d_k and VP = d_v rounded up to 16 (KT = KP / 16, VT = VP / 16): the tiles
 // are padded with zeros to whole 16 x 16 MFMA tiles.  Backward workspace: ds, the
 // state adjoint at each chunk end, packed like st, and, with a score adjoint, sc,
 // the coefficients c and c' per token [2][16], for the window of chunks w0 .. w0 +
 // wn - 1 of each (batch, head) (index bh * wn + c - w0; all nc chunks unless the
 // scalar-gate path walks windows); carry is the adjoint before the window, packed,
-// one state per (batch, head).  st and ds are zero outside K x V.  Every array
+// one state per (batch, head), and wbad the backward's counterpart of bad, at the
+// workspace's end.  st and ds are zero outside K x V.  Every array
 // starts on a 16-byte boundary when the caller's buffer does.
 struct FcArgs {
     SeqArgs s;
@@ -44,10 +49,11 @@ struct FcArgs {
     int vec;      // every input of the call passes fc_vec_view
     int scalar;   // scalar gates
     int nonneg;   // a negative alpha poisons its sequence with NaN
-    float *st, *tm, *pm, *dm, *fw, *fk, *fq, *fu, *gv, *gb;
+    float *st, *fu, *tm, *pm, *dm, *fw, *fk, *fq, *gv, *gb;
     float *ds, *sc;
     int w0, wn;
     float *carry;
+    int *bad, *wbad;  // null with channel-wise gates
 };
 
 inline int64_t fc_chunks(int64_t B, int64_t T, int64_t H) { return B * H * ((T + FC_C - 1) / FC_C); }
@@ -67,19 +73,29 @@ constexpr int FC_PARTS = 10;
 inline void fc_checkpoint_parts(int64_t n, int K, int V, bool scalar, size_t part[FC_PARTS]) {
     const size_t KP = fc_kp(K), VP = fc_kp(V);
     part[0] = n * KP * VP;                      // st
-    part[1] = part[2] = n * FC_C * FC_C;        // tm, pm
-    part[3] = scalar ? n * FC_C * FC_C : 0;     // dm
-    part[4] = part[5] = part[6] = n * FC_C * KP;  // fw, fk, fq
-    part[7] = n * FC_C * VP;                    // fu
+    part[1] = n * FC_C * VP;                    // fu
+    part[2] = part[3] = n * FC_C * FC_C;        // tm, pm
+    part[4] = scalar ? n * FC_C * FC_C : 0;     // dm
+    part[5] = part[6] = part[7] = n * FC_C * KP;  // fw, fk, fq
     part[8] = n * KP;                           // gv
     part[9] = n * FC_C * 8;                     // gb
 }
+
+// Bytes of one word per (batch, head), whole 16-byte pieces.
+inline size_t fc_word_bytes(int64_t B, int64_t H) { return ((size_t)(B * H) * 4 + 15) & ~(size_t)15; }
 
 inline size_t fc_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V, bool scalar) {
     size_t part[FC_PARTS], total = 0;
     fc_checkpoint_parts(fc_chunks(B, T, H), K, V, scalar, part);
     for (size_t x : part) total += x;
-    return total * sizeof(float);
+    return total * sizeof(float) + (scalar ? fc_word_bytes(B, H) : 0);
+}
+
+// What the token walk keeps: st and fu.
+inline size_t fc_walk_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V) {
+    size_t part[FC_PARTS];
+    fc_checkpoint_parts(fc_chunks(B, T, H), K, V, true, part);
+    return (part[0] + part[1]) * sizeof(float);
 }
 
 // Floats of the workspace per chunk.
@@ -94,11 +110,12 @@ inline void fc_bind(FcArgs &a, void *ck, void *ws) {
     size_t part[FC_PARTS];
     fc_checkpoint_parts(n, a.s.K, a.s.V, a.scalar != 0, part);
     float *p = static_cast<float *>(ck);
-    float **dst[FC_PARTS] = {&a.st, &a.tm, &a.pm, &a.dm, &a.fw, &a.fk, &a.fq, &a.fu, &a.gv, &a.gb};
+    float **dst[FC_PARTS] = {&a.st, &a.fu, &a.tm, &a.pm, &a.dm, &a.fw, &a.fk, &a.fq, &a.gv, &a.gb};
     for (int i = 0; i < FC_PARTS; ++i) {
         *dst[i] = p;
         p += part[i];
     }
+    a.bad = a.scalar ? reinterpret_cast<int *>(p) : nullptr;
     a.w0 = 0;
     a.wn = a.nc;
     if (ws) {
@@ -115,8 +132,9 @@ void launch_fc_adjoint(const FcArgs &a, hipStream_t stream);
 
 hipError_t launch_fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
 hipError_t launch_fc_bwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
-// Scalar gates.  The backward takes any workspace that holds one chunk window
-// and the carry; the whole of fc_workspace_bytes is one window.
+// Scalar gates.  The backward takes any workspace that holds one chunk window, the
+// carry and the words, and the words behind the token walk's workspace; with
+// fc_workspace_bytes and the words it is one window.
 hipError_t launch_fs_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev);
 hipError_t launch_fs_bwd(const FcArgs &a, size_t ws_bytes, hipStream_t stream, const hipEvent_t *ev);
 

@@ -260,6 +260,7 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
     const bool jv = j < V, has_do = REV && s.dout.data != nullptr;
     const View dov = has_do ? s.dout : s.v;  // a missing dO reads v, zeroed where it is used
     const int steps = REV ? a.wn : a.nc;
+    if (REV && a.wbad && a.w0 + a.wn == a.nc && cg == 0 && threadIdx.x == 0) a.wbad[bh] = a.bad[bh];
     float *carry = a.carry + (((int64_t)bh * VT + cg) * KT + tau) * 256;
     f32x4 X;
     if (REV && a.w0 + a.wn < a.nc) {
@@ -438,6 +439,7 @@ __global__ void __launch_bounds__(512) fc_out_kernel(FcArgs a) {
     const f32x4 on4 = fc_gb4(a, ci, 0);
     const f32x4 o = fc_mma_tree<KM>(q, s0) + fc_mma4(p, dl, zero4());
     fc_put<false, VEC>(s.out, s.out_bf16, s, b, h, c, V, vt, fc_keep4(o, on4));
+    if (a.bad && !fc_finite(o + dl)) a.bad[bh] = 1;
     if (!s.scores) return;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {

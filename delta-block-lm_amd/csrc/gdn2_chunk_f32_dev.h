@@ -74,6 +74,10 @@ __device__ __forceinline__ f32x4 fc_mma_tree(const f32x4 (&a)[N], const f32x4 (&
 __device__ __forceinline__ f32x4 fc_rows(float x, int g) {  // rows 4 g + i of a per-token value (lane n: token n)
     return f32x4{__shfl(x, 4 * g), __shfl(x, 4 * g + 1), __shfl(x, 4 * g + 2), __shfl(x, 4 * g + 3)};
 }
+__device__ __forceinline__ bool fc_finite(const f32x4 &x) {  // every element (a sum that overflows counts as not)
+    const float z = (x[0] + x[1]) + (x[2] + x[3]);
+    return z - z == 0.f;
+}
 __device__ __forceinline__ f32x4 fc_keep(f32x4 x, bool on) { return on ? x : zero4(); }
 __device__ __forceinline__ f32x4 fc_keep4(f32x4 x, const f32x4 &on) {
 #pragma unroll

@@ -11,6 +11,13 @@
 // needs no special case.  The map's factors, the states, the scans and out are
 // gdn2_chunk_f32.hip's; prep and bgrad are here.
 //
+// A chunk's products multiply the terms past a token by zero, so a NaN or an
+// infinity at one token reaches the other tokens of its chunk, on both sides, which
+// the recurrence does not.  Out and bgrad therefore mark every (batch, head) that
+// gave a value that is not finite, and the token-sequential kernels (gdn2_seq.hip),
+// launched behind them, walk the marked ones again (the rest return at once): such
+// a sequence gets what the recurrence gives, token by token.
+//
 // At B8 T512 H8 K = V = 64 in f32, forward + backward takes 121 us of kernels
 // (prep 17, scans 20 and 29, out 11, bgrad 43) against 885 us of the
 // token-sequential kernels, which walk a head's tokens in one workgroup
@@ -80,6 +87,7 @@ __global__ void __launch_bounds__(64) fs_prep_kernel(FcArgs a) {
     const int K = s.K, V = s.V, KP = fc_kp(K), KT = KP >> 4, VT = (V + 15) >> 4;
     const int l = lane_id(), g = l >> 4, n = l & 15, tg = c * C + n;
     const FcSrc<BF, VEC> sk(s.k, b, h, c, s.T, K), sq(s.q, b, h, c, s.T, K), sv(s.v, b, h, c, s.T, V);
+    if (c == 0 && l == 0) a.bad[bh] = 0;
     bool on, rst;
     fc_flags(s, b, c, on, rst);
     const int tc = min(tg, s.T - 1);
@@ -202,7 +210,9 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
             const float x = fc_row_sum(v[r] * dr[r]);
             if (n == 0) sm.vd[w][4 * g + r] = x;
         }
-        if (s.dv) fc_put<BF, VEC>(s.dv, BF, s, b, h, c, V, w, fc_keep4(be4 * dr, on4));
+        const f32x4 dvt = fc_keep4(be4 * dr, on4);
+        if (s.dv) fc_put<BF, VEC>(s.dv, BF, s, b, h, c, V, w, dvt);
+        if (!fc_finite(dvt)) a.wbad[bh] = 1;
     }
     f32x4 yf[KM];  // dO rows
 #pragma unroll
@@ -283,8 +293,10 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
     if (w < KT) {
         const f32x4 dq = Qb[0] + fc_mma4(sm.m[0][l], kb, zero4()), de = Ab[0] + fc_mma4(sm.m[1][l], kb, zero4());
         const f32x4 dk = Kl[0] + (fc_mma4(sm.m[2][l], qb, zero4()) + fc_mma4(sm.m[3][l], kb, zero4()));
-        if (s.dq) fc_put<BF, VEC>(s.dq, BF, s, b, h, c, K, w, fc_keep4(dq, on4));
-        if (s.dk) fc_put<BF, VEC>(s.dk, BF, s, b, h, c, K, w, fc_keep4(dk + be4 * de + ck4 * kb, on4));
+        const f32x4 dqt = fc_keep4(dq, on4), dkt = fc_keep4(dk + be4 * de + ck4 * kb, on4);
+        if (s.dq) fc_put<BF, VEC>(s.dq, BF, s, b, h, c, K, w, dqt);
+        if (s.dk) fc_put<BF, VEC>(s.dk, BF, s, b, h, c, K, w, dkt);
+        if (!fc_finite(dqt + dkt)) a.wbad[bh] = 1;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float ys = fc_row_sum(be4[i] * kb[i] * Ab[0][i] + qb[i] * Qb[0][i]);
@@ -319,6 +331,7 @@ __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fs_bgrad_kernel(FcAr
         const int64_t o = ((int64_t)b * s.T + tg) * s.H + h;
         if (s.dbeta) s.dbeta[o] = on ? (float)db : 0.f;
         if (s.dg) s.dg[o] = (on && fc_gb(a, ci, 1) == 0.f) ? (float)dg : 0.f;
+        if (on && !(db - db == 0. && dg - dg == 0.)) a.wbad[bh] = 1;
     }
 }
 
@@ -333,6 +346,15 @@ static void fs_bgrad(const FcArgs &a, hipStream_t stream) {
                        stream, a);
 }
 
+// The token walk of the marked (batch, head)s on this call's checkpoint.
+static SeqArgs fs_walk(const FcArgs &a, const int *marked) {
+    SeqArgs s = a.s;
+    s.st = a.st;
+    s.fu = a.fu;
+    s.only = marked;
+    return s;
+}
+
 hipError_t launch_fs_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev) {
     fc_mark(ev, 0, stream);
     FC_DISPATCH(fc_kp(a.s.K) / 16, fs_prep, a, stream);
@@ -343,7 +365,7 @@ hipError_t launch_fs_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *
     fc_mark(ev, 4, stream);
     launch_fc_out(a, stream);
     fc_mark(ev, 5, stream);
-    return hipGetLastError();
+    return launch_seq_fwd(fs_walk(a, a.bad), a.in_bf16, stream);
 }
 
 hipError_t launch_fs_bwd(const FcArgs &whole, size_t ws_bytes, hipStream_t stream, const hipEvent_t *ev) {
@@ -352,9 +374,12 @@ hipError_t launch_fs_bwd(const FcArgs &whole, size_t ws_bytes, hipStream_t strea
     // Chunk windows, last first: as many chunks as the workspace holds, the
     // adjoint between two windows in the carry.
     const int64_t state = (int64_t)KT * VT * 256, carry = bh * state * 4, per = bh * fc_ws_chunk(a.s.K, a.s.V) * 4;
-    int64_t wn = (int64_t)ws_bytes / per;
-    if (wn < a.nc) wn = ((int64_t)ws_bytes - carry) / per;
-    if (wn < 1) return hipErrorInvalidValue;
+    const int64_t words = fc_word_bytes(a.s.B, a.s.H);
+    const int64_t room = ((int64_t)ws_bytes - words) & ~(int64_t)15;  // the words lie behind it
+    int64_t wn = room / per;
+    if (wn < a.nc) wn = (room - carry) / per;
+    if (wn < 1 || room < (int64_t)seq_workspace_floats(a.s.B, a.s.H, a.s.K, a.s.V) * 4) return hipErrorInvalidValue;
+    a.wbad = reinterpret_cast<int *>(reinterpret_cast<char *>(a.ds) + room);
     wn = std::min<int64_t>(wn, a.nc);
     a.sc = a.ds + wn * bh * state;
     a.carry = a.sc + wn * bh * 2 * C;
@@ -371,7 +396,9 @@ hipError_t launch_fs_bwd(const FcArgs &whole, size_t ws_bytes, hipStream_t strea
         FC_DISPATCH(std::max(KT, VT), fs_bgrad, a, stream);
         fc_mark(e, 5, stream);
     }
-    return hipGetLastError();
+    SeqArgs walk = fs_walk(a, a.wbad);
+    walk.replay = a.ds;  // the windows are done with it
+    return launch_seq_bwd(walk, a.in_bf16, stream);
 }
 
 }  // namespace gdn2

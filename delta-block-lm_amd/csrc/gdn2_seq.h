@@ -24,12 +24,13 @@ struct SeqArgs {
     void *out;
     int out_bf16;
     float *final_state, *scores;
-    // Checkpoint (null = not written, decode), carved by seq_bind_checkpoint:
-    //   ck       [B*H][nck][K_pad][V_pad]  state at the start of every block
-    //   ck_delta [B*H][nck*SEQ_CT][V_pad]  the edit delta of every token
-    //   ck_norm  [B*H][nck*SEQ_CT][2]      |k| and |delta| of every token
-    float *ck, *ck_delta, *ck_norm;
+    // Checkpoint (null: not written), the arrays of the same names of the f32
+    // chunk kernels (gdn2_chunk_f32.h): the state at the start of every block and
+    // the edit delta of every token, in packed 16 x 16 tiles.
+    float *st, *fu;
     int nck;
+    // The (batch, head)s to walk: those whose word is not zero (null: all).
+    const int *only;
     // backward
     View dout;
     const float *dfinal, *dscores;
@@ -42,24 +43,17 @@ struct SeqArgs {
 inline int seq_pad(int n) { return n <= 32 ? 32 : (n <= 64 ? 64 : 128); }
 inline int64_t seq_state_floats(int K, int V) { return (int64_t)seq_pad(K) * seq_pad(V); }
 
-inline int64_t seq_checkpoint_floats(int64_t B, int64_t T, int64_t H, int K, int V) {
-    const int64_t nck = (T + SEQ_CT - 1) / SEQ_CT, tp = nck * SEQ_CT;
-    return B * H * (nck * seq_state_floats(K, V) + tp * seq_pad(V) + tp * 2);
+// Offsets of S[i][j] in a block's state tiles (KT key tiles) and of token t's delta[j]
+// in its edit tiles.
+__host__ __device__ inline int seq_state_at(int i, int j, int KT) {
+    return ((j >> 4) * KT + (i >> 4)) * 256 + ((i & 15) >> 2) * 64 + (j & 15) * 4 + (i & 3);
+}
+__host__ __device__ inline int seq_edit_at(int t, int j) {
+    return (j >> 4) * 256 + (t >> 2) * 64 + (j & 15) * 4 + (t & 3);
 }
 
 inline int64_t seq_workspace_floats(int64_t B, int64_t H, int K, int V) {
     return B * H * SEQ_CT * seq_state_floats(K, V);
-}
-
-inline void seq_bind_checkpoint(SeqArgs &a, const void *ck) {
-    a.ck = static_cast<float *>(const_cast<void *>(ck));
-    if (!ck) {
-        a.ck_delta = a.ck_norm = nullptr;
-        return;
-    }
-    const int64_t bh = (int64_t)a.B * a.H, tp = (int64_t)a.nck * SEQ_CT;
-    a.ck_delta = a.ck + bh * a.nck * seq_state_floats(a.K, a.V);
-    a.ck_norm = a.ck_delta + bh * tp * seq_pad(a.V);
 }
 
 hipError_t launch_seq_fwd(const SeqArgs &a, bool in_bf16, hipStream_t stream);

@@ -29,8 +29,8 @@
 // block's global loads are issued before the current block's token loop and
 // written to LDS after it, so their latency hides behind the loop.
 //
-// Checkpoints: the forward stores the state at the start of every block
-// (row-major fp32), the edit delta of every token and the norms |k|, |delta|.
+// Checkpoints: the forward stores the state at the start of every block and the
+// edit delta of every token, in the tile layout of the f32 chunk kernels.
 // The backward walks blocks in reverse and replays a block from its
 // checkpoint with the forward's own deltas (the same rounded operations, so
 // the replayed states are the forward's), keeping the pre-token states in a
@@ -129,6 +129,8 @@ __device__ __forceinline__ void lds_get(const float *p, float (&x)[N]) {
     }
 }
 
+typedef float seq_f4 __attribute__((ext_vector_type(4), aligned(4)));  // the checkpoint takes any alignment
+
 template <int N>
 __device__ __forceinline__ void lds_put(float *p, const float (&x)[N]) {
     static_assert(N % 2 == 0, "even runs");
@@ -162,8 +164,8 @@ struct TokenRegs {
     uint32_t v[NV], w[NV];
     uint32_t dy[BWD ? NV : 1], d[BWD ? NV : 1];
     // Per-token words (threads tid < SEQ_CT): doc limits (start, end) or the
-    // valid/reset masks; dscores and the forward's |k|, |delta|.
-    uint32_t f0, f1, sa, nk, nd;
+    // valid/reset masks; dscores.
+    uint32_t f0, f1, sa;
     bool in;
 };
 
@@ -227,14 +229,15 @@ __device__ __forceinline__ uint32_t ld_s(const Stream &s, int64_t t, int64_t c) 
 
 // The per-workgroup scalars the block loads need besides the streams.
 struct BlockCtx {
-    int T, K, V, scalar, doc, H, b, h, bh;
-    int64_t tp;
-    const float *ck_delta, *ck_norm, *dscores;
+    int T, K, V, scalar, doc, H, b, h;
+    const float *fu;  // the head's edit tiles
+    const float *dscores;
 };
 
 __device__ __forceinline__ BlockCtx make_ctx(const SeqArgs &a, int b, int h, int bh) {
-    return BlockCtx{a.T, a.K, a.V, a.scalar, a.doc, a.H, b, h, bh, (int64_t)a.nck * SEQ_CT,
-                    a.ck_delta, a.ck_norm, a.dscores};
+    const int64_t vt = (a.V + 15) >> 4;
+    return BlockCtx{a.T, a.K, a.V, a.scalar, a.doc, a.H, b, h, a.fu ? a.fu + bh * a.nck * vt * 256 : nullptr,
+                    a.dscores};
 }
 
 template <int KP, int VP, int NT, bool BWD, typename TIN>
@@ -268,21 +271,19 @@ __device__ __forceinline__ void load_tokens(const TokenSrc &src, const BlockCtx 
             r.w[n] = ld_s<float>(src.w, t, cv);
             if constexpr (BWD) {
                 if (src.dy.p) r.dy[n] = ld_s<TIN>(src.dy, t, cv);
-                r.d[n] = __float_as_uint(x.ck_delta[((int64_t)x.bh * x.tp + t) * VP + cv]);
+                r.d[n] = __float_as_uint(x.fu[(int64_t)(t0 >> 4) * ((x.V + 15) >> 4) * 256 + seq_edit_at(t - t0, cv)]);
             }
         }
     }
     const int t = t0 + tid;
     r.in = tid < SEQ_CT && t < x.T;
     r.f0 = x.doc ? 0u : ONE_BITS;
-    r.f1 = r.sa = r.nk = r.nd = 0u;
+    r.f1 = r.sa = 0u;
     if (r.in) {
         if (src.f0.p) r.f0 = ld_s<float>(src.f0, t, 0);
         if (src.f1.p) r.f1 = ld_s<float>(src.f1, t, 0);
         if constexpr (BWD) {
             if (x.dscores) r.sa = __float_as_uint(x.dscores[((int64_t)x.b * x.T + t) * x.H + x.h]);
-            r.nk = __float_as_uint(x.ck_norm[((int64_t)x.bh * x.tp + t) * 2]);
-            r.nd = __float_as_uint(x.ck_norm[((int64_t)x.bh * x.tp + t) * 2 + 1]);
         }
     }
 }
@@ -403,7 +404,8 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
     const int rg = lane / CLN, cl = lane % CLN;
     const int r0 = RL * rg, c0 = 16 * w + CL * cl;  // first key row / value column of this lane
     const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
-    const int64_t tp = (int64_t)a.nck * CT;
+    if (a.only && a.only[bh] == 0) return;
+    const int KT = (a.K + 15) >> 4, VT = (a.V + 15) >> 4;  // the checkpoint's tiles
 
     // Initial state, coalesced through the transpose slab.
     for (int idx = tid; idx < KP * VP; idx += NT) {
@@ -432,10 +434,18 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
     for (int blk = 0; blk < a.nck; ++blk) {
         const int t0 = blk * CT, nt = min(CT, a.T - t0);
         const FwdTokens<KP, VP> &B = s.buf[blk & 1];
-        if (a.ck) {
-            float *ck = a.ck + ((int64_t)bh * a.nck + blk) * KP * VP;
+        if (a.st) {
+            float *st = a.st + ((int64_t)bh * a.nck + blk) * KT * VT * 256;
+            static_assert(RL % 4 == 0, "whole pieces");
 #pragma unroll
-            for (int ri = 0; ri < RL; ++ri) lds_put<CL>(ck + (r0 + ri) * VP + c0, S[ri]);
+            for (int cj = 0; cj < CL; ++cj)
+#pragma unroll
+                for (int ri = 0; ri < RL; ri += 4) {
+                    const int i = r0 + ri, j = c0 + cj;
+                    if (i < 16 * KT && j < 16 * VT)
+                        *reinterpret_cast<seq_f4 *>(st + seq_state_at(i, j, KT)) =
+                            seq_f4{S[ri][cj], S[ri + 1][cj], S[ri + 2][cj], S[ri + 3][cj]};
+                }
         }
         if (blk + 1 < a.nck) load_tokens<KP, VP, NT, false, TIN>(src, ctx, t0 + CT, tid, nx);
         // One token: S <- a S, delta = w v - S^T (e k), S += k delta^T,
@@ -499,15 +509,12 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
         }
         for (int idx = tid; idx < CT * VP; idx += NT) {
             const int tt = idx / VP, c = idx % VP;
-            if (tt < nt) {
-                if (c < a.V)
-                    store_out(a.out, a.out_bf16, (((int64_t)b * a.T + t0 + tt) * a.H + h) * a.V + c,
-                              s.o[tt][c]);
-                if (a.ck) a.ck_delta[((int64_t)bh * tp + t0 + tt) * VP + c] = s.d[tt][c];
-            }
+            if (tt < nt && c < a.V)
+                store_out(a.out, a.out_bf16, (((int64_t)b * a.T + t0 + tt) * a.H + h) * a.V + c, s.o[tt][c]);
+            if (a.fu && c < 16 * VT)
+                a.fu[((int64_t)bh * a.nck + blk) * VT * 256 + seq_edit_at(tt, c)] = tt < nt ? s.d[tt][c] : 0.f;
         }
-        // Scores |k| |delta| (zero on padding) and the checkpoint norms: one
-        // 16-lane row per token.
+        // Scores |k| |delta| (zero on padding): one 16-lane row per token.
         for (int tt = tid >> 4; tt < CT; tt += NT / 16) {
             const int l = tid & 15;
             float kk = 0.f, dd = 0.f;
@@ -515,15 +522,8 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
             for (int c = l; c < VP; c += 16) dd = __builtin_fmaf(s.d[tt][c], s.d[tt][c], dd);
             kk = row16_sum(kk);
             dd = row16_sum(dd);
-            if (l == 0 && tt < nt) {
-                const int t = t0 + tt;
-                if (a.scores)
-                    a.scores[((int64_t)b * a.T + t) * a.H + h] = B.val[tt] != 0.f ? sqrtf(kk * dd) : 0.f;
-                if (a.ck) {
-                    a.ck_norm[((int64_t)bh * tp + t) * 2] = sqrtf(kk);
-                    a.ck_norm[((int64_t)bh * tp + t) * 2 + 1] = sqrtf(dd);
-                }
-            }
+            if (l == 0 && tt < nt && a.scores)
+                a.scores[((int64_t)b * a.T + t0 + tt) * a.H + h] = B.val[tt] != 0.f ? sqrtf(kk * dd) : 0.f;
         }
         __syncthreads();
     }
@@ -584,12 +584,8 @@ __device__ __forceinline__ void store_bwd_flags(const SeqArgs &a,
         token_flags(a, r, t0 + tid, val, rst);
         s.val[tid] = val;
         s.rst[tid] = rst;
-        // Score VJP (zero subgradient at |k| |delta| = 0): ddelta += cs delta,
-        // dk += ks k.
-        const float sa = __uint_as_float(r.sa), nk = __uint_as_float(r.nk), nd = __uint_as_float(r.nd);
-        const bool ok = val != 0.f && nk > 0.f && nd > 0.f;
-        s.cs[tid] = ok ? sa * nk / nd : 0.f;
-        s.ks[tid] = ok ? sa * nd / nk : 0.f;
+        s.cs[tid] = __uint_as_float(r.sa);  // until score_coefs
+        s.ks[tid] = 0.f;
     }
 }
 
@@ -619,12 +615,41 @@ __device__ __forceinline__ void store_bwd_data(const SeqArgs &a,
     }
 }
 
-template <int KP, int VP, int RL, int CL>
+// The staged block's score VJP coefficients (zero subgradient at |k| |delta| = 0):
+// ddelta += cs delta, dk += ks k.  One 16-lane row per token.
+template <int KP, int VP, int NT>
+__device__ __forceinline__ void score_coefs(SeqBwdSmem<KP, VP> &s, int tid) {
+    for (int tt = tid >> 4; tt < SEQ_CT; tt += NT / 16) {
+        const int l = tid & 15;
+        float kk = 0.f, dd = 0.f;
+        for (int c = l; c < KP; c += 16) kk = __builtin_fmaf(s.k[tt][c], s.k[tt][c], kk);
+        for (int c = l; c < VP; c += 16) dd = __builtin_fmaf(s.d[tt][c], s.d[tt][c], dd);
+        const float nk = sqrtf(row16_sum(kk)), nd = sqrtf(row16_sum(dd));
+        if (l == 0) {
+            const bool ok = s.val[tt] != 0.f && nk > 0.f && nd > 0.f;
+            const float sa = s.cs[tt];
+            s.cs[tt] = ok ? sa * nk / nd : 0.f;
+            s.ks[tt] = ok ? sa * nd / nk : 0.f;
+        }
+    }
+}
+
+template <int RL, int CL>
 __device__ __forceinline__ void load_ck(const SeqArgs &a, int bh, int blk, int r0, int c0,
                                         float (&S)[RL][CL]) {
-    const float *ck = a.ck + ((int64_t)bh * a.nck + blk) * KP * VP;
+    const int KT = (a.K + 15) >> 4, VT = (a.V + 15) >> 4;
+    const float *st = a.st + ((int64_t)bh * a.nck + blk) * KT * VT * 256;
+    constexpr int R = RL < 4 ? RL : 4;  // rows of a piece
 #pragma unroll
-    for (int ri = 0; ri < RL; ++ri) lds_get<CL>(ck + (r0 + ri) * VP + c0, S[ri]);
+    for (int cj = 0; cj < CL; ++cj)
+#pragma unroll
+        for (int ri = 0; ri < RL; ri += R) {
+            const int i = r0 + ri, j = c0 + cj;
+            const bool in = i < 16 * KT && j < 16 * VT;
+            const float *p = st + (in ? seq_state_at(i, j, KT) : 0);
+#pragma unroll
+            for (int e = 0; e < R; ++e) S[ri + e][cj] = in ? p[e] : 0.f;
+        }
 }
 
 // One token's operands for a backward lane.
@@ -701,6 +726,7 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
     const int rg = lane >> 2, cl = lane & 3;
     const int r0 = RL * rg, c0 = 4 * CL * w + CL * cl;  // first key row / value column of this lane
     const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
+    if (a.only && a.only[bh] == 0) return;
     const int64_t KV = (int64_t)a.K * a.V;
 
     float adj[RL][CL];
@@ -722,18 +748,22 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
     TokenRegs<KP, VP, NT, true> nx;
     float ckn[RL][CL];
     load_tokens<KP, VP, NT, true, TIN>(src, ctx, (a.nck - 1) * CT, tid, nx);
-    if (AHEAD) load_ck<KP, VP, RL, CL>(a, bh, a.nck - 1, r0, c0, ckn);
+    if (AHEAD) load_ck<RL, CL>(a, bh, a.nck - 1, r0, c0, ckn);
     store_bwd_flags<KP, VP, NT, TIN>(a, nx, s, (a.nck - 1) * CT, tid);
     __syncthreads();
     store_bwd_data<KP, VP, NT, TIN>(a, nx, s, tid);
     __syncthreads();
+    if (a.dscores) {
+        score_coefs<KP, VP, NT>(s, tid);
+        __syncthreads();
+    }
 
     for (int blk = a.nck - 1; blk >= 0; --blk) {
         const int t0 = blk * CT, nt = min(CT, a.T - t0);
         // Resets as a wave-uniform bit mask.
         const uint64_t rm = __ballot(lane < CT && s.rst[lane & (CT - 1)] != 0.f &&
                                      s.val[lane & (CT - 1)] != 0.f);
-        if (!AHEAD) load_ck<KP, VP, RL, CL>(a, bh, blk, r0, c0, ckn);
+        if (!AHEAD) load_ck<RL, CL>(a, bh, blk, r0, c0, ckn);
         float S[RL][CL];
 #pragma unroll
         for (int ri = 0; ri < RL; ++ri)
@@ -743,7 +773,7 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
         // token loop.
         if (blk > 0) {
             load_tokens<KP, VP, NT, true, TIN>(src, ctx, t0 - CT, tid, nx);
-            if (AHEAD) load_ck<KP, VP, RL, CL>(a, bh, blk - 1, r0, c0, ckn);
+            if (AHEAD) load_ck<RL, CL>(a, bh, blk - 1, r0, c0, ckn);
         }
         // Replay the block with the forward's deltas: padding leaves S as is
         // (a = 1, k = 0, delta = 0); a reset zeroes it first.
@@ -867,6 +897,10 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
             __syncthreads();
             store_bwd_data<KP, VP, NT, TIN>(a, nx, s, tid);
             __syncthreads();
+            if (a.dscores) {
+                score_coefs<KP, VP, NT>(s, tid);
+                __syncthreads();
+            }
         }
     }
     // Initial-state adjoint.
@@ -1031,7 +1065,7 @@ hipError_t launch_seq_decode(const SeqArgs &a, bool bf16, hipStream_t st) {
 }
 
 hipError_t launch_seq_bwd(const SeqArgs &a, bool bf16, hipStream_t st) {
-    if (!a.ck || !a.replay) return hipErrorInvalidValue;
+    if (!a.st || !a.fu || !a.replay) return hipErrorInvalidValue;
     GDN2_SEQ_DISPATCH(bwd_typed)
 }
 
