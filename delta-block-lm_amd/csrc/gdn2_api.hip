@@ -417,51 +417,7 @@ int gdn2_backward(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *
 
 }  // extern "C"
 
-static bool use_seq_path(const gdn2_shape *shape) { return shape->time <= FC_C; }
-
-// The scalar-gate backward's workspace without the f32 chunk kernels' words (one per
-// batch and head).  Their backward walks windows of chunks that fit whatever
-// workspace it is given, so its share is capped: 64 MiB holds 4064 chunks of
-// 64 x 64, enough to fill the chip, and keeps every shape whose other needs fit
-// the library's fixed scratch within it (gdn_scalar_backward_noalloc).
-static size_t scalar_workspace_base(const gdn2_shape *shape, int chunk) {
-    size_t c = 0;
-    if (chunk_eligible_shape(shape, chunk))
-        c = chunk_workspace_bytes(shape->batch, shape->time, shape->heads);
-    else if (wide_eligible_shape(shape, chunk))
-        c = wide_workspace_bytes(shape->batch, shape->time, shape->heads);
-    const size_t f = fc_workspace_bytes(shape->batch, shape->time, shape->heads, (int)shape->keys,
-                                        (int)shape->values);
-    return std::max(std::max(c, std::min(f, (size_t)GDN2_NOALLOC_SCRATCH_BYTES)), seq_workspace_bytes(shape));
-}
-
-extern "C" {
-
-size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
-    if (check_shape(shape) || check_chunk(chunk)) return 0;
-    size_t c = 0;
-    if (chunk_eligible_shape(shape, chunk))
-        c = chunk_checkpoint_bytes(shape->batch, shape->time, shape->heads);
-    else if (wide_eligible_shape(shape, chunk))
-        c = wide_checkpoint_bytes(shape->batch, shape->time, shape->heads);
-    const int K = (int)shape->keys, V = (int)shape->values;
-    return std::max(c, use_seq_path(shape)
-                           ? fc_walk_checkpoint_bytes(shape->batch, shape->time, shape->heads, K, V)
-                           : fc_checkpoint_bytes(shape->batch, shape->time, shape->heads, K, V, true));
-}
-
-size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
-    if (check_shape(shape) || check_chunk(chunk)) return 0;
-    const size_t base = scalar_workspace_base(shape, chunk);
-    if (use_seq_path(shape)) return base;
-    const size_t words = fc_word_bytes(shape->batch, shape->heads);
-    const size_t f = fc_workspace_bytes(shape->batch, shape->time, shape->heads, (int)shape->keys,
-                                        (int)shape->values) + words;
-    return std::max(base, std::max(std::min(f, (size_t)GDN2_NOALLOC_SCRATCH_BYTES),
-                                   seq_workspace_bytes(shape) + words));
-}
-
-// The chunk-WY MFMA kernels take bf16 q/k/v with d_k = d_v = 64 (gdn2_chunk.hip)
+// Kernels of a scalar-gate call.  The chunk-WY MFMA kernels take bf16 q/k/v with d_k = d_v = 64 (gdn2_chunk.hip)
 // or 128 (gdn2_chunk_wide.hip), chunk 64, unit channel stride and 16-byte
 // aligned token rows.  Everything else runs the f32 scalar-gate chunk kernels
 // (gdn2_chunk_fs.hip) from 17 tokens on, and the token-sequential kernels
@@ -471,12 +427,90 @@ size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
 // and 19 at 32, 62 and 30 at 128; backward 18 and 26, 29 and 25, 49 and 28, 172
 // and 42; at 2048 heads T = 16 takes 58 and 74 forward).  Forward and backward
 // apply the same rule, so the checkpoint format always matches.
+enum class ScalarPath { chunk, wide, walk, f32 };
 
-static bool use_chunk_path(const gdn2_shape *shape, int chunk, const gdn2_view *q,
-                           const gdn2_view *k, const gdn2_view *v) {
-    return (chunk_eligible_shape(shape, chunk) || wide_eligible_shape(shape, chunk)) &&
-           q->dtype == GDN2_BF16 && rows_aligned(q) && rows_aligned(k) && rows_aligned(v);
+static bool use_seq_path(const gdn2_shape *shape) { return shape->time <= FC_C; }
+
+static ScalarPath scalar_path(const gdn2_shape *shape, int chunk, const gdn2_view *q, const gdn2_view *k,
+                              const gdn2_view *v) {
+    if (q->dtype == GDN2_BF16 && rows_aligned(q) && rows_aligned(k) && rows_aligned(v)) {
+        if (chunk_eligible_shape(shape, chunk)) return ScalarPath::chunk;
+        if (wide_eligible_shape(shape, chunk)) return ScalarPath::wide;
+    }
+    return use_seq_path(shape) ? ScalarPath::walk : ScalarPath::f32;
 }
+
+static size_t path_checkpoint_bytes(ScalarPath path, const gdn2_shape *s) {
+    const int K = (int)s->keys, V = (int)s->values;
+    switch (path) {
+        case ScalarPath::chunk: return chunk_checkpoint_bytes(s->batch, s->time, s->heads);
+        case ScalarPath::wide: return wide_checkpoint_bytes(s->batch, s->time, s->heads);
+        case ScalarPath::walk: return fc_walk_checkpoint_bytes(s->batch, s->time, s->heads, K, V);
+        default: return fc_checkpoint_bytes(s->batch, s->time, s->heads, K, V, true);
+    }
+}
+
+// The f32 chunk kernels' backward walks windows of chunks that fit whatever
+// workspace it is given, so its share is capped: 64 MiB holds 4064 chunks of
+// 64 x 64, enough to fill the chip, and keeps every shape whose other needs fit
+// the library's fixed scratch within it (gdn_scalar_backward_noalloc).  words: with
+// the kernels' words, one per batch and head.
+static size_t path_workspace_bytes(ScalarPath path, const gdn2_shape *s, bool words = true) {
+    if (path == ScalarPath::chunk) return chunk_workspace_bytes(s->batch, s->time, s->heads);
+    if (path == ScalarPath::wide) return wide_workspace_bytes(s->batch, s->time, s->heads);
+    if (path == ScalarPath::walk) return seq_workspace_bytes(s);
+    const size_t n = words ? fc_word_bytes(s->batch, s->heads) : 0;
+    const size_t f = fc_workspace_bytes(s->batch, s->time, s->heads, (int)s->keys, (int)s->values) + n;
+    return std::max(std::min(f, (size_t)GDN2_NOALLOC_SCRATCH_BYTES), seq_workspace_bytes(s) + n);
+}
+
+// The most that any call of a shape needs, whatever its dtype and alignment.
+template <typename F>
+static size_t shape_bytes(const gdn2_shape *shape, int chunk, F bytes) {
+    size_t n = bytes(use_seq_path(shape) ? ScalarPath::walk : ScalarPath::f32);
+    if (chunk_eligible_shape(shape, chunk)) n = std::max(n, bytes(ScalarPath::chunk));
+    if (wide_eligible_shape(shape, chunk)) n = std::max(n, bytes(ScalarPath::wide));
+    return n;
+}
+
+static size_t scalar_workspace_shape(const gdn2_shape *shape, int chunk, bool words) {
+    return shape_bytes(shape, chunk, [&](ScalarPath p) { return path_workspace_bytes(p, shape, words); });
+}
+
+static int check_call(const gdn2_shape *shape, int chunk, const gdn2_view *q, const gdn2_view *k,
+                      const gdn2_view *v) {
+    GDN2_TRY(check_shape(shape));
+    GDN2_TRY(check_chunk(chunk));
+    GDN2_TRY(check_view(q, "q", -1, true));
+    GDN2_TRY(check_view(k, "k", q->dtype, true));
+    return check_view(v, "v", q->dtype, true);
+}
+
+extern "C" {
+
+size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk) {
+    if (check_shape(shape) || check_chunk(chunk)) return 0;
+    return shape_bytes(shape, chunk, [&](ScalarPath p) { return path_checkpoint_bytes(p, shape); });
+}
+
+size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk) {
+    if (check_shape(shape) || check_chunk(chunk)) return 0;
+    return scalar_workspace_shape(shape, chunk, true);
+}
+
+size_t gdn_scalar_call_checkpoint_bytes(const gdn2_shape *shape, int chunk, const gdn2_view *q,
+                                        const gdn2_view *k, const gdn2_view *v) {
+    if (check_call(shape, chunk, q, k, v)) return 0;
+    return path_checkpoint_bytes(scalar_path(shape, chunk, q, k, v), shape);
+}
+
+size_t gdn_scalar_call_workspace_bytes(const gdn2_shape *shape, int chunk, const gdn2_view *q,
+                                       const gdn2_view *k, const gdn2_view *v) {
+    if (check_call(shape, chunk, q, k, v)) return 0;
+    return path_workspace_bytes(scalar_path(shape, chunk, q, k, v), shape);
+}
+
+}  // extern "C"
 
 static ChunkArgs chunk_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_view *k,
                             const gdn2_view *v, const gdn2_view *beta, const gdn2_view *g,
@@ -531,6 +565,8 @@ static int check_scalar_inputs(const gdn2_view *q, const gdn2_view *k, const gdn
     return GDN2_OK;
 }
 
+extern "C" {
+
 int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, const gdn2_view *k,
                     const gdn2_view *v, const gdn2_view *beta, const gdn2_view *g,
                     const gdn2_view *valid, const gdn2_view *reset, const gdn2_view *initial,
@@ -544,10 +580,11 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
     if (!output || !final_state || !scores)
         return fail(GDN2_ERR_ARGUMENT, "output, final_state and scores must be non-null");
     if (!checkpoint) return fail(GDN2_ERR_ARGUMENT, "checkpoint is null");
-    if (checkpoint_bytes < gdn_scalar_checkpoint_bytes(shape, chunk))
+    const ScalarPath path = scalar_path(shape, chunk, q, k, v);
+    if (checkpoint_bytes < path_checkpoint_bytes(path, shape))
         return fail(GDN2_ERR_WORKSPACE, "checkpoint needs %zu bytes, got %zu",
-                    gdn_scalar_checkpoint_bytes(shape, chunk), checkpoint_bytes);
-    if (use_chunk_path(shape, chunk, q, k, v)) {
+                    path_checkpoint_bytes(path, shape), checkpoint_bytes);
+    if (path == ScalarPath::chunk || path == ScalarPath::wide) {
         ChunkArgs c = chunk_args(shape, q, k, v, beta, g, valid, reset);
         c.initial = make_view(initial);
         c.out = output;
@@ -555,7 +592,7 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
         c.final_state = final_state;
         c.scores = scores;
         const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
-        if (wide_eligible_shape(shape, chunk)) {
+        if (path == ScalarPath::wide) {
             wide_bind_checkpoint(c, checkpoint);
             return launch_status(launch_wide_fwd(c, (hipStream_t)stream, ev), "gdn_scalar_scan");
         }
@@ -568,7 +605,7 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
     a.out_bf16 = output_dtype == GDN2_BF16;
     a.final_state = final_state;
     a.scores = scores;
-    if (use_seq_path(shape)) {
+    if (path == ScalarPath::walk) {
         bind_walk(a, checkpoint);
         return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_scan");
@@ -601,7 +638,7 @@ int gdn_scalar_backward_noalloc(const gdn2_shape *shape, int chunk, const gdn2_v
                                 void *stream) {
     GDN2_TRY(check_shape(shape));
     GDN2_TRY(check_chunk(chunk));
-    const size_t need = scalar_workspace_base(shape, chunk);
+    const size_t need = scalar_workspace_shape(shape, chunk, false);
     if (need > GDN2_NOALLOC_SCRATCH_BYTES)
         return fail(GDN2_ERR_WORKSPACE,
                     "gdn_scalar_backward_noalloc: this shape needs %zu bytes of scratch, above "
@@ -630,20 +667,21 @@ static int scalar_backward_impl(const gdn2_shape *shape, int chunk, const gdn2_v
     GDN2_TRY(check_scalar_inputs(q, k, v, beta, g, valid, reset));
     if (d_output) GDN2_TRY(check_view(d_output, "d_output", q->dtype, true));
     if (!checkpoint) return fail(GDN2_ERR_ARGUMENT, "checkpoint is null");
-    if (checkpoint_bytes < gdn_scalar_checkpoint_bytes(shape, chunk))
+    const ScalarPath path = scalar_path(shape, chunk, q, k, v);
+    if (checkpoint_bytes < path_checkpoint_bytes(path, shape))
         return fail(GDN2_ERR_WORKSPACE, "checkpoint needs %zu bytes, got %zu",
-                    gdn_scalar_checkpoint_bytes(shape, chunk), checkpoint_bytes);
+                    path_checkpoint_bytes(path, shape), checkpoint_bytes);
     if (!workspace) return fail(GDN2_ERR_ARGUMENT, "workspace is null");
-    if (workspace_bytes < gdn_scalar_workspace_bytes(shape, chunk))
+    if (workspace_bytes < path_workspace_bytes(path, shape))
         return fail(GDN2_ERR_WORKSPACE, "workspace needs %zu bytes, got %zu",
-                    gdn_scalar_workspace_bytes(shape, chunk), workspace_bytes);
-    if (use_chunk_path(shape, chunk, q, k, v)) {
+                    path_workspace_bytes(path, shape), workspace_bytes);
+    if (path == ScalarPath::chunk || path == ScalarPath::wide) {
         if (d_output && d_output->data && !rows_aligned(d_output))
             return fail(GDN2_ERR_ARGUMENT,
                         "d_output needs unit channel stride and 16-byte aligned rows on the "
                         "chunked path (chunk 64, bf16, d_k = d_v = 64 or 128)");
         ChunkArgs c = chunk_args(shape, q, k, v, beta, g, valid, reset);
-        const bool wide = wide_eligible_shape(shape, chunk);
+        const bool wide = path == ScalarPath::wide;
         if (wide) {
             wide_bind_checkpoint(c, const_cast<void *>(checkpoint));
             wide_bind_workspace(c, workspace);
@@ -678,7 +716,7 @@ static int scalar_backward_impl(const gdn2_shape *shape, int chunk, const gdn2_v
     a.dbeta = dbeta;
     a.dg = dg;
     a.dinitial = d_initial;
-    if (use_seq_path(shape)) {
+    if (path == ScalarPath::walk) {
         bind_walk(a, checkpoint);
         a.replay = (float *)workspace;
         return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),

@@ -339,11 +339,12 @@ def gdn_scalar_forward(q, k, v, beta, g, valid, reset, initial=None, chunk: int 
     out = torch.empty((B, T, H, V), dtype=q.dtype, device=dev)
     final = torch.empty((B, H, K, V), dtype=torch.float32, device=dev)
     scores = torch.empty((B, T, H), dtype=torch.float32, device=dev)
-    nck = L.gdn_scalar_checkpoint_bytes(ctypes.byref(shape), chunk)
-    if nck == 0:
-        check("gdn_scalar_checkpoint_bytes", 1)
-    ck = torch.empty((nck,), dtype=torch.uint8, device=dev)
     views = [_view(x) for x in (q, k, v, beta, g, valid, reset, initial)]
+    nck = L.gdn_scalar_call_checkpoint_bytes(ctypes.byref(shape), chunk,
+                                             *[ctypes.byref(x) for x in views[:3]])
+    if nck == 0:
+        check("gdn_scalar_call_checkpoint_bytes", 1)
+    ck = torch.empty((nck,), dtype=torch.uint8, device=dev)
     with on_device(dev):
         rc = L.gdn_scalar_scan(ctypes.byref(shape), chunk, *[ctypes.byref(x) for x in views],
                                _ptr(out), _code(out), _ptr(final), _ptr(scores), _ptr(ck), nck,
@@ -366,7 +367,9 @@ def gdn_scalar_backward(q, k, v, beta, g, valid, reset, checkpoint, chunk: int =
     db = torch.empty((B, T, H), dtype=torch.float32, device=dev)
     dg = torch.empty((B, T, H), dtype=torch.float32, device=dev)
     dinit = torch.empty((B, H, K, V), dtype=torch.float32, device=dev)
-    nws = L.gdn_scalar_workspace_bytes(ctypes.byref(shape), chunk)
+    views = [_view(x) for x in (q, k, v, beta, g, valid, reset)]
+    nws = L.gdn_scalar_call_workspace_bytes(ctypes.byref(shape), chunk,
+                                            *[ctypes.byref(x) for x in views[:3]])
     ws = torch.empty((max(nws, 1),), dtype=torch.uint8, device=dev)
     if d_output is not None:
         if d_output.dtype != q.dtype:
@@ -377,7 +380,6 @@ def gdn_scalar_backward(q, k, v, beta, g, valid, reset, checkpoint, chunk: int =
             d_output = d_output.contiguous()
     dfin = None if d_final_state is None else d_final_state.float().contiguous()
     dsc = None if d_scores is None else d_scores.float().contiguous()
-    views = [_view(x) for x in (q, k, v, beta, g, valid, reset)]
     dov = _view(d_output)
     with on_device(dev):
         rc = L.gdn_scalar_backward(
