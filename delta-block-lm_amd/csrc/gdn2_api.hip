@@ -66,13 +66,17 @@ using namespace gdn2;
 namespace {
 
 // Stage timing (gdn2_stage_timing): six stages, an event pair each; the
-// forward records pairs 0-2, the backward pairs 3-5.  A measurement hook for
+// forward records pairs 0-2, the backward pairs 3-5; the scalar-gate op's f32 chunk
+// kernels have six of their own behind them, so that a call's stages tell which
+// kernels it ran.  A measurement hook for
 // benchmarks only: the events and flags below are process-wide (not thread
 // safe), and no event is recorded on a stream that is being captured, so a
 // graph never holds them.
-constexpr int kStages = 6;
-const char *const kStageNames[kStages] = {"chunk_prep", "state_scan", "chunk_out",
-                                          "chunk_bprep", "adjoint_scan", "chunk_bgrad"};
+constexpr int kScalarF32 = 6, kStages = 12;
+const char *const kStageNames[kStages] = {
+    "chunk_prep", "state_scan", "chunk_out", "chunk_bprep", "adjoint_scan", "chunk_bgrad",
+    "scalar_f32_prep", "scalar_f32_state_scan", "scalar_f32_out",
+    "scalar_f32_bprep", "scalar_f32_adjoint_scan", "scalar_f32_bgrad"};
 hipEvent_t g_stage_ev[2 * kStages];
 bool g_stage_ready = false;  // events created
 bool g_stage_on = false;
@@ -610,7 +614,7 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
         return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_scan");
     }
-    const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
+    const hipEvent_t *ev = stage_events(kScalarF32, (hipStream_t)stream);
     return launch_status(launch_fs_fwd(fc_args(a, q, false, checkpoint, nullptr), (hipStream_t)stream, ev),
                          "gdn_scalar_scan");
 }
@@ -722,7 +726,7 @@ static int scalar_backward_impl(const gdn2_shape *shape, int chunk, const gdn2_v
         return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_backward");
     }
-    const hipEvent_t *ev = stage_events(3, (hipStream_t)stream);
+    const hipEvent_t *ev = stage_events(kScalarF32 + 3, (hipStream_t)stream);
     return launch_status(launch_fs_bwd(fc_args(a, q, false, const_cast<void *>(checkpoint), workspace), workspace_bytes,
                                        (hipStream_t)stream, ev),
                          "gdn_scalar_backward");

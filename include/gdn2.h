@@ -505,14 +505,16 @@ GDN2_API int gdn2_hola_backward(const gdn2_hola_shape *shape, const gdn2_view *q
                                 size_t workspace_bytes, void *stream);
 
 /* Measurement hook.  No counterpart in the reference: it serves benchmarks
- * that need the duration of each kernel of the chunk-WY path, measured on the
- * stream the kernels run on.  After gdn2_stage_timing(1), every chunk-path
- * call of gdn_scalar_scan / gdn_scalar_backward records a pair of HIP events
- * around each of its kernels on the call's stream; gdn2_stage_ms(i) returns
+ * that need the duration of each kernel of the chunked paths, measured on the
+ * stream the kernels run on.  After gdn2_stage_timing(1), every chunked
+ * call of the scans and their backwards records a pair of HIP events around each of its kernels on the call's stream; gdn2_stage_ms(i) returns
  * the duration of stage i in the most recent call that ran it (the caller
  * synchronises the stream first), or a negative value if stage i has not run
  * since timing was enabled.  Stages: 0 prep, 1 state scan, 2 output
- * (forward); 3 backward prep, 4 adjoint scan, 5 gradients (backward).
+ * (forward); 3 backward prep, 4 adjoint scan, 5 gradients (backward), of the
+ * chunk-WY kernels and of the channel-wise op's f32 chunk kernels; 6 to 11 the same
+ * of the scalar-gate op's f32 chunk kernels (their stage 9 is empty, as stage 3 is
+ * on the channel-wise op).
  * Process-wide state for the current device, not thread safe: enable it only
  * in single-threaded measurement runs.  A call whose stream is being captured
  * into a graph records no events (the stage then keeps its last duration).

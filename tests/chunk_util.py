@@ -11,7 +11,8 @@ from oracle import oracle
 def chunk_stages(D):
     """Stage-timer names of the chunk-WY path at d_k = d_v = D (64 or 128):
     prep, state scan and output forward; prep, adjoint scan and gradients
-    backward."""
+    backward.  The scalar-gate op's f32 chunk kernels, which take every other
+    call, report names of their own (tests/test_gpu_dispatch.py)."""
     assert D in (64, 128)
     return {"chunk_prep", "state_scan", "chunk_out", "chunk_bprep", "adjoint_scan", "chunk_bgrad"}
 

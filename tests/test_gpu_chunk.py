@@ -1,6 +1,7 @@
 """GPU parity of the chunk-WY MFMA path (scalar gates, bf16, d_k = d_v = 64,
-chunk 64) against the f64 oracle, and against the token-sequential GPU kernels
-at the full BASELINE configs[1] size through size-independent properties."""
+chunk 64) against the f64 oracle, at the full language-model size (16 x 512
+tokens, 8 heads) on two of its sequences, and there against the f32 chunk
+kernels."""
 import numpy as np
 import pytest
 
@@ -36,9 +37,7 @@ def test_chunk_forward_matches_oracle(dk, B, T, H, masks):
     gate("scores", sc, o_sc, TOL_BF16, exact_zero=pad)
 
 
-def test_chunk_forward_full_size_matches_sequential_kernel(dk):
-    """BASELINE configs[1] inputs: chunk-WY MFMA forward vs the token-sequential
-    GPU kernel (chunk 16 selects it) on the same bf16 inputs."""
+def _full_size():
     from delta_mixers.synthetic import CONFIGS, generate
     cfg = CONFIGS[1]
     p = generate(cfg)
@@ -46,11 +45,28 @@ def test_chunk_forward_full_size_matches_sequential_kernel(dk):
     p["valid"] = np.ones((B, T), np.float32)
     p["reset"] = np.zeros((B, T), np.float32)
     p["initial"] = None
+    p["dO"] = p["d_output"]
+    p["dF"] = np.zeros((B, H, 64, 64), np.float32)
+    p["dS"] = np.zeros((B, T, H), np.float32)
+    return p, [0, B - 1]
+
+
+def test_chunk_forward_full_size(dk):
+    """16 x 512 tokens, 8 heads: the chunk-WY MFMA forward against the recurrence (the f64 oracle)
+    on two sequences, and whole against the f32 chunk kernels (chunk 16 selects them) on the
+    same bf16 inputs."""
+    p, rows = _full_size()
     o64, f64_, s64 = run_fwd(dk, p, 64)
     o16, f16_, s16 = run_fwd(dk, p, 16)
-    gate("output vs sequential", o64, host(o16), TOL_BF16)
-    gate("final_state vs sequential", f64_, host(f16_), TOL_BF16)
-    gate("scores vs sequential", s64, host(s16), TOL_BF16)
+    gate("output vs f32 kernels", o64, host(o16), TOL_BF16)
+    gate("final_state vs f32 kernels", f64_, host(f16_), TOL_BF16)
+    gate("scores vs f32 kernels", s64, host(s16), TOL_BF16)
+    x = {n: p[n][rows] for n in ("q", "k", "v", "beta", "g", "valid", "reset")}
+    a, e, w = oracle.scalar_gates(x["beta"], x["g"], 64, 64)
+    o_out, o_fin, o_sc = oracle.scan(x["q"], x["k"], x["v"], a, e, w, x["valid"], x["reset"])
+    gate("output", o64[rows], o_out, TOL_BF16)
+    gate("final_state", f64_[rows], o_fin, TOL_BF16)
+    gate("scores", s64[rows], o_sc, TOL_BF16)
 
 
 @pytest.mark.parametrize("B,T,H", [(1, 64, 1), (2, 200, 2), (1, 130, 3)])
@@ -79,23 +95,20 @@ def test_chunk_backward_output_adjoint_only(dk):
         gate(name, got, ref, TOL_BF16)
 
 
-def test_chunk_backward_full_size_matches_sequential_kernel(dk):
-    """chunk-WY MFMA backward vs the token-sequential GPU
-    backward on the same bf16 inputs and upstream dO."""
-    from delta_mixers.synthetic import CONFIGS, generate
-    cfg = CONFIGS[1]
-    p = generate(cfg)
-    B, T, H = cfg.batch, cfg.time, cfg.heads
-    p["valid"] = np.ones((B, T), np.float32)
-    p["reset"] = np.zeros((B, T), np.float32)
-    p["initial"] = None
-    p["dO"] = p["d_output"]
-    p["dF"] = np.zeros((B, H, 64, 64), np.float32)
-    p["dS"] = np.zeros((B, T, H), np.float32)
+def test_chunk_backward_full_size(dk):
+    """16 x 512 tokens, 8 heads: the chunk-WY MFMA backward against the recurrence's gradients (the
+    f64 oracle) on two sequences, and whole against the f32 chunk kernels on the same bf16
+    inputs and upstream dO."""
+    p, rows = _full_size()
     g64 = run_bwd(dk, p, 64, use_final=False, use_scores=False)
     g16 = run_bwd(dk, p, 16, use_final=False, use_scores=False)
     for name, a, b in zip(("dq", "dk", "dv", "dbeta", "dg"), g64[:5], g16[:5]):
-        gate(f"{name} vs sequential", a, host(b), TOL_BF16)
+        gate(f"{name} vs f32 kernels", a, host(b), TOL_BF16)
+    og, odb, odg = scalar_oracle_grads({n: x[rows] for n, x in p.items()
+                                        if isinstance(x, np.ndarray)} | {"initial": None})
+    for name, a, b in zip(("dq", "dk", "dv", "dbeta", "dg"), g64[:5],
+                          (og["q"], og["k"], og["v"], odb, odg)):
+        gate(name, a[rows], b, TOL_BF16)
 
 
 @pytest.mark.parametrize("B,T,H", [(2, 200, 2)])
