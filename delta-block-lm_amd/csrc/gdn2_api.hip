@@ -449,7 +449,7 @@ static size_t path_checkpoint_bytes(ScalarPath path, const gdn2_shape *s) {
     switch (path) {
         case ScalarPath::chunk: return chunk_checkpoint_bytes(s->batch, s->time, s->heads);
         case ScalarPath::wide: return wide_checkpoint_bytes(s->batch, s->time, s->heads);
-        case ScalarPath::walk: return fc_walk_checkpoint_bytes(s->batch, s->time, s->heads, K, V);
+        case ScalarPath::walk: return (size_t)seq_checkpoint_floats(s->batch, s->heads, K, V) * 4;
         default: return fc_checkpoint_bytes(s->batch, s->time, s->heads, K, V, true);
     }
 }
@@ -550,12 +550,6 @@ static SeqArgs scalar_args(const gdn2_shape *s, const gdn2_view *q, const gdn2_v
     return a;
 }
 
-// The token walk's arrays of a checkpoint.
-static void bind_walk(SeqArgs &a, const void *checkpoint) {
-    a.st = (float *)const_cast<void *>(checkpoint);
-    a.fu = a.st + (int64_t)a.B * a.H * a.nck * fc_kp(a.K) * fc_kp(a.V);
-}
-
 static int check_scalar_inputs(const gdn2_view *q, const gdn2_view *k, const gdn2_view *v,
                                const gdn2_view *beta, const gdn2_view *g,
                                const gdn2_view *valid, const gdn2_view *reset) {
@@ -610,7 +604,7 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
     a.final_state = final_state;
     a.scores = scores;
     if (path == ScalarPath::walk) {
-        bind_walk(a, checkpoint);
+        seq_bind_checkpoint(a, checkpoint);
         return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_scan");
     }
@@ -721,7 +715,7 @@ static int scalar_backward_impl(const gdn2_shape *shape, int chunk, const gdn2_v
     a.dg = dg;
     a.dinitial = d_initial;
     if (path == ScalarPath::walk) {
-        bind_walk(a, checkpoint);
+        seq_bind_checkpoint(a, checkpoint);
         a.replay = (float *)workspace;
         return launch_status(launch_seq_bwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
                              "gdn_scalar_backward");

@@ -32,7 +32,6 @@ constexpr int FC_C = 16;  // tokens per chunk
 // and, with scalar gates, one word per (batch, head):
 //   bad    the forward gave a value that is not finite (out); such a (batch, head)
 //          is walked by token afterwards (gdn2_chunk_fs.hip)
-// st and fu come first: they are all that the token walk keeps.
 // KP = d_k and VP = d_v rounded up to 16 (KT = KP / 16, VT = VP / 16): the tiles
 // are padded with zeros to whole 16 x 16 MFMA tiles.  Backward workspace: ds, the
 // state adjoint at each chunk end, packed like st, and, with a score adjoint, sc,
@@ -89,13 +88,6 @@ inline size_t fc_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V,
     fc_checkpoint_parts(fc_chunks(B, T, H), K, V, scalar, part);
     for (size_t x : part) total += x;
     return total * sizeof(float) + (scalar ? fc_word_bytes(B, H) : 0);
-}
-
-// What the token walk keeps: st and fu.
-inline size_t fc_walk_checkpoint_bytes(int64_t B, int64_t T, int64_t H, int K, int V) {
-    size_t part[FC_PARTS];
-    fc_checkpoint_parts(fc_chunks(B, T, H), K, V, true, part);
-    return (part[0] + part[1]) * sizeof(float);
 }
 
 // Floats of the workspace per chunk.

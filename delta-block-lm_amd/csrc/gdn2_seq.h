@@ -1,4 +1,5 @@
-// Token-sequential GDN-2 kernels (general channel-wise surface, decode).
+// Token-sequential GDN-2 kernels (the scalar-gate walk, channel-wise decode), and the
+// argument block that the chunk kernels' launchers share with them.
 #pragma once
 
 #include "gdn2_common.h"
@@ -11,8 +12,8 @@ struct SeqArgs {
     int B, T, H, K, V;
     View q, k, v, alpha, erase, write, valid, reset, initial;
     // Document limits (int32 [batch, time] views, inclusive; end < start marks
-    // padding, start == t resets the state).  When set they replace
-    // valid/reset; the backward is the exact VJP, as with masks.
+    // padding, start == t resets the state; the f32 chunk kernels).  When set they
+    // replace valid/reset; the backward is the exact VJP, as with masks.
     int doc;
     View doc_start, doc_end;
     // Scalar-gate mode: alpha[i] = exp(g), erase[i] = write[j] = beta, with
@@ -24,12 +25,15 @@ struct SeqArgs {
     void *out;
     int out_bf16;
     float *final_state, *scores;
-    // Checkpoint (null: not written), the arrays of the same names of the f32
-    // chunk kernels (gdn2_chunk_f32.h): the state at the start of every block and
-    // the edit delta of every token, in packed 16 x 16 tiles.
+    // Checkpoint: the state at the start of every block and the edit delta of every
+    // token.  A call that only walks has one block (T <= SEQ_CT): row-major
+    // [B*H][K_pad][V_pad] and [B*H][SEQ_CT][V_pad].  Behind the f32 chunk kernels the
+    // walk takes the (batch, head)s whose word in `only` is not zero, and these are
+    // the chunk kernels' arrays of the same names, in packed 16 x 16 tiles
+    // (gdn2_chunk_f32.h; whole lines a wave there, but pieces of 16 bytes in the walk's
+    // own layout: at 1024 heads of 128 x 128 its forward took 62 us of them, for 53).
     float *st, *fu;
     int nck;
-    // The (batch, head)s to walk: those whose word is not zero (null: all).
     const int *only;
     // backward
     View dout;
@@ -42,6 +46,16 @@ struct SeqArgs {
 // Padded widths used by the kernels: 32, 64 or 128.
 inline int seq_pad(int n) { return n <= 32 ? 32 : (n <= 64 ? 64 : 128); }
 inline int64_t seq_state_floats(int K, int V) { return (int64_t)seq_pad(K) * seq_pad(V); }
+
+// A call of one block's checkpoint.
+inline int64_t seq_checkpoint_floats(int64_t B, int64_t H, int K, int V) {
+    return B * H * (seq_state_floats(K, V) + SEQ_CT * seq_pad(V));
+}
+
+inline void seq_bind_checkpoint(SeqArgs &a, const void *ck) {
+    a.st = static_cast<float *>(const_cast<void *>(ck));
+    a.fu = a.st + (int64_t)a.B * a.H * seq_state_floats(a.K, a.V);
+}
 
 // Offsets of S[i][j] in a block's state tiles (KT key tiles) and of token t's delta[j]
 // in its edit tiles.

@@ -1,12 +1,10 @@
-// Token-sequential GDN-2 scan for gfx950: the general channel-wise surface.
+// Token-sequential GDN-2 kernels for gfx950: the scalar-gate scan (alpha = exp(g),
+// erase = write = beta) and its backward, and the channel-wise decode step.  The scan
+// takes the scalar-gate calls of up to 16 tokens, and any length for the (batch,
+// head)s that the f32 chunk kernels mark (gdn2_chunk_fs.hip).
 //
-// Semantics follow crates/mixers/src/reference.rs:41-257 (forward and VJP),
-// the stateful fused kernels crates/kernels/src/gdn_training.rs:12-284 and,
-// with document limits, the forward of crates/mixers/src/gdn2_reference.rs:51-103
-// (a token is live when end >= start and resets the state when start == t)
-// with the exact VJP of that forward, as the reference's chunked kernels
-// compute it (crates/kernels/src/gdn2.rs:24-65, :288-490): the adjoint never
-// crosses a reset.
+// Semantics follow crates/mixers/src/reference.rs:41-257 (forward and VJP) and the
+// stateful fused kernels crates/kernels/src/gdn_training.rs:12-284.
 //
 // One workgroup per (batch, head).  Value columns evolve independently in the
 // recurrence, so each wave owns a block of value columns and walks the tokens
@@ -30,8 +28,8 @@
 // written to LDS after it, so their latency hides behind the loop.
 //
 // Checkpoints: the forward stores the state at the start of every block and the
-// edit delta of every token, in the tile layout of the f32 chunk kernels.
-// The backward walks blocks in reverse and replays a block from its
+// edit delta of every token (row-major, or in the tile layout of the f32 chunk
+// kernels for the heads that they mark).  The backward walks blocks in reverse and replays a block from its
 // checkpoint with the forward's own deltas (the same rounded operations, so
 // the replayed states are the forward's), keeping the pre-token states in a
 // thread-major scratch area that the reverse token loop reads one token
@@ -163,8 +161,7 @@ struct TokenRegs {
     uint32_t q[NK], k[NK], a[NK], e[NK];
     uint32_t v[NV], w[NV];
     uint32_t dy[BWD ? NV : 1], d[BWD ? NV : 1];
-    // Per-token words (threads tid < SEQ_CT): doc limits (start, end) or the
-    // valid/reset masks; dscores.
+    // Per-token words (threads tid < SEQ_CT): the valid/reset masks; dscores.
     uint32_t f0, f1, sa;
     bool in;
 };
@@ -194,25 +191,24 @@ __device__ __forceinline__ Stream make_stream(const View &v, int b, int h, int e
                   v.s1, broadcast ? 0 : v.s3};
 }
 
-// Token inputs of one (batch, head): q, k, the key gates a (alpha, or g in
-// scalar mode) and e (erase, or beta), v, the write gate w (write, or beta),
-// the output adjoint dy, and the per-token words f0/f1 (valid/reset masks,
-// or the document limits start/end).
+// Token inputs of one (batch, head): q, k, the key gates a (alpha, or g of a scalar
+// gate) and e (erase, or beta), v, the write gate w (write, or beta), the output
+// adjoint dy, and the per-token words f0/f1 (valid/reset masks).
 struct TokenSrc {
     Stream q, k, a, e, v, w, dy, f0, f1;
 };
 
-template <typename TIN>
+template <typename TIN, bool SCALAR>
 __device__ __forceinline__ TokenSrc make_src(const SeqArgs &a, int b, int h) {
     TokenSrc s;
     s.q = make_stream(a.q, b, h, sizeof(TIN));
     s.k = make_stream(a.k, b, h, sizeof(TIN));
-    s.a = a.scalar ? make_stream(a.g, b, h, 4, true) : make_stream(a.alpha, b, h, 4);
-    s.e = a.scalar ? make_stream(a.beta, b, h, 4, true) : make_stream(a.erase, b, h, 4);
+    s.a = SCALAR ? make_stream(a.g, b, h, 4, true) : make_stream(a.alpha, b, h, 4);
+    s.e = SCALAR ? make_stream(a.beta, b, h, 4, true) : make_stream(a.erase, b, h, 4);
     s.v = make_stream(a.v, b, h, sizeof(TIN));
-    s.w = a.scalar ? make_stream(a.beta, b, h, 4, true) : make_stream(a.write, b, h, 4);
+    s.w = SCALAR ? make_stream(a.beta, b, h, 4, true) : make_stream(a.write, b, h, 4);
     s.dy = make_stream(a.dout, b, h, sizeof(TIN));
-    const View &f0 = a.doc ? a.doc_start : a.valid, &f1 = a.doc ? a.doc_end : a.reset;
+    const View &f0 = a.valid, &f1 = a.reset;
     s.f0 = f0.data ? Stream{static_cast<const char *>(f0.data) + (int64_t)b * f0.s0 * 4, f0.s1, 0}
                    : Stream{nullptr, 0, 0};
     s.f1 = f1.data ? Stream{static_cast<const char *>(f1.data) + (int64_t)b * f1.s0 * 4, f1.s1, 0}
@@ -229,18 +225,18 @@ __device__ __forceinline__ uint32_t ld_s(const Stream &s, int64_t t, int64_t c) 
 
 // The per-workgroup scalars the block loads need besides the streams.
 struct BlockCtx {
-    int T, K, V, scalar, doc, H, b, h;
-    const float *fu;  // the head's edit tiles
+    int T, K, V, H, b, h;
+    const float *fu;  // the head's edits
     const float *dscores;
 };
 
+template <int VP, bool MARKED>
 __device__ __forceinline__ BlockCtx make_ctx(const SeqArgs &a, int b, int h, int bh) {
-    const int64_t vt = (a.V + 15) >> 4;
-    return BlockCtx{a.T, a.K, a.V, a.scalar, a.doc, a.H, b, h, a.fu ? a.fu + bh * a.nck * vt * 256 : nullptr,
-                    a.dscores};
+    const int64_t edits = MARKED ? (int64_t)a.nck * ((a.V + 15) >> 4) * 256 : SEQ_CT * VP;
+    return BlockCtx{a.T, a.K, a.V, a.H, b, h, a.fu + bh * edits, a.dscores};
 }
 
-template <int KP, int VP, int NT, bool BWD, typename TIN>
+template <int KP, int VP, int NT, bool BWD, bool MARKED, typename TIN>
 __device__ __forceinline__ void load_tokens(const TokenSrc &src, const BlockCtx &x, int t0, int tid,
                                             TokenRegs<KP, VP, NT, BWD> &r) {
     using R = TokenRegs<KP, VP, NT, BWD>;
@@ -253,7 +249,7 @@ __device__ __forceinline__ void load_tokens(const TokenSrc &src, const BlockCtx 
     for (int n = 0; n < R::NK; ++n) {
         const int t = tk + n * KS;
         r.q[n] = r.k[n] = r.e[n] = 0u;
-        r.a[n] = x.scalar ? NEG_INF_BITS : 0u;  // exp(-inf) = 0 beyond the sequence
+        r.a[n] = NEG_INF_BITS;  // exp(-inf) = 0 beyond the sequence
         if (t < x.T && ck < x.K) {
             r.q[n] = ld_s<TIN>(src.q, t, ck);
             r.k[n] = ld_s<TIN>(src.k, t, ck);
@@ -271,13 +267,15 @@ __device__ __forceinline__ void load_tokens(const TokenSrc &src, const BlockCtx 
             r.w[n] = ld_s<float>(src.w, t, cv);
             if constexpr (BWD) {
                 if (src.dy.p) r.dy[n] = ld_s<TIN>(src.dy, t, cv);
-                r.d[n] = __float_as_uint(x.fu[(int64_t)(t0 >> 4) * ((x.V + 15) >> 4) * 256 + seq_edit_at(t - t0, cv)]);
+                r.d[n] = __float_as_uint(
+                    x.fu[MARKED ? (int64_t)(t0 >> 4) * ((x.V + 15) >> 4) * 256 + seq_edit_at(t - t0, cv)
+                                  : t * VP + cv]);
             }
         }
     }
     const int t = t0 + tid;
     r.in = tid < SEQ_CT && t < x.T;
-    r.f0 = x.doc ? 0u : ONE_BITS;
+    r.f0 = ONE_BITS;
     r.f1 = r.sa = 0u;
     if (r.in) {
         if (src.f0.p) r.f0 = ld_s<float>(src.f0, t, 0);
@@ -290,18 +288,11 @@ __device__ __forceinline__ void load_tokens(const TokenSrc &src, const BlockCtx 
 
 // Token flags (valid, reset) from a thread's per-token words.
 template <int KP, int VP, int NT, bool BWD>
-__device__ __forceinline__ void token_flags(const SeqArgs &a, const TokenRegs<KP, VP, NT, BWD> &r,
-                                            int t, float &val, float &rst) {
+__device__ __forceinline__ void token_flags(const TokenRegs<KP, VP, NT, BWD> &r, float &val, float &rst) {
     val = rst = 0.f;
     if (!r.in) return;
-    if (a.doc) {
-        const int32_t st = (int32_t)r.f0, en = (int32_t)r.f1;
-        val = en >= st ? 1.f : 0.f;
-        rst = st == t ? 1.f : 0.f;
-    } else {
-        val = __uint_as_float(r.f0);
-        rst = __uint_as_float(r.f1);
-    }
+    val = __uint_as_float(r.f0);
+    rst = __uint_as_float(r.f1);
 }
 
 // ---- forward ---------------------------------------------------------------------
@@ -325,15 +316,15 @@ struct FwdTokens {
     float val[SEQ_CT], rst[SEQ_CT];
 };
 
-template <int KP, int VP>
+template <int KP, int VP, bool MARKED>
 struct alignas(16) SeqFwdSmem {
-    FwdTokens<KP, VP> buf[2];
+    FwdTokens<KP, VP> buf[MARKED ? 2 : 1];  // the next block's beside this one's
     float o[SEQ_CT][VP], d[SEQ_CT][VP];
 };
 
-template <int KP, int VP>
+template <int KP, int VP, bool MARKED>
 union SeqFwdShared {
-    SeqFwdSmem<KP, VP> s;
+    SeqFwdSmem<KP, VP, MARKED> s;
     float st[KP * (VP + 1)];  // state transpose slab (row stride VP+1)
 };
 
@@ -344,21 +335,17 @@ union SeqFwdShared {
 // edit and output are zero.  A reset token gets a = 0, which zeroes the
 // carried state before the edit.
 template <int KP, int VP, int NT, typename TIN>
-__device__ __forceinline__ void store_fwd_flags(const SeqArgs &a,
-                                                const TokenRegs<KP, VP, NT, false> &r,
-                                                FwdTokens<KP, VP> &s, int t0, int tid) {
+__device__ __forceinline__ void store_fwd_flags(const TokenRegs<KP, VP, NT, false> &r, FwdTokens<KP, VP> &s, int tid) {
     if (tid < SEQ_CT) {
         float val, rst;
-        token_flags(a, r, t0 + tid, val, rst);
+        token_flags(r, val, rst);
         s.val[tid] = val;
         s.rst[tid] = rst;
     }
 }
 
 template <int KP, int VP, int NT, typename TIN>
-__device__ __forceinline__ void store_fwd_data(const SeqArgs &a,
-                                               const TokenRegs<KP, VP, NT, false> &r,
-                                               FwdTokens<KP, VP> &s, int tid) {
+__device__ __forceinline__ void store_fwd_data(const TokenRegs<KP, VP, NT, false> &r, FwdTokens<KP, VP> &s, int tid) {
     using R = TokenRegs<KP, VP, NT, false>;
 #pragma unroll
     for (int n = 0; n < R::NK; ++n) {
@@ -367,7 +354,7 @@ __device__ __forceinline__ void store_fwd_data(const SeqArgs &a,
         const float kf = raw_f<TIN>(r.k[n]), af = __uint_as_float(r.a[n]);
         s.q[tt][c] = on ? raw_f<TIN>(r.q[n]) : 0.f;
         s.k[tt][c] = on ? kf : 0.f;
-        s.a[tt][c] = on ? (rs ? 0.f : (a.scalar ? expf(af) : af)) : 1.f;
+        s.a[tt][c] = on ? (rs ? 0.f : expf(af)) : 1.f;
         s.ek[tt][c] = on ? __uint_as_float(r.e[n]) * kf : 0.f;
     }
 #pragma unroll
@@ -394,17 +381,18 @@ __device__ __forceinline__ void fetch_fwd(const FwdTokens<KP, VP> &B, int tt, in
 }
 
 #pragma clang fp contract(off)
-template <int KP, int VP, typename TIN>
+template <int KP, int VP, bool MARKED, typename TIN>
 __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
     using L = FwdLayout<KP>;
     constexpr int RL = L::RL, CL = L::CL, CLN = L::CLN, NT = 4 * VP, CT = SEQ_CT;
-    __shared__ SeqFwdShared<KP, VP> sh;
-    SeqFwdSmem<KP, VP> &s = sh.s;
+    __shared__ SeqFwdShared<KP, VP, MARKED> sh;
+    SeqFwdSmem<KP, VP, MARKED> &s = sh.s;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int rg = lane / CLN, cl = lane % CLN;
     const int r0 = RL * rg, c0 = 16 * w + CL * cl;  // first key row / value column of this lane
     const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
-    if (a.only && a.only[bh] == 0) return;
+    if (MARKED && a.only[bh] == 0) return;
+    const int nck = MARKED ? a.nck : 1;
     const int KT = (a.K + 15) >> 4, VT = (a.V + 15) >> 4;  // the checkpoint's tiles
 
     // Initial state, coalesced through the transpose slab.
@@ -422,19 +410,19 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
         for (int cj = 0; cj < CL; ++cj) S[ri][cj] = sh.st[(r0 + ri) * (VP + 1) + c0 + cj];
     __syncthreads();
 
-    const TokenSrc src = make_src<TIN>(a, b, h);
-    const BlockCtx ctx = make_ctx(a, b, h, bh);
+    const TokenSrc src = make_src<TIN, true>(a, b, h);
+    const BlockCtx ctx = make_ctx<VP, MARKED>(a, b, h, bh);
     TokenRegs<KP, VP, NT, false> nx;
-    load_tokens<KP, VP, NT, false, TIN>(src, ctx, 0, tid, nx);
-    store_fwd_flags<KP, VP, NT, TIN>(a, nx, s.buf[0], 0, tid);
+    load_tokens<KP, VP, NT, false, MARKED, TIN>(src, ctx, 0, tid, nx);
+    store_fwd_flags<KP, VP, NT, TIN>(nx, s.buf[0], tid);
     __syncthreads();
-    store_fwd_data<KP, VP, NT, TIN>(a, nx, s.buf[0], tid);
+    store_fwd_data<KP, VP, NT, TIN>(nx, s.buf[0], tid);
     __syncthreads();
 
-    for (int blk = 0; blk < a.nck; ++blk) {
+    for (int blk = 0; blk < nck; ++blk) {
         const int t0 = blk * CT, nt = min(CT, a.T - t0);
-        const FwdTokens<KP, VP> &B = s.buf[blk & 1];
-        if (a.st) {
+        const FwdTokens<KP, VP> &B = s.buf[MARKED ? blk & 1 : 0];
+        if constexpr (MARKED) {
             float *st = a.st + ((int64_t)bh * a.nck + blk) * KT * VT * 256;
             static_assert(RL % 4 == 0, "whole pieces");
 #pragma unroll
@@ -446,8 +434,12 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
                         *reinterpret_cast<seq_f4 *>(st + seq_state_at(i, j, KT)) =
                             seq_f4{S[ri][cj], S[ri + 1][cj], S[ri + 2][cj], S[ri + 3][cj]};
                 }
+        } else {
+            float *st = a.st + (int64_t)bh * KP * VP;
+#pragma unroll
+            for (int ri = 0; ri < RL; ++ri) lds_put<CL>(st + (r0 + ri) * VP + c0, S[ri]);
         }
-        if (blk + 1 < a.nck) load_tokens<KP, VP, NT, false, TIN>(src, ctx, t0 + CT, tid, nx);
+        if (blk + 1 < nck) load_tokens<KP, VP, NT, false, MARKED, TIN>(src, ctx, t0 + CT, tid, nx);
         // One token: S <- a S, delta = w v - S^T (e k), S += k delta^T,
         // o = S^T q.  Key sums keep two partial chains per column.
         auto step = [&](int tt, const FwdTok<RL, CL> &x) {
@@ -502,17 +494,21 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
         // Stage the next block first: its loads are the oldest memory
         // operations still in flight, so waiting for them does not wait for
         // this block's output stores.
-        if (blk + 1 < a.nck) {
-            store_fwd_flags<KP, VP, NT, TIN>(a, nx, s.buf[(blk + 1) & 1], t0 + CT, tid);
+        if (blk + 1 < nck) {
+            store_fwd_flags<KP, VP, NT, TIN>(nx, s.buf[MARKED ? (blk + 1) & 1 : 0], tid);
             __syncthreads();
-            store_fwd_data<KP, VP, NT, TIN>(a, nx, s.buf[(blk + 1) & 1], tid);
+            store_fwd_data<KP, VP, NT, TIN>(nx, s.buf[MARKED ? (blk + 1) & 1 : 0], tid);
         }
         for (int idx = tid; idx < CT * VP; idx += NT) {
             const int tt = idx / VP, c = idx % VP;
             if (tt < nt && c < a.V)
                 store_out(a.out, a.out_bf16, (((int64_t)b * a.T + t0 + tt) * a.H + h) * a.V + c, s.o[tt][c]);
-            if (a.fu && c < 16 * VT)
-                a.fu[((int64_t)bh * a.nck + blk) * VT * 256 + seq_edit_at(tt, c)] = tt < nt ? s.d[tt][c] : 0.f;
+            if constexpr (MARKED) {
+                if (c < 16 * VT)
+                    a.fu[((int64_t)bh * a.nck + blk) * VT * 256 + seq_edit_at(tt, c)] = tt < nt ? s.d[tt][c] : 0.f;
+            } else if (tt < nt) {
+                a.fu[(int64_t)bh * CT * VP + tt * VP + c] = s.d[tt][c];
+            }
         }
         // Scores |k| |delta| (zero on padding): one 16-lane row per token.
         for (int tt = tid >> 4; tt < CT; tt += NT / 16) {
@@ -576,12 +572,10 @@ struct alignas(16) SeqBwdSmem {
 // passes unchanged and every gradient but dalpha comes out zero (the flush
 // zeroes dalpha).  A reset token gets a = 0, which cuts the adjoint.
 template <int KP, int VP, int NT, typename TIN>
-__device__ __forceinline__ void store_bwd_flags(const SeqArgs &a,
-                                                const TokenRegs<KP, VP, NT, true> &r,
-                                                SeqBwdSmem<KP, VP> &s, int t0, int tid) {
+__device__ __forceinline__ void store_bwd_flags(const TokenRegs<KP, VP, NT, true> &r, SeqBwdSmem<KP, VP> &s, int tid) {
     if (tid < SEQ_CT) {
         float val, rst;
-        token_flags(a, r, t0 + tid, val, rst);
+        token_flags(r, val, rst);
         s.val[tid] = val;
         s.rst[tid] = rst;
         s.cs[tid] = __uint_as_float(r.sa);  // until score_coefs
@@ -590,9 +584,7 @@ __device__ __forceinline__ void store_bwd_flags(const SeqArgs &a,
 }
 
 template <int KP, int VP, int NT, typename TIN>
-__device__ __forceinline__ void store_bwd_data(const SeqArgs &a,
-                                               const TokenRegs<KP, VP, NT, true> &r,
-                                               SeqBwdSmem<KP, VP> &s, int tid) {
+__device__ __forceinline__ void store_bwd_data(const TokenRegs<KP, VP, NT, true> &r, SeqBwdSmem<KP, VP> &s, int tid) {
     using R = TokenRegs<KP, VP, NT, true>;
 #pragma unroll
     for (int n = 0; n < R::NK; ++n) {
@@ -601,7 +593,7 @@ __device__ __forceinline__ void store_bwd_data(const SeqArgs &a,
         const float af = __uint_as_float(r.a[n]);
         s.q[tt][c] = on ? raw_f<TIN>(r.q[n]) : 0.f;
         s.k[tt][c] = on ? raw_f<TIN>(r.k[n]) : 0.f;
-        s.a[tt][c] = on ? (cut ? 0.f : (a.scalar ? expf(af) : af)) : 1.f;
+        s.a[tt][c] = on ? (cut ? 0.f : expf(af)) : 1.f;
         s.e[tt][c] = on ? __uint_as_float(r.e[n]) : 0.f;
     }
 #pragma unroll
@@ -634,21 +626,25 @@ __device__ __forceinline__ void score_coefs(SeqBwdSmem<KP, VP> &s, int tid) {
     }
 }
 
-template <int RL, int CL>
+template <int KP, int VP, int RL, int CL, bool MARKED>
 __device__ __forceinline__ void load_ck(const SeqArgs &a, int bh, int blk, int r0, int c0,
                                         float (&S)[RL][CL]) {
+    if constexpr (!MARKED) {
+        const float *st = a.st + (int64_t)bh * KP * VP;
+#pragma unroll
+        for (int ri = 0; ri < RL; ++ri) lds_get<CL>(st + (r0 + ri) * VP + c0, S[ri]);
+        return;
+    }
     const int KT = (a.K + 15) >> 4, VT = (a.V + 15) >> 4;
     const float *st = a.st + ((int64_t)bh * a.nck + blk) * KT * VT * 256;
-    constexpr int R = RL < 4 ? RL : 4;  // rows of a piece
 #pragma unroll
     for (int cj = 0; cj < CL; ++cj)
 #pragma unroll
-        for (int ri = 0; ri < RL; ri += R) {
+        for (int ri = 0; ri < RL; ++ri) {
             const int i = r0 + ri, j = c0 + cj;
             const bool in = i < 16 * KT && j < 16 * VT;
-            const float *p = st + (in ? seq_state_at(i, j, KT) : 0);
-#pragma unroll
-            for (int e = 0; e < R; ++e) S[ri + e][cj] = in ? p[e] : 0.f;
+            const float x = st[in ? seq_state_at(i, j, KT) : 0];
+            S[ri][cj] = in ? x : 0.f;
         }
 }
 
@@ -672,8 +668,8 @@ __device__ __forceinline__ void fetch_bwd(const SeqBwdSmem<KP, VP> &s, int tt, i
 }
 
 // Sum the per-wave partials of tokens g0 .. g0+FT-1 (those below nt) and
-// store dq, dk, dalpha, derase, dv, dwrite; scalar-gate mode keeps derase and
-// dalpha in the consumed e/a rows of LDS for the per-token chain rule.
+// store dq, dk, dv; the per-channel derase and dalpha stay in the consumed e/a rows
+// of LDS for the per-token chain rule.
 template <int KP, int VP, typename TIN>
 __device__ __forceinline__ void flush_group(const SeqArgs &a, SeqBwdSmem<KP, VP> &s, int b, int h,
                                             int t0, int g0, int nt, int tid) {
@@ -697,26 +693,20 @@ __device__ __forceinline__ void flush_group(const SeqArgs &a, SeqBwdSmem<KP, VP>
             const int64_t o = (((int64_t)b * a.T + t0 + tt) * a.H + h) * a.K + i;
             if (a.dq) store_in<TIN>(a.dq, o, gq);
             if (a.dk) store_in<TIN>(a.dk, o, dk);
-            if (a.dalpha) a.dalpha[o] = ga;
-            if (a.derase) a.derase[o] = de;
         }
-        if (a.scalar) {
-            s.a[tt][i] = i < a.K ? ga : 0.f;
-            s.e[tt][i] = i < a.K ? de : 0.f;
-        }
+        s.a[tt][i] = i < a.K ? ga : 0.f;
+        s.e[tt][i] = i < a.K ? de : 0.f;
     }
     for (int idx = tid; idx < Cfg::FT * VP; idx += Cfg::NT) {
         const int sl = idx / VP, j = idx % VP, tt = g0 + sl;
         if (tt >= nt || j >= a.V) continue;
-        const float dd = s.dd[tt][j];
         const int64_t o = (((int64_t)b * a.T + t0 + tt) * a.H + h) * a.V + j;
-        if (a.dv) store_in<TIN>(a.dv, o, s.w[tt][j] * dd);
-        if (a.dwrite) a.dwrite[o] = s.v[tt][j] * dd;
+        if (a.dv) store_in<TIN>(a.dv, o, s.w[tt][j] * s.dd[tt][j]);
     }
 }
 
 #pragma clang fp contract(off)
-template <int KP, int VP, typename TIN>
+template <int KP, int VP, bool MARKED, typename TIN>
 __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArgs a) {
     using Cfg = SeqBwdCfg<KP, VP>;
     constexpr int NT = Cfg::NT, RL = Cfg::RL, CL = Cfg::CL, FT = Cfg::FT, CT = SEQ_CT;
@@ -726,7 +716,8 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
     const int rg = lane >> 2, cl = lane & 3;
     const int r0 = RL * rg, c0 = 4 * CL * w + CL * cl;  // first key row / value column of this lane
     const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
-    if (a.only && a.only[bh] == 0) return;
+    if (MARKED && a.only[bh] == 0) return;
+    const int nck = MARKED ? a.nck : 1;
     const int64_t KV = (int64_t)a.K * a.V;
 
     float adj[RL][CL];
@@ -743,27 +734,27 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
     // rp + ((tt * RL + ri) * NT + tid) * CL.
     float *rp = a.replay + (int64_t)bh * CT * KP * VP;
 
-    const TokenSrc src = make_src<TIN>(a, b, h);
-    const BlockCtx ctx = make_ctx(a, b, h, bh);
+    const TokenSrc src = make_src<TIN, true>(a, b, h);
+    const BlockCtx ctx = make_ctx<VP, MARKED>(a, b, h, bh);
     TokenRegs<KP, VP, NT, true> nx;
     float ckn[RL][CL];
-    load_tokens<KP, VP, NT, true, TIN>(src, ctx, (a.nck - 1) * CT, tid, nx);
-    if (AHEAD) load_ck<RL, CL>(a, bh, a.nck - 1, r0, c0, ckn);
-    store_bwd_flags<KP, VP, NT, TIN>(a, nx, s, (a.nck - 1) * CT, tid);
+    load_tokens<KP, VP, NT, true, MARKED, TIN>(src, ctx, (nck - 1) * CT, tid, nx);
+    if (AHEAD) load_ck<KP, VP, RL, CL, MARKED>(a, bh, nck - 1, r0, c0, ckn);
+    store_bwd_flags<KP, VP, NT, TIN>(nx, s, tid);
     __syncthreads();
-    store_bwd_data<KP, VP, NT, TIN>(a, nx, s, tid);
+    store_bwd_data<KP, VP, NT, TIN>(nx, s, tid);
     __syncthreads();
     if (a.dscores) {
         score_coefs<KP, VP, NT>(s, tid);
         __syncthreads();
     }
 
-    for (int blk = a.nck - 1; blk >= 0; --blk) {
+    for (int blk = nck - 1; blk >= 0; --blk) {
         const int t0 = blk * CT, nt = min(CT, a.T - t0);
         // Resets as a wave-uniform bit mask.
         const uint64_t rm = __ballot(lane < CT && s.rst[lane & (CT - 1)] != 0.f &&
                                      s.val[lane & (CT - 1)] != 0.f);
-        if (!AHEAD) load_ck<RL, CL>(a, bh, blk, r0, c0, ckn);
+        if (!AHEAD) load_ck<KP, VP, RL, CL, MARKED>(a, bh, blk, r0, c0, ckn);
         float S[RL][CL];
 #pragma unroll
         for (int ri = 0; ri < RL; ++ri)
@@ -772,8 +763,8 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
         // The earlier block's inputs: issued here, written to LDS after the
         // token loop.
         if (blk > 0) {
-            load_tokens<KP, VP, NT, true, TIN>(src, ctx, t0 - CT, tid, nx);
-            if (AHEAD) load_ck<RL, CL>(a, bh, blk - 1, r0, c0, ckn);
+            load_tokens<KP, VP, NT, true, MARKED, TIN>(src, ctx, t0 - CT, tid, nx);
+            if (AHEAD) load_ck<KP, VP, RL, CL, MARKED>(a, bh, blk - 1, r0, c0, ckn);
         }
         // Replay the block with the forward's deltas: padding leaves S as is
         // (a = 1, k = 0, delta = 0); a reset zeroes it first.
@@ -870,32 +861,31 @@ __global__ void __launch_bounds__((SeqBwdCfg<KP, VP>::NT)) seq_bwd_kernel(SeqArg
             }
             step(tt - 1, pb, xb);
         }
-        if (a.scalar) {  // chain rule onto beta and the log gate g
-            for (int tt = tid >> 4; tt < CT; tt += NT / 16) {
-                const int l = tid & 15;
-                float de = 0.f, da = 0.f, dw = 0.f;
-                for (int c = l; c < KP; c += 16) {
-                    de += s.e[tt][c];
-                    da += s.a[tt][c];
-                }
-                for (int c = l; c < VP; c += 16) dw = __builtin_fmaf(s.v[tt][c], s.dd[tt][c], dw);
-                de = row16_sum(de);
-                da = row16_sum(da);
-                dw = row16_sum(dw);
-                if (l == 0 && tt < nt) {
-                    const int t = t0 + tt;
-                    const int64_t tok = ((int64_t)b * a.T + t) * a.H + h;
-                    const bool on = s.val[tt] != 0.f;
-                    if (a.dbeta) a.dbeta[tok] = on ? de + dw : 0.f;
-                    if (a.dg) a.dg[tok] = on ? expf(ld4<float>(a.g, b, t, h, 0)) * da : 0.f;
-                }
+        // Chain rule onto beta and the log gate g.
+        for (int tt = tid >> 4; tt < CT; tt += NT / 16) {
+            const int l = tid & 15;
+            float de = 0.f, da = 0.f, dw = 0.f;
+            for (int c = l; c < KP; c += 16) {
+                de += s.e[tt][c];
+                da += s.a[tt][c];
             }
-            __syncthreads();
+            for (int c = l; c < VP; c += 16) dw = __builtin_fmaf(s.v[tt][c], s.dd[tt][c], dw);
+            de = row16_sum(de);
+            da = row16_sum(da);
+            dw = row16_sum(dw);
+            if (l == 0 && tt < nt) {
+                const int t = t0 + tt;
+                const int64_t tok = ((int64_t)b * a.T + t) * a.H + h;
+                const bool on = s.val[tt] != 0.f;
+                if (a.dbeta) a.dbeta[tok] = on ? de + dw : 0.f;
+                if (a.dg) a.dg[tok] = on ? expf(ld4<float>(a.g, b, t, h, 0)) * da : 0.f;
+            }
         }
+        __syncthreads();
         if (blk > 0) {
-            store_bwd_flags<KP, VP, NT, TIN>(a, nx, s, t0 - CT, tid);
+            store_bwd_flags<KP, VP, NT, TIN>(nx, s, tid);
             __syncthreads();
-            store_bwd_data<KP, VP, NT, TIN>(a, nx, s, tid);
+            store_bwd_data<KP, VP, NT, TIN>(nx, s, tid);
             __syncthreads();
             if (a.dscores) {
                 score_coefs<KP, VP, NT>(s, tid);
@@ -930,7 +920,7 @@ __global__ void __launch_bounds__(VP < 64 ? 64 : VP) seq_decode_kernel(SeqArgs a
     constexpr int NTD = VP < 64 ? 64 : VP, RGN = L::RGN, RL = L::RL;
     __shared__ float sq[KP], sk[KP], sa[KP], sek[KP], sd[VP];
     const int j = threadIdx.x, bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
-    const TokenSrc src = make_src<TIN>(a, b, h);
+    const TokenSrc src = make_src<TIN, false>(a, b, h);
     const bool jin = j < a.V;
     float S[KP];
 #pragma unroll
@@ -946,11 +936,8 @@ __global__ void __launch_bounds__(VP < 64 ? 64 : VP) seq_decode_kernel(SeqArgs a
         if (i < a.K) {
             qf = raw_f<TIN>(ld_s<TIN>(src.q, 0, i));
             kf = raw_f<TIN>(ld_s<TIN>(src.k, 0, i));
-            const float g = __uint_as_float(ld_s<float>(src.a, 0, i));
-            af = a.scalar ? expf(g) : g;
+            af = __uint_as_float(ld_s<float>(src.a, 0, i));
             ef = __uint_as_float(ld_s<float>(src.e, 0, i));
-        } else if (a.scalar) {
-            af = 0.f;
         }
         sq[i] = on ? qf : 0.f;
         sk[i] = on ? kf : 0.f;
@@ -1023,23 +1010,25 @@ static hipError_t decode_typed(const SeqArgs &a, bool bf16, hipStream_t st) {
     return hipGetLastError();
 }
 
+template <int KP, int VP, bool MARKED, typename TIN>
+static void fwd_kernel(const SeqArgs &a, hipStream_t st) {
+    hipLaunchKernelGGL((seq_fwd_kernel<KP, VP, MARKED, TIN>), dim3(a.B * a.H), dim3(4 * VP), 0, st, a);
+}
 template <int KP, int VP>
 static hipError_t fwd_typed(const SeqArgs &a, bool bf16, hipStream_t st) {
-    constexpr int NT = 4 * VP;
-    if (bf16)
-        hipLaunchKernelGGL((seq_fwd_kernel<KP, VP, bf16_t>), dim3(a.B * a.H), dim3(NT), 0, st, a);
-    else
-        hipLaunchKernelGGL((seq_fwd_kernel<KP, VP, float>), dim3(a.B * a.H), dim3(NT), 0, st, a);
+    if (a.only) bf16 ? fwd_kernel<KP, VP, true, bf16_t>(a, st) : fwd_kernel<KP, VP, true, float>(a, st);
+    else bf16 ? fwd_kernel<KP, VP, false, bf16_t>(a, st) : fwd_kernel<KP, VP, false, float>(a, st);
     return hipGetLastError();
 }
 
+template <int KP, int VP, bool MARKED, typename TIN>
+static void bwd_kernel(const SeqArgs &a, hipStream_t st) {
+    hipLaunchKernelGGL((seq_bwd_kernel<KP, VP, MARKED, TIN>), dim3(a.B * a.H), dim3(SeqBwdCfg<KP, VP>::NT), 0, st, a);
+}
 template <int KP, int VP>
 static hipError_t bwd_typed(const SeqArgs &a, bool bf16, hipStream_t st) {
-    constexpr int NT = SeqBwdCfg<KP, VP>::NT;
-    if (bf16)
-        hipLaunchKernelGGL((seq_bwd_kernel<KP, VP, bf16_t>), dim3(a.B * a.H), dim3(NT), 0, st, a);
-    else
-        hipLaunchKernelGGL((seq_bwd_kernel<KP, VP, float>), dim3(a.B * a.H), dim3(NT), 0, st, a);
+    if (a.only) bf16 ? bwd_kernel<KP, VP, true, bf16_t>(a, st) : bwd_kernel<KP, VP, true, float>(a, st);
+    else bf16 ? bwd_kernel<KP, VP, false, bf16_t>(a, st) : bwd_kernel<KP, VP, false, float>(a, st);
     return hipGetLastError();
 }
 
@@ -1056,16 +1045,17 @@ static hipError_t bwd_typed(const SeqArgs &a, bool bf16, hipStream_t st) {
     return FN<128, 128>(a, bf16, st);
 
 hipError_t launch_seq_fwd(const SeqArgs &a, bool bf16, hipStream_t st) {
+    if (!a.st || !a.fu || (!a.only && a.T > SEQ_CT)) return hipErrorInvalidValue;
     GDN2_SEQ_DISPATCH(fwd_typed)
 }
 
 hipError_t launch_seq_decode(const SeqArgs &a, bool bf16, hipStream_t st) {
-    if (a.T != 1 || a.doc) return hipErrorInvalidValue;
+    if (a.T != 1) return hipErrorInvalidValue;
     GDN2_SEQ_DISPATCH(decode_typed)
 }
 
 hipError_t launch_seq_bwd(const SeqArgs &a, bool bf16, hipStream_t st) {
-    if (!a.st || !a.fu || !a.replay) return hipErrorInvalidValue;
+    if (!a.st || !a.fu || !a.replay || (!a.only && a.T > SEQ_CT)) return hipErrorInvalidValue;
     GDN2_SEQ_DISPATCH(bwd_typed)
 }
 
