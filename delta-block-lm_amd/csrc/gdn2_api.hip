@@ -6,6 +6,7 @@
 // an unsupported shape, dtype or buffer size is an error, never a fallback.
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <mutex>
@@ -421,16 +422,18 @@ int gdn2_backward(const gdn2_shape *shape, const gdn2_view *q, const gdn2_view *
 
 }  // extern "C"
 
-// Kernels of a scalar-gate call.  The chunk-WY MFMA kernels take bf16 q/k/v with d_k = d_v = 64 (gdn2_chunk.hip)
-// or 128 (gdn2_chunk_wide.hip), chunk 64, unit channel stride and 16-byte
-// aligned token rows.  Everything else runs the f32 scalar-gate chunk kernels
-// (gdn2_chunk_fs.hip) from 17 tokens on, and the token-sequential kernels
-// (gdn2_seq.hip) up to 16: there one workgroup per head walks one chunk's tokens
-// in less time than three launches take (forward at 64 heads of 64 x 64 f32,
-// token-sequential against chunked: 11 and 17 us at T = 8, 13 and 17 at 16, 21
-// and 19 at 32, 62 and 30 at 128; backward 18 and 26, 29 and 25, 49 and 28, 172
-// and 42; at 2048 heads T = 16 takes 58 and 74 forward).  Forward and backward
-// apply the same rule, so the checkpoint format always matches.
+// Kernels of a scalar-gate call.  The chunk-WY MFMA kernels take bf16 q/k/v with d_k =
+// d_v = 64 (gdn2_chunk.hip) or 128 (gdn2_chunk_wide.hip), chunk 64, unit channel
+// stride and 16-byte aligned token rows.  Everything else runs the f32 scalar-gate
+// chunk kernels (gdn2_chunk_fs.hip) from 17 tokens on, and the token walk
+// (gdn2_seq.hip) of one workgroup per head up to 16, one block of its checkpoint.
+// Forward + backward in us, f32, walked against chunked: 64 heads of 64 x 64, T = 8
+// 10 + 17 and 16 + 18, T = 16 13 + 27 and 16 + 18; 2048 heads, T = 8 32 + 158 and
+// 67 + 93, T = 16 43 + 262 and 68 + 95; at T = 32 (the walk with a checkpoint of two
+// blocks, since removed) 64 heads 21 + 50 and 18 + 19.  The line keeps a short call's
+// forward, which serving makes alone, at its fastest; the backward would gain from a
+// lower one.  Forward and backward apply the same rule, so the checkpoint format
+// always matches.
 enum class ScalarPath { chunk, wide, walk, f32 };
 
 static bool use_seq_path(const gdn2_shape *shape) { return shape->time <= FC_C; }
@@ -442,6 +445,35 @@ static ScalarPath scalar_path(const gdn2_shape *shape, int chunk, const gdn2_vie
         if (wide_eligible_shape(shape, chunk)) return ScalarPath::wide;
     }
     return use_seq_path(shape) ? ScalarPath::walk : ScalarPath::f32;
+}
+
+// Whether the token walk's forward alone takes less time than the f32 chunk kernels',
+// which write 36 KiB a chunk of 64 x 64 that only a backward reads.  Both times in
+// microseconds: a start, and a slope that is the serial chain's or, with more heads
+// than it takes to fill the chip, the throughput of all of them.  P is the walk's padded
+// state and Q the chunks' in units of 64 x 64, F the floats of a chunk's arrays.
+// Measured, f32, walk against chunked: 64 heads of 64 x 64, T = 24 16.4 and 18.0, 48
+// 24.5 and 19.0, 512 205 and 51; 256 heads, T = 17 15.1 and 28.9, 64 32.8 and 36.7,
+// 128 59 and 50; 1024 heads, T = 17 30 and 53, 128 129 and 197, 1024 908 and 1331;
+// 256 heads of 128 x 128, T = 64 76 and 88, 512 494 and 595; 1024 heads of 16 x 16,
+// T = 32 20 and 23, 256 117 and 69.
+static bool walk_is_faster(const gdn2_shape *s) {
+    const int K = (int)s->keys, V = (int)s->values, KP = fc_kp(K), VP = fc_kp(V);
+    const double heads = (double)(s->batch * s->heads), T = (double)s->time, chunks = (double)((s->time + FC_C - 1) / FC_C);
+    const double P = seq_state_floats(K, V) / 4096., Q = KP * VP / 4096.;
+    const double F = KP * VP + 3 * FC_C * FC_C + FC_C * (3 * KP + VP) + KP + 8 * FC_C;
+    const double full = P < 1. ? 13.7e-3 * std::sqrt(P) : 14.5e-3 * P;  // of 16 tokens of a head
+    const double walk = 6. + 1.3 * P + T * std::max(.22 + .175 * P, heads * full / FC_C);
+    const double ragged = K % FC_C || V % FC_C ? 4.5 : 0.;  // element reads
+    const double chunked = 12. + 2.5 * Q + ragged + chunks * std::max(.25 + .0052 * KP, heads * 2.2e-6 * F);
+    return walk < 1.05 * chunked;
+}
+
+// The same for a call that no backward follows.
+static ScalarPath outputs_path(const gdn2_shape *shape, int chunk, const gdn2_view *q, const gdn2_view *k,
+                               const gdn2_view *v) {
+    const ScalarPath path = scalar_path(shape, chunk, q, k, v);
+    return path == ScalarPath::f32 && walk_is_faster(shape) ? ScalarPath::walk : path;
 }
 
 static size_t path_checkpoint_bytes(ScalarPath path, const gdn2_shape *s) {
@@ -563,6 +595,52 @@ static int check_scalar_inputs(const gdn2_view *q, const gdn2_view *k, const gdn
     return GDN2_OK;
 }
 
+// The forward on the kernels of `path`.  keep: with their arrays in `buffer` (named
+// `what`); otherwise the walk's outputs alone.
+static int scalar_forward(ScalarPath path, bool keep, const char *what, const gdn2_shape *shape,
+                          const gdn2_view *q, const gdn2_view *k, const gdn2_view *v, const gdn2_view *beta,
+                          const gdn2_view *g, const gdn2_view *valid, const gdn2_view *reset,
+                          const gdn2_view *initial, void *output, int32_t output_dtype, float *final_state,
+                          float *scores, void *buffer, size_t buffer_bytes, void *stream) {
+    GDN2_TRY(check_view(initial, "initial", GDN2_F32, true));
+    GDN2_TRY(check_out_dtype(output_dtype));
+    if (!output || !final_state || !scores)
+        return fail(GDN2_ERR_ARGUMENT, "output, final_state and scores must be non-null");
+    if (keep && !buffer) return fail(GDN2_ERR_ARGUMENT, "%s is null", what);
+    if (keep && buffer_bytes < path_checkpoint_bytes(path, shape))
+        return fail(GDN2_ERR_WORKSPACE, "%s needs %zu bytes, got %zu", what, path_checkpoint_bytes(path, shape),
+                    buffer_bytes);
+    if (path == ScalarPath::chunk || path == ScalarPath::wide) {
+        ChunkArgs c = chunk_args(shape, q, k, v, beta, g, valid, reset);
+        c.initial = make_view(initial);
+        c.out = output;
+        c.out_bf16 = output_dtype == GDN2_BF16;
+        c.final_state = final_state;
+        c.scores = scores;
+        const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
+        if (path == ScalarPath::wide) {
+            wide_bind_checkpoint(c, buffer);
+            return launch_status(launch_wide_fwd(c, (hipStream_t)stream, ev), "gdn_scalar_scan");
+        }
+        chunk_bind_checkpoint(c, buffer);
+        return launch_status(launch_chunk_fwd(c, (hipStream_t)stream, ev), "gdn_scalar_scan");
+    }
+    SeqArgs a = scalar_args(shape, q, k, v, beta, g, valid, reset);
+    a.initial = make_view(initial);
+    a.out = output;
+    a.out_bf16 = output_dtype == GDN2_BF16;
+    a.final_state = final_state;
+    a.scores = scores;
+    if (path == ScalarPath::walk) {
+        if (keep) seq_bind_checkpoint(a, buffer);
+        return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
+                             "gdn_scalar_scan");
+    }
+    const hipEvent_t *ev = stage_events(kScalarF32, (hipStream_t)stream);
+    return launch_status(launch_fs_fwd(fc_args(a, q, false, buffer, nullptr), (hipStream_t)stream, ev),
+                         "gdn_scalar_scan");
+}
+
 extern "C" {
 
 int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, const gdn2_view *k,
@@ -573,44 +651,29 @@ int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view *q, cons
     GDN2_TRY(check_shape(shape));
     GDN2_TRY(check_chunk(chunk));
     GDN2_TRY(check_scalar_inputs(q, k, v, beta, g, valid, reset));
-    GDN2_TRY(check_view(initial, "initial", GDN2_F32, true));
-    GDN2_TRY(check_out_dtype(output_dtype));
-    if (!output || !final_state || !scores)
-        return fail(GDN2_ERR_ARGUMENT, "output, final_state and scores must be non-null");
-    if (!checkpoint) return fail(GDN2_ERR_ARGUMENT, "checkpoint is null");
-    const ScalarPath path = scalar_path(shape, chunk, q, k, v);
-    if (checkpoint_bytes < path_checkpoint_bytes(path, shape))
-        return fail(GDN2_ERR_WORKSPACE, "checkpoint needs %zu bytes, got %zu",
-                    path_checkpoint_bytes(path, shape), checkpoint_bytes);
-    if (path == ScalarPath::chunk || path == ScalarPath::wide) {
-        ChunkArgs c = chunk_args(shape, q, k, v, beta, g, valid, reset);
-        c.initial = make_view(initial);
-        c.out = output;
-        c.out_bf16 = output_dtype == GDN2_BF16;
-        c.final_state = final_state;
-        c.scores = scores;
-        const hipEvent_t *ev = stage_events(0, (hipStream_t)stream);
-        if (path == ScalarPath::wide) {
-            wide_bind_checkpoint(c, checkpoint);
-            return launch_status(launch_wide_fwd(c, (hipStream_t)stream, ev), "gdn_scalar_scan");
-        }
-        chunk_bind_checkpoint(c, checkpoint);
-        return launch_status(launch_chunk_fwd(c, (hipStream_t)stream, ev), "gdn_scalar_scan");
-    }
-    SeqArgs a = scalar_args(shape, q, k, v, beta, g, valid, reset);
-    a.initial = make_view(initial);
-    a.out = output;
-    a.out_bf16 = output_dtype == GDN2_BF16;
-    a.final_state = final_state;
-    a.scores = scores;
-    if (path == ScalarPath::walk) {
-        seq_bind_checkpoint(a, checkpoint);
-        return launch_status(launch_seq_fwd(a, q->dtype == GDN2_BF16, (hipStream_t)stream),
-                             "gdn_scalar_scan");
-    }
-    const hipEvent_t *ev = stage_events(kScalarF32, (hipStream_t)stream);
-    return launch_status(launch_fs_fwd(fc_args(a, q, false, checkpoint, nullptr), (hipStream_t)stream, ev),
-                         "gdn_scalar_scan");
+    return scalar_forward(scalar_path(shape, chunk, q, k, v), true, "checkpoint", shape, q, k, v, beta, g, valid,
+                          reset, initial, output, output_dtype, final_state, scores, checkpoint,
+                          checkpoint_bytes, stream);
+}
+
+size_t gdn_scalar_outputs_bytes(const gdn2_shape *shape, int chunk, const gdn2_view *q,
+                                const gdn2_view *k, const gdn2_view *v) {
+    if (check_call(shape, chunk, q, k, v)) return 0;
+    const ScalarPath path = outputs_path(shape, chunk, q, k, v);
+    return path == ScalarPath::walk ? 0 : path_checkpoint_bytes(path, shape);
+}
+
+int gdn_scalar_outputs(const gdn2_shape *shape, int chunk, const gdn2_view *q, const gdn2_view *k,
+                       const gdn2_view *v, const gdn2_view *beta, const gdn2_view *g,
+                       const gdn2_view *valid, const gdn2_view *reset, const gdn2_view *initial,
+                       void *output, int32_t output_dtype, float *final_state, float *scores,
+                       void *workspace, size_t workspace_bytes, void *stream) {
+    GDN2_TRY(check_shape(shape));
+    GDN2_TRY(check_chunk(chunk));
+    GDN2_TRY(check_scalar_inputs(q, k, v, beta, g, valid, reset));
+    const ScalarPath path = outputs_path(shape, chunk, q, k, v);
+    return scalar_forward(path, path != ScalarPath::walk, "workspace", shape, q, k, v, beta, g, valid, reset,
+                          initial, output, output_dtype, final_state, scores, workspace, workspace_bytes, stream);
 }
 
 int gdn_scalar_backward(const gdn2_shape *shape, int chunk, const gdn2_view *q,

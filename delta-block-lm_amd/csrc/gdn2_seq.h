@@ -70,6 +70,7 @@ inline int64_t seq_workspace_floats(int64_t B, int64_t H, int K, int V) {
     return B * H * SEQ_CT * seq_state_floats(K, V);
 }
 
+// Without a checkpoint (st and fu null) the outputs alone, of any length.
 hipError_t launch_seq_fwd(const SeqArgs &a, bool in_bf16, hipStream_t stream);
 // One token (T == 1, masks only) on a carried state; no checkpoint.
 hipError_t launch_seq_decode(const SeqArgs &a, bool in_bf16, hipStream_t stream);

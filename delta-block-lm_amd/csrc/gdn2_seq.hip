@@ -233,7 +233,7 @@ struct BlockCtx {
 template <int VP, bool MARKED>
 __device__ __forceinline__ BlockCtx make_ctx(const SeqArgs &a, int b, int h, int bh) {
     const int64_t edits = MARKED ? (int64_t)a.nck * ((a.V + 15) >> 4) * 256 : SEQ_CT * VP;
-    return BlockCtx{a.T, a.K, a.V, a.H, b, h, a.fu + bh * edits, a.dscores};
+    return BlockCtx{a.T, a.K, a.V, a.H, b, h, a.fu ? a.fu + bh * edits : nullptr, a.dscores};
 }
 
 template <int KP, int VP, int NT, bool BWD, bool MARKED, typename TIN>
@@ -297,6 +297,10 @@ __device__ __forceinline__ void token_flags(const TokenRegs<KP, VP, NT, BWD> &r,
 
 // ---- forward ---------------------------------------------------------------------
 
+// What the forward is for: a call of one block, with its checkpoint; the marked heads,
+// with theirs; or the outputs alone, of any length.
+enum { SEQ_BLOCK, SEQ_MARKED, SEQ_PLAIN };
+
 // Forward lane tile: RL key rows x CL value columns per lane, RGN row groups
 // and CLN column lanes per wave (16 value columns per wave).  Eight row groups
 // keep the per-token LDS reads of the key-side rows (a, e.k, k, q) at
@@ -316,15 +320,16 @@ struct FwdTokens {
     float val[SEQ_CT], rst[SEQ_CT];
 };
 
-template <int KP, int VP, bool MARKED>
+template <int KP, int VP, int MODE>
 struct alignas(16) SeqFwdSmem {
-    FwdTokens<KP, VP> buf[MARKED ? 2 : 1];  // the next block's beside this one's
+    static constexpr int NB = MODE == SEQ_BLOCK ? 1 : 2;
+    FwdTokens<KP, VP> buf[NB];  // the next block's beside this one's
     float o[SEQ_CT][VP], d[SEQ_CT][VP];
 };
 
-template <int KP, int VP, bool MARKED>
+template <int KP, int VP, int MODE>
 union SeqFwdShared {
-    SeqFwdSmem<KP, VP, MARKED> s;
+    SeqFwdSmem<KP, VP, MODE> s;
     float st[KP * (VP + 1)];  // state transpose slab (row stride VP+1)
 };
 
@@ -381,18 +386,20 @@ __device__ __forceinline__ void fetch_fwd(const FwdTokens<KP, VP> &B, int tt, in
 }
 
 #pragma clang fp contract(off)
-template <int KP, int VP, bool MARKED, typename TIN>
+template <int KP, int VP, int MODE, typename TIN>
 __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
     using L = FwdLayout<KP>;
     constexpr int RL = L::RL, CL = L::CL, CLN = L::CLN, NT = 4 * VP, CT = SEQ_CT;
-    __shared__ SeqFwdShared<KP, VP, MARKED> sh;
-    SeqFwdSmem<KP, VP, MARKED> &s = sh.s;
+    constexpr bool MARKED = MODE == SEQ_MARKED;
+    __shared__ SeqFwdShared<KP, VP, MODE> sh;
+    SeqFwdSmem<KP, VP, MODE> &s = sh.s;
+    constexpr int NB = SeqFwdSmem<KP, VP, MODE>::NB;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int rg = lane / CLN, cl = lane % CLN;
     const int r0 = RL * rg, c0 = 16 * w + CL * cl;  // first key row / value column of this lane
     const int bh = blockIdx.x, b = bh / a.H, h = bh % a.H;
     if (MARKED && a.only[bh] == 0) return;
-    const int nck = MARKED ? a.nck : 1;
+    const int nck = MODE == SEQ_BLOCK ? 1 : a.nck;
     const int KT = (a.K + 15) >> 4, VT = (a.V + 15) >> 4;  // the checkpoint's tiles
 
     // Initial state, coalesced through the transpose slab.
@@ -421,7 +428,7 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
 
     for (int blk = 0; blk < nck; ++blk) {
         const int t0 = blk * CT, nt = min(CT, a.T - t0);
-        const FwdTokens<KP, VP> &B = s.buf[MARKED ? blk & 1 : 0];
+        const FwdTokens<KP, VP> &B = s.buf[blk % NB];
         if constexpr (MARKED) {
             float *st = a.st + ((int64_t)bh * a.nck + blk) * KT * VT * 256;
             static_assert(RL % 4 == 0, "whole pieces");
@@ -434,7 +441,7 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
                         *reinterpret_cast<seq_f4 *>(st + seq_state_at(i, j, KT)) =
                             seq_f4{S[ri][cj], S[ri + 1][cj], S[ri + 2][cj], S[ri + 3][cj]};
                 }
-        } else {
+        } else if constexpr (MODE == SEQ_BLOCK) {
             float *st = a.st + (int64_t)bh * KP * VP;
 #pragma unroll
             for (int ri = 0; ri < RL; ++ri) lds_put<CL>(st + (r0 + ri) * VP + c0, S[ri]);
@@ -495,9 +502,9 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
         // operations still in flight, so waiting for them does not wait for
         // this block's output stores.
         if (blk + 1 < nck) {
-            store_fwd_flags<KP, VP, NT, TIN>(nx, s.buf[MARKED ? (blk + 1) & 1 : 0], tid);
+            store_fwd_flags<KP, VP, NT, TIN>(nx, s.buf[(blk + 1) % NB], tid);
             __syncthreads();
-            store_fwd_data<KP, VP, NT, TIN>(nx, s.buf[MARKED ? (blk + 1) & 1 : 0], tid);
+            store_fwd_data<KP, VP, NT, TIN>(nx, s.buf[(blk + 1) % NB], tid);
         }
         for (int idx = tid; idx < CT * VP; idx += NT) {
             const int tt = idx / VP, c = idx % VP;
@@ -506,7 +513,7 @@ __global__ void __launch_bounds__(4 * VP) seq_fwd_kernel(SeqArgs a) {
             if constexpr (MARKED) {
                 if (c < 16 * VT)
                     a.fu[((int64_t)bh * a.nck + blk) * VT * 256 + seq_edit_at(tt, c)] = tt < nt ? s.d[tt][c] : 0.f;
-            } else if (tt < nt) {
+            } else if (MODE == SEQ_BLOCK && tt < nt) {
                 a.fu[(int64_t)bh * CT * VP + tt * VP + c] = s.d[tt][c];
             }
         }
@@ -1010,17 +1017,22 @@ static hipError_t decode_typed(const SeqArgs &a, bool bf16, hipStream_t st) {
     return hipGetLastError();
 }
 
-template <int KP, int VP, bool MARKED, typename TIN>
+template <int KP, int VP, int MODE, typename TIN>
 static void fwd_kernel(const SeqArgs &a, hipStream_t st) {
-    hipLaunchKernelGGL((seq_fwd_kernel<KP, VP, MARKED, TIN>), dim3(a.B * a.H), dim3(4 * VP), 0, st, a);
+    hipLaunchKernelGGL((seq_fwd_kernel<KP, VP, MODE, TIN>), dim3(a.B * a.H), dim3(4 * VP), 0, st, a);
+}
+template <int KP, int VP, int MODE>
+static void fwd_mode(const SeqArgs &a, bool bf16, hipStream_t st) {
+    if (bf16) fwd_kernel<KP, VP, MODE, bf16_t>(a, st);
+    else fwd_kernel<KP, VP, MODE, float>(a, st);
 }
 template <int KP, int VP>
 static hipError_t fwd_typed(const SeqArgs &a, bool bf16, hipStream_t st) {
-    if (a.only) bf16 ? fwd_kernel<KP, VP, true, bf16_t>(a, st) : fwd_kernel<KP, VP, true, float>(a, st);
-    else bf16 ? fwd_kernel<KP, VP, false, bf16_t>(a, st) : fwd_kernel<KP, VP, false, float>(a, st);
+    if (a.only) fwd_mode<KP, VP, SEQ_MARKED>(a, bf16, st);
+    else if (a.st) fwd_mode<KP, VP, SEQ_BLOCK>(a, bf16, st);
+    else fwd_mode<KP, VP, SEQ_PLAIN>(a, bf16, st);
     return hipGetLastError();
 }
-
 template <int KP, int VP, bool MARKED, typename TIN>
 static void bwd_kernel(const SeqArgs &a, hipStream_t st) {
     hipLaunchKernelGGL((seq_bwd_kernel<KP, VP, MARKED, TIN>), dim3(a.B * a.H), dim3(SeqBwdCfg<KP, VP>::NT), 0, st, a);
@@ -1045,7 +1057,7 @@ static hipError_t bwd_typed(const SeqArgs &a, bool bf16, hipStream_t st) {
     return FN<128, 128>(a, bf16, st);
 
 hipError_t launch_seq_fwd(const SeqArgs &a, bool bf16, hipStream_t st) {
-    if (!a.st || !a.fu || (!a.only && a.T > SEQ_CT)) return hipErrorInvalidValue;
+    if (!a.st != !a.fu || (a.only && !a.st) || (a.st && !a.only && a.T > SEQ_CT)) return hipErrorInvalidValue;
     GDN2_SEQ_DISPATCH(fwd_typed)
 }
 

@@ -331,6 +331,11 @@ def gdn2_scan(q, k, v, alpha, erase, write, doc_start, doc_end):
 def gdn_scalar_forward(q, k, v, beta, g, valid, reset, initial=None, chunk: int = 64):
     """Raw forward of the scalar-gate scan.  Returns (output, final_state,
     scores, checkpoint); the checkpoint is private storage for the backward."""
+    return _scalar_forward("gdn_scalar_call_checkpoint_bytes", "gdn_scalar_scan", q, k, v, beta, g,
+                           valid, reset, initial, chunk)
+
+
+def _scalar_forward(size, scan, q, k, v, beta, g, valid, reset, initial, chunk):
     L = lib()
     shape = _shape(q, v)
     B, T, H, K = q.shape
@@ -340,17 +345,14 @@ def gdn_scalar_forward(q, k, v, beta, g, valid, reset, initial=None, chunk: int 
     final = torch.empty((B, H, K, V), dtype=torch.float32, device=dev)
     scores = torch.empty((B, T, H), dtype=torch.float32, device=dev)
     views = [_view(x) for x in (q, k, v, beta, g, valid, reset, initial)]
-    nck = L.gdn_scalar_call_checkpoint_bytes(ctypes.byref(shape), chunk,
-                                             *[ctypes.byref(x) for x in views[:3]])
-    if nck == 0:
-        check("gdn_scalar_call_checkpoint_bytes", 1)
-    ck = torch.empty((nck,), dtype=torch.uint8, device=dev)
+    n = getattr(L, size)(ctypes.byref(shape), chunk, *[ctypes.byref(x) for x in views[:3]])
+    buf = torch.empty((n,), dtype=torch.uint8, device=dev)
     with on_device(dev):
-        rc = L.gdn_scalar_scan(ctypes.byref(shape), chunk, *[ctypes.byref(x) for x in views],
-                               _ptr(out), _code(out), _ptr(final), _ptr(scores), _ptr(ck), nck,
-                               _stream(q))
-    check("gdn_scalar_scan", rc)
-    return out, final, scores, ck
+        rc = getattr(L, scan)(ctypes.byref(shape), chunk, *[ctypes.byref(x) for x in views],
+                              _ptr(out), _code(out), _ptr(final), _ptr(scores), _ptr(buf), n,
+                              _stream(q))
+    check(scan, rc)
+    return out, final, scores, buf
 
 
 def gdn_scalar_backward(q, k, v, beta, g, valid, reset, checkpoint, chunk: int = 64,
@@ -393,7 +395,10 @@ def gdn_scalar_backward(q, k, v, beta, g, valid, reset, checkpoint, chunk: int =
 
 class _ScalarScan(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, q, k, v, beta, g, valid, reset, initial, chunk):
+    def forward(ctx, q, k, v, beta, g, valid, reset, initial, chunk, grad):
+        if not (grad and any(ctx.needs_input_grad)):
+            return _scalar_forward("gdn_scalar_outputs_bytes", "gdn_scalar_outputs", q, k, v, beta,
+                                   g, valid, reset, initial, chunk)[:3]
         out, final, scores, ck = gdn_scalar_forward(q, k, v, beta, g, valid, reset, initial,
                                                     chunk)
         # Unused outputs reach backward as None (not zero tensors), so the
@@ -411,7 +416,7 @@ class _ScalarScan(torch.autograd.Function):
         dq, dk, dv, db, dg, dinit = gdn_scalar_backward(q, k, v, beta, g, valid, reset,
                                                         ctx.checkpoint, ctx.chunk, d_out,
                                                         d_final, d_scores)
-        return dq, dk, dv, db, dg, None, None, (dinit if ctx.has_initial else None), None
+        return dq, dk, dv, db, dg, None, None, (dinit if ctx.has_initial else None), None, None
 
 
 def gdn_scalar_scan(q, k, v, beta, g, valid=None, reset=None, initial=None,
@@ -432,7 +437,8 @@ def gdn_scalar_scan(q, k, v, beta, g, valid=None, reset=None, initial=None,
     g = g if g.dtype == torch.float32 else g.float()
     if initial is not None and initial.dtype != torch.float32:
         initial = initial.float()
-    return _ScalarScan.apply(q, k, v, beta, g, valid, reset, initial, chunk_size)
+    return _ScalarScan.apply(q, k, v, beta, g, valid, reset, initial, chunk_size,
+                             torch.is_grad_enabled())
 
 
 # ---- decode ---------------------------------------------------------------------

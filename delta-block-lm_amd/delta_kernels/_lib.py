@@ -107,6 +107,8 @@ SIGNATURES = {
     "gdn_scalar_call_checkpoint_bytes": (_Z, [_S, _I] + [_V] * 3),
     "gdn_scalar_call_workspace_bytes": (_Z, [_S, _I] + [_V] * 3),
     "gdn_scalar_scan": (_I, [_S, _I] + [_V] * 8 + [_P, ctypes.c_int32, _F, _F, _P, _Z, _P]),
+    "gdn_scalar_outputs_bytes": (_Z, [_S, _I] + [_V] * 3),
+    "gdn_scalar_outputs": (_I, [_S, _I] + [_V] * 8 + [_P, ctypes.c_int32, _F, _F, _P, _Z, _P]),
     "gdn_scalar_backward": (_I, [_S, _I] + [_V] * 7 + [_P, _Z, _V, _F, _F] + [_P] * 3
                             + [_F] * 3 + [_P, _Z, _P]),
     "gdn_scalar_backward_noalloc": (_I, [_S, _I] + [_V] * 7 + [_P, _Z, _V, _F, _F] + [_P] * 3

@@ -203,6 +203,19 @@ GDN2_API int gdn_scalar_scan(const gdn2_shape *shape, int chunk, const gdn2_view
                     float *final_state, float *scores, void *checkpoint,
                     size_t checkpoint_bytes, void *stream);
 
+/* The same forward for a caller that no backward follows: no checkpoint, and a
+ * workspace (gdn_scalar_outputs_bytes; may be zero, then workspace may be NULL)
+ * that is free again when the call has run.  It picks its kernels for the forward
+ * alone. */
+GDN2_API size_t gdn_scalar_outputs_bytes(const gdn2_shape *shape, int chunk, const gdn2_view *q,
+                                         const gdn2_view *k, const gdn2_view *v);
+GDN2_API int gdn_scalar_outputs(const gdn2_shape *shape, int chunk, const gdn2_view *q,
+                       const gdn2_view *k, const gdn2_view *v, const gdn2_view *beta,
+                       const gdn2_view *g, const gdn2_view *valid, const gdn2_view *reset,
+                       const gdn2_view *initial, void *output, int32_t output_dtype,
+                       float *final_state, float *scores, void *workspace,
+                       size_t workspace_bytes, void *stream);
+
 GDN2_API size_t gdn_scalar_workspace_bytes(const gdn2_shape *shape, int chunk);
 
 GDN2_API int gdn_scalar_backward(const gdn2_shape *shape, int chunk, const gdn2_view *q,
