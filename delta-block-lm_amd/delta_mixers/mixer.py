@@ -42,28 +42,52 @@ class GdnMixerConfig:
 
 
 class _Projections(torch.autograd.Function):
-    """x W_i^T for every weight [width_i, D], side by side on the last axis."""
+    """x W_i^T for every weight [width_i, D], side by side on the last axis.  With a tuple of
+    widths and a number behind the weights: the same columns in pieces of these widths, the last
+    so many of them through a sigmoid."""
 
     @staticmethod
-    def forward(ctx, x, *weights):
-        ctx.save_for_backward(x, *weights)
-        return F.linear(x, torch.cat(weights))
+    def forward(ctx, x, *args):
+        weights, pieces, gates = args, None, 0
+        if not torch.is_tensor(args[-1]):
+            *weights, pieces, gates = args
+        ctx.extra, ctx.gates = len(args) - len(weights), gates
+        z = F.linear(x, torch.cat(weights))
+        if pieces is None:
+            ctx.save_for_backward(x, *weights)
+            return z
+        out = z.split(pieces, -1)
+        if gates:  # the last columns are one strided block
+            n = sum(pieces[-gates:])
+            z.narrow(-1, z.shape[-1] - n, n).sigmoid_()
+        ctx.save_for_backward(x, *weights, *out[len(out) - gates:])
+        return out
 
     @staticmethod
-    def backward(ctx, dz):
+    def backward(ctx, *dz):
         x, *weights = ctx.saved_tensors
+        if ctx.gates:
+            weights, y = weights[:-ctx.gates], weights[-ctx.gates:]
+            dz = dz[:-ctx.gates] + tuple(torch.ops.aten.sigmoid_backward(d, s)
+                                         for d, s in zip(dz[-ctx.gates:], y))
+        dz = dz[0] if len(dz) == 1 else torch.cat(dz, -1)
         widths = [w.shape[0] for w in weights]
         dz = dz.reshape(-1, dz.shape[-1])
-        dx, dw = None, [None] * len(weights)
+        dx, need = None, ctx.needs_input_grad[1:1 + len(weights)]
         if ctx.needs_input_grad[0]:
             # One projection after another: a single product over all columns is a longer sum
             # in f32 (the pass's error against 64 bits rises from 2.1e-6 to 2.9e-6).
             for d, w in zip(dz.split(widths, 1), weights):
                 dx = d @ w if dx is None else dx.addmm_(d, w)
             dx = dx.view(x.shape)
-        if any(ctx.needs_input_grad[1:]):
-            dw = (dz.t() @ x.reshape(-1, x.shape[-1])).split(widths)
-        return (dx, *dw)
+        x = x.reshape(-1, x.shape[-1])
+        if not all(need):
+            dw = [d.t() @ x if n else None for d, n in zip(dz.split(widths, 1), need)]
+        else:
+            # One product, then each weight's rows copied to memory of their own: a gradient that
+            # is kept keeps no other.
+            dw = torch._foreach_mul((dz.t() @ x).split(widths), 1.0)
+        return (dx, *dw, *[None] * ctx.extra)
 
 
 class GdnMixer(torch.nn.Module):
@@ -117,13 +141,14 @@ class GdnMixer(torch.nn.Module):
         x = x * valid[..., None]
         docs = torch.cumsum(reset * valid, dim=1)
 
-        # One GEMM for the seven projections, one convolution for q, k and v, one L2 norm for q
-        # and k: the host took longer to launch them one by one (66 kernels, 1.6 ms a training
-        # pass at 8 x 512 tokens) than they ran.  Every operator reads its columns in place.
+        # One GEMM for the seven projections (erase and write leave it as sigmoids: the products
+        # themselves are not kept), one convolution for q, k and v, one L2 norm for q and k: the
+        # host took longer to launch them one by one (66 kernels, 1.6 ms a training pass at
+        # 8 x 512 tokens) than they ran.  Every operator reads its columns in place.
         kw, vw = H * K, H * V
-        z = _Projections.apply(x, self.q, self.k, self.v, self.decay, self.erase, self.write,
-                               self.output_gate)
-        qkv, z_decay, z_erase, z_write, z_gate = z.split([2 * kw + vw, kw, kw, vw, vw], -1)
+        qkv, z_decay, z_gate, erase, write = _Projections.apply(
+            x, self.q, self.k, self.v, self.decay, self.output_gate, self.erase, self.write,
+            (2 * kw + vw, kw, vw, kw, vw), 2)
         qkv = dk.causal_conv(qkv, torch.cat([self.q_conv, self.k_conv, self.v_conv], 1), valid,
                              docs, activation="silu")
         qk, v = qkv.split([2 * kw, vw], -1)
@@ -131,8 +156,7 @@ class GdnMixer(torch.nn.Module):
         q, k = dk.l2_norm(qk.view(B, T, 2 * H, K)).view(B, T, 2, H, K).unbind(2)
         v = v.view(B, T, H, V)
         alpha = dk.decay(z_decay.view(B, T, H, K), self.decay_bias, self.decay_scale)
-        erase = torch.sigmoid(z_erase).view(B, T, H, K)
-        write = torch.sigmoid(z_write).view(B, T, H, V)
+        erase, write = erase.view(B, T, H, K), write.view(B, T, H, V)
         scan = dk.gdn_training_scan(q, k, v, alpha, erase, write, valid, reset, None,
                                     cfg.chunk_size)
         out = scan.output
