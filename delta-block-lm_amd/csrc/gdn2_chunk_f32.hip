@@ -242,6 +242,7 @@ struct FcScanOps {
     f32x4 g, k, a;     // gv rows; Ktil or W', A operand over the tokens; U or Qhat
     f32x4 d, p;        // reverse: dO columns j, P rows
     f32x4 on;
+    f32x4 c, e;        // reverse with a score adjoint: the coefficients c, the edits
 };
 
 // The workgroups of one (batch, head) read the same factors, so they take block
@@ -299,6 +300,10 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
             o.d = FcSrc<BF, VEC>(dov, b, h, c, s.T, V).col(cg);
             o.p = oc.get(a.pm + ci * C * C);
             o.on = fc_gb4(a, ci, 0);
+            if (SC) {
+                o.c = fc_g4(a.sc + ((int64_t)bh * a.wn + chunk_at(step)) * 2 * C, 16 * g);
+                o.e = fc_g4(a.fu + (ci * VT + cg) * 256, 16 * l);
+            }
         }
     };
     // The loads are issued in ring order, the order in which the steps wait for
@@ -312,22 +317,16 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
     // A step's masked dO and the terms of v known before X: U, or in tile 0 P^T dO
     // + c delta.
     f32x4 dnext = zero4(), base = zero4();
-    auto prepare = [&](int step, const FcScanOps<REV> &o) {
+    auto prepare = [&](const FcScanOps<REV> &o) {
         if (!REV) {
             base = o.a;
             return;
         }
         dnext = fc_keep(fc_keep4(o.d, o.on), has_do);
         if (tau != 0) return;
-        base = zero4();
-        if (SC) {
-            const int cw = chunk_at(step);
-            base = fc_g4(a.sc + ((int64_t)bh * a.wn + cw) * 2 * C, 16 * g) *
-                   fc_g4(a.fu + (((int64_t)bh * a.nc + a.w0 + cw) * VT + cg) * 256, 16 * l);
-        }
-        base = fc_mma4(o.p, dnext, base);
+        base = fc_mma4(o.p, dnext, SC ? o.c * o.e : zero4());
     };
-    prepare(0, ring[0]);
+    prepare(ring[0]);
     float *keep = REV ? a.ds : a.st;
     auto advance = [&](int step, int d) __attribute__((always_inline)) {
         const int cw = chunk_at(step);
@@ -352,7 +351,7 @@ __global__ void __launch_bounds__(64 * KT) fc_scan_kernel(FcArgs a) {
         // in the shadow of the exchange: what depends on neither X nor v
         f32x4 x = cur.g * X, v = vp;
         if (REV) x = fc_mma4(cur.a, dnow, x);
-        prepare(step + 1, ring[(d + 1) % D]);
+        prepare(ring[(d + 1) % D]);
         if (KT > 1) {
             __syncthreads();
             float4 t0 = vpart[par][0][l];
@@ -692,20 +691,18 @@ static void fc_scan(const FcArgs &a, hipStream_t stream) {
 
 void launch_fc_scan(const FcArgs &a, hipStream_t stream) { fc_scan<false, false, false, false>(a, stream); }
 
+template <bool SC>
+static void fc_adjoint(const FcArgs &a, hipStream_t stream) {
+    if (a.in_bf16 && a.vec) fc_scan<true, true, true, SC>(a, stream);
+    else if (a.in_bf16) fc_scan<true, true, false, SC>(a, stream);
+    else if (a.vec) fc_scan<true, false, true, SC>(a, stream);
+    else fc_scan<true, false, false, SC>(a, stream);
+}
+
 void launch_fc_adjoint(const FcArgs &a, hipStream_t stream) {
-    if (a.s.dscores) {  // the reads of any layout only
-        hipLaunchKernelGGL(fc_score_kernel, dim3(a.s.B * a.s.H * a.wn), dim3(64), 0, stream, a);
-        if (a.in_bf16) fc_scan<true, true, false, true>(a, stream);
-        else fc_scan<true, false, false, true>(a, stream);
-    } else if (a.in_bf16 && a.vec) {
-        fc_scan<true, true, true, false>(a, stream);
-    } else if (a.in_bf16) {
-        fc_scan<true, true, false, false>(a, stream);
-    } else if (a.vec) {
-        fc_scan<true, false, true, false>(a, stream);
-    } else {
-        fc_scan<true, false, false, false>(a, stream);
-    }
+    if (!a.s.dscores) return fc_adjoint<false>(a, stream);
+    hipLaunchKernelGGL(fc_score_kernel, dim3(a.s.B * a.s.H * a.wn), dim3(64), 0, stream, a);
+    fc_adjoint<true>(a, stream);
 }
 
 hipError_t launch_fc_fwd(const FcArgs &a, hipStream_t stream, const hipEvent_t *ev) {
