@@ -141,8 +141,11 @@ struct FcSrc {
         }
     }
     __device__ __forceinline__ float at(int t, int ch) const {
-        if (t0 + t >= T || ch >= W) return 0.f;
-        return BF ? ld4<bf16_t>(v, b, t0 + t, h, ch) : ld4<float>(v, b, t0 + t, h, ch);
+        // Loaded whether wanted or not (the sequence's last row, the last channel), so
+        // that no load waits behind a branch.
+        const int tt = min(t0 + t, T - 1), cc = min(ch, W - 1);
+        const float x = BF ? ld4<bf16_t>(v, b, tt, h, cc) : ld4<float>(v, b, tt, h, cc);
+        return t0 + t < T && ch < W ? x : 0.f;
     }
     __device__ __forceinline__ f32x4 frag(int tau) const {
         if (VEC) {
