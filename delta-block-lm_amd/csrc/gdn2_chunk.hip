@@ -483,14 +483,17 @@ __global__ void __launch_bounds__(AS_THREADS) affine_scan_kernel(AsArgs p) {
                                                  16, 0, 0);
             }
         };
-        for (int s = 0; s < AS_MRING; ++s) issue(s);
-        __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_MRING - 1) * AS_MOPS));
+        for (int s = 0; s < AS_MRING && s < p.nc; ++s) issue(s);
+        // Near the end fewer maps than the ring holds are in flight: wait for them all.
+        if (AS_MRING <= p.nc) __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_MRING - 1) * AS_MOPS));
+        else __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
         as_barrier();  // chunk 0 has landed
         for (int s = 0; s < p.nc; ++s) {
             // chunk s + 1 has landed once no more than the AS_MRING - 2 later maps are in flight
-            __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_MRING - 2) * AS_MOPS));
+            if (s + AS_MRING <= p.nc) __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_MRING - 2) * AS_MOPS));
+            else __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
             as_barrier();
-            issue(s + AS_MRING);  // into the slot that held chunk s
+            if (s + AS_MRING < p.nc) issue(s + AS_MRING);  // into the slot that held chunk s
         }
         __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
         return;
@@ -506,13 +509,15 @@ __global__ void __launch_bounds__(AS_THREADS) affine_scan_kernel(AsArgs p) {
                                                  0, 0);
             }
         };
-        for (int s = 0; s < AS_NRING; ++s) issue(s);
-        __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_NRING - 1) * AS_NOPS));
+        for (int s = 0; s < AS_NRING && s < p.nc; ++s) issue(s);
+        if (AS_NRING <= p.nc) __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_NRING - 1) * AS_NOPS));
+        else __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
         as_barrier();
         for (int s = 0; s < p.nc; ++s) {
-            __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_NRING - 2) * AS_NOPS));
+            if (s + AS_NRING <= p.nc) __builtin_amdgcn_s_waitcnt(as_vmcnt((AS_NRING - 2) * AS_NOPS));
+            else __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
             as_barrier();
-            issue(s + AS_NRING);
+            if (s + AS_NRING < p.nc) issue(s + AS_NRING);
         }
         __builtin_amdgcn_s_waitcnt(as_vmcnt(0));
         return;
