@@ -28,10 +28,13 @@
 namespace gdn2 {
 namespace {
 
-constexpr int kGroupRows = 8;       // time steps per 16-lane group of a convolution wave
-constexpr int kWaveRows = 4 * kGroupRows;
-constexpr int kInWaves = 4;
-constexpr int kSegRows = kWaveRows * kInWaves;  // time steps per segment (one workgroup)
+// Time steps of a 16-lane group, a wave and a segment (one workgroup) of the convolution.
+template <int GROUP, int WAVES>
+struct InTile {
+    static constexpr int group = GROUP, wave = 4 * GROUP, waves = WAVES, seg = wave * WAVES;
+};
+using InWide = InTile<8, 4>;
+using InShort = InTile<4, 1>;
 constexpr int kBwdBlocks = 1024;    // workgroups of the persistent row VJPs (fixed: deterministic)
 constexpr int kSumWaves = 16;
 
@@ -257,7 +260,7 @@ struct InArgs {
     float *gpart;  // [B nseg][2 H]
 };
 
-__host__ __device__ inline int64_t in_segments(int64_t T) { return (T + kSegRows - 1) / kSegRows; }
+__host__ __device__ inline int64_t in_segments(int64_t T, int seg) { return (T + seg - 1) / seg; }
 
 // Four bf16 channels of a row, packed.  VEC: one 8-byte access (bases 8-byte
 // aligned; the row strides always are, z_stride being a multiple of 4).
@@ -292,40 +295,51 @@ __device__ __forceinline__ void unpack_here(uint2 u, float *f) {
 struct RowSpan {
     int64_t t0;
     int lo, hi;
-    __device__ __forceinline__ RowSpan(const InArgs &a, int W) {
-        t0 = (blockIdx.x % in_segments(a.T)) * kSegRows;
+    __device__ __forceinline__ RowSpan(const InArgs &a, int W, int seg) {
+        t0 = (blockIdx.x % in_segments(a.T, seg)) * seg;
         lo = t0 == 0 ? 0 : -(W - 1);
-        hi = (int)min(a.T - 1 - t0, (int64_t)(kSegRows + W - 2));
+        hi = (int)min(a.T - 1 - t0, (int64_t)(seg + W - 2));
     }
 };
 
 // Lag masks of a wave's rows: the mask of the lag from row s to row r is
 // valid[s] valid[r] [docs[s] == docs[r]], 0 outside [0, T).  Slot j is row
-// tw - (W - 1) + j; lane j fetches slot j (kWaveRows + 2 (W - 1) <= 64 of
-// them).  Where every row in [0, T) is valid and of one document, each mask in
+// tw - (W - 1) + j; lane j takes slot j (rows + 2 (W - 1) <= 64 of them) and leaves its
+// W lags in LDS, side by side: a row's masks are one or two 16-byte reads there.
+// Where every row in [0, T) is valid and of one document, each mask in
 // range is one (rows outside hold x = 0 and gradient 0): `plain`, wave-uniform,
 // and nothing is multiplied.
+template <int W, class R>
 struct LagMasks {
-    const float *v, *d;  // LDS, 64 each
+    static constexpr int slots = R::wave + 2 * (W - 1), pitch = (W + 3) & ~3;
+    const float *lag;  // LDS, [slots][pitch]
     bool plain;
 
-    __device__ __forceinline__ void fetch(const InArgs &a, int64_t b, int64_t tw, int W, int lane,
-                                          float *lds) {
+    __device__ __forceinline__ void fetch(const InArgs &a, int64_t b, int64_t tw, int lane, float *lds) {
         const int64_t t = tw - (W - 1) + lane;
-        const bool in = t >= 0 && t < a.T && lane < kWaveRows + 2 * (W - 1);
+        const bool in = t >= 0 && t < a.T && lane < slots;
         const float vt = in ? a.valid[b * a.T + t] : 0.f, dt = in ? a.docs[b * a.T + t] : 0.f;
         const float ref = __shfl(dt, W - 1);  // row tw, in range
         plain = __all(!in || (vt == 1.f && dt == ref));
-        lds[lane] = vt;
-        lds[64 + lane] = dt;
+        lag = lds;
+        if (plain) return;
+#pragma unroll
+        for (int l = 0; l < W; ++l) {
+            const float vs = __shfl(vt, lane - l), ds = __shfl(dt, lane - l);  // below slot 0: not read
+            if (lane < slots) lds[lane * pitch + l] = ds == dt ? vs * vt : 0.f;
+        }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read by the wave's other lanes
         __builtin_amdgcn_wave_barrier();
-        v = lds;
-        d = lds + 64;
     }
-    __device__ __forceinline__ float at(int from, int to) const {
-        return d[from] == d[to] ? v[from] * v[to] : 0.f;
+    // The masks of every lag to slot `to`.
+    __device__ __forceinline__ void row(int to, float (&m)[pitch]) const {
+#pragma unroll
+        for (int l = 0; l < pitch; l += 4) {
+            const float4 x = *reinterpret_cast<const float4 *>(&lag[to * pitch + l]);
+            m[l] = x.x, m[l + 1] = x.y, m[l + 2] = x.z, m[l + 3] = x.w;
+        }
     }
+    __device__ __forceinline__ float at(int to, int l) const { return lag[to * pitch + l]; }
 };
 
 // Gate columns of a wave's rows [t0, t1): lane h = lane % H handles every
@@ -333,7 +347,7 @@ struct LagMasks {
 __device__ void gates_forward(const InArgs &a, int64_t b, int64_t t0, int64_t t1, int lane) {
     const int H = a.H;
     const int64_t cb = a.C + (int64_t)H * a.V;  // beta column; decay follows at cb + H
-    for (int i = lane; i < kWaveRows * H; i += 64) {
+    for (int i = lane; i < (int)(t1 - t0) * H; i += 64) {
         const int64_t t = t0 + i / H;
         const int h = i % H;
         if (t >= t1) break;
@@ -349,33 +363,32 @@ __device__ void gates_forward(const InArgs &a, int64_t b, int64_t t0, int64_t t1
 
 // Pre-activation of the row in slot r + W - 1 of xs, its lag masks m[].
 template <int W, bool PLAIN>
-__device__ __forceinline__ void conv_row(const float (*xs)[4], const float (*w)[4],
-                                         const LagMasks &mk, int slot, int r, float *p) {
+__device__ __forceinline__ void conv_row(const float (*xs)[4], const float (*w)[4], const float *m,
+                                         int r, float *p) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) p[e] = 0.f;
 #pragma unroll
-    for (int l = 0; l < W; ++l) {
-        const float m = PLAIN ? 1.f : mk.at(slot + r + W - 1 - l, slot + r + W - 1);
+    for (int l = 0; l < W; ++l)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const float t = xs[r + W - 1 - l][e] * w[l][e];
-            p[e] += PLAIN ? t : t * m;
+            p[e] += PLAIN ? t : t * m[l];
         }
-    }
 }
 
-template <int W, bool VEC, bool PLAIN>
+template <int W, bool VEC, class R, bool PLAIN>
 __device__ __forceinline__ void in_fwd_rows(const InArgs &a, const uint2 *xq, const float (*w)[4],
-                                            const LagMasks &mk, int grp, bool l2, int64_t tg,
-                                            bf16_t *out) {
-    constexpr int NR = kGroupRows + W - 1;
+                                            const LagMasks<W, R> &mk, int grp, bool l2,
+                                            int64_t tg, bf16_t *out) {
+    constexpr int NR = R::group + W - 1;
     float x[NR][4];
 #pragma unroll
     for (int i = 0; i < NR; ++i) unpack4(xq[i], x[i]);
 #pragma unroll
-    for (int i = 0; i < kGroupRows; ++i) {
-        float p[4], ss = 0.f;
-        conv_row<W, PLAIN>(x, w, mk, grp * kGroupRows, i, p);
+    for (int i = 0; i < R::group; ++i) {
+        float p[4], ss = 0.f, m[LagMasks<W, R>::pitch];
+        if (!PLAIN) mk.row(grp * R::group + i + W - 1, m);
+        conv_row<W, PLAIN>(x, w, m, i, p);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             p[e] = p[e] * sigm(p[e]);
@@ -392,29 +405,31 @@ __device__ __forceinline__ void in_fwd_rows(const InArgs &a, const uint2 *xq, co
 
 // Both kernels: grid (B nseg, C / 64 + 1).  Block column y < C / 64 holds 64
 // channels (one head of q, k or v): a lane owns four of them, 16 lanes a row
-// (its L2 sum is four DPP steps), and each 16-lane group walks kGroupRows time
+// (its L2 sum is four DPP steps), and each 16-lane group walks R::group time
 // steps with the rows it needs fetched up front as 8-byte loads.  The groups
 // share nothing: the W - 1 rows on either side are read again (from cache) and
 // their gradients formed again, which costs less than the wave-wide sums and
 // the LDS exchange of one lane per channel.  The last column does the gates.
 // Bound by VALU work (SiLU and its VJP).  At 16 x 512 tokens, H = 8, 4 taps:
-// forward 24.9 -> 16.5 us, VJP 60.7 -> 31.4 us against one lane per channel.
-template <int W, bool VEC>
-__global__ void __launch_bounds__(64 * kInWaves) lm_in_fwd_kernel(InArgs a) {
-    constexpr int NR = kGroupRows + W - 1;
-    const int64_t nseg = in_segments(a.T);
+// forward 24.9 -> 16.5 us, VJP 60.7 -> 31.4 us against one lane per channel; with
+// padding and documents (masks multiplied) 37.7, and 45.3 with each mask formed from
+// its two rows where it is used.
+template <int W, bool VEC, class R>
+__global__ void __launch_bounds__(64 * R::waves) lm_in_fwd_kernel(InArgs a) {
+    constexpr int NR = R::group + W - 1;
+    const int64_t nseg = in_segments(a.T, R::seg);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, grp = lane >> 4;
     const int64_t b = blockIdx.x / nseg;
-    const int64_t tw = (blockIdx.x % nseg) * kSegRows + kWaveRows * wv;  // this wave's first row
+    const int64_t tw = (blockIdx.x % nseg) * R::seg + R::wave * wv;  // this wave's first row
     if (tw >= a.T) return;  // no barrier below: the waves are independent
     if ((int)blockIdx.y == a.C / 64) {
-        gates_forward(a, b, tw, min(tw + kWaveRows, a.T), lane);
+        gates_forward(a, b, tw, min(tw + R::wave, a.T), lane);
         return;
     }
     const int c = blockIdx.y * 64 + 4 * (lane & 15);
     const bool l2 = c < 2 * a.H * a.K;  // q and k heads: block-uniform
-    const int64_t tg = tw + kGroupRows * grp;
-    const RowSpan sp(a, W);
+    const int64_t tg = tw + R::group * grp;
+    const RowSpan sp(a, W, R::seg);
     const int r0 = (int)(tg - sp.t0), lo = sp.lo, hi = sp.hi;
     const bf16_t *zb = a.z + (b * a.T + sp.t0 + lo) * a.zs;
     uint2 xq[NR];
@@ -429,12 +444,13 @@ __global__ void __launch_bounds__(64 * kInWaves) lm_in_fwd_kernel(InArgs a) {
     for (int l = 0; l < W; ++l)
 #pragma unroll
         for (int e = 0; e < 4; ++e) w[l][e] = a.w[l * a.C + c + e];
-    __shared__ float mv[kInWaves][128];
-    LagMasks mk;
-    mk.fetch(a, b, tw, W, lane, mv[wv]);
+    using Masks = LagMasks<W, R>;
+    __shared__ __align__(16) float mv[R::waves][Masks::slots * Masks::pitch];
+    Masks mk;
+    mk.fetch(a, b, tw, lane, mv[wv]);
     bf16_t *out = a.qkv + (b * a.T + tg) * a.C + c;
-    if (mk.plain) in_fwd_rows<W, VEC, true>(a, xq, w, mk, grp, l2, tg, out);
-    else in_fwd_rows<W, VEC, false>(a, xq, w, mk, grp, l2, tg, out);
+    if (mk.plain) in_fwd_rows<W, VEC, R, true>(a, xq, w, mk, grp, l2, tg, out);
+    else in_fwd_rows<W, VEC, R, false>(a, xq, w, mk, grp, l2, tg, out);
 }
 
 __device__ void gates_backward(const InArgs &a, int64_t b, int64_t t0, int64_t t1, int lane,
@@ -442,7 +458,7 @@ __device__ void gates_backward(const InArgs &a, int64_t b, int64_t t0, int64_t t
     const int H = a.H;
     const int64_t cb = a.C + (int64_t)H * a.V;
     float pb = 0.f, ps = 0.f;
-    for (int i = lane; i < kWaveRows * H; i += 64) {
+    for (int i = lane; i < (int)(t1 - t0) * H; i += 64) {
         const int64_t t = t0 + i / H;
         const int h = i % H;
         if (t >= t1) break;
@@ -473,15 +489,15 @@ __device__ void gates_backward(const InArgs &a, int64_t b, int64_t t0, int64_t t
 }
 
 // The VJP of a group's rows: gr (the gradient at the pre-activation,
-// recomputed: window, SiLU, L2) of rows tg .. tg + kGroupRows + W - 2 in turn,
+// recomputed: window, SiLU, L2) of rows tg .. tg + R::group + W - 2 in turn,
 // dz of row t as soon as gr of row t + W - 1 is there.
-template <int W, bool VEC, bool PLAIN>
+template <int W, bool VEC, class R, bool PLAIN>
 __device__ __forceinline__ void in_bwd_rows(const InArgs &a, const uint2 *xq, const uint2 *uq,
-                                            const float (*w)[4], const LagMasks &mk, int grp,
+                                            const float (*w)[4], const LagMasks<W, R> &mk, int grp,
                                             bool l2, int64_t tw, int64_t tg, bf16_t *dz,
                                             float (*dw)[4]) {
-    constexpr int NG = kGroupRows + W - 1, NR = NG + W - 1;
-    const int slot = grp * kGroupRows;  // mask slot of x row 0
+    constexpr int NG = R::group + W - 1, NR = NG + W - 1;
+    const int slot = grp * R::group;  // mask slot of x row 0
     float x[NR][4], g[NG][4];
 #pragma unroll
     for (int i = 0; i < W - 1; ++i) unpack_here(xq[i], x[i]);
@@ -491,10 +507,11 @@ __device__ __forceinline__ void in_bwd_rows(const InArgs &a, const uint2 *xq, co
         for (int e = 0; e < 4; ++e) x[i + W - 1][e] = g[i][e] = 0.f;
         // Wave-uniform; and a block of its own for each row keeps the rows in order.
         if (tw + i < a.T) {
-            float p[4], sg[4], s[4], u[4];
+            float p[4], sg[4], s[4], u[4], m[LagMasks<W, R>::pitch];
+            if (!PLAIN) mk.row(slot + i + W - 1, m);
             unpack_here(xq[i + W - 1], x[i + W - 1]);
             unpack_here(uq[i], u);
-            conv_row<W, PLAIN>(x, w, mk, slot, i, p);
+            conv_row<W, PLAIN>(x, w, m, i, p);
             float ss = 0.f, us = 0.f;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -515,14 +532,13 @@ __device__ __forceinline__ void in_bwd_rows(const InArgs &a, const uint2 *xq, co
                 const float gv = u[e] * sg[e] * (1.f + p[e] * (1.f - sg[e]));
                 g[i][e] = in ? gv : 0.f;
             }
-            if (i < kGroupRows) {
+            if (i < R::group) {
 #pragma unroll
                 for (int l = 0; l < W; ++l) {
-                    const float m = PLAIN ? 1.f : mk.at(slot + i + W - 1 - l, slot + i + W - 1);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float t = g[i][e] * x[i + W - 1 - l][e];
-                        dw[l][e] += PLAIN ? t : t * m;
+                        dw[l][e] += PLAIN ? t : t * m[l];
                     }
                 }
             }
@@ -532,7 +548,7 @@ __device__ __forceinline__ void in_bwd_rows(const InArgs &a, const uint2 *xq, co
             float sum[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int l = 0; l < W; ++l) {
-                const float m = PLAIN ? 1.f : mk.at(slot + o + W - 1, slot + o + W - 1 + l);
+                const float m = PLAIN ? 1.f : mk.at(slot + o + W - 1 + l, l);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float t = g[o + l][e] * w[l][e];
@@ -549,23 +565,25 @@ __device__ __forceinline__ void in_bwd_rows(const InArgs &a, const uint2 *xq, co
 //   dz[t]  = sum_l gr[t + l] w[l] mask(t -> t + l)
 //   dw[l] += gr[t] z[t - l] mask(t - l -> t)     (t in this group)
 // The 16 groups' dw are added in order into one partial per workgroup.
-template <int W, bool VEC>
-__global__ void __launch_bounds__(64 * kInWaves) lm_in_bwd_kernel(InArgs a) {
-    constexpr int NG = kGroupRows + W - 1;  // gradient rows of a group
+template <int W, bool VEC, class R>
+__global__ void __launch_bounds__(64 * R::waves) lm_in_bwd_kernel(InArgs a) {
+    constexpr int NG = R::group + W - 1;  // gradient rows of a group
     constexpr int NR = NG + W - 1;          // rows read: tg - (W - 1) .. tg + NG - 1
-    const int64_t nseg = in_segments(a.T);
+    const int64_t nseg = in_segments(a.T, R::seg);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, grp = lane >> 4;
     const int64_t b = blockIdx.x / nseg;
-    const int64_t tw = (blockIdx.x % nseg) * kSegRows + kWaveRows * wv;  // this wave's first row
-    __shared__ __align__(16) float dwr[4 * kInWaves][W][64];
-    __shared__ float mv[kInWaves][128];
+    const int64_t tw = (blockIdx.x % nseg) * R::seg + R::wave * wv;  // this wave's first row
+    __shared__ __align__(16) float dwr[4 * R::waves][W][64];
+    using Masks = LagMasks<W, R>;
+    constexpr int MV = Masks::slots * Masks::pitch;
+    __shared__ __align__(16) float mv[R::waves][MV > 64 ? MV : 64];  // masks; the gates' sums, 2 H <= 64
     if ((int)blockIdx.y == a.C / 64) {
         if (lane < 2 * a.H) mv[wv][lane] = 0.f;
-        if (tw < a.T) gates_backward(a, b, tw, min(tw + kWaveRows, a.T), lane, mv[wv]);
+        if (tw < a.T) gates_backward(a, b, tw, min(tw + R::wave, a.T), lane, mv[wv]);
         __syncthreads();
         if ((int)threadIdx.x < 2 * a.H) {
             float t = mv[0][threadIdx.x];
-            for (int q = 1; q < kInWaves; ++q) t += mv[q][threadIdx.x];
+            for (int q = 1; q < R::waves; ++q) t += mv[q][threadIdx.x];
             a.gpart[(int64_t)blockIdx.x * 2 * a.H + threadIdx.x] = t;
         }
         return;
@@ -582,8 +600,8 @@ __global__ void __launch_bounds__(64 * kInWaves) lm_in_bwd_kernel(InArgs a) {
         const bf16_t *src = c < HK ? a.dq : (l2 ? a.dk : a.dv);
         const int64_t width = l2 ? HK : (int64_t)a.H * a.V;
         const int uc = c < HK ? c : (l2 ? c - HK : c - 2 * HK);
-        const int64_t tg = tw + kGroupRows * grp;
-        const RowSpan sp(a, W);
+        const int64_t tg = tw + R::group * grp;
+        const RowSpan sp(a, W, R::seg);
         const int r0 = (int)(tg - sp.t0), lo = sp.lo, hi = sp.hi;
         const bf16_t *zb = a.z + (b * a.T + sp.t0 + lo) * a.zs;
         const bf16_t *ub = src + (b * a.T + sp.t0) * width;
@@ -603,21 +621,21 @@ __global__ void __launch_bounds__(64 * kInWaves) lm_in_bwd_kernel(InArgs a) {
         for (int l = 0; l < W; ++l)
 #pragma unroll
             for (int e = 0; e < 4; ++e) w[l][e] = a.w[l * a.C + c + e];
-        LagMasks mk;
-        mk.fetch(a, b, tw, W, lane, mv[wv]);
+        Masks mk;
+        mk.fetch(a, b, tw, lane, mv[wv]);
         bf16_t *dz = a.dz + (b * a.T + tg) * a.zs + c;
-        if (mk.plain) in_bwd_rows<W, VEC, true>(a, xq, uq, w, mk, grp, l2, tw, tg, dz, dw);
-        else in_bwd_rows<W, VEC, false>(a, xq, uq, w, mk, grp, l2, tw, tg, dz, dw);
+        if (mk.plain) in_bwd_rows<W, VEC, R, true>(a, xq, uq, w, mk, grp, l2, tw, tg, dz, dw);
+        else in_bwd_rows<W, VEC, R, false>(a, xq, uq, w, mk, grp, l2, tw, tg, dz, dw);
     }
 #pragma unroll
     for (int l = 0; l < W; ++l)
         st_f4(&dwr[4 * wv + grp][l][4 * l16], make_float4(dw[l][0], dw[l][1], dw[l][2], dw[l][3]));
     __syncthreads();
     float *part = a.wpart + (int64_t)blockIdx.x * W * a.C + blockIdx.y * 64;
-    for (int i = threadIdx.x; i < W * 64; i += 64 * kInWaves) {
+    for (int i = threadIdx.x; i < W * 64; i += 64 * R::waves) {
         const int l = i >> 6, k = i & 63;
         float t = dwr[0][l][k];
-        for (int q = 1; q < 4 * kInWaves; ++q) t += dwr[q][l][k];
+        for (int q = 1; q < 4 * R::waves; ++q) t += dwr[q][l][k];
         part[l * a.C + k] = t;
     }
 }
@@ -824,34 +842,40 @@ InArgs in_args(const gdn2_lm_mixer_shape *s, const void *z, const float *conv_w,
     return a;
 }
 
-template <template <int, bool> class K, bool VEC>
-void launch_taps(int W, dim3 grid, hipStream_t st, const InArgs &a) {
-    const dim3 block(64 * kInWaves);
+template <template <int, bool, class> class K, bool VEC, class R>
+void launch_taps(int W, hipStream_t st, const InArgs &a) {
+    const dim3 grid((unsigned)(a.B * in_segments(a.T, R::seg)), (unsigned)(a.C / 64 + 1)), block(64 * R::waves);
     switch (W) {
-        case 1: hipLaunchKernelGGL((K<1, VEC>::fn), grid, block, 0, st, a); break;
-        case 2: hipLaunchKernelGGL((K<2, VEC>::fn), grid, block, 0, st, a); break;
-        case 3: hipLaunchKernelGGL((K<3, VEC>::fn), grid, block, 0, st, a); break;
-        case 4: hipLaunchKernelGGL((K<4, VEC>::fn), grid, block, 0, st, a); break;
-        case 5: hipLaunchKernelGGL((K<5, VEC>::fn), grid, block, 0, st, a); break;
-        case 6: hipLaunchKernelGGL((K<6, VEC>::fn), grid, block, 0, st, a); break;
-        case 7: hipLaunchKernelGGL((K<7, VEC>::fn), grid, block, 0, st, a); break;
-        default: hipLaunchKernelGGL((K<8, VEC>::fn), grid, block, 0, st, a); break;
+        case 1: hipLaunchKernelGGL((K<1, VEC, R>::fn), grid, block, 0, st, a); break;
+        case 2: hipLaunchKernelGGL((K<2, VEC, R>::fn), grid, block, 0, st, a); break;
+        case 3: hipLaunchKernelGGL((K<3, VEC, R>::fn), grid, block, 0, st, a); break;
+        case 4: hipLaunchKernelGGL((K<4, VEC, R>::fn), grid, block, 0, st, a); break;
+        case 5: hipLaunchKernelGGL((K<5, VEC, R>::fn), grid, block, 0, st, a); break;
+        case 6: hipLaunchKernelGGL((K<6, VEC, R>::fn), grid, block, 0, st, a); break;
+        case 7: hipLaunchKernelGGL((K<7, VEC, R>::fn), grid, block, 0, st, a); break;
+        default: hipLaunchKernelGGL((K<8, VEC, R>::fn), grid, block, 0, st, a); break;
     }
 }
-template <int W, bool VEC> struct InFwd { static constexpr auto fn = lm_in_fwd_kernel<W, VEC>; };
-template <int W, bool VEC> struct InBwd { static constexpr auto fn = lm_in_bwd_kernel<W, VEC>; };
+template <int W, bool VEC, class R> struct InFwd { static constexpr auto fn = lm_in_fwd_kernel<W, VEC, R>; };
+template <int W, bool VEC, class R> struct InBwd { static constexpr auto fn = lm_in_bwd_kernel<W, VEC, R>; };
 
 // 8-byte accesses where every bf16 base allows them (the strides always do);
 // bases at odd elements take the same kernel with 2-byte accesses.
-template <template <int, bool> class K>
-void launch_in(int W, bool vec, dim3 grid, hipStream_t st, const InArgs &a) {
-    if (vec) launch_taps<K, true>(W, grid, st, a);
-    else launch_taps<K, false>(W, grid, st, a);
+template <template <int, bool, class> class K, class R>
+void launch_in(int W, bool vec, hipStream_t st, const InArgs &a) {
+    if (vec) launch_taps<K, true, R>(W, st, a);
+    else launch_taps<K, false, R>(W, st, a);
 }
 
-dim3 in_grid(const InArgs &a) {
-    return dim3((unsigned)(a.B * in_segments(a.T)), (unsigned)(a.C / 64 + 1));
+// The VJP in short segments (one wave, four rows a group): where the wide ones would
+// leave most of a segment's waves without rows, or the chip without waves.  Wide and
+// short, 4 taps, H = 8, in us: T = 16 x 64 22 and 16, 33 x 256 59 and 42, 100 x 4 12.7
+// and 11.6, 100 x 8 13.2 and 13.6, 512 x 1 13.8 and 11.8, 512 x 16 34 and 36 (one lane
+// per channel took 21, 101, 13.9, 16.1, 14.9 and 62).
+bool in_short(int64_t B, int64_t T, int64_t C) {
+    return T <= 64 || B * in_segments(T, InWide::seg) * (C / 64) < 160;
 }
+int in_bwd_seg(int64_t B, int64_t T, int64_t C) { return in_short(B, T, C) ? InShort::seg : InWide::seg; }
 
 // Row widths of the norm kernels: 4 G NV with G = 64 (multiples of 256 up to
 // 1024) or G = 32 (width 128).
@@ -974,15 +998,15 @@ int gdn2_lm_mixer_in_forward(const gdn2_lm_mixer_shape *shape, const void *z, co
     a.qkv = static_cast<bf16_t *>(qkv);
     a.beta = beta;
     a.g = g;
-    launch_in<InFwd>((int)shape->taps, al(z, 8) && al(qkv, 8), in_grid(a), (hipStream_t)stream, a);
+    launch_in<InFwd, InWide>((int)shape->taps, al(z, 8) && al(qkv, 8), (hipStream_t)stream, a);
     return launch_status(hipGetLastError(), "gdn2_lm_mixer_in_forward");
 }
 
 size_t gdn2_lm_mixer_in_workspace_bytes(const gdn2_lm_mixer_shape *shape) {
     if (!shape || shape->batch < 1 || shape->time < 1 || shape->heads < 1 || shape->taps < 1)
         return 0;
-    const int64_t segs = shape->batch * in_segments(shape->time);
     const int64_t C = 3 * shape->heads * 64;
+    const int64_t segs = shape->batch * in_segments(shape->time, in_bwd_seg(shape->batch, shape->time, C));
     return (size_t)segs * (shape->taps * C + 2 * shape->heads) * sizeof(float);
 }
 
@@ -1006,12 +1030,13 @@ int gdn2_lm_mixer_in_backward(const gdn2_lm_mixer_shape *shape, const void *z,
     a.dbeta = dbeta;
     a.dg = dg;
     a.dz = static_cast<bf16_t *>(dz);
-    const int64_t segs = a.B * in_segments(a.T);
+    const int64_t segs = a.B * in_segments(a.T, in_bwd_seg(a.B, a.T, a.C));
     a.wpart = static_cast<float *>(workspace);
     a.gpart = a.wpart + segs * shape->taps * a.C;
     hipStream_t st = (hipStream_t)stream;
-    launch_in<InBwd>((int)shape->taps, al(z, 8) && al(dz, 8) && al(dq, 8) && al(dk, 8) && al(dv, 8),
-                     in_grid(a), st, a);
+    const bool vec = al(z, 8) && al(dz, 8) && al(dq, 8) && al(dk, 8) && al(dv, 8);
+    if (in_short(a.B, a.T, a.C)) launch_in<InBwd, InShort>((int)shape->taps, vec, st, a);
+    else launch_in<InBwd, InWide>((int)shape->taps, vec, st, a);
     colsum(a.wpart, shape->taps * a.C, segs, dconv_w, st);
     hipLaunchKernelGGL(lm_gate_sum_kernel, dim3(1), dim3(64 * kSumWaves), 0, st, a.gpart, a.H,
                        segs, decay_scale, ddecay_bias, ddecay_scale);

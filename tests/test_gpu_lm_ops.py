@@ -246,6 +246,40 @@ def test_mixer_in_segments(T, taps, masked, odd):
         _normwise(name, got, ref, tol)
 
 
+@pytest.mark.parametrize("T,taps,masked,odd", [
+    (65, 4, True, False), (73, 1, False, True), (97, 3, True, False), (127, 8, True, False),
+    (128, 4, False, False), (129, 4, True, True), (131, 8, False, True), (260, 2, True, False)])
+def test_mixer_in_wide_segments(T, taps, masked, odd):
+    """The same with enough sequences that the VJP takes its wide segments (test_mixer_in_segments'
+    few take the short ones: groups of 4 rows, one wave): edges of 8, 32 and 128 rows."""
+    lm = _lm()
+    B, H = 32, 2
+    gen = _gen(T * 10 + taps)
+    z = (torch.randn(B * T, _zstride(H), generator=gen) * 1.5).to(BF)
+    conv_w = torch.rand(taps, 3 * H * 64, generator=gen) - 0.5
+    valid, docs = _masks(B, T, gen) if masked else (torch.ones(B, T), torch.full((B, T), 3.0))
+    ds, db = torch.rand(H, generator=gen) - 0.5, torch.rand(H, generator=gen) * 4 - 3
+    up = [torch.randn(B, T, H, 64, generator=gen).to(BF) for _ in range(3)]
+    dbeta, dg = (torch.randn(B, T, H, generator=gen) for _ in range(2))
+    put = _odd if odd else (lambda t: t.cuda())
+    args = [put(z)] + [t.cuda() for t in (conv_w, valid, docs, ds, db)]
+    qkv, beta, g = lm.mixer_in_forward(*args, B, T, H)
+    dz = put(torch.zeros_like(z))
+    dconv, dds, ddb = lm.mixer_in_backward(*args, *[put(t) for t in up], dbeta.cuda(), dg.cuda(),
+                                           dz, B, T, H)
+    zd, cwd, dsd, dbd = (t.double().requires_grad_(True) for t in (z, conv_w, ds, db))
+    rq, rb, rg = _in_ref(zd, cwd, valid, docs, dsd, dbd, B, T, H)
+    ((rq * torch.cat(up, 2).double()).sum() + (rb * dbeta.double()).sum()
+     + (rg * dg.double()).sum()).backward()
+    _bf16_close("qkv", qkv, rq.detach())
+    _bf16_close("dz", dz, zd.grad, slack=1e-5)
+    for name, got, ref, tol in (("beta", beta, rb.detach(), 1e-6), ("g", g, rg.detach(), 1e-6),
+                                ("dconv", dconv, cwd.grad, 1e-5),
+                                ("ddecay_scale", dds, dsd.grad, 1e-5),
+                                ("ddecay_bias", ddb, dbd.grad, 1e-5)):
+        _normwise(name, got, ref, tol)
+
+
 @pytest.mark.parametrize("B,T,H", [(2, 131, 2), (3, 33, 8), (1, 1, 1)])
 def test_mixer_out_forward_backward(B, T, H):
     lm = _lm()
