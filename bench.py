@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """GDN scan forward+backward throughput on one MI355X.
 
-Workload: BASELINE configs[1] ("lm512" scan shape): B=16, T=512, H=8,
+Workload: the "lm512" scan shape: B=16, T=512, H=8,
 d_k=d_v=64, chunk 64, bf16 q/k/v/dO with f32 gates and state, scalar gates
 beta and g generated by SplitMix64 seed 0 (delta_mixers.synthetic).
 A step is one forward plus one backward of the scan over the whole batch
@@ -186,7 +186,7 @@ def main():
                     help="the document-limit op gdn2_scan (channel-wise gates, packed "
                          "documents) fwd+bwd at the lm512 head shape")
     ap.add_argument("--decode", action="store_true",
-                    help="BASELINE configs[3]: decode steps (one token per sequence) on 256 x 8 "
+                    help="decode steps (one token per sequence) on 256 x 8 "
                          "carried fp32 states, d_k = d_v = 64")
     ap.add_argument("--ref-shape", action="store_true",
                     help="the reference's isolated-scan benchmark (kron_benchmark.rs:73-116): "
@@ -443,7 +443,7 @@ def train_flops_per_token(cfg, T):
 
 
 def bench_train(args):
-    """one AdamW training step of the 8-block lm512 GDN
+    """One AdamW training step of the 8-block lm512 GDN
     model (random-init weights, uniform random token ids) over B=16 x T=512."""
     import torch
 
@@ -944,9 +944,9 @@ def mfma_from_counters(pmc_dir, out_path):
 
 
 def bench_decode(args):
-    """BASELINE configs[3]: B=256 sequences x H=8 heads, d_k = d_v = 64 fp32
+    """B=256 sequences x H=8 heads, d_k = d_v = 64 fp32
     states drawn N(0, 0.02); one token per sequence per step (q, k, v, beta, g
-    from the configs[0] generator), gdn2_decode_step on the carried state.  A
+    from the generator of delta_mixers.synthetic), gdn2_decode_step on the carried state.  A
     step reads and writes every state once: compulsory bytes
     2 B H K V 4 + token I/O, HBM-bound."""
     import numpy as np

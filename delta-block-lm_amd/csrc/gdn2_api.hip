@@ -247,7 +247,7 @@ static size_t training_workspace_bytes(const gdn2_shape *s) {
     return fc_workspace_bytes(s->batch, s->time, s->heads, (int)s->keys, (int)s->values);
 }
 
-// The f32 chunk path's argument block over the token-sequential one.
+// The f32 chunk path's argument block over the token walk's.
 static FcArgs fc_args(const SeqArgs &s, const gdn2_view *q, bool rows64, void *checkpoint, void *workspace) {
     FcArgs f{};
     f.s = s;

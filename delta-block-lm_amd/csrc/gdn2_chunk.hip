@@ -15,17 +15,18 @@
 // nilpotent series replaced by a blocked substitution inverse (C > 16).
 //
 // Forward = three launches:
-//   prep  (one workgroup per chunk): gates, A, T -> checkpoint (T bf16, gates)
-//   state (one workgroup per (batch, head), chunks in order): the only
-//         sequential part; fp32 S lives in MFMA accumulators, next chunk's
-//         K/V/T/gates are prefetched into registers; writes S at each chunk start
+//   prep  (one workgroup per chunk): gates, A, T and the dense state map ->
+//         checkpoint (T bf16, gates, the map as hi/lo pairs and f32)
+//   scan  (two workgroups per (batch, head), chunks in order): the only
+//         sequential part; fp32 S lives in MFMA accumulators, the maps stream
+//         through an LDS ring; writes S at each chunk start
 //   out   (one workgroup per chunk): delta from the chunk-start state, O, scores
 // Workgroups are 8 waves; wave w owns output tiles (w/2, 2(w%2)) and
 // (w/2, 2(w%2)+1) of every 64x64 product.  All GEMMs are
 // v_mfma_f32_16x16x32_bf16 on LDS tiles; the inverse is fp32 (diagonal 16x16
 // blocks by forward substitution, off-diagonal blocks by a 2x2 recursion on
-// v_mfma_f32_16x16x4_f32).  R, delta and P enter the GEMMs that consume them
-// as two-term bf16 splits (hi + lo); S0, T, Q, K, V as single bf16 terms.
+// v_mfma_f32_16x16x4_f32).  R, delta and P and S0 enter the GEMMs that consume
+// them as two-term bf16 splits (hi + lo); T, Q, K, V as single bf16 terms.
 #include "gdn2_chunk_tile.h"
 
 #include <algorithm>

@@ -467,6 +467,7 @@ __global__ void __launch_bounds__(512) fc_out_kernel(FcArgs a) {
 // and dalpha from the adjoints of every F and G (b and lam, whose adjoints are
 // eh.Ag + q.Qg [+ rowsum(S0 . dS) at token 15] and k.Kg, are the last level's).
 // Wave w takes value tile w up to dR, then key tile w; blockDim is 64 max(KT, VT).
+// Four waves a SIMD leave 128 registers, of which 1 spills (4 in the f32 element form).
 template <int KM, bool BF, bool VEC>
 __global__ void __launch_bounds__(64 * KM, KM == 8 ? 2 : 4) fc_bgrad_kernel(FcArgs a) {
     __shared__ FcGradSmem<KM> sm;

@@ -18,10 +18,10 @@
 // launched behind them, walk the marked ones again (the rest return at once): such
 // a sequence gets what the recurrence gives, token by token.
 //
-// At B8 T512 H8 K = V = 64 in f32, forward + backward takes 121 us of kernels
-// (prep 17, scans 20 and 29, out 11, bgrad 43) against 885 us of the
-// token-sequential kernels, which walk a head's tokens in one workgroup
-// (forward 226, backward 658); the floor of its 69 MB is 14 us.
+// At B8 T512 H8 K = V = 64 in f32, forward + backward takes 126 us of kernels
+// (prep 18, scans 20 and 29, out 11, bgrad 44, the two launches for marked heads
+// 2 each) against 885 us of the token-sequential kernels, which walk a head's tokens
+// in one workgroup (forward 226, backward 658); the floor of its 69 MB is 14 us.
 #include "gdn2_chunk_f32_dev.h"
 
 #include <algorithm>

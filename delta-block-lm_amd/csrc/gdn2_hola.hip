@@ -9,9 +9,9 @@
 // query/key VJPs) and the scalar oracle of crates/mixers/src/hola_checks.rs.
 //
 // Layout and work split:
-//   * schedule: one wave per (batch, head), chunks in order; each candidate's
-//     rank is the number of eligible candidates that beat it (exact top-k with
-//     no sort); it writes the cache positions before/after every chunk and the
+//   * schedule: two waves per (batch, head), chunks in order; one ranks a chunk's
+//     eligible tokens, one chunk ahead, the other keeps the cache sorted and merges
+//     them into it; it writes the cache positions before/after every chunk and the
 //     end of each key's visibility ("expiry");
 //   * read, query VJP: one wave per (batch, head, chunk); the rows of the chunk's
 //     slots (cache positions from the schedule + the chunk's own tokens) go from
@@ -500,7 +500,8 @@ __device__ __forceinline__ void visible_logits(const HolaArgs &a, const SlotInfo
 // a chunk at 64 slots + 16 and widths of 64, out of the caches) and its latency.
 // B16 T512 H8, widths of 64: 31 us, against 86 with the tiles in LDS (four waves a
 // chunk) and VALU products; the rows and results alone are 14 us at copy rate.  Four
-// waves a SIMD hold all 4096 chunks at once (three: 33 us).
+// waves a SIMD hold all 4096 chunks at once (three: 33 us); they cost 1 to 12 spilled
+// registers where keys or values are 64 wide (10 at 64 x 64), which is in the 31 us.
 template <int DK, int DV, bool VEC>
 __global__ void __launch_bounds__(64, DK + DV > 128 ? 2 : 4) hola_forward_kernel(HolaArgs a) {
     __shared__ SlotInfo s;
@@ -553,7 +554,9 @@ __global__ void __launch_bounds__(64, DK + DV > 128 ? 2 : 4) hola_forward_kernel
 // One wave per (batch, head, chunk); bound as the read, plus the pairs that it
 // leaves for the key VJP (8 bytes a query and slot).
 // B16 T512 H8, widths of 64: 53 us, against 127 with the tiles in LDS; rows, pairs and
-// results are 29 us at copy rate.  Three waves a SIMD: four would spill.
+// results are 29 us at copy rate.  Three waves a SIMD: four would spill.  The element
+// form spills 34 to 93 registers where keys or values are 128 wide: B16 T512 H8 128 x
+// 127, the whole call, takes 778 us, against 1466 with the tiles in LDS.
 template <int DK, int DV, bool VEC>
 __global__ void __launch_bounds__(64, DK + DV > 128 ? 2 : 3) hola_query_backward_kernel(HolaArgs a) {
     __shared__ SlotInfo s;

@@ -1,12 +1,12 @@
-"""The lm512 GDN language model and its training step (BASELINE configuration 4).
+"""The lm512 GDN language model and its training step.
 
 Each of the `layers` blocks is pre-norm residual
     x += mixer(rms_norm(x));  x += swiglu(rms_norm(x))
 followed by a final RMSNorm and the tied embedding as output head, with AdamW
 (block structure: crates/experiment/src/model.rs:300-364; train step:
-crates/experiment/src/train.rs:335-357; optimizer: update.rs:43-96).  Widths
-follow configuration 4, which is not the reference's own lm512 (d_model 512,
-8 layers, H8 K64 V64, SwiGLU 1408, vocab 32768, tied head).  The mixer is the scalar-gate gated delta rule:
+crates/experiment/src/train.rs:335-357; optimizer: update.rs:43-96).  The
+widths are not the reference's own lm512's: d_model 512, 8 layers, H8 K64 V64,
+SwiGLU 1408, vocab 32768, tied head.  The mixer is the scalar-gate gated delta rule:
     q = l2(silu(conv(x Wq)))   k = l2(silu(conv(x Wk)))   v = silu(conv(x Wv))
     beta = sigmoid(x Wb)       g = -exp(decay_scale) * softplus(x Wg + decay_bias)
     o = scan(q, k, v, beta, g)                       chunk-WY HIP kernels

@@ -83,20 +83,22 @@ GDN2_API const char *gdn2_last_error(void);
  * packed + B*T*H*V, scores = packed + B*T*H*V + B*H*K*V with an f32 output
  * reproduces that packing exactly.  The reference's private `checkpoint` and
  * `auxiliary` tensors are replaced by one opaque checkpoint buffer written by
- * the forward and read by the backward.
+ * the forward and read by the backward.  Here and below a checkpoint belongs to
+ * the build of the library that wrote it: its layout is no part of the ABI and
+ * changes without a change of gdn2_abi_version, so none is stored across builds.
  *
  * q, k, v: F32 or BF16 (same dtype); alpha, erase, write, valid, reset,
  * initial: F32.  initial.data may be NULL (zero state).  chunk: 1..64, the
  * checkpoint interval of the reference (1..16, gdn_training.rs:370-373; up to
- * 64 accepted here); results do not depend on it.  bf16 q/k/v with keys =
- * values = 64, unit channel stride and 16-byte aligned token rows run the
- * 16-token chunk-WY MFMA kernels; every other shape (keys, values <= 128, f32
- * or bf16, any strides) runs the 16-token f32 chunk kernels, which read bf16
- * inputs as their exact f32 values.  The bf16 MFMA kernels need alpha >= 0 on
- * valid tokens: a negative alpha gives NaN outputs, state and gradients for
- * its sequence (the f32 chunk kernels accept any alpha).  alpha = 0 and tiny
- * alphas get their exact gradient on both.  On the MFMA kernels d_output must
- * have aligned rows too.  checkpoint (and the backward's workspace) must be
+ * 64 accepted here); results do not depend on it.  Every call (keys, values <=
+ * 128, f32 or bf16, any strides) runs the 16-token f32 chunk kernels, which read
+ * bf16 inputs as their exact f32 values and take any alpha; alpha = 0 and tiny
+ * alphas get their exact gradient.  One form of call keeps two restrictions that
+ * the kernels themselves do not have, so that callers see what they always saw:
+ * with bf16 q/k/v, keys = values = 64, unit channel stride and 16-byte aligned
+ * token rows, a negative alpha on a valid token gives NaN outputs, state and
+ * gradients for its sequence, and d_output must have aligned rows too
+ * (GDN2_ERR_ARGUMENT).  checkpoint (and the backward's workspace) must be
  * 16-byte aligned. */
 GDN2_API size_t gdn2_training_checkpoint_bytes(const gdn2_shape *shape, int chunk);
 
@@ -143,11 +145,10 @@ GDN2_API int gdn2_training_backward(const gdn2_shape *shape, int chunk, const gd
  * limits every packed batch carries) and differ only for limits where a reset
  * has no preceding end or an end no following reset.  Zero initial state; no
  * final state or score outputs.  q, k, v: F32 or BF16 (same dtype); alpha,
- * erase, write: F32.  bf16 q/k/v with keys = values = 64 and 16-byte aligned
- * rows run the 16-token chunk-WY MFMA kernels, every other shape (keys, values
- * <= 128) the 16-token f32 chunk kernels.  The MFMA kernels need alpha >= 0 on
- * live tokens (a negative alpha gives NaN results for its sequence); the f32
- * chunk kernels accept any alpha.  The checkpoint (opaque, 16-byte aligned, as
+ * erase, write: F32.  Every call (keys, values <= 128) runs the
+ * 16-token f32 chunk kernels, with the training scan's two restrictions on bf16
+ * calls of keys = values = 64 with aligned rows: a negative alpha on a live token
+ * gives NaN results for its sequence, and d_output needs aligned rows.  The checkpoint (opaque, 16-byte aligned, as
  * is the backward's workspace) replaces the reference's [B, H, T/16, 48, 64]
  * checkpoint tensor. */
 GDN2_API size_t gdn2_scan_checkpoint_bytes(const gdn2_shape *shape);
@@ -175,11 +176,15 @@ GDN2_API int gdn2_backward(const gdn2_shape *shape, const gdn2_view *q, const gd
  * erase[i] = write[j] = beta for every channel.  beta and g are [B,T,H] F32
  * (g is the log decay, finite).  No counterpart entry exists in the reference
  * (it reaches this case only through the channel-wise op with broadcast
- * gates); this is the chunk-WY fast path the north-star benchmark measures.
+ * gates).
  * The chunk-WY MFMA kernels run when chunk == 64, d_k == d_v (64 or 128) and
  * q, k, v are BF16 with unit channel stride, 16-byte aligned data and every
- * other stride a multiple of 8 elements; any other call takes the
- * token-sequential kernels.  On the chunk-WY path d_output must satisfy the
+ * other stride a multiple of 8 elements.  Any other call runs the 16-token f32
+ * chunk kernels from 17 tokens on and the token-sequential kernels up to 16.  A
+ * NaN or an infinity reaches the tokens that the recurrence takes it to: a chunk's
+ * products spread it over 16 tokens, so the sequences whose results are not finite
+ * are walked again token by token.  (On the chunk-WY path it may reach all 64 tokens of
+ * its chunk.)  On the chunk-WY path d_output must satisfy the
  * same row rule (a stride-0 broadcast upstream is rejected with
  * GDN2_ERR_ARGUMENT: pass a dense copy). */
 GDN2_API size_t gdn_scalar_checkpoint_bytes(const gdn2_shape *shape, int chunk);
@@ -232,8 +237,8 @@ GDN2_API int gdn_scalar_backward(const gdn2_shape *shape, int chunk, const gdn2_
  * harnesses that forbid hipMalloc).  No counterpart in the reference.  It
  * calls no allocating routine: its scratch is a fixed device array of
  * GDN2_NOALLOC_SCRATCH_BYTES inside the library (one per device, held until
- * the process ends), and a shape whose gdn_scalar_workspace_bytes exceeds
- * that size is rejected with GDN2_ERR_WORKSPACE.  Every call on a device
+ * the process ends), and a shape whose gdn_scalar_workspace_bytes, less a word
+ * per batch and head, exceeds that size is rejected with GDN2_ERR_WORKSPACE.  Every call on a device
  * shares that device's array, so calls that overlap in time on one device
  * (other streams, other threads) race; calls in order on one stream do not.
  * Arguments and results are those of gdn_scalar_backward. */

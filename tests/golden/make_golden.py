@@ -5,7 +5,7 @@ f64 oracle's answers (oracle/gdn2_oracle.c, a restatement of
 crates/mixers/src/reference.rs:41-257) on the inputs below, stored with the
 inputs so that the GPU tests and later builds check against fixed numbers:
 
-  cfg0.npz           BASELINE configs[0]: B1 H2 T256 K=V=32 fp32, SplitMix64
+  cfg0.npz           B1 H2 T256 K=V=32 fp32, SplitMix64
                      seed 0 (delta_mixers.synthetic), scalar gates; forward
                      outputs plus the VJP for an upstream drawn from seed 1.
   reset_padding.npz  crates/mixers/src/chunk_tests.rs:25-75 (B2 T5 H2 K3 V4),

@@ -4,7 +4,7 @@ f64 sequential oracle: the reference's own fixtures (masks, resets on and off
 padding, zero alpha on one and on all channels, exactly zero edits, zero key
 and value norms, a nonzero initial state) and random bf16-style inputs, at
 chunk sizes 1, 5, 16 and 64 (the solver's result must not depend on the
-chunk).  Gate: the north-star f32 tolerance, rms-floored."""
+chunk).  Gate: the f32 tolerance (1e-4), rms-floored."""
 import numpy as np
 import pytest
 

@@ -1,7 +1,7 @@
 """The committed golden vectors (tests/golden/) against the generators that
 made their inputs and the f64 oracle that made their outputs.
 
-Inputs must regenerate bit-exactly (SplitMix64 seed 0 for BASELINE configs[0];
+Inputs must regenerate bit-exactly (SplitMix64 seed 0 for cfg0;
 the fixture restatements of crates/mixers/src/chunk_tests.rs:25-75 and
 kron_checks.rs:124-188), and the oracle must reproduce every stored output to
 float32 rounding.  A change of generator or oracle that moves any of them fails

@@ -1,12 +1,12 @@
-"""Parity at BASELINE.json's full sizes (configs 1-3; config 0 is the golden
-vector set of tests/test_gpu_golden.py).
+"""Parity at the full sizes of the benchmark's workloads (scalar scans at d = 64 and
+128, decode; the small f32 one is the golden vector set of tests/test_gpu_golden.py).
 
 Every (batch, head) sequence of the scan is an independent recurrence, so the
 full-size GPU result is checked against the f64 oracle on whole sequences cut
 out of the batch (oracle slices), and through size-independent properties:
 split continuation (scanning [0, T/2) then [T/2, T) from the carried state
 equals one scan) and, for the decode configuration, step-by-step equality with
-the scan.  Inputs come from the BASELINE generator (SplitMix64 seed 0).
+the scan.  Inputs come from the benchmark's generator (SplitMix64 seed 0).
 """
 import numpy as np
 import pytest

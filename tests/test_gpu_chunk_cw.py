@@ -1,11 +1,10 @@
-"""GPU parity of the channel-wise chunk-WY MFMA path (the training op
-gdn_training_scan with bf16 q/k/v and d_k = d_v = 64; csrc/gdn2_chunk_cw.hip)
+"""GPU parity of the channel-wise training op (gdn_training_scan, the f32 chunk
+kernels of csrc/gdn2_chunk_f32.hip) with bf16 q/k/v and d_k = d_v = 64
 against the f64 oracle: per-channel gates, masks, resets (on valid and on
 padded tokens, at chunk starts), an initial state, every adjoint (output,
 final state, scores), ragged lengths, several heads, sequences past 16 chunks
 (the scan's rolled loop), broadcast gate views and strong decays.  The stage
-timers show that the chunk kernels, not the token-sequential kernels,
-produced each result."""
+timers show that the channel-wise chunk kernels produced each result."""
 import numpy as np
 import pytest
 
@@ -164,10 +163,10 @@ def test_cw_alpha_zero_exact_gradient(dk):
 
 
 def test_cw_negative_alpha_fails_loudly(dk):
-    """A negative alpha is outside the chunk kernels' log-domain decays: the
-    sequence that holds it gets NaN outputs (never finite wrong values), the
-    other sequences are untouched, and the f32 chunk kernels give the oracle's
-    values for the same inputs."""
+    """A negative alpha in a bf16 call of this shape gives its sequence NaN outputs
+    (kept from when this shape had kernels with log-domain decays), the other
+    sequences are untouched, and with f32 inputs the same gates give the oracle's
+    values."""
     p = cw_problem(83, 2, 40, 1, masks=False)
     p["alpha"][1, 12, 0, 5] = -0.5
     x, init = _inputs(p, grad=False)

@@ -12,9 +12,8 @@ q/k/v and d_k, d_v <= 128, in 16-token chunks, against the f64 oracle.
    p = 16, so the exact alpha gradient at alpha = 0 is gated too.
 3. Gates the chunk kernels handle with no special case, because they form every
    decay as a product of the gates: negative alpha, alpha = 0 on a whole
-   chunk, tiny alpha; and ragged widths (d_k, d_v in 1..128: the kernels built
-   for 64-wide tiles up to 64, for 128-wide tiles above, where bgrad walks the
-   value axis in two blocks) with padding and resets inside chunks and sequence
+   chunk, tiny alpha; and ragged widths (d_k, d_v in 1..128, padded to tiles of
+   16, read element by element where they are not whole tiles) with padding and resets inside chunks and sequence
    ends off the chunk grid.
 4. Slow decay over 256 chunks (T = 4096) at K32/V64, and over 128 chunks
    (T = 2048) at K = V = 128, at both gates.

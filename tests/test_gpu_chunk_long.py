@@ -4,10 +4,10 @@ against the f64 oracle, and through the split-continuation property.
 T = 1000, 2048 and 8192 give 16, 32 and 128 chunks per sequence: the state and
 adjoint scans' straight-line instantiation for 16 chunks and the rolled loop
 that every longer sequence takes.  The checkpoint holds the chunk-start state
-and the state maps in bf16, so these sizes also show whether those single
+and the state maps as bf16 hi/lo pairs, so these sizes also show whether those
 roundings stay inside the bf16 gate over 128 chained chunks.  Each test
-asserts through the stage timers that the chunk kernels (not the
-token-sequential fallback) produced the result.
+asserts through the stage timers that the chunk kernels (not the f32 chunk
+kernels, which time their own stages) produced the result.
 """
 import numpy as np
 import pytest

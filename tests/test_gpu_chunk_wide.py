@@ -2,7 +2,8 @@
 chunk 64; csrc/gdn2_chunk_wide.hip) against the f64 oracle, with masks,
 resets, an initial state and every adjoint (output, final state, scores), on
 ragged lengths and several heads.  The stage timers show that the chunk
-kernels, not the token-sequential fallback, produced each result."""
+kernels, not the f32 chunk kernels (which time their own stages), produced each
+result."""
 import pytest
 
 torch = pytest.importorskip("torch")

@@ -1,8 +1,8 @@
 """GPU parity against the committed golden vectors (tests/golden/*.npz).
 
-cfg0 (BASELINE configs[0]: B1 H2 T256 K=V=32 fp32, chunk 32) runs the
+cfg0 (B1 H2 T256 K=V=32 fp32, chunk 32) runs the
 scalar-gate op forward and backward; the reference fixtures run the
-channel-wise training op.  Gates: the north-star rms-floored 1e-4 for fp32
+channel-wise training op.  Gates: rms-floored 1e-4 for fp32
 and the reference's own 2e-5 + 3e-4|ref| (crates/mixers/src/checks.rs:73-74);
 padding entries must be exactly zero.
 """

@@ -8,7 +8,7 @@ and adjoints; and the cancellation check (hola_checks.rs:466-512, analytic VJP
 of the observed forward probability).  Outputs and gradients (q, k, v, sink) at
 the reference's gate 2e-5 + 3e-4|ref| (checks.rs:73-74); final cache
 positions and the positions-only schedule exactly.  Wider heads (K = V = 64,
-128) against the oracle at the north-star fp32 gate.
+128) against the oracle at the fp32 gate (1e-4).
 """
 import numpy as np
 import pytest

@@ -6,8 +6,8 @@ masked lags, the norms from their formulas, and the scalar-gate recurrence of
 crates/mixers/src/reference.rs:68-111 (alpha = exp(g) on every key channel,
 erase = write = beta) as a differentiable token loop.
 
-float32 model (token-sequential scan, float32 GEMMs) against the exact
-float64 composition: the loss within the north-star fp32 gate (1e-4); each
+float32 model (the scalar-gate f32 kernels, float32 GEMMs) against the exact
+float64 composition: the loss within the fp32 gate (1e-4); each
 parameter gradient within 1e-4 normwise and 5e-4 elementwise (rms-floored).
 The model composes two scans, each within 1e-4 of its oracle, and ~30 other
 f32 operators; measured on two initialisations: worst normwise 2.2e-5,

@@ -1,4 +1,4 @@
-"""BASELINE configs[4] at its full workload: the 8-block lm512 language model
+"""The language-model training step at its full workload: the 8-block lm512 model
 (d_model 512, H8, K = V = 64, conv taps 4, SwiGLU width 1408, tied vocab
 32768, B16 T512) on the fused bf16 step operators and the chunk-WY scan.
 
@@ -9,8 +9,8 @@ tests/test_gpu_lm.py pin the semantics at a reduced shape):
     variance of its logits (the tied head's logits are O(0.5) here);
   * every parameter gradient is finite and nonzero;
   * the fused bf16 model, the unfused bf16 composition of the
-    reference-mirrored operators and the float32 model (token-sequential
-    scan, f32 GEMMs; within 1e-4 of exact float64 at the reduced shape) agree
+    reference-mirrored operators and the float32 model (f32 chunk
+    kernels, f32 GEMMs; within 1e-4 of exact float64 at the reduced shape) agree
     on the loss, and per parameter the fused gradient is at most 1.5 x as far
     from the float32 one as the unfused bf16 gradient is (bf16 rounding alone
     moves these gradients 2-10 % at the reduced shape, more for the per-head
@@ -81,7 +81,7 @@ def test_full_shape_loss_and_gradients(full):
     assert abs(loss.item() - lp.item()) <= 2e-3 * abs(lp.item()), (loss.item(), lp.item())
     plain_grads = {n: t.grad.float().clone() for n, t in plain.named_parameters()}
     del plain
-    # float32 model (token-sequential scan, f32 GEMMs): within 1e-4 of exact
+    # float32 model (f32 chunk kernels, f32 GEMMs): within 1e-4 of exact
     # float64 at the reduced shape, the stand-in for exact gradients here.
     exact = GdnLM(replace(cfg, fused=False, compute_dtype=torch.float32), device="cuda")
     exact.load_state_dict(model.state_dict())

@@ -4,7 +4,7 @@ float64 CPU composition of the same block from plain torch operations
 the norms and decay from their formulas, and the recurrence of
 crates/mixers/src/reference.rs:41-119 as a differentiable token loop.
 Output, input gradient and every parameter gradient are compared with the
-north-star fp32 gate (1e-4, rms-floored).
+fp32 gate (1e-4, rms-floored).
 """
 import numpy as np
 import pytest

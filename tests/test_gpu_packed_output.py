@@ -5,9 +5,8 @@ GdnTrainingOps returns one f32 buffer [output ; final_state ; scores]
 that passing output = packed, final_state = packed + B*T*H*V and scores =
 packed + B*T*H*V + B*H*K*V with an f32 output reproduces that packing; this
 test calls gdn2_training_scan both ways and requires the packed buffer's
-three slices to equal the separate buffers bit for bit, on the
-token-sequential kernels (f32, d = 32) and on the chunk kernels (bf16 q/k/v,
-d = 64, f32 output), with the packed tail left untouched."""
+three slices to equal the separate buffers bit for bit, with f32 q/k/v at
+d = 32 and with bf16 q/k/v at d = 64 (f32 output), with the packed tail left untouched."""
 import ctypes
 
 import numpy as np
