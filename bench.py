@@ -622,12 +622,13 @@ def ref_shape_bytes_per_token_head(K, V):
     """Compulsory HBM bytes per token-head of each f32 chunk kernel: the inputs
     it must read and the outputs it must write (4-byte elements), no
     intermediates.  prep reads k, alpha, erase, v, write; out reads q, k,
-    alpha, erase, v, write and writes the output and the score; bprep reads q,
-    k, alpha and dO; bgrad reads q, k, alpha, erase, v, write, dO and writes dq,
-    dk, dalpha, derase, dv, dwrite.  The scans move only chunk states."""
+    alpha, erase, v, write and writes the output and the score; the adjoint scan
+    reads dO and forms its additive term from it (no kernel runs in the bprep
+    stage); bgrad reads q, k, alpha, erase, v, write, dO and writes dq, dk, dalpha,
+    derase, dv, dwrite.  Beyond that the scans move only chunk states."""
     return {"chunk_prep": 4 * (3 * K + 2 * V), "chunk_out": 4 * (4 * K + 3 * V + 1),
-            "chunk_bprep": 4 * (3 * K + V), "chunk_bgrad": 4 * (8 * K + 5 * V),
-            "state_scan": 0.0, "adjoint_scan": 0.0}
+            "chunk_bprep": 0.0, "chunk_bgrad": 4 * (8 * K + 5 * V),
+            "state_scan": 0.0, "adjoint_scan": 4 * V}
 
 
 def bench_ref_shape(args):
